@@ -2414,26 +2414,17 @@ __global__ void k_em2_edges(const DModel* __restrict__ models, const DShot* __re
 // ELASTIC25: seismic25, legacy/fortran/seismicfdtd.f95:388-949
 // Two launches per step: stresses, then velocities.  A wavefront takes one
 // z plane k, 64 adjacent columns (lanes 1..EW25 are owned; lanes 0 and 63
-// only supply x neighbours, which travel by lane shuffles) and a chunk of at
-// most Y25 rows in y, which it walks with its y neighbours kept in registers.
+// only supply x neighbours, which travel by lane shuffles) and a chunk of
+// rows in y (rows25), which it walks with its y neighbours kept in registers.
 // The 2-D (y-invariant) coefficients of its columns are loaded once per
-// chunk; z neighbours are plain loads of the adjacent planes.  A block is
-// XW25 x KB25 wavefronts (columns x planes).  Chunks end at the y-slab edges,
+// chunk; z neighbours are plain loads of the adjacent planes.  A block is one
+// wavefront.  Chunks end at the y-slab edges,
 // and a wavefront clear of every slab runs a body without memory variables.
 // psi slabs (per shot):
 //   x [nz][ny][2lx]: dvx_dx dvy_dx dvz_dx dsxx_dx dsxy_dx dsxz_dx
 //   y [nz][2ly][nx]: dvx_dy dvy_dy dvz_dy dsyy_dy dsxy_dy dsyz_dy
 //   z [2lz][ny][nx]: dvx_dz dvy_dz dvz_dz dszz_dz dsxz_dz dsyz_dz
 // ===========================================================================
-#ifndef SDT_EL25_PLANES
-#define SDT_EL25_PLANES 1
-#endif
-#ifndef SDT_EL25_ROWS
-#define SDT_EL25_ROWS 32
-#endif
-#ifndef SDT_EL25_XW
-#define SDT_EL25_XW 1
-#endif
 // (56, which puts every row of stores on a 32-byte boundary, measured slower
 // here: 1.319 against 1.309 ms per aniso25 step, 0.640 against 0.593 ms per
 // gpr25 step; the lanes lost cost more than the aligned stores gain)
@@ -2442,10 +2433,7 @@ __global__ void k_em2_edges(const DModel* __restrict__ models, const DShot* __re
 #endif
 constexpr int EW25 = SDT_EL25_EW;      // owned columns per wavefront
 static_assert(EW25 >= 1 && EW25 <= 62, "2.5-D wavefront: one halo lane on each side");
-constexpr int KB25 = SDT_EL25_PLANES;  // z planes per block
-constexpr int XW25 = SDT_EL25_XW;      // wavefronts side by side in x per block
-constexpr int NT25 = 64 * KB25 * XW25;
-constexpr int Y25 = SDT_EL25_ROWS;     // y rows per work item
+constexpr int NT25 = 64;               // a block is one wavefront
 
 // The y chunk [j0, j1) of a 2.5-D work item travels in one int as two
 // unsigned 16-bit halves (ny <= 65535 is checked at plan creation); the
@@ -2455,6 +2443,14 @@ __host__ __device__ inline int ychunk_pack(int j0, int j1) {
 }
 __host__ __device__ inline int ychunk_j0(int w) { return (int)((unsigned)w & 0xffffu); }
 __host__ __device__ inline int ychunk_j1(int w) { return (int)((unsigned)w >> 16); }
+
+// The work item of this block in a launch over n consecutive items, -1 for
+// none (the grid is n rounded up to a multiple of 8): each XCD (blockIdx % 8)
+// takes a contiguous run of them.
+__device__ __forceinline__ int item25(int n) {
+  const int run = (int)(gridDim.x >> 3), q = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
+  return q < n ? q : -1;
+}
 
 struct Slab3 {
   long SX, SY, SZ;       // elements per memory-variable array on each axis
@@ -2501,18 +2497,12 @@ __device__ __forceinline__ void el25_stress_tile(const DModel* __restrict__ mode
   const DShot& S = shots[s];
   const DModel& M = models[S.model];
   const int nx = M.nx, ny = M.ny, nz = M.nz;
-  // a wavefront past the last plane stays (clamped, storing nothing) so that
-  // every wavefront of the block takes the same barriers
-  const int wx_ = (int)(threadIdx.x >> 6) % XW25;  // x slot in the block
-  const int wv_ = (int)(threadIdx.x >> 6) / XW25;  // plane slot in the block
-  const int kw = __builtin_amdgcn_readfirstlane(wv.z) + wv_;
-  const bool live = kw < nz;
-  const int k = live ? kw : nz - 1;
+  const int k = __builtin_amdgcn_readfirstlane(wv.z);
   const int lane = threadIdx.x & 63;
-  const int i = __builtin_amdgcn_readfirstlane(wv.y) + wx_ * EW25 - 1 + lane;
+  const int i = __builtin_amdgcn_readfirstlane(wv.y) - 1 + lane;
   const bool incol = (i >= 0 && i < nx);
   const int ic = incol ? i : (i < 0 ? 0 : nx - 1);  // clamped column: loads stay in bounds
-  const bool own = live && incol && lane >= 1 && lane <= EW25;
+  const bool own = incol && lane >= 1 && lane <= EW25;
   const int j0 = ychunk_j0(__builtin_amdgcn_readfirstlane(wv.w)), j1 = ychunk_j1(__builtin_amdgcn_readfirstlane(wv.w));
   const long nxy = (long)nx * ny;
   const uint32_t p = (uint32_t)k * nx + ic;
@@ -2736,13 +2726,13 @@ __device__ __forceinline__ void el25_stress_tile(const DModel* __restrict__ mode
 template <typename T>
 __global__ void __launch_bounds__(NT25, sizeof(T) == 4 ? SDT_EL25S_WAVES : 2)
 k_el25_stress(const DModel* __restrict__ models, const DShot* __restrict__ shots,
-          const int4* __restrict__ work, const int* __restrict__ base, int rel) {
-  const int4 wv = work[blockIdx.x];
+          const int4* __restrict__ work, int n, const int* __restrict__ base, int rel) {
+  const int q = item25(n);
+  if (q < 0) return;
+  const int4 wv = work[q];
   const int s = __builtin_amdgcn_readfirstlane(wv.x);
-  if (s < 0) return;
   const DModel& M = models[shots[s].model];
-  const int xo = __builtin_amdgcn_readfirstlane(wv.y) + (int)((threadIdx.x >> 6) % XW25) * EW25;
-  const int k = __builtin_amdgcn_readfirstlane(wv.z) + (int)(threadIdx.x >> 6) / XW25;
+  const int xo = __builtin_amdgcn_readfirstlane(wv.y), k = __builtin_amdgcn_readfirstlane(wv.z);
   const int j0 = ychunk_j0(__builtin_amdgcn_readfirstlane(wv.w)), j1 = ychunk_j1(__builtin_amdgcn_readfirstlane(wv.w));
   const bool interior = xo - 1 >= M.lx && xo + 62 < M.nx - M.lx && k >= M.lz && k < M.nz - M.lz &&
                         j0 >= M.ly && j1 <= M.ny - M.ly;
@@ -2761,18 +2751,12 @@ __device__ __forceinline__ void el25_vel_tile(const DModel* __restrict__ models,
   const DShot& S = shots[s];
   const DModel& M = models[S.model];
   const int nx = M.nx, ny = M.ny, nz = M.nz;
-  // a wavefront past the last plane stays (clamped, storing nothing) so that
-  // every wavefront of the block takes the same barriers
-  const int wx_ = (int)(threadIdx.x >> 6) % XW25;  // x slot in the block
-  const int wv_ = (int)(threadIdx.x >> 6) / XW25;  // plane slot in the block
-  const int kw = __builtin_amdgcn_readfirstlane(wv.z) + wv_;
-  const bool live = kw < nz;
-  const int k = live ? kw : nz - 1;
+  const int k = __builtin_amdgcn_readfirstlane(wv.z);
   const int lane = threadIdx.x & 63;
-  const int i = __builtin_amdgcn_readfirstlane(wv.y) + wx_ * EW25 - 1 + lane;
+  const int i = __builtin_amdgcn_readfirstlane(wv.y) - 1 + lane;
   const bool incol = (i >= 0 && i < nx);
   const int ic = incol ? i : (i < 0 ? 0 : nx - 1);
-  const bool own = live && incol && lane >= 1 && lane <= EW25;
+  const bool own = incol && lane >= 1 && lane <= EW25;
   const int j0 = ychunk_j0(__builtin_amdgcn_readfirstlane(wv.w)), j1 = ychunk_j1(__builtin_amdgcn_readfirstlane(wv.w));
   const int it = *base + rel;
   const long nxy = (long)nx * ny;
@@ -2899,13 +2883,13 @@ __device__ __forceinline__ void el25_vel_tile(const DModel* __restrict__ models,
 template <typename T>
 __global__ void __launch_bounds__(NT25, sizeof(T) == 4 ? SDT_EL25V_WAVES : 2)
 k_el25_vel(const DModel* __restrict__ models, const DShot* __restrict__ shots,
-          const int4* __restrict__ work, const int* __restrict__ base, int rel) {
-  const int4 wv = work[blockIdx.x];
+          const int4* __restrict__ work, int n, const int* __restrict__ base, int rel) {
+  const int q = item25(n);
+  if (q < 0) return;
+  const int4 wv = work[q];
   const int s = __builtin_amdgcn_readfirstlane(wv.x);
-  if (s < 0) return;
   const DModel& M = models[shots[s].model];
-  const int xo = __builtin_amdgcn_readfirstlane(wv.y) + (int)((threadIdx.x >> 6) % XW25) * EW25;
-  const int k = __builtin_amdgcn_readfirstlane(wv.z) + (int)(threadIdx.x >> 6) / XW25;
+  const int xo = __builtin_amdgcn_readfirstlane(wv.y), k = __builtin_amdgcn_readfirstlane(wv.z);
   const int j0 = ychunk_j0(__builtin_amdgcn_readfirstlane(wv.w)), j1 = ychunk_j1(__builtin_amdgcn_readfirstlane(wv.w));
   const bool interior = xo - 1 >= M.lx && xo + 62 < M.nx - M.lx && k >= M.lz && k < M.nz - M.lz &&
                         j0 >= M.ly && j1 <= M.ny - M.ly;
@@ -3489,10 +3473,11 @@ __device__ __forceinline__ bool em25_interior(const DModel& M, int xo, int k, in
 template <typename T>
 __global__ void __launch_bounds__(64)
 k_em25_h(const DModel* __restrict__ models, const DShot* __restrict__ shots,
-         const int4* __restrict__ work) {
-  const int4 wv = work[blockIdx.x];
+         const int4* __restrict__ work, int n) {
+  const int q = item25(n);
+  if (q < 0) return;
+  const int4 wv = work[q];
   const int s = __builtin_amdgcn_readfirstlane(wv.x);
-  if (s < 0) return;
   const DModel& M = models[shots[s].model];
   const int j0 = ychunk_j0(__builtin_amdgcn_readfirstlane(wv.w)), j1 = ychunk_j1(__builtin_amdgcn_readfirstlane(wv.w));
   if (em25_interior(M, __builtin_amdgcn_readfirstlane(wv.y), __builtin_amdgcn_readfirstlane(wv.z), j0, j1))
@@ -3504,10 +3489,11 @@ k_em25_h(const DModel* __restrict__ models, const DShot* __restrict__ shots,
 template <typename T>
 __global__ void __launch_bounds__(64)
 k_em25_e(const DModel* __restrict__ models, const DShot* __restrict__ shots,
-         const int4* __restrict__ work, const int* __restrict__ base, int rel) {
-  const int4 wv = work[blockIdx.x];
+         const int4* __restrict__ work, int n, const int* __restrict__ base, int rel) {
+  const int q = item25(n);
+  if (q < 0) return;
+  const int4 wv = work[q];
   const int s = __builtin_amdgcn_readfirstlane(wv.x);
-  if (s < 0) return;
   const DModel& M = models[shots[s].model];
   const int it = *base + rel;
   const int j0 = ychunk_j0(__builtin_amdgcn_readfirstlane(wv.w)), j1 = ychunk_j1(__builtin_amdgcn_readfirstlane(wv.w));
@@ -3546,7 +3532,6 @@ __global__ void __launch_bounds__(64)
 k_em25_edges(const DModel* __restrict__ models, const DShot* __restrict__ shots,
              const int4* __restrict__ work) {
   const int4 wv = work[blockIdx.x];
-  if (wv.x < 0) return;
   const DShot& S = shots[wv.x];
   const DModel& M = models[S.model];
   const int nx = M.nx, ny = M.ny, nz = M.nz;
@@ -3910,48 +3895,97 @@ std::vector<int4> el2_work(const Plan* p, int ew = EW, int which = 0) {
   return work;
 }
 
-// Work list of the ELASTIC25 kernels: one item (shot, x0, k0, j0 | j1 << 16)
-// per block of KB25 planes k0.. x XW25 * EW25 columns x0.. x rows j0..j1-1
-// (at most Y25, cut at the y-slab edges), x fastest.
-// The items of each shot are cut into 8 contiguous runs, one per XCD (item w
-// runs on XCD w % 8), so the blocks an XCD runs at a time cover whole rows
-// of a few planes (long contiguous runs of addresses in each array).
-std::vector<int4> el25_work(const Plan* p, int planes, int xstep) {
+// Where the y chunks of at most `rows` rows of one model start, and ny: chunks
+// end at the y-slab edges, so a chunk lies inside a slab or outside both.
+std::vector<int> cuts25(const sdt_model& M, int rows) {
+  std::vector<int> cuts = {0};
+  const int ya = std::min(M.ly, M.ny), yb = std::max(ya, M.ny - M.ly);
+  auto cut = [&](int a, int b) {  // rows a .. b-1 in chunks of nearly equal height
+    const int nc = b > a ? (b - a + rows - 1) / rows : 0;
+    for (int c = 1; c <= nc; ++c) cuts.push_back(a + (int)((long long)(b - a) * c / nc));
+  };
+  cut(0, ya);
+  cut(ya, yb);
+  cut(yb, M.ny);
+  return cuts;
+}
+
+// Rows per y chunk of a 2.5-D plan.  A wavefront walks its rows one after the
+// other, waiting for each row's loads, so tall chunks leave a small grid
+// bound by the latency of that walk with most of the device idle; short ones
+// reload the row above and below, and, in the elastic passes, the column's 39
+// coefficients, per chunk.  Measured per step (us, chunks of 32 / 16 / 8 / 4 /
+// 2 rows): EM 544x96x416 FP32 580 / 532 / 504 / 495 / -, 332x72x182 FP64 246 /
+// 257 / 231 / 219 / 220, 112x56x82 FP32 74 / 64 / 40 / 30 / 23; elastic
+// 832x96x432 FP32 1309 / 1281 / 1322 / 1474 / 1872, 332x72x182 FP32 170 / 191 /
+// 171 / 174 / 203, 182x69x107 FP64 145 / 146 / 125 / 126 / 135, 112x56x82 FP64
+// 137 / 127 / 82 / 62 / 70.  So the EM passes take 4 rows, the elastic ones 16,
+// or 8 and 4 where that leaves fewer than 12000 and 2500 wavefronts; either
+// takes 2 below 2000.
+int rows25(const Plan* p) {
+  auto waves = [&](int rows) {
+    long long n = 0;
+    for (const sdt_shot& S : p->hshots) {
+      const sdt_model& M = p->hmodels[S.model];
+      n += (long long)(cuts25(M, rows).size() - 1) * ((M.nx + EW25 - 1) / EW25) * M.nz;
+    }
+    return n;
+  };
+  if (p->kind == SDT_ELASTIC25) {
+    if (waves(16) >= 12000) return 16;
+    if (waves(8) >= 2500) return 8;
+  }
+  return waves(4) >= 2000 ? 4 : 2;
+}
+
+// Work list of the 2.5-D kernels: one item (shot, x0, k, j0 | j1 << 16) per
+// wavefront of EW25 columns x0.. of plane k and one y chunk, plane by plane,
+// chunk by chunk, x fastest.  The kernels give each XCD a contiguous run of
+// them, so the wavefronts an XCD runs at a time cover whole rows of a few
+// planes (long contiguous runs of addresses in each array).
+// `least`: the fewest rows per chunk (a shorter list for the fixed scratch).
+std::vector<int4> el25_work(const Plan* p, int least) {
   std::vector<int4> all;
+  const int rows = std::max(rows25(p), least);
   for (int s = 0; s < p->nshots; ++s) {
     const sdt_model& M = p->hmodels[p->hshots[s].model];
-    // y chunks of at most Y25 rows, cut at the y-slab edges
-    std::vector<int> cuts = {0};
-    const int ya = std::min(M.ly, M.ny), yb = std::max(ya, M.ny - M.ly);
-    if (ya > 0) cuts.push_back(ya);
-    for (int j = ya + Y25; j < yb; j += Y25) cuts.push_back(j);
-    if (yb > cuts.back()) cuts.push_back(yb);
-    if (M.ny > cuts.back()) cuts.push_back(M.ny);
-    for (size_t c = 0; c + 1 < cuts.size(); ++c)
-      for (int k0 = 0; k0 < M.nz; k0 += planes)
-        for (int x0 = 0; x0 < M.nx; x0 += xstep)
-          all.push_back(make_int4(s, x0, k0, ychunk_pack(cuts[c], cuts[c + 1])));
+    const std::vector<int> cuts = cuts25(M, rows);
+    for (int k = 0; k < M.nz; ++k)
+      for (size_t c = 0; c + 1 < cuts.size(); ++c)
+        for (int x0 = 0; x0 < M.nx; x0 += EW25)
+          all.push_back(make_int4(s, x0, k, ychunk_pack(cuts[c], cuts[c + 1])));
   }
-  const size_t run = (all.size() + 7) / 8;
-  std::vector<int4> work(run * 8, make_int4(-1, 0, 0, 0));
-  for (size_t q = 0; q < all.size(); ++q) work[(q % run) * 8 + q / run] = all[q];
-  return work;
+  return all;
+}
+
+// Kernel `which` (0 stress / H, 1 velocity / E, 2 receiver gather) of step
+// base + rel of a 2.5-D plan.
+template <typename T>
+void launch_one25(Plan* p, hipStream_t st, int rel, int which) {
+  const int n = p->nwork;
+  const dim3 grd((n + 7) / 8 * 8), blk(NT25);
+  if (which == 2) {
+    if (p->maxrec > 0)
+      hipLaunchKernelGGL(k_gather<T>, dim3((p->maxrec + 63) / 64, p->nshots), dim3(64), 0, st, p->dmodels,
+                         p->dshots, p->nshots, p->ncomp, p->dbase, rel);
+  } else if (p->kind == SDT_ELASTIC25) {
+    if (which == 0)
+      hipLaunchKernelGGL(k_el25_stress<T>, grd, blk, 0, st, p->dmodels, p->dshots, p->dwork, n, p->dbase, rel);
+    else
+      hipLaunchKernelGGL(k_el25_vel<T>, grd, blk, 0, st, p->dmodels, p->dshots, p->dwork, n, p->dbase, rel);
+  } else if (which == 0) {
+    hipLaunchKernelGGL(k_em25_h<T>, grd, blk, 0, st, p->dmodels, p->dshots, p->dwork, n);
+  } else {
+    hipLaunchKernelGGL(k_em25_e<T>, grd, blk, 0, st, p->dmodels, p->dshots, p->dwork, n, p->dbase, rel);
+  }
 }
 
 // Launch kernel `which` (0: first field update, 1: second field update,
 // 2: receiver gather) of one step.
 template <typename T>
 void launch_one(Plan* p, hipStream_t st, int rel, int which) {
-  const dim3 grd(p->nwork);
-  if (which == 2) {
-    // the 2-D step kernels write their receiver samples themselves
-    if (p->maxrec > 0 && kind_3d(p->kind)) {
-      const dim3 gg((p->maxrec + 63) / 64, p->nshots);
-      hipLaunchKernelGGL(k_gather<T>, gg, dim3(64), 0, st, p->dmodels, p->dshots, p->nshots,
-                         p->ncomp, p->dbase, rel);
-    }
-    return;
-  }
+  if (kind_3d(p->kind)) return launch_one25<T>(p, st, rel, which);
+  if (which == 2) return;  // the 2-D step kernels write their receiver samples themselves
   switch (p->kind * 2 + which) {
     case SDT_ELASTIC2 * 2:
       if (p->split)
@@ -3966,21 +4000,6 @@ void launch_one(Plan* p, hipStream_t st, int rel, int which) {
       break;
     case SDT_EM2 * 2 + 1:
       break;  // the fused step kernel does both phases
-    case SDT_ELASTIC25 * 2:
-      hipLaunchKernelGGL(k_el25_stress<T>, grd, dim3(NT25), 0, st, p->dmodels, p->dshots, p->dwork,
-                         p->dbase, rel);
-      break;
-    case SDT_ELASTIC25 * 2 + 1:
-      hipLaunchKernelGGL(k_el25_vel<T>, grd, dim3(NT25), 0, st, p->dmodels, p->dshots, p->dwork,
-                         p->dbase, rel);
-      break;
-    case SDT_EM25 * 2:
-      hipLaunchKernelGGL(k_em25_h<T>, grd, dim3(64), 0, st, p->dmodels, p->dshots, p->dwork);
-      break;
-    case SDT_EM25 * 2 + 1:
-      hipLaunchKernelGGL(k_em25_e<T>, grd, dim3(64), 0, st, p->dmodels, p->dshots, p->dwork, p->dbase,
-                         rel);
-      break;
   }
 }
 
@@ -4343,7 +4362,7 @@ struct Stage {
 // settings and everything of `S` except the receivers-by-row index.  Reads
 // no device memory.
 int stage_host(Plan* p, int kind, int prec, const sdt_model* models, int nmodels,
-               const sdt_shot* shots, int nshots, int nt, Stage& S) {
+               const sdt_shot* shots, int nshots, int nt, Stage& S, int least_rows25 = 0) {
   const bool split = (kind & SDT_SPLIT_CPML) != 0;
   kind &= ~SDT_SPLIT_CPML;
   if (split && kind != SDT_ELASTIC2) return fail(SDT_EINVAL, "SDT_SPLIT_CPML applies to ELASTIC2 only");
@@ -4398,8 +4417,7 @@ int stage_host(Plan* p, int kind, int prec, const sdt_model* models, int nmodels
     D.rxid = nullptr;
   }
   // work lists: (shot, x0, z0); all shots of one tile share blockIdx % 8 (XCD)
-  if (kind == SDT_ELASTIC25) S.work = el25_work(p, KB25, EW25 * XW25);
-  if (kind == SDT_EM25) S.work = el25_work(p, 1, EW25);  // one plane, one wavefront per item
+  if (kind_3d(kind)) S.work = el25_work(p, least_rows25);
   if (pingpong(kind)) {
     p->el2_eh = default_rows(p);
     S.work = el2_work(p);
@@ -4742,7 +4760,15 @@ int sdt_run_noalloc(int kind, int prec, const sdt_model* models, int nmodels,
   Stage S;
   int rc = stage_host(p, kind, prec, models, nmodels, shots, nshots, nt, S);
   if (rc) return rc;
-  const ScratchLayout L = scratch_layout(p, S);
+  ScratchLayout L = scratch_layout(p, S);
+  // a 2.5-D list too long for the scratch: taller chunks, as far as that helps
+  for (int rows = 8; kind_3d(p->kind) && L.total > (size_t)SDT_NOALLOC_SCRATCH_BYTES && rows <= 65536; rows *= 2) {
+    P = Plan();
+    S = Stage();
+    rc = stage_host(p, kind, prec, models, nmodels, shots, nshots, nt, S, rows);
+    if (rc) return rc;
+    L = scratch_layout(p, S);
+  }
   if (L.total > (size_t)SDT_NOALLOC_SCRATCH_BYTES)
     return fail(SDT_EINVAL, "sdt_run_noalloc: this run needs " + std::to_string(L.total) +
                                 " bytes of scratch (descriptors, work lists, receiver index) but the "

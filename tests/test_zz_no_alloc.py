@@ -94,3 +94,15 @@ def test_noalloc_reports_instability_and_rejects_oversize():
     c, _ = _pair([many], "fp32")
     with pytest.raises(_hip.SeidartHipError, match="scratch"):
         c.run_noalloc()
+
+
+def test_noalloc_25d_list_longer_than_the_scratch():
+    """A 2.5-D grid whose work list of 4-row chunks does not fit the scratch
+    (525,000 items of 16 bytes): the call takes taller chunks and equals the
+    plan path bit for bit."""
+    probs = [tiny_problem("em25", seed=330, npml=6, nt=3, nx=64, ny=600, nz=1750)]
+    _near_source_receivers(probs)
+    a, b = _pair(probs, "fp32")
+    a.run(graph_block=0).check()
+    b.run_noalloc()
+    _same(a, b)
