@@ -175,17 +175,18 @@ int sdt_plan_run(void* plan, int it0, int nsteps, int graph_block, void* stream)
  * waves_per_block (1, 2 or 4) wavefronts side by side, each owning 61
  * columns (56 in the two-step ELASTIC2 kernel, 60 in the two-step EM2
  * one), walks `rows` rows (1..256).
- * Default: 4 wavefronts and the tallest of 32, 16, 8, 4 rows that gives the
- * plan at least 1024 blocks (else 2).  Results do not depend on the shape.
+ * Default: by the number of wavefronts the plan has (short tiles for small
+ * plans, so that they fill the device).  Results do not depend on the shape.
+ * The adjoint's trail recomputation has a tile shape of its own.
  * Synchronises the device when the shape changes. */
 int sdt_plan_set_tiles(void* plan, int waves_per_block, int rows);
 int sdt_plan_get_tiles(void* plan, int* waves_per_block, int* rows);
 
 /* ELASTIC2 / EM2 order of the step kernels' work lists (no counterpart in
  * the reference; the autotuner's third knob beside the tile shape and the
- * steps per launch).  0 (the default) deals a model's tiles to the eight
- * XCDs in turn, so every XCD covers the whole model; 1 lists the tiles
- * column by column and gives each XCD a contiguous run of them, so a tile
+ * steps per launch).  0 (the default of large plans) deals a model's tiles to the eight
+ * XCDs in turn, so every XCD covers the whole model; 1 (the default of the
+ * others) lists the tiles column by column and gives each XCD a contiguous run of them, so a tile
  * and the one below it, which read the same halo rows, run on one XCD one
  * after the other, and each XCD keeps to one part of the model from step
  * to step (small single-shot grids gain; the large batched plans do not).
@@ -195,8 +196,8 @@ int sdt_plan_set_tile_order(void* plan, int order);
 int sdt_plan_get_tile_order(void* plan, int* order);
 
 /* ELASTIC2 / EM2 steps per launch of the step kernel (no counterpart in the
- * reference): 2 (the default for plans of at least 4M cells per step,
- * summed over shots; smaller plans default to 1) advances two time steps in
+ * reference): 2 (the default, except for elastic plans so small that tiles of
+ * one row and one step per launch are faster) advances two time steps in
  * one launch, keeping the state of the first in registers, so the state
  * crosses HBM once per two steps; 1 is the one-step kernel.  Results are
  * identical bit for bit.  A run of an odd number of steps ends with one

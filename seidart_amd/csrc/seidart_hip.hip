@@ -675,9 +675,6 @@ static_assert(EW2 >= 1 && EW2 <= 58, "two-step wavefront: 2 halo lanes left, 4 r
 #ifndef SDT_EL2X2_WAVES
 #define SDT_EL2X2_WAVES 4   // FP32 wavefronts per SIMD the register budget allows
 #endif
-#ifndef SDT_EL2X2_MIN_CELLS
-#define SDT_EL2X2_MIN_CELLS 4000000LL  // cells per step from which plans default to two steps per launch
-#endif
 #ifndef SDT_EL2X2_PREFETCH
 #define SDT_EL2X2_PREFETCH 0
 #endif
@@ -1907,12 +1904,12 @@ template <typename T, bool SPLIT, bool PML>
 __device__ __forceinline__ void el2_adj_tile(const DModel* __restrict__ models,
                                              const DShot* __restrict__ shots,
                                              const DAdj* __restrict__ adj, const int s, const int xo,
-                                             const int zo, const int t, const int t0,
+                                             const int zo, const int eh, const int t, const int t0,
                                              const unsigned gmask, const int lane, const int tb) {
   const DShot& S = shots[s];
   const DModel& M = models[S.model];
   const DAdj& A = adj[s];
-  const int zend = min(zo + AH, M.nz);
+  const int zend = min(zo + eh, M.nz);
   const A32<const T> Lin(A.lam[(t + 1) & 1]);
   const A32<T> Lout(A.lam[t & 1]);
   const T* trail = static_cast<const T*>(A.trail[tb]);
@@ -1941,18 +1938,18 @@ k_el2_adj(const DModel* __restrict__ models, const DShot* __restrict__ shots,
     const int4 wv = work[w];
     const int s = __builtin_amdgcn_readfirstlane(wv.x);
     const int xo = __builtin_amdgcn_readfirstlane(wv.y) + wave * AW;
-    const int zo = __builtin_amdgcn_readfirstlane(wv.z);
+    const int zo = __builtin_amdgcn_readfirstlane(wv.z), eh = __builtin_amdgcn_readfirstlane(wv.w);
     if (s < 0) continue;
     const DModel& M = models[shots[s].model];
     if (xo >= M.nx) continue;
     // a wave whose columns and rows (halo included) avoid every C-PML slab
     // runs the body without memory variables
     const bool interior = xo - 2 >= M.lx && xo + 61 < M.nx - M.lx && zo - 3 >= M.lz &&
-                          zo + AH + 2 < M.nz - M.lz;
+                          zo + eh + 2 < M.nz - M.lz;
     if (interior)
-      el2_adj_tile<T, SPLIT, false>(models, shots, adj, s, xo, zo, t, t0, gmask, threadIdx.x & 63, tb);
+      el2_adj_tile<T, SPLIT, false>(models, shots, adj, s, xo, zo, eh, t, t0, gmask, threadIdx.x & 63, tb);
     else
-      el2_adj_tile<T, SPLIT, true>(models, shots, adj, s, xo, zo, t, t0, gmask, threadIdx.x & 63, tb);
+      el2_adj_tile<T, SPLIT, true>(models, shots, adj, s, xo, zo, eh, t, t0, gmask, threadIdx.x & 63, tb);
   }
 }
 
@@ -3618,6 +3615,8 @@ struct Plan {
   DAdj* dadj = nullptr;          // adjoint descriptors (sdt_adjoint_setup)
   std::vector<DAdj> hadj;
   int4* dadjwork = nullptr;      // work list of the fused adjoint kernel
+  int4* dtrwork = nullptr;       // work list of the trail recomputation, with its own tile shape
+  int ntrwork = 0, tr_grid = 0, tr_wb = 4, tr_eh = 4;
   int* dtbase = nullptr;         // first step of the trail (adjoint kernels)
   int* dtsel_trail = nullptr;    // trail buffer the recomputation writes
   int* dtsel_adj = nullptr;      // trail buffer the adjoint reads
@@ -3681,36 +3680,39 @@ long long psi_elems(int kind, long long nx, long long ny, long long nz, long lon
 template <typename T, bool TRAIL, bool SPLIT>
 void launch_el2(Plan* p, hipStream_t st, int rel, const int* tsel, const int* prun = nullptr) {
   const DAdj* adj = TRAIL ? p->dadj : nullptr;
-  const dim3 g(p->el2_grid);
-  if (!TRAIL && p->el2_eh == 1) {  // tiles of one row: all loads at once
-    switch (p->el2_wb) {
+  const dim3 g(TRAIL ? p->tr_grid : p->el2_grid);
+  const int4* w = TRAIL ? p->dtrwork : p->dwork;
+  const int n = TRAIL ? p->ntrwork : p->nwork, wb = TRAIL ? p->tr_wb : p->el2_wb;
+  const int eh = TRAIL ? p->tr_eh : p->el2_eh;
+  if (!TRAIL && eh == 1) {  // tiles of one row: all loads at once
+    switch (wb) {
       case 1:
         hipLaunchKernelGGL((k_el2_step<T, false, SPLIT, 1, true>), g, dim3(64), 0, st, p->dmodels,
-                           p->dshots, p->dwork, p->nwork, p->dbase, rel, adj, tsel, 1, prun);
+                           p->dshots, w, n, p->dbase, rel, adj, tsel, 1, prun);
         break;
       case 2:
         hipLaunchKernelGGL((k_el2_step<T, false, SPLIT, 2, true>), g, dim3(128), 0, st, p->dmodels,
-                           p->dshots, p->dwork, p->nwork, p->dbase, rel, adj, tsel, 1, prun);
+                           p->dshots, w, n, p->dbase, rel, adj, tsel, 1, prun);
         break;
       default:
         hipLaunchKernelGGL((k_el2_step<T, false, SPLIT, 4, true>), g, dim3(256), 0, st, p->dmodels,
-                           p->dshots, p->dwork, p->nwork, p->dbase, rel, adj, tsel, 1, prun);
+                           p->dshots, w, n, p->dbase, rel, adj, tsel, 1, prun);
         break;
     }
     return;
   }
-  switch (p->el2_wb) {
+  switch (wb) {
     case 1:
       hipLaunchKernelGGL((k_el2_step<T, TRAIL, SPLIT, 1>), g, dim3(64), 0, st, p->dmodels,
-                         p->dshots, p->dwork, p->nwork, p->dbase, rel, adj, tsel, p->el2_eh, prun);
+                         p->dshots, w, n, p->dbase, rel, adj, tsel, eh, prun);
       break;
     case 2:
       hipLaunchKernelGGL((k_el2_step<T, TRAIL, SPLIT, 2>), g, dim3(128), 0, st, p->dmodels,
-                         p->dshots, p->dwork, p->nwork, p->dbase, rel, adj, tsel, p->el2_eh, prun);
+                         p->dshots, w, n, p->dbase, rel, adj, tsel, eh, prun);
       break;
     default:
       hipLaunchKernelGGL((k_el2_step<T, TRAIL, SPLIT, 4>), g, dim3(256), 0, st, p->dmodels,
-                         p->dshots, p->dwork, p->nwork, p->dbase, rel, adj, tsel, p->el2_eh, prun);
+                         p->dshots, w, n, p->dbase, rel, adj, tsel, eh, prun);
       break;
   }
 }
@@ -3746,19 +3748,22 @@ void launch_el2x2(Plan* p, hipStream_t st, int rel) {
 template <typename T, bool TRAIL>
 void launch_em2(Plan* p, hipStream_t st, int rel, const int* tsel, const int* prun = nullptr) {
   const DAdj* adj = TRAIL ? p->dadj : nullptr;
-  const dim3 g(p->el2_grid);
-  switch (p->el2_wb) {
+  const dim3 g(TRAIL ? p->tr_grid : p->el2_grid);
+  const int4* w = TRAIL ? p->dtrwork : p->dwork;
+  const int n = TRAIL ? p->ntrwork : p->nwork, wb = TRAIL ? p->tr_wb : p->el2_wb;
+  const int eh = TRAIL ? p->tr_eh : p->el2_eh;
+  switch (wb) {
     case 1:
       hipLaunchKernelGGL((k_em2_step<T, TRAIL, 1>), g, dim3(64), 0, st, p->dmodels, p->dshots,
-                         p->dwork, p->nwork, p->dbase, rel, adj, tsel, p->el2_eh, prun);
+                         w, n, p->dbase, rel, adj, tsel, eh, prun);
       break;
     case 2:
       hipLaunchKernelGGL((k_em2_step<T, TRAIL, 2>), g, dim3(128), 0, st, p->dmodels, p->dshots,
-                         p->dwork, p->nwork, p->dbase, rel, adj, tsel, p->el2_eh, prun);
+                         w, n, p->dbase, rel, adj, tsel, eh, prun);
       break;
     default:
       hipLaunchKernelGGL((k_em2_step<T, TRAIL, 4>), g, dim3(256), 0, st, p->dmodels, p->dshots,
-                         p->dwork, p->nwork, p->dbase, rel, adj, tsel, p->el2_eh, prun);
+                         w, n, p->dbase, rel, adj, tsel, eh, prun);
       break;
   }
 }
@@ -3801,20 +3806,69 @@ bool el2x2_interior(const sdt_model& M, int x0, int z0, int wb, int eh) {
   return true;
 }
 
-// Default rows per tile of the 2-D step kernels: the tallest of 32, 16, 8, 4
-// rows that still gives the plan 1024 blocks or more (4 per CU), else 2 --
-// a single shot on a small grid needs short tiles to fill the device.
-int default_rows(const Plan* p) {
-  const int bw = EW * p->el2_wb;
-  for (int rows : {32, 16, 8, 4}) {
-    long long blocks = 0;
-    for (const sdt_shot& S : p->hshots) {
-      const sdt_model& M = p->hmodels[S.model];
-      blocks += (long long)((M.nx + bw - 1) / bw) * ((M.nz + rows - 1) / rows);
-    }
-    if (blocks >= 1024) return rows;
+// Wavefronts of a 2-D plan with ew owned columns each and tiles of `rows` rows.
+long long waves2d(const Plan* p, int ew, int rows) {
+  long long n = 0;
+  for (const sdt_shot& S : p->hshots) {
+    const sdt_model& M = p->hmodels[S.model];
+    n += (long long)((M.nx + ew - 1) / ew) * ((M.nz + rows - 1) / rows);
   }
-  return 2;
+  return n;
+}
+
+// Default launch shape of a 2-D plan: steps per launch, wavefronts per block,
+// rows per tile and tile order, from how many wavefronts the plan has and
+// whether its ping-pong fields fit the 256 MB last-level cache.  Fitted to the
+// times of every shape on 30 plans (6 k to 27 M cells per step, 1 to 36 shots)
+// per kind and precision: within 2 to 4 % of the fastest shape in the mean.
+// Against tiles of 32 .. 2 rows for 1024 blocks of four wavefronts, one step
+// per launch below 4 M cells and order 0 (us per step, then and now): elastic
+// FP64 127x103 12.1 -> 7.1, 296^2 15.3 -> 9.0, 1064x808 40.5 -> 28.3, 640x440 x
+// 12 shots 119 -> 74; EM FP64 296^2 8.9 -> 5.0, 1064x808 22.8 -> 12.3; EM FP32
+// 1064x808 16.4 -> 8.4.
+//  - EM2 always takes two steps per launch (also the smallest grid, 80x70:
+//    4.1 against 5.9 us per step).  The elastic two-step walk reads six halo
+//    rows per tile, so below 2000 (FP64) and 6000 (FP32) wavefronts of one row
+//    the one-step kernel's one-row tiles win (296^2 FP64 9.0 against 12.4).
+//  - Rows: the tallest of 8, 4, 2 (EM also 1) that still give 2000 (FP64) or
+//    4000 (elastic FP32; EM 2800) wavefronts; 16 and 32 only with many of them
+//    (1064x808 x 6 shots EM FP64 46.6 with 8, 51.4 with 16).
+//  - Column strips per XCD (order 1) while the fields fit the cache, tiles
+//    dealt in turn beyond (1064x808 x 12 shots elastic FP64 157 against 178).
+//  - Wide blocks waste wavefronts at the edge of a narrow grid and take its
+//    interior tiles for edge tiles: fewer wavefronts per block below 400
+//    columns, and (but for EM FP64) where the fields do not fit the cache.
+void default_shape(Plan* p) {
+  const bool em = p->kind == SDT_EM2, f64 = p->prec == SDT_FP64;
+  const int ew = em ? EW2E : EW2;
+  long long cells = 0;
+  int maxnx = 0;
+  for (const sdt_shot& S : p->hshots) {
+    const sdt_model& M = p->hmodels[S.model];
+    cells += (long long)M.nx * M.nz;
+    maxnx = std::max(maxnx, M.nx);
+  }
+  const bool big = cells * kind_fields(p->kind) * 2 * (f64 ? 8 : 4) >= 250000000LL;
+  p->spl = 2;
+  p->el2_order = big ? 0 : 1;
+  if (!em && waves2d(p, EW, 1) <= (f64 ? 2000 : 6000)) {
+    p->spl = 1;
+    p->el2_wb = 2;
+    p->el2_eh = 1;
+  } else if (waves2d(p, ew, 32) >= 16000) {
+    p->el2_wb = 4;
+    p->el2_eh = 32;
+  } else {
+    const bool narrow = maxnx < 400;
+    if (big)
+      p->el2_wb = em ? (f64 ? 4 : 2) : (f64 ? 1 : 2);
+    else
+      p->el2_wb = !narrow ? 4 : em ? 1 : f64 ? 2 : 4;
+    p->el2_eh = em ? 1 : 2;
+    for (int rows : {2, 4, 8})
+      if (waves2d(p, ew, rows) >= (f64 ? 2000 : em ? 2800 : 4000)) p->el2_eh = rows;
+    if (waves2d(p, ew, 16) >= (em ? 12000 : 8000)) p->el2_eh = 16;
+  }
 }
 
 // Row cuts of one model's tiles: rows of at most eh, and with zt < zb also
@@ -3840,16 +3894,16 @@ std::vector<int> row_cuts(int nz, int eh, int zt, int zb) {
 // others.  ew: owned columns per wavefront; two-step lists (ew = EW2, EW2E)
 // cut their rows at the interior limits of their kernel and carry each
 // tile's height in .w (0: the plan's rows); one-step lists (ew = EW) carry
-// the shot's model index in .w.  Order (p->el2_order): 0 deals a model's
+// the shot's model index in .w.  Order: 0 deals a model's
 // tiles to the XCDs in turn (tile k of the list on XCD k % 8), every XCD
 // covering the whole model; 1 lists them column by column and gives each
 // XCD a contiguous run, so a tile and the one below it, which share halo
 // rows, run on one XCD one after the other, and each XCD keeps to one part
 // of the model from step to step.  Either way all shots of a tile run on
 // one XCD, one after another.
-std::vector<int4> el2_work(const Plan* p, int ew = EW, int which = 0) {
+std::vector<int4> el2_work(const Plan* p, int wb, int eh, int order, int ew = EW, int which = 0) {
   std::vector<int4> work;
-  const int bw = ew * p->el2_wb, eh = p->el2_eh;
+  const int bw = ew * wb;
   for (int m = 0; m < p->nmodels; ++m) {
     const sdt_model& M = p->hmodels[m];
     // first and last-plus-one interior rows of k_el2_step2 / k_em2_step2
@@ -3864,10 +3918,10 @@ std::vector<int4> el2_work(const Plan* p, int ew = EW, int which = 0) {
     std::vector<int> tl;
     auto take = [&](int t) {
       const int z0 = cuts[t / tx], h = cuts[t / tx + 1] - z0;
-      if (which == 0 || el2x2_interior(M, (t % tx) * bw, z0, p->el2_wb, h) == (which == 1))
+      if (which == 0 || el2x2_interior(M, (t % tx) * bw, z0, wb, h) == (which == 1))
         tl.push_back(t);
     };
-    if (p->el2_order) {
+    if (order) {
       for (int x = 0; x < tx; ++x)
         for (int z = 0; z < tz; ++z) take(z * tx + x);
     } else {
@@ -3877,7 +3931,7 @@ std::vector<int4> el2_work(const Plan* p, int ew = EW, int which = 0) {
     // tile of slot tg of XCD tt (-1: none)
     const int chunk = (nt + 7) / 8;
     auto tile_at = [&](int tg, int tt) {
-      const int k = p->el2_order ? tt * chunk + tg : tg * 8 + tt;
+      const int k = order ? tt * chunk + tg : tg * 8 + tt;
       return k < nt ? tl[k] : -1;
     };
     for (int tg = 0; tg < chunk; ++tg)
@@ -4291,9 +4345,10 @@ void drop_adjoint_graphs(Plan* p) {
 // interior blocks first (their count in *ni), then the others; EM2: one list.
 std::vector<int4> build_work2(const Plan* p, int* ni) {
   const bool em = p->kind == SDT_EM2;
-  std::vector<int4> work = em ? std::vector<int4>() : el2_work(p, EW2, 1);
+  auto list = [&](int ew, int which) { return el2_work(p, p->el2_wb, p->el2_eh, p->el2_order, ew, which); };
+  std::vector<int4> work = em ? std::vector<int4>() : list(EW2, 1);
   *ni = (int)work.size();
-  const std::vector<int4> edge = em ? el2_work(p, EW2E, 0) : el2_work(p, EW2, 2);
+  const std::vector<int4> edge = em ? list(EW2E, 0) : list(EW2, 2);
   work.insert(work.end(), edge.begin(), edge.end());
   if (work.empty()) work.push_back(make_int4(-1, 0, 0, 0));
   return work;
@@ -4362,7 +4417,7 @@ struct Stage {
 // settings and everything of `S` except the receivers-by-row index.  Reads
 // no device memory.
 int stage_host(Plan* p, int kind, int prec, const sdt_model* models, int nmodels,
-               const sdt_shot* shots, int nshots, int nt, Stage& S, int least_rows25 = 0) {
+               const sdt_shot* shots, int nshots, int nt, Stage& S, int least_rows = 0) {
   const bool split = (kind & SDT_SPLIT_CPML) != 0;
   kind &= ~SDT_SPLIT_CPML;
   if (split && kind != SDT_ELASTIC2) return fail(SDT_EINVAL, "SDT_SPLIT_CPML applies to ELASTIC2 only");
@@ -4417,21 +4472,19 @@ int stage_host(Plan* p, int kind, int prec, const sdt_model* models, int nmodels
     D.rxid = nullptr;
   }
   // work lists: (shot, x0, z0); all shots of one tile share blockIdx % 8 (XCD)
-  if (kind_3d(kind)) S.work = el25_work(p, least_rows25);
+  if (kind_3d(kind)) S.work = el25_work(p, least_rows);
   if (pingpong(kind)) {
-    p->el2_eh = default_rows(p);
-    S.work = el2_work(p);
+    default_shape(p);
+    if (least_rows > p->el2_eh) {  // shorter lists for the fixed scratch
+      p->el2_eh = least_rows;
+      p->el2_wb = 4;
+    }
+    S.work = el2_work(p, p->el2_wb, p->el2_eh, p->el2_order);
     const int nblk = (int)S.work.size();
     p->el2_grid = std::max(8, std::min(nblk, SDT_EL2_GRID) / 8 * 8);
     int ni = 0;
     S.work2 = build_work2(p, &ni);
     set_work2_grids(p, (int)S.work2.size(), ni);
-    // Two steps per launch pay off once the plan has enough tiles to fill the
-    // device; a small plan is bound by the latency of one tile's walk, which
-    // the two-step kernel lengthens (measured: 4M cells per step and above).
-    long long cells = 0;
-    for (int s = 0; s < nshots; ++s) cells += (long long)models[shots[s].model].nx * models[shots[s].model].nz;
-    p->spl = cells >= SDT_EL2X2_MIN_CELLS ? 2 : 1;
   }
   if (S.work.empty()) S.work.push_back(make_int4(-1, 0, 0, 0));
   p->nwork = (int)S.work.size();
@@ -4761,8 +4814,8 @@ int sdt_run_noalloc(int kind, int prec, const sdt_model* models, int nmodels,
   int rc = stage_host(p, kind, prec, models, nmodels, shots, nshots, nt, S);
   if (rc) return rc;
   ScratchLayout L = scratch_layout(p, S);
-  // a 2.5-D list too long for the scratch: taller chunks, as far as that helps
-  for (int rows = 8; kind_3d(p->kind) && L.total > (size_t)SDT_NOALLOC_SCRATCH_BYTES && rows <= 65536; rows *= 2) {
+  // work lists too long for the scratch: taller tiles, as far as that helps
+  for (int rows = 4; L.total > (size_t)SDT_NOALLOC_SCRATCH_BYTES && rows <= 65536; rows *= 2) {
     P = Plan();
     S = Stage();
     rc = stage_host(p, kind, prec, models, nmodels, shots, nshots, nt, S, rows);
@@ -4853,7 +4906,7 @@ static int retile(Plan* p, int waves_per_block, int rows, int order) {
   p->el2_wb = waves_per_block;
   p->el2_eh = rows;
   p->el2_order = order;
-  const std::vector<int4> work = el2_work(p);
+  const std::vector<int4> work = el2_work(p, p->el2_wb, p->el2_eh, p->el2_order);
   int4* dw = nullptr;
   int rc = SDT_OK;
   if (hipMalloc(&dw, sizeof(int4) * work.size()) != hipSuccess) {
@@ -5034,6 +5087,27 @@ int sdt_adjoint_setup(void* plan, const sdt_adj_shot* adj, int nshots, unsigned 
   if (!p->dtbase) HIP_TRY(hipMalloc(&p->dtbase, sizeof(int)));
   if (!p->dtsel_trail) HIP_TRY(hipMalloc(&p->dtsel_trail, sizeof(int)));
   if (!p->dtsel_adj) HIP_TRY(hipMalloc(&p->dtsel_adj, sizeof(int)));
+  if (!p->dtrwork) {
+    // The recomputation has a tile shape of its own (it steps one at a time,
+    // beside the adjoint kernel): 4 rows, 2 where the plan then has fewer than
+    // 4000 wavefronts, tiles dealt to the XCDs in turn.  Measured for one
+    // backward pass (ms, tiles of 1 / 2 / 4 / 8 / 32 rows): 16 shots of
+    // 1064x552 FP32 86.5 / 73.9 / 70.1 / 71.2 / 75.0 (73.6 with 4 rows in column
+    // strips), 6 shots of 740x440 FP64 32.7 / 30.0 / 28.9 / 29.0 / 32.2 with two
+    // wavefronts per block (30.1 with four).
+    p->tr_wb = p->prec == SDT_FP64 ? 2 : 4;
+    p->tr_eh = waves2d(p, EW, 4) >= 4000 ? 4 : 2;
+    const std::vector<int4> work = el2_work(p, p->tr_wb, p->tr_eh, 0);
+    int4* dw = nullptr;
+    HIP_TRY(hipMalloc(&dw, sizeof(int4) * work.size()));
+    if (hipMemcpy(dw, work.data(), sizeof(int4) * work.size(), hipMemcpyHostToDevice) != hipSuccess) {
+      (void)hipFree(dw);
+      return fail(SDT_EDEVICE, "hipMemcpy failed (work list)");
+    }
+    p->dtrwork = dw;
+    p->ntrwork = (int)work.size();
+    p->tr_grid = std::max(8, std::min(p->ntrwork, SDT_EL2_GRID) / 8 * 8);
+  }
   if (!p->dadjwork) {
     // (shot, x0, z0, rows) items of AWB * AW columns x rows; the items of one
     // tile over all shots of its model share blockIdx % 8 (one XCD's L2).
@@ -5148,6 +5222,7 @@ void sdt_plan_destroy(void* plan) {
   if (p->dnpsi) (void)hipFree(p->dnpsi);
   if (p->dadj) (void)hipFree(p->dadj);
   if (p->dadjwork) (void)hipFree(p->dadjwork);
+  if (p->dtrwork) (void)hipFree(p->dtrwork);
   if (p->dtbase) (void)hipFree(p->dtbase);
   if (p->dtsel_trail) (void)hipFree(p->dtsel_trail);
   if (p->dtsel_adj) (void)hipFree(p->dtsel_adj);

@@ -228,8 +228,8 @@ class Simulation:
     @property
     def steps_per_launch(self) -> int:
         """Time steps one launch of the ELASTIC2 / EM2 step kernel advances
-        (2 by default for plans of at least 4M cells per step, else 1;
-        ``autotune`` times both); results do not depend on it."""
+        (2 by default, 1 for small ELASTIC2 plans; ``autotune`` times both);
+        results do not depend on it."""
         v = C.c_int()
         _hip.check(_hip.lib().sdt_plan_get_steps_per_launch(self._plan, C.byref(v)))
         return v.value

@@ -190,3 +190,23 @@ def test_em2_two_step_segments_and_oracle(oracle_lib):
             exp = o.field(n)
             if np.abs(exp).max() > 0:
                 assert rel_l2(s.field(k, n), exp) < FP64_TOL, n
+
+
+@pytest.mark.parametrize("kind,precision,nx,nz,nshots", [
+    ("elastic2", "fp64", 30, 28, 1), ("elastic2", "fp64", 500, 250, 1), ("elastic2", "fp32", 400, 90, 3),
+    ("elastic2", "fp32", 700, 500, 1), ("em2", "fp64", 30, 28, 1), ("em2", "fp32", 410, 380, 2),
+    ("em2", "fp64", 1300, 1100, 5)])
+def test_default_shape_keeps_results(kind, precision, nx, nz, nshots):
+    """The launch shape a plan picks by its size (one or two steps, short or
+    tall tiles, either order) against one step of 4 x 32 tiles, order 0."""
+    p = tiny_problem(kind, seed=340, nx=nx, nz=nz, npml=6, nt=11, nshots=nshots, nrec=9)
+    a = _sim(p, precision, 1)
+    a.use((1, 4, 32, 0))
+    ref = _snap(a.run(graph_block=4).check())
+    from seidart_amd.solver import Simulation
+    for gb in (0, 4):
+        b = Simulation(p, precision=precision)
+        assert (b.steps_per_launch, *b.tiles(), b.tile_order) != (1, 4, 32, 0)
+        _assert_same(ref, _snap(b.run(graph_block=gb).check()))
+        b.close()
+    a.close()

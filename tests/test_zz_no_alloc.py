@@ -106,3 +106,14 @@ def test_noalloc_25d_list_longer_than_the_scratch():
     a.run(graph_block=0).check()
     b.run_noalloc()
     _same(a, b)
+
+
+def test_noalloc_2d_lists_longer_than_the_scratch_leaves():
+    """Receivers that leave 52 KB of the scratch, on a grid whose default
+    tiles need 64 KB of work lists: the call takes taller tiles and equals the
+    plan path bit for bit."""
+    p = tiny_problem("em2", seed=331, npml=6, nt=3, nx=64, nz=2000, nrec=1_041_000)
+    a, b = _pair([p], "fp64")
+    a.run(graph_block=0).check()
+    b.run_noalloc()
+    _same(a, b)
