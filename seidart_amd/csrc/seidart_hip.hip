@@ -1540,7 +1540,7 @@ k_el2_adj_g(const DModel* __restrict__ models, const DShot* __restrict__ shots,
 // ---------------------------------------------------------------------------
 // Fused adjoint step: the same transpose as the three kernels above, in one
 // pass.  A wavefront owns AW columns (lanes 2..AW+1; two halo lanes on each
-// side) of AH rows of one shot and marches down them.  At march row r it
+// side) of eh rows of one shot and marches down them.  At march row r it
 // does V^T of row r, the stress gathers with S^T / N^T of row r-1 and the
 // velocity gather of row r-2, keeping the few rows each phase needs from
 // the previous ones in registers and taking x neighbours from the
@@ -1557,10 +1557,6 @@ k_el2_adj_g(const DModel* __restrict__ models, const DShot* __restrict__ shots,
 constexpr int AW = SDT_ADJ_AW;   // owned columns per wavefront
 static_assert(AW >= 1 && AW <= 60, "adjoint wavefront: two halo lanes on each side");
 constexpr int AWB = 4;   // wavefronts per block, side by side in x
-#ifndef SDT_ADJ_ROWS
-#define SDT_ADJ_ROWS SDT_EL2_ROWS
-#endif
-constexpr int AH = SDT_ADJ_ROWS;
 
 // One march row of the fused adjoint, shared by the one-step kernel and by
 // both stages of the two-step kernel.  Inputs of march row r: lambda_{t+1}
@@ -5111,21 +5107,35 @@ int sdt_adjoint_setup(void* plan, const sdt_adj_shot* adj, int nshots, unsigned 
   if (!p->dadjwork) {
     // (shot, x0, z0, rows) items of AWB * AW columns x rows; the items of one
     // tile over all shots of its model share blockIdx % 8 (one XCD's L2).
-    // The elastic kernel walks AH rows; the EM kernel takes the tallest of
-    // AH, 16, 8, 4, 2 rows that gives the plan 1000 tiles or more (its
-    // single-shot grids are small and stay in the cache, so the walk's
-    // latency is what a tile costs).
+    // Rows per tile: a tile is a serial walk, so a small plan needs short
+    // ones to fill the device, a large one tall ones (the elastic walk reads
+    // five halo rows per tile).  Elastic: the rows whose walk, times the rounds
+    // the device needs for all blocks at three (FP64 two) blocks per CU, is
+    // shortest.  EM: the tallest that give 1300 blocks.  Measured for one
+    // backward pass of 128 steps (ms; 1 / 2 / 4 / 8 / 16 / 32 / 64 rows): elastic
+    // FP32 160x130 2.6 / 3.0 / 4.3 / 5.1 / 7.7 / 13.3 / 23.1, FP64 740x440 x 2
+    // shots 15.8 / 12.3 / 10.7 / 9.8 / 12.1 / 18.0 / 29.7, x 6 shots 43.1 / 32.4 /
+    // 28.4 / 25.4 / 24.8 / 30.1 / 36.8; EM FP64 1064x808 x 2 shots 12.8 / 11.7 /
+    // 11.9 / 14.1 / 18.2 / 27.5 / 45.8.
     const int bw = AW * AWB;
-    int eh = AH;
+    auto blocks = [&](int rows) {
+      long long n = 0;
+      for (const sdt_shot& S : p->hshots) {
+        const sdt_model& M = p->hmodels[S.model];
+        n += (long long)((M.nx + bw - 1) / bw) * ((M.nz + rows - 1) / rows);
+      }
+      return n;
+    };
+    int eh = 1;
     if (p->kind == SDT_EM2) {
-      for (int rows : {AH, 16, 8, 4, 2}) {
-        eh = rows;
-        long long tiles = 0;
-        for (const sdt_shot& S : p->hshots) {
-          const sdt_model& M = p->hmodels[S.model];
-          tiles += (long long)((M.nx + bw - 1) / bw) * ((M.nz + rows - 1) / rows);
-        }
-        if (tiles >= 1000) break;
+      for (int rows : {2, 4, 8, 16, 32})
+        if (blocks(rows) >= 1300) eh = rows;
+    } else {
+      const double room = 256.0 * (p->prec == SDT_FP32 ? 3 : 2);
+      double best = 1e300;
+      for (int rows : {1, 2, 4, 8, 16, 24, 32, 64}) {
+        const double cost = std::max(1.0, blocks(rows) / room) * (rows + 5);
+        if (cost < best) { best = cost; eh = rows; }
       }
     }
     std::vector<int4> work;

@@ -576,3 +576,31 @@ def test_em_gradient_finite_differences():
             errs.append(abs((J(up) - J(dn)) / (2 * h) - g[j, i]) / abs(g[j, i]))
         worst[k] = max(errs)
     assert all(v < 1e-3 for v in worst.values()), worst
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,nx,nz,nshots", [
+    ("elastic2", 62, 9, 1), ("elastic2", 250, 131, 4), ("elastic2", 500, 333, 9),
+    ("em2", 62, 9, 1), ("em2", 500, 333, 5)])
+def test_adjoint_tile_heights_match_reference_kernels(kind, nx, nz, nshots):
+    """The fused adjoint with the tile heights that plans of these sizes take
+    (1 to 32 rows, remainders included) against the unfused kernels, whose
+    launches do not tile: gradients and lambda_0 to FP64 rounding."""
+    p = tiny_problem(kind, seed=95, nx=nx, nz=nz, npml=3, nt=10, nshots=nshots, nrec=5,
+                     src=(nx // 2, 0, nz // 2), gamma=1e-3 if kind == "elastic2" else 0.0)
+    p.cpml_split = kind == "elastic2"
+    out = []
+    for ref in (False, True):
+        eng = _engine(p, "fp64", every=4, reference=ref)
+        g = torch.Generator().manual_seed(12)
+        for s in range(eng.nshots):
+            eng.init[s].copy_(torch.randn(eng.init[s].numel(), generator=g, dtype=torch.float64))
+        tr = eng.forward()
+        grad, _ = eng.backward([torch.randn(t.shape, generator=g, dtype=torch.float64) for t in tr])
+        out.append((grad[0].cpu().numpy(), [eng.adjoint_state(s).cpu().numpy() for s in range(nshots)]))
+        eng.close()
+    (g0, l0), (g1, l1) = out
+    for q in range(g0.shape[0]):
+        assert rel_l2(g0[q], g1[q]) < 1e-12, (q, rel_l2(g0[q], g1[q]))
+    for a, b in zip(l0, l1):
+        assert rel_l2(a, b) < 1e-12
