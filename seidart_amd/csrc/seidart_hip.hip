@@ -3260,10 +3260,19 @@ k_em2_adj(const DModel* __restrict__ models, const DShot* __restrict__ shots,
 //            y [nz][2ly][nx]: dEz_dy dEx_dy dHz_dy dHx_dy
 //            z [2lz][ny][nx]: dEy_dz dEx_dz dHy_dz dHx_dz
 // H boundary zeroing (:1059-1078) is applied by the next H update.
-// Two launches per step (H, then E) in the layout of the 2.5-D elastic
-// kernels: a wavefront takes one plane, 64 columns (62 owned; x neighbours by
-// lane shuffles) and a chunk of rows, walking y with the y neighbours in
-// registers; the z neighbours are loads of the adjacent plane.
+// Two launches per step (H, then E): a wavefront takes one plane, 64 columns
+// (62 owned; x neighbours by DPP lane shifts) and a chunk of rows, R = 4 (FP64
+// 2) rows at a time; the z neighbours are loads of the adjacent plane.
+// What bounds it is the latency of a row's loads, with the fields streaming
+// from HBM on large grids: so all loads of the R rows, C-PML memory included,
+// are issued before the first use (34 field loads per lane in flight in FP32),
+// and the y neighbours among them come from registers.  A walk of one row at a
+// time, whose memory variables were loaded after the wait for the row's fields,
+// took (us per step, same chunks) 495 against 429 on 544x96x416 FP32 (3.8
+// against 4.4 TB/s of traffic), 865 against 850 in FP64, 219 against 202 on
+// 332x72x182 FP64, 37.6 against 30.7 on 133x57x79 FP64, 30 against 19.6 on
+// 112x56x82 FP32.  Four rows in FP64 need 180 registers (two wavefronts per
+// SIMD): 841 and 32.4 on the large and the small grid.
 // ===========================================================================
 struct Slab3e {
   long SX, SY, SZ, bx, by, bz;
@@ -3277,9 +3286,26 @@ struct Slab3e {
   }
 };
 
+// rows whose loads an EM 2.5-D wavefront has in flight at once
+template <typename T>
+constexpr int RE25 = sizeof(T) == 4 ? 4 : 2;
+
+// C-PML memory of the EM 2.5-D passes on one plane: arrays q and q + 1 of each
+// axis (q = 0 for the H pass, 2 for the E pass).  The bases are wave-uniform,
+// the offsets 32-bit: x[j * 2lx + xs], y[slab row * nx + i], z[j * nx + i].
+template <typename T>
+struct Psi25 {
+  const A32<T> x0, x1, y0, y1, z0, z1;
+  __device__ __forceinline__ Psi25(void* psi, const Slab3e& L, int q, int nx, int ny, int lx, int ly, int k, int zs)
+      : x0((T*)psi + L.bx + q * L.SX + (long)k * ny * 2 * lx), x1((T*)psi + L.bx + (q + 1) * L.SX + (long)k * ny * 2 * lx),
+        y0((T*)psi + L.by + q * L.SY + (long)k * 2 * ly * nx), y1((T*)psi + L.by + (q + 1) * L.SY + (long)k * 2 * ly * nx),
+        z0((T*)psi + L.bz + q * L.SZ + (long)zs * ny * nx), z1((T*)psi + L.bz + (q + 1) * L.SZ + (long)zs * ny * nx) {}
+};
+
 template <typename T, bool PML>
 __device__ __forceinline__ void em25_h_tile(const DModel* __restrict__ models,
                                            const DShot* __restrict__ shots, const int4 wv) {
+  constexpr int R = RE25<T>;
   const int s = __builtin_amdgcn_readfirstlane(wv.x);
   const DShot& S = shots[s];
   const DModel& M = models[S.model];
@@ -3296,65 +3322,97 @@ __device__ __forceinline__ void em25_h_tile(const DModel* __restrict__ models,
   const long nxy = (long)nx * ny;
   const T idx = T(1.0 / M.dx), idy = T(1.0 / M.dy), idz = T(1.0 / M.dz), dbH = T(M.scal[0]);
   const int lx = M.lx, ly = M.ly, lz = M.lz;
+  // a chunk lies inside a y slab or outside both
   const bool inx = PML && incol && in_slab(i, nx, lx), inz = PML && in_slab(k, nz, lz);
+  const bool iny = PML && in_slab(j0, ny, ly);
   const Prof<T> P(&M.prof[0][0]);
   const T bx_i = P[PB][ic], ax_i = P[PA][ic], ikx_i = P[PK][ic];
-  const T bz_k = P[12 + PB][k], az_k = P[12 + PA][k], ikz_k = P[12 + PK][k];
-  const T bzh_k = P[12 + PBH][k], azh_k = P[12 + PAH][k], ikzh_k = P[12 + PKH][k];
-  gcptr<T> by = P[6 + PB], ay = P[6 + PA], iky = P[6 + PK];
-  gcptr<T> byh = P[6 + PBH], ayh = P[6 + PAH], ikyh = P[6 + PKH];
+  const auto pz = kp<T>(M.prof[2][PK]), pza = kp<T>(M.prof[2][PA]), pzb = kp<T>(M.prof[2][PB]);
+  const T ikz_k = pz[k], az_k = pza[k], bz_k = pzb[k];
+  const T ikzh_k = kp<T>(M.prof[2][PKH])[k], azh_k = kp<T>(M.prof[2][PAH])[k], bzh_k = kp<T>(M.prof[2][PBH])[k];
+  const auto iky = kp<T>(M.prof[1][PK]), ay = kp<T>(M.prof[1][PA]), by = kp<T>(M.prof[1][PB]);
+  const auto ikyh = kp<T>(M.prof[1][PKH]), ayh = kp<T>(M.prof[1][PAH]), byh = kp<T>(M.prof[1][PBH]);
   const int ku = k + 1 < nz ? k + 1 : k;
   const A32<const T> EX = cplane<T>(S.f[0], nxy, k), EY = cplane<T>(S.f[1], nxy, k);
   const A32<const T> EZ = cplane<T>(S.f[2], nxy, k);
   const A32<const T> EXU = cplane<T>(S.f[0], nxy, ku), EYU = cplane<T>(S.f[1], nxy, ku);
   const A32<T> HX = plane<T>(S.f[3], nxy, k), HY = plane<T>(S.f[4], nxy, k), HZ = plane<T>(S.f[5], nxy, k);
-  auto psi = mp<T>(S.psi);
-  const Slab3e L(nx, ny, nz, lx, ly, lz);
   const int xs = inx ? slab_pos(i, nx, lx) : 0, zs = inz ? slab_pos(k, nz, lz) : 0;
-  if (j0 >= j1) return;
-  // y window: Ex, Ez of row j
-  uint32_t c = (uint32_t)j0 * nx + ic;
-  T exc = EX[c], ezc = EZ[c];
+  const Psi25<T> W(S.psi, Slab3e(nx, ny, nz, lx, ly, lz), 0, nx, ny, lx, ly, k, zs);
 #pragma unroll 1
-  for (int j = j0; j < j1; ++j, c += nx) {
-    const T exn = EX[c + nx], ezn = EZ[c + nx];  // row j+1 (j <= ny-2)
-    const T eyc = EY[c];
-    const T eyu = EYU[c], exu = EXU[c];          // plane k+1
-    const T eze = lane_next(ezc), eye = lane_next(eyc);
-    const T hx0 = HX[c], hy0 = HY[c], hz0 = HZ[c];
-    if (own) {
-      const bool iny = PML && in_slab(j, ny, ly);
-      const long ox = L.bx + ((long)k * ny + j) * 2 * lx + xs;
-      const long oy = L.by + ((long)k * 2 * ly + (iny ? slab_pos(j, ny, ly) : 0)) * nx + ic;
-      const long oz = L.bz + ((long)zs * ny + j) * nx + ic;
-      const bool lo = (i == 0 || j == 0 || k == 0);
-      {  // Hx, :901-920
-        T a = (ezc - ezn) * idy;  // dEz_dy
-        if (iny) { T m = byh[j] * psi[oy] + ayh[j] * a; a = a * ikyh[j] + m; psi[oy] = m; }
-        T b = (eyu - eyc) * idz;  // dEy_dz
-        if (inz) { T m = bzh_k * psi[oz] + azh_k * b; b = b * ikzh_k + m; psi[oz] = m; }
-        const bool edge = lo || i == nx - 1 || j == ny - 2 || k == nz - 2;
-        HX[c] = (edge ? T(0) : hx0) + dbH * (b + a);
-      }
-      {  // Hy, :922-942
-        T a = (exc - exu) * idz;  // dEx_dz
-        if (inz) { T m = bz_k * psi[oz + L.SZ] + az_k * a; a = a * ikz_k + m; psi[oz + L.SZ] = m; }
-        T b = (eze - ezc) * idx;  // dEz_dx
-        if (inx) { T m = bx_i * psi[ox] + ax_i * b; b = b * ikx_i + m; psi[ox] = m; }
-        const bool edge = lo || i == nx - 2 || j == ny - 1 || k == nz - 2;
-        HY[c] = (edge ? T(0) : hy0) + dbH * (b + a);
-      }
-      if (k >= 1) {  // Hz, :944-962
-        T a = (exn - exc) * idy;  // dEx_dy
-        if (iny) { T m = by[j] * psi[oy + L.SY] + ay[j] * a; a = a * iky[j] + m; psi[oy + L.SY] = m; }
-        T b = (eyc - eye) * idx;  // dEy_dx
-        if (inx) { T m = bx_i * psi[ox + L.SX] + ax_i * b; b = b * ikx_i + m; psi[ox + L.SX] = m; }
-        const bool edge = lo || i == nx - 2 || j == ny - 2 || k == nz - 1;
-        HZ[c] = (edge ? T(0) : hz0) + dbH * (b + a);
+  for (int jb = j0; jb < j1; jb += R) {
+    // every load of the R rows before the first use; rows past the chunk
+    // reload its last row (E: the row below it, j1 <= ny - 1)
+    T ex[R + 1], ez[R + 1], ey[R], eyu[R], exu[R], hx[R], hy[R], hz[R];
+    T mx0[R], mx1[R], my0[R], my1[R], mz0[R], mz1[R];
+    uint32_t c[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const uint32_t ce = (uint32_t)min(jb + q, j1) * nx + ic;
+      c[q] = (uint32_t)min(jb + q, j1 - 1) * nx + ic;
+      ex[q] = EX[ce]; ez[q] = EZ[ce]; ey[q] = EY[c[q]];
+      eyu[q] = EYU[c[q]]; exu[q] = EXU[c[q]];
+      hx[q] = HX[c[q]]; hy[q] = HY[c[q]]; hz[q] = HZ[c[q]];
+    }
+    const uint32_t cl = (uint32_t)min(jb + R, j1) * nx + ic;
+    ex[R] = EX[cl]; ez[R] = EZ[cl];
+    if (PML && iny) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const uint32_t o = (uint32_t)slab_pos(min(jb + q, j1 - 1), ny, ly) * nx + ic;
+        my0[q] = W.y0[o]; my1[q] = W.y1[o];
       }
     }
-    exc = exn;
-    ezc = ezn;
+    if (PML && inz) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) { mz0[q] = W.z0[c[q]]; mz1[q] = W.z1[c[q]]; }
+    }
+    if (PML && inx) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const uint32_t o = (uint32_t)min(jb + q, j1 - 1) * 2 * lx + xs;
+        mx0[q] = W.x0[o]; mx1[q] = W.x1[o];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const int j = jb + q;
+      if (j >= j1) break;
+      const T exc = ex[q], ezc = ez[q], exn = ex[q + 1], ezn = ez[q + 1], eyc = ey[q];
+      const T eze = dpp_next(ezc), eye = dpp_next(eyc);
+      T ay_ = (ezc - ezn) * idy, bz_ = (eyu[q] - eyc) * idz;   // Hx: dEz_dy, dEy_dz (:901-920)
+      T az_ = (exc - exu[q]) * idz, bx_ = (eze - ezc) * idx;   // Hy: dEx_dz, dEz_dx (:922-942)
+      T cy_ = (exn - exc) * idy, cx_ = (eyc - eye) * idx;      // Hz: dEx_dy, dEy_dx (:944-962)
+      if (PML && iny) {
+        my0[q] = byh[j] * my0[q] + ayh[j] * ay_; ay_ = ay_ * ikyh[j] + my0[q];
+        my1[q] = by[j] * my1[q] + ay[j] * cy_; cy_ = cy_ * iky[j] + my1[q];
+      }
+      if (PML && inz) {
+        mz0[q] = bzh_k * mz0[q] + azh_k * bz_; bz_ = bz_ * ikzh_k + mz0[q];
+        mz1[q] = bz_k * mz1[q] + az_k * az_; az_ = az_ * ikz_k + mz1[q];
+      }
+      if (PML && inx) {
+        mx0[q] = bx_i * mx0[q] + ax_i * bx_; bx_ = bx_ * ikx_i + mx0[q];
+        mx1[q] = bx_i * mx1[q] + ax_i * cx_; cx_ = cx_ * ikx_i + mx1[q];
+      }
+      if (own) {
+        const bool lo = (i == 0 || j == 0 || k == 0);
+        HX[c[q]] = (lo || i == nx - 1 || j == ny - 2 || k == nz - 2 ? T(0) : hx[q]) + dbH * (bz_ + ay_);
+        HY[c[q]] = (lo || i == nx - 2 || j == ny - 1 || k == nz - 2 ? T(0) : hy[q]) + dbH * (bx_ + az_);
+        if (k >= 1) HZ[c[q]] = (lo || i == nx - 2 || j == ny - 2 || k == nz - 1 ? T(0) : hz[q]) + dbH * (cx_ + cy_);
+        if (PML && iny) {
+          const uint32_t o = (uint32_t)slab_pos(j, ny, ly) * nx + ic;
+          W.y0[o] = my0[q];
+          if (k >= 1) W.y1[o] = my1[q];
+        }
+        if (PML && inz) { W.z0[c[q]] = mz0[q]; W.z1[c[q]] = mz1[q]; }
+        if (PML && inx) {
+          const uint32_t o = (uint32_t)j * 2 * lx + xs;
+          W.x0[o] = mx0[q];
+          if (k >= 1) W.x1[o] = mx1[q];
+        }
+      }
+    }
   }
 }
 
@@ -3362,6 +3420,7 @@ template <typename T, bool PML>
 __device__ __forceinline__ void em25_e_tile(const DModel* __restrict__ models,
                                            const DShot* __restrict__ shots, const int4 wv,
                                            const int it) {
+  constexpr int R = RE25<T>;
   const int s = __builtin_amdgcn_readfirstlane(wv.x);
   const DShot& S = shots[s];
   const DModel& M = models[S.model];
@@ -3379,81 +3438,117 @@ __device__ __forceinline__ void em25_e_tile(const DModel* __restrict__ models,
   const T idx = T(1.0 / M.dx), idy = T(1.0 / M.dy), idz = T(1.0 / M.dz);
   const int lx = M.lx, ly = M.ly, lz = M.lz;
   const bool inx = PML && incol && in_slab(i, nx, lx), inz = PML && in_slab(k, nz, lz);
+  const bool iny = PML && in_slab(j0, ny, ly);
   const Prof<T> P(&M.prof[0][0]);
   const T bxh_i = P[PBH][ic], axh_i = P[PAH][ic], ikxh_i = P[PKH][ic];
-  const T bz_k = P[12 + PB][k], az_k = P[12 + PA][k], ikz_k = P[12 + PK][k];
-  const T bzh_k = P[12 + PBH][k], azh_k = P[12 + PAH][k], ikzh_k = P[12 + PKH][k];
-  gcptr<T> byh = P[6 + PBH], ayh = P[6 + PAH], ikyh = P[6 + PKH];
+  const T ikz_k = kp<T>(M.prof[2][PK])[k], az_k = kp<T>(M.prof[2][PA])[k], bz_k = kp<T>(M.prof[2][PB])[k];
+  const T ikzh_k = kp<T>(M.prof[2][PKH])[k], azh_k = kp<T>(M.prof[2][PAH])[k], bzh_k = kp<T>(M.prof[2][PBH])[k];
+  const auto ikyh = kp<T>(M.prof[1][PKH]), ayh = kp<T>(M.prof[1][PAH]), byh = kp<T>(M.prof[1][PBH]);
   // loop ranges of :968-1029
   const bool ux = own && k >= 1 && k <= nz - 2 && i <= nx - 2;
   const bool uy = own && k >= 1 && k <= nz - 2 && i >= 1 && i <= nx - 2;
   const bool uz = own && k <= nz - 2 && i >= 1 && i <= nx - 2;
-  const T cax = ux ? A32<const T>(M.coef[0])[p] : T(0), cbx = ux ? A32<const T>(M.coef[1])[p] : T(0);
-  const T cay = uy ? A32<const T>(M.coef[2])[p] : T(0), cby = uy ? A32<const T>(M.coef[3])[p] : T(0);
-  const T caz = uz ? A32<const T>(M.coef[4])[p] : T(0), cbz = uz ? A32<const T>(M.coef[5])[p] : T(0);
+  const T cax = A32<const T>(M.coef[0])[p], cbx = A32<const T>(M.coef[1])[p];
+  const T cay = A32<const T>(M.coef[2])[p], cby = A32<const T>(M.coef[3])[p];
+  const T caz = A32<const T>(M.coef[4])[p], cbz = A32<const T>(M.coef[5])[p];
   const int kd = k >= 1 ? k - 1 : 0;
   const A32<const T> HX = cplane<T>(S.f[3], nxy, k), HY = cplane<T>(S.f[4], nxy, k);
   const A32<const T> HZ = cplane<T>(S.f[5], nxy, k);
   const A32<const T> HXD = cplane<T>(S.f[3], nxy, kd), HYD = cplane<T>(S.f[4], nxy, kd);
   const A32<T> EX = plane<T>(S.f[0], nxy, k), EY = plane<T>(S.f[1], nxy, k), EZ = plane<T>(S.f[2], nxy, k);
-  auto psi = mp<T>(S.psi);
-  const Slab3e L(nx, ny, nz, lx, ly, lz);
   const int xs = inx ? slab_pos(i, nx, lx) : 0, zs = inz ? slab_pos(k, nz, lz) : 0;
+  const Psi25<T> W(S.psi, Slab3e(nx, ny, nz, lx, ly, lz), 2, nx, ny, lx, ly, k, zs);
   const bool srccol = (i == S.isrc && k == S.ksrc);
-  // y window: Hx, Hz of row j-1
-  uint32_t c = (uint32_t)j0 * nx + ic;
-  T hxm = 0, hzm = 0;
-  if (j0 >= 1) { hxm = HX[c - nx]; hzm = HZ[c - nx]; }
+  bool bad = false;
 #pragma unroll 1
-  for (int j = j0; j < j1; ++j, c += nx) {
-    const T hxc = HX[c], hyc = HY[c], hzc = HZ[c];
-    const T hyd = HYD[c], hxd = HXD[c];          // plane k-1
-    const T hzw = lane_prev(hzc), hyw = lane_prev(hyc);
-    T ex = EX[c], ey = EY[c], ez = EZ[c];
-    if (own) {
-      const bool iny = PML && in_slab(j, ny, ly);
-      const long ox = L.bx + ((long)k * ny + j) * 2 * lx + xs;
-      const long oy = L.by + ((long)k * 2 * ly + (iny ? slab_pos(j, ny, ly) : 0)) * nx + ic;
-      const long oz = L.bz + ((long)zs * ny + j) * nx + ic;
-      if (ux && j >= 1 && j <= ny - 2) {  // Ex, :968-985
-        T a = (hzc - hzm) * idy;  // dHz_dy
-        if (iny) { T m = byh[j] * psi[oy + 2 * L.SY] + ayh[j] * a; a = a * ikyh[j] + m; psi[oy + 2 * L.SY] = m; }
-        T b = (hyd - hyc) * idz;  // dHy_dz
-        if (inz) { T m = bz_k * psi[oz + 2 * L.SZ] + az_k * b; b = b * ikz_k + m; psi[oz + 2 * L.SZ] = m; }
-        ex = cax * ex + cbx * (a + b);
+  for (int jb = j0; jb < j1; jb += R) {
+    T hx[R + 1], hz[R + 1], hy[R], hyd[R], hxd[R], ex[R], ey[R], ez[R];
+    T mx0[R], mx1[R], my0[R], my1[R], mz0[R], mz1[R];
+    uint32_t c[R];
+    const uint32_t cm = (uint32_t)max(jb - 1, 0) * nx + ic;  // the row above (row 0 uses none)
+    hx[0] = HX[cm]; hz[0] = HZ[cm];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      c[q] = (uint32_t)min(jb + q, j1 - 1) * nx + ic;
+      hx[q + 1] = HX[c[q]]; hy[q] = HY[c[q]]; hz[q + 1] = HZ[c[q]];
+      hyd[q] = HYD[c[q]]; hxd[q] = HXD[c[q]];
+      ex[q] = EX[c[q]]; ey[q] = EY[c[q]]; ez[q] = EZ[c[q]];
+    }
+    if (PML && iny) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const uint32_t o = (uint32_t)slab_pos(min(jb + q, j1 - 1), ny, ly) * nx + ic;
+        my0[q] = W.y0[o]; my1[q] = W.y1[o];
       }
-      if (uy && j <= ny - 2) {  // Ey, :988-1006
-        T a = (hzw - hzc) * idx;  // dHz_dx
-        if (inx) { T m = bxh_i * psi[ox + 2 * L.SX] + axh_i * a; a = a * ikxh_i + m; psi[ox + 2 * L.SX] = m; }
-        T b = (hxc - hxd) * idz;  // dHx_dz
-        if (inz) { T m = bzh_k * psi[oz + 3 * L.SZ] + azh_k * b; b = b * ikzh_k + m; psi[oz + 3 * L.SZ] = m; }
-        ey = cay * ey + cby * (a + b);
+    }
+    if (PML && inz) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) { mz0[q] = W.z0[c[q]]; mz1[q] = W.z1[c[q]]; }
+    }
+    if (PML && inx) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const uint32_t o = (uint32_t)min(jb + q, j1 - 1) * 2 * lx + xs;
+        mx0[q] = W.x0[o]; mx1[q] = W.x1[o];
       }
-      if (uz && j >= 1 && j <= ny - 2) {  // Ez, :1011-1029
-        T a = (hxm - hxc) * idy;  // dHx_dy
-        if (iny) { T m = byh[j] * psi[oy + 3 * L.SY] + ayh[j] * a; a = a * ikyh[j] + m; psi[oy + 3 * L.SY] = m; }
-        T b = (hyc - hyw) * idx;  // dHy_dx
-        if (inx) { T m = bxh_i * psi[ox + 3 * L.SX] + axh_i * b; b = b * ikxh_i + m; psi[ox + 3 * L.SX] = m; }
-        ez = caz * ez + cbz * (a + b);
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const int j = jb + q;
+      if (j >= j1) break;
+      const T hxc = hx[q + 1], hyc = hy[q], hzc = hz[q + 1], hxm = hx[q], hzm = hz[q];
+      const T hzw = dpp_prev(hzc), hyw = dpp_prev(hyc);
+      const bool jx = j >= 1 && j <= ny - 2, jy = j <= ny - 2;
+      T exn = ex[q], eyn = ey[q], ezn = ez[q];
+      if (ux && jx) {  // Ex, :968-985
+        T a = (hzc - hzm) * idy, b = (hyd[q] - hyc) * idz;  // dHz_dy, dHy_dz
+        if (PML && iny) {
+          my0[q] = byh[j] * my0[q] + ayh[j] * a; a = a * ikyh[j] + my0[q];
+          W.y0[(uint32_t)slab_pos(j, ny, ly) * nx + ic] = my0[q];
+        }
+        if (PML && inz) { mz0[q] = bz_k * mz0[q] + az_k * b; b = b * ikz_k + mz0[q]; W.z0[c[q]] = mz0[q]; }
+        exn = cax * exn + cbx * (a + b);
       }
-      if (srccol && j == S.jsrc) {  // source, :1033-1035
-        if (S.src[0]) ex += cp<T>(S.src[0])[it];
-        if (S.src[1]) ey += cp<T>(S.src[1])[it];
-        if (S.src[2]) ez += cp<T>(S.src[2])[it];
+      if (uy && jy) {  // Ey, :988-1006
+        T a = (hzw - hzc) * idx, b = (hxc - hxd[q]) * idz;  // dHz_dx, dHx_dz
+        if (PML && inx) {
+          mx0[q] = bxh_i * mx0[q] + axh_i * a; a = a * ikxh_i + mx0[q];
+          W.x0[(uint32_t)j * 2 * lx + xs] = mx0[q];
+        }
+        if (PML && inz) { mz1[q] = bzh_k * mz1[q] + azh_k * b; b = b * ikzh_k + mz1[q]; W.z1[c[q]] = mz1[q]; }
+        eyn = cay * eyn + cby * (a + b);
+      }
+      if (uz && jx) {  // Ez, :1011-1029
+        T a = (hxm - hxc) * idy, b = (hyc - hyw) * idx;  // dHx_dy, dHy_dx
+        if (PML && iny) {
+          my1[q] = byh[j] * my1[q] + ayh[j] * a; a = a * ikyh[j] + my1[q];
+          W.y1[(uint32_t)slab_pos(j, ny, ly) * nx + ic] = my1[q];
+        }
+        if (PML && inx) {
+          mx1[q] = bxh_i * mx1[q] + axh_i * b; b = b * ikxh_i + mx1[q];
+          W.x1[(uint32_t)j * 2 * lx + xs] = mx1[q];
+        }
+        ezn = caz * ezn + cbz * (a + b);
+      }
+      if (srccol && j == S.jsrc && own) {  // source, :1033-1035
+        if (S.src[0]) exn += cp<T>(S.src[0])[it];
+        if (S.src[1]) eyn += cp<T>(S.src[1])[it];
+        if (S.src[2]) ezn += cp<T>(S.src[2])[it];
       }
       // Dirichlet faces, :1038-1057 (and cells outside each staggered field's extent)
       const bool lo = (i == 0 || j == 0 || k == 0);
-      if (lo || i >= nx - 2 || j == ny - 1 || k == nz - 1) ex = 0;
-      if (lo || i == nx - 1 || j >= ny - 2 || k == nz - 1) ey = 0;
-      if (lo || i == nx - 1 || j == ny - 1 || k >= nz - 2) ez = 0;
-      check_blowup((double)ex * ex + (double)ey * ey + (double)ez * ez, S.blowup, it);
-      EX[c] = ex;
-      EY[c] = ey;
-      EZ[c] = ez;
+      if (lo || i >= nx - 2 || j == ny - 1 || k == nz - 1) exn = 0;
+      if (lo || i == nx - 1 || j >= ny - 2 || k == nz - 1) eyn = 0;
+      if (lo || i == nx - 1 || j == ny - 1 || k >= nz - 2) ezn = 0;
+      if (own) {
+        bad |= !((double)exn * exn + (double)eyn * eyn + (double)ezn * ezn <= 1.0e50);
+        EX[c[q]] = exn;
+        EY[c[q]] = eyn;
+        EZ[c[q]] = ezn;
+      }
     }
-    hxm = hxc;
-    hzm = hzc;
   }
+  if (bad) atomicMin(S.blowup, it);
 }
 
 // A wavefront whose columns, plane and rows (with the neighbours it reads)
@@ -3960,18 +4055,17 @@ std::vector<int> cuts25(const sdt_model& M, int rows) {
   return cuts;
 }
 
-// Rows per y chunk of a 2.5-D plan.  A wavefront walks its rows one after the
-// other, waiting for each row's loads, so tall chunks leave a small grid
-// bound by the latency of that walk with most of the device idle; short ones
-// reload the row above and below, and, in the elastic passes, the column's 39
-// coefficients, per chunk.  Measured per step (us, chunks of 32 / 16 / 8 / 4 /
-// 2 rows): EM 544x96x416 FP32 580 / 532 / 504 / 495 / -, 332x72x182 FP64 246 /
-// 257 / 231 / 219 / 220, 112x56x82 FP32 74 / 64 / 40 / 30 / 23; elastic
+// Rows per y chunk of a 2.5-D plan.  A wavefront takes its rows in turn,
+// waiting for their loads, so tall chunks leave a small grid bound by the
+// latency of that walk with most of the device idle; short ones reload the
+// row above and below, and, in the elastic passes, the column's 39
+// coefficients, per chunk.  EM: 4 rows (measured per step in us, 8 / 4 / 2 rows:
+// 332x72x182 FP32 90 / 84 / 86, FP64 207 / 202 / 203, 133x57x79 FP64 35 / 31 /
+// 31; 544x96x416 FP32 439 / 428 / -).  Elastic (32 / 16 / 8 / 4 / 2 rows):
 // 832x96x432 FP32 1309 / 1281 / 1322 / 1474 / 1872, 332x72x182 FP32 170 / 191 /
 // 171 / 174 / 203, 182x69x107 FP64 145 / 146 / 125 / 126 / 135, 112x56x82 FP64
-// 137 / 127 / 82 / 62 / 70.  So the EM passes take 4 rows, the elastic ones 16,
-// or 8 and 4 where that leaves fewer than 12000 and 2500 wavefronts; either
-// takes 2 below 2000.
+// 137 / 127 / 82 / 62 / 70: 16 rows, 8 where that leaves fewer than 12000
+// wavefronts, 4 below 2500 and 2 below 2000.
 int rows25(const Plan* p) {
   auto waves = [&](int rows) {
     long long n = 0;
@@ -3981,10 +4075,9 @@ int rows25(const Plan* p) {
     }
     return n;
   };
-  if (p->kind == SDT_ELASTIC25) {
-    if (waves(16) >= 12000) return 16;
-    if (waves(8) >= 2500) return 8;
-  }
+  if (p->kind == SDT_EM25) return 4;
+  if (waves(16) >= 12000) return 16;
+  if (waves(8) >= 2500) return 8;
   return waves(4) >= 2000 ? 4 : 2;
 }
 

@@ -122,6 +122,21 @@ def test_3d_tiles_and_y_chunks(oracle_lib, kind):
     _compare(sim, p, oracle_lib, FP64_TOL)
 
 
+@pytest.mark.parametrize("ny,npml", [(4, 1), (7, 2), (9, 3), (13, 5), (20, 4), (21, 8)])
+def test_em25_row_groups(oracle_lib, ny, npml):
+    """The EM 2.5-D passes take the rows of a chunk in groups (4 in FP32, 2 in
+    FP64): chunks of 1 to 4 rows, slabs with a remainder, a last row that the
+    H pass leaves out; against the oracle with the bars of the other tests."""
+    p = tiny_problem("em25", seed=68 + ny, nx=70, ny=ny, nz=19, npml=npml, nt=25, nrec=9,
+                     src=(35, ny // 2, 9))
+    _compare(_sim(p, "fp64").run().check(), p, oracle_lib, FP64_TOL)
+    sim = _sim(p, "fp32").run(graph_block=5).check()
+    ref = oracle_lib.OracleRun(p).run()
+    assert rel_l2(sim.traces()[0], ref.trace) < FP32_TOL
+    for n, exp in zip(ref.names, ref.fields):
+        assert rel_l2(sim.field(0, n), exp) < FP32_TOL, n
+
+
 @pytest.mark.parametrize("kind", ["elastic25", "em25"])
 def test_3d_y_rows_above_32767(oracle_lib, kind):
     """A 2.5-D grid 32,832 rows long in y: the work items whose y chunk ends
