@@ -3597,15 +3597,14 @@ k_em25_e(const DModel* __restrict__ models, const DShot* __restrict__ shots,
 // ===========================================================================
 template <typename T>
 __global__ void k_gather(const DModel* __restrict__ models, const DShot* __restrict__ shots,
-                         int nshots, int ncomp, const int* __restrict__ base, int rel) {
-  const int s = blockIdx.y;
-  if (s >= nshots) return;
-  const DShot& S = shots[s];
+                         int s0, int ncomp, const int* __restrict__ base, int rel, int k0, int k1) {
+  const DShot& S = shots[s0 + blockIdx.y];
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= S.nrec || S.trace == nullptr) return;
   const DModel& M = models[S.model];
   const int it = *base + rel;
   const auto q = cp<int>(S.rec) + 3 * r;
+  if (q[2] < k0 || q[2] >= k1) return;  // only planes k0 .. k1-1 are at this step
   const long c = ((long)q[2] * M.ny + q[1]) * M.nx + q[0];
   auto tr = mp<T>(S.trace) + ((long)it * ncomp) * S.nrec + r;
   for (int f = 0; f < ncomp; ++f) tr[(long)f * S.nrec] = cp<T>(S.f[f])[c];
@@ -3672,6 +3671,12 @@ __global__ void __launch_bounds__(256) k_hbm_probe(const float* __restrict__ src
 // ===========================================================================
 // Plan
 // ===========================================================================
+// A block of the 2.5-D schedule (set_blocks25): shots s0..s1-1, or of one shot
+// the planes from the previous block's `top` to below this one's (INT_MAX: nz).
+struct Block25 {
+  int s0, s1, top;
+};
+
 struct Plan {
   int kind = 0, prec = 0, nmodels = 0, nshots = 0, nt = 0, ncomp = 2;
   bool split = false;  // SDT_SPLIT_CPML
@@ -3682,6 +3687,9 @@ struct Plan {
   DShot* dshots = nullptr;
   int4* dwork = nullptr;
   int nwork = 0;
+  std::vector<int> item25;                // 2.5-D: first work item of each shot, and their number
+  std::vector<Block25> blocks25;          // 2.5-D: schedule (set_blocks25)
+  std::vector<std::pair<int, int>> reck;  // per shot: lowest and highest receiver plane
   int el2_grid = 0;  // persistent grid of the ELASTIC2 step kernel
   int el2_wb = SDT_EL2_WAVES_PER_BLOCK;  // tile: wavefronts per block
   int el2_eh = SDT_EL2_ROWS;             // tile: rows
@@ -4087,8 +4095,9 @@ int rows25(const Plan* p) {
 // them, so the wavefronts an XCD runs at a time cover whole rows of a few
 // planes (long contiguous runs of addresses in each array).
 // `least`: the fewest rows per chunk (a shorter list for the fixed scratch).
-std::vector<int4> el25_work(const Plan* p, int least) {
+std::vector<int4> el25_work(Plan* p, int least) {
   std::vector<int4> all;
+  p->item25.assign(1, 0);
   const int rows = std::max(rows25(p), least);
   for (int s = 0; s < p->nshots; ++s) {
     const sdt_model& M = p->hmodels[p->hshots[s].model];
@@ -4097,29 +4106,119 @@ std::vector<int4> el25_work(const Plan* p, int least) {
       for (size_t c = 0; c + 1 < cuts.size(); ++c)
         for (int x0 = 0; x0 < M.nx; x0 += EW25)
           all.push_back(make_int4(s, x0, k, ychunk_pack(cuts[c], cuts[c + 1])));
+    p->item25.push_back((int)all.size());
   }
   return all;
 }
 
-// Kernel `which` (0 stress / H, 1 velocity / E, 2 receiver gather) of step
-// base + rel of a 2.5-D plan.
+// Bytes of a shot's state.
+double shot_bytes(const Plan* p, int s) {
+  const sdt_model& M = p->hmodels[p->hshots[s].model];
+  const double n = kind_fields(p->kind) * (double)M.nx * M.ny * M.nz +
+                   psi_elems(p->kind | (p->split ? SDT_SPLIT_CPML : 0), M.nx, M.ny, M.nz, M.lx, M.ly, M.lz);
+  return n * (p->prec == SDT_FP64 ? 8 : 4);
+}
+
+// The schedule of the EM 2.5-D steps.  Each pass streams the whole state, so a
+// plan larger than the 256 MB last-level cache reads everything from HBM twice
+// per step.  Blocks of planes of at most 160 MB go through both passes of up to
+// 16 time steps before the next block starts, and what the first pass of a
+// block left in the cache the following ones find there.  Nothing is computed
+// twice: the H pass reads E of the plane above, so a block's upper bound moves
+// down by one plane per step, and the next block takes those planes.  Shots
+// that fit the cache go in groups of at most 200 MB.  Same kernels and results.
+// Measured per step (us, whole plan per pass, then blocks): 544x96x416 FP32 428
+// -> 350, FP64 831 -> 744; 832x96x432 FP32 682 -> 582; 432x96x282 FP64 468 ->
+// 409; 6 shots of 232x96x182 FP32 508 -> 476; 24 shots of 152x62x112 FP64 1156 ->
+// 1064 (groups of 150 MB: 1257; a launch over four of them leaves the device
+// half empty at its end).  100 and 200 MB for blocks of planes: 378 and 357 on
+// the first grid, 600 and 613 on the third.  The elastic passes gain nothing
+// (832x96x432 FP32 1281 whole, 1398 .. 1750 in blocks of 40 .. 140 planes):
+// resident in the cache they run at 41 instead of 35 Gcell-updates/s, less than
+// the launches' tails cost.
+constexpr int STEPS25 = 16;
+constexpr double PLANES25_BYTES = 160e6, SHOTS25_BYTES = 200e6;
+
+void set_blocks25(Plan* p) {
+  p->blocks25.clear();
+  double total = 0;
+  for (int s = 0; s < p->nshots; ++s) total += shot_bytes(p, s);
+  if (p->kind != SDT_EM25 || total < 250e6) {
+    p->blocks25.push_back({0, p->nshots, INT_MAX});
+    return;
+  }
+  for (int s = 0; s < p->nshots;) {
+    const int nz = p->hmodels[p->hshots[s].model].nz;
+    // a block keeps more planes than its bounds move in STEPS25 steps
+    const int nb = shot_bytes(p, s) < 250e6 ? 1
+                   : (int)std::min((double)(nz / (2 * STEPS25)), std::ceil(shot_bytes(p, s) / PLANES25_BYTES));
+    if (nb > 1) {
+      for (int b = 0; b < nb; ++b)
+        p->blocks25.push_back({s, s + 1, b == nb - 1 ? INT_MAX : (int)((long long)nz * (b + 1) / nb)});
+      ++s;
+      continue;
+    }
+    int e = s;
+    for (double sum = 0; e < p->nshots && (e == s || sum + shot_bytes(p, e) <= SHOTS25_BYTES); ++e)
+      sum += shot_bytes(p, e);
+    p->blocks25.push_back({s, e, INT_MAX});
+    s = e;
+  }
+}
+
+// One pass (0 stress / H, 1 velocity / E) of step base + rel over n items of
+// the 2.5-D work list from item `off`.
 template <typename T>
-void launch_one25(Plan* p, hipStream_t st, int rel, int which) {
-  const int n = p->nwork;
+void launch_pass25(Plan* p, hipStream_t st, int rel, int pass, int off, int n) {
   const dim3 grd((n + 7) / 8 * 8), blk(NT25);
-  if (which == 2) {
-    if (p->maxrec > 0)
-      hipLaunchKernelGGL(k_gather<T>, dim3((p->maxrec + 63) / 64, p->nshots), dim3(64), 0, st, p->dmodels,
-                         p->dshots, p->nshots, p->ncomp, p->dbase, rel);
-  } else if (p->kind == SDT_ELASTIC25) {
-    if (which == 0)
-      hipLaunchKernelGGL(k_el25_stress<T>, grd, blk, 0, st, p->dmodels, p->dshots, p->dwork, n, p->dbase, rel);
+  const int4* w = p->dwork + off;
+  if (p->kind == SDT_ELASTIC25) {
+    if (pass == 0)
+      hipLaunchKernelGGL(k_el25_stress<T>, grd, blk, 0, st, p->dmodels, p->dshots, w, n, p->dbase, rel);
     else
-      hipLaunchKernelGGL(k_el25_vel<T>, grd, blk, 0, st, p->dmodels, p->dshots, p->dwork, n, p->dbase, rel);
-  } else if (which == 0) {
-    hipLaunchKernelGGL(k_em25_h<T>, grd, blk, 0, st, p->dmodels, p->dshots, p->dwork, n);
+      hipLaunchKernelGGL(k_el25_vel<T>, grd, blk, 0, st, p->dmodels, p->dshots, w, n, p->dbase, rel);
+  } else if (pass == 0) {
+    hipLaunchKernelGGL(k_em25_h<T>, grd, blk, 0, st, p->dmodels, p->dshots, w, n);
   } else {
-    hipLaunchKernelGGL(k_em25_e<T>, grd, blk, 0, st, p->dmodels, p->dshots, p->dwork, n, p->dbase, rel);
+    hipLaunchKernelGGL(k_em25_e<T>, grd, blk, 0, st, p->dmodels, p->dshots, w, n, p->dbase, rel);
+  }
+}
+
+// Receiver samples of step base + rel of shots s0..s1-1 on planes k0..k1-1.
+template <typename T>
+void launch_gather25(Plan* p, hipStream_t st, int rel, int s0, int s1, int k0, int k1) {
+  int nrec = 0;
+  for (int s = s0; s < s1; ++s)
+    if (p->reck[s].first < k1 && p->reck[s].second >= k0) nrec = std::max(nrec, p->hshots[s].nrec);
+  if (nrec > 0)
+    hipLaunchKernelGGL(k_gather<T>, dim3((nrec + 63) / 64, s1 - s0), dim3(64), 0, st, p->dmodels, p->dshots,
+                       s0, p->ncomp, p->dbase, rel, k0, k1);
+}
+
+template <typename T>
+void launch_steps25(Plan* p, hipStream_t st, int n) {
+  const bool one = p->blocks25.size() == 1;
+  const int runs = one ? 1 : (n + STEPS25 - 1) / STEPS25;  // of nearly equal length
+  for (int q = 0; q < runs; ++q) {
+    const int r0 = (int)((long long)n * q / runs), r1 = (int)((long long)n * (q + 1) / runs);
+    for (size_t b = 0; b < p->blocks25.size(); ++b) {
+      const Block25& B = p->blocks25[b];
+      const int i0 = p->item25[B.s0], ni = p->item25[B.s1] - i0;
+      const bool first = b == 0 || p->blocks25[b - 1].s1 <= B.s0;  // of its shots
+      for (int r = r0; r < r1; ++r) {
+        int off = i0, m = ni, k0 = 0, k1 = INT_MAX;
+        if (!first || B.top != INT_MAX) {  // planes k0 .. k1-1 of one shot
+          const int nz = p->hmodels[p->hshots[B.s0].model].nz, per = ni / nz;
+          k0 = first ? 0 : p->blocks25[b - 1].top - (r - r0);
+          k1 = B.top == INT_MAX ? nz : B.top - (r - r0);
+          off += k0 * per;
+          m = (k1 - k0) * per;
+        }
+        launch_pass25<T>(p, st, r, 0, off, m);
+        launch_pass25<T>(p, st, r, 1, off, m);
+        launch_gather25<T>(p, st, r, B.s0, B.s1, k0, k1);
+      }
+    }
   }
 }
 
@@ -4127,7 +4226,13 @@ void launch_one25(Plan* p, hipStream_t st, int rel, int which) {
 // 2: receiver gather) of one step.
 template <typename T>
 void launch_one(Plan* p, hipStream_t st, int rel, int which) {
-  if (kind_3d(p->kind)) return launch_one25<T>(p, st, rel, which);
+  if (kind_3d(p->kind)) {
+    if (which == 2)
+      launch_gather25<T>(p, st, rel, 0, p->nshots, 0, INT_MAX);
+    else
+      launch_pass25<T>(p, st, rel, which, 0, p->nwork);
+    return;
+  }
   if (which == 2) return;  // the 2-D step kernels write their receiver samples themselves
   switch (p->kind * 2 + which) {
     case SDT_ELASTIC2 * 2:
@@ -4167,6 +4272,13 @@ void launch_step(Plan* p, hipStream_t st, int rel) {
 }
 
 void launch_steps(Plan* p, hipStream_t st, int n) {
+  if (kind_3d(p->kind)) {
+    if (p->prec == SDT_FP64)
+      launch_steps25<double>(p, st, n);
+    else
+      launch_steps25<float>(p, st, n);
+    return;
+  }
   for (int r = 0; r < n; ++r) {
     if (p->prec == SDT_FP64)
       launch_step<double>(p, st, r);
@@ -4561,7 +4673,10 @@ int stage_host(Plan* p, int kind, int prec, const sdt_model* models, int nmodels
     D.rxid = nullptr;
   }
   // work lists: (shot, x0, z0); all shots of one tile share blockIdx % 8 (XCD)
-  if (kind_3d(kind)) S.work = el25_work(p, least_rows);
+  if (kind_3d(kind)) {
+    S.work = el25_work(p, least_rows);
+    set_blocks25(p);
+  }
   if (pingpong(kind)) {
     default_shape(p);
     if (least_rows > p->el2_eh) {  // shorter lists for the fixed scratch
@@ -4592,7 +4707,8 @@ int stage_host(Plan* p, int kind, int prec, const sdt_model* models, int nmodels
 // check them against the grid, and build the receivers-by-row index of the
 // 2-D kinds: per shot rrow[nz + 1] then (column, index) pairs sorted by
 // (row, column).
-int stage_receivers(const Plan* p, Stage& S) {
+int stage_receivers(Plan* p, Stage& S) {
+  p->reck.assign(p->nshots, {INT_MAX, -1});
   S.rows_cols.clear();
   S.rows_cols.reserve((size_t)S.rows_cols_size);
   for (int s = 0; s < p->nshots; ++s) {
@@ -4607,6 +4723,7 @@ int stage_receivers(const Plan* p, Stage& S) {
       if (i < 0 || i >= M.nx || k < 0 || k >= M.nz || j < 0 || j >= M.ny)
         return fail(SDT_EINVAL, "shot " + std::to_string(s) + ": receiver " + std::to_string(r) +
                                     " outside the padded grid");
+      p->reck[s] = {std::min(p->reck[s].first, k), std::max(p->reck[s].second, k)};
     }
     if (S.rec_off[s] < 0) continue;
     std::vector<int> order(H.nrec);
