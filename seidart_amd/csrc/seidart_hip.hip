@@ -2405,14 +2405,23 @@ __global__ void k_em2_edges(const DModel* __restrict__ models, const DShot* __re
 
 // ===========================================================================
 // ELASTIC25: seismic25, legacy/fortran/seismicfdtd.f95:388-949
-// Two launches per step: stresses, then velocities.  A wavefront takes one
-// z plane k, 64 adjacent columns (lanes 1..EW25 are owned; lanes 0 and 63
-// only supply x neighbours, which travel by lane shuffles) and a chunk of
-// rows in y (rows25), which it walks with its y neighbours kept in registers.
-// The 2-D (y-invariant) coefficients of its columns are loaded once per
-// chunk; z neighbours are plain loads of the adjacent planes.  A block is one
-// wavefront.  Chunks end at the y-slab edges,
-// and a wavefront clear of every slab runs a body without memory variables.
+// Two launches per step: stresses, then velocities.  A wavefront (a block of
+// its own) takes one z plane k, 64 adjacent columns (lanes 1..EW25 are owned;
+// lanes 0 and 63 only supply x neighbours, which travel by DPP lane shifts) and
+// a chunk of rows in y (rows25), R rows at a time.  Chunks end at the y-slab
+// edges, and a wavefront clear of every slab runs a body without memory
+// variables.  z neighbours are plain loads of the adjacent planes.
+// What bounds it: on large grids the bytes (the second pass re-reads what the
+// first wrote; 832x96x432 FP32 moves 5.0 GB per step at 4.3 TB/s, a copy
+// reaches 4.9 .. 5.3), on small ones the latency of a row's loads.  So the loads
+// of a row group, C-PML memory included, are all issued before the first use,
+// and the stress pass reads the 33 y-invariant coefficients of its column from
+// LDS once per group.  Loading the memory variables after the wait for the
+// fields, with the next row's fields prefetched only where there are none, and
+// x neighbours by ds_bpermute, measured (us per step) 1302 against 1160 on
+// 832x96x432 FP32, 2402 against 2179 in FP64, 433 against 342 on 332x72x182
+// FP64, 177 against 135 in FP32, 86 against 68 on 171x57x95 FP64, 48 against 27
+// on 112x56x82 FP32.
 // psi slabs (per shot):
 //   x [nz][ny][2lx]: dvx_dx dvy_dx dvz_dx dsxx_dx dsxy_dx dsxz_dx
 //   y [nz][2ly][nx]: dvx_dy dvy_dy dvz_dy dsyy_dy dsxy_dy dsyz_dy
@@ -2468,24 +2477,40 @@ __device__ __forceinline__ A32<const T> cplane(const void* f, long nxy, int k) {
   return A32<const T>(static_cast<const T*>(f) + (long)k * nxy);
 }
 
-// waves per SIMD the register budget is sized for (FP32; FP64 takes 2)
-#ifndef SDT_EL25S_WAVES
-#define SDT_EL25S_WAVES 3
-#endif
-#ifndef SDT_EL25V_WAVES
-#define SDT_EL25V_WAVES 4
-#endif
-// the C-PML body of the stress pass with two rows of loads in flight too
-// (measured no faster: 1.312 against 1.310 ms per FP32 aniso25 step, at more
-// registers)
-#ifndef SDT_EL25_PF_PML
-#define SDT_EL25_PF_PML 0
-#endif
+// Rows whose loads a wavefront has in flight at once (stress, velocity), and
+// the wavefronts per SIMD that the register budgets are sized for.  Measured on
+// 832x96x432 (us per step): FP32 stress rows / waves 1 / 4 1160, 1 / 5 1187, 2 / 3
+// 1166, 2 / 4 1167; FP32 velocity 2 / 5 and 2 / 6 1160, 4 / 4 (spills) 1210;
+// FP64 stress 1 / 2 2213, 2 / 2 2179; FP64 velocity 1 / 4 2211, 2 / 3 2179, 2 / 4
+// (spills) 2271.  On 112x56x82 FP32 one stress row 27.2, two 29.2.
+template <typename T>
+constexpr int RS25 = sizeof(T) == 4 ? 1 : 2;
+constexpr int RV25 = 2;
+template <typename T>
+constexpr int WS25 = sizeof(T) == 4 ? 4 : 2;
+template <typename T>
+constexpr int WV25 = sizeof(T) == 4 ? 5 : 3;
+
+// C-PML memory of an elastic 2.5-D pass on one plane: arrays q .. q + 2 of each
+// axis (q = 0 stress, 3 velocity).  The bases are wave-uniform, the offsets
+// 32-bit: x[j * 2lx + xs], y[slab row * nx + i], z[j * nx + i].
+template <typename T>
+struct PsiEl25 {
+  const A32<T> x0, x1, x2, y0, y1, y2, z0, z1, z2;
+  __device__ __forceinline__ PsiEl25(void* psi, const Slab3& L, int q, int nx, int ny, int lx, int ly, int k, int zs)
+      : x0((T*)psi + L.bx + q * L.SX + (long)k * ny * 2 * lx), x1((T*)psi + L.bx + (q + 1) * L.SX + (long)k * ny * 2 * lx),
+        x2((T*)psi + L.bx + (q + 2) * L.SX + (long)k * ny * 2 * lx),
+        y0((T*)psi + L.by + q * L.SY + (long)k * 2 * ly * nx), y1((T*)psi + L.by + (q + 1) * L.SY + (long)k * 2 * ly * nx),
+        y2((T*)psi + L.by + (q + 2) * L.SY + (long)k * 2 * ly * nx),
+        z0((T*)psi + L.bz + q * L.SZ + (long)zs * ny * nx), z1((T*)psi + L.bz + (q + 1) * L.SZ + (long)zs * ny * nx),
+        z2((T*)psi + L.bz + (q + 2) * L.SZ + (long)zs * ny * nx) {}
+};
 
 template <typename T, bool PML>
 __device__ __forceinline__ void el25_stress_tile(const DModel* __restrict__ models,
                                               const DShot* __restrict__ shots, const int4 wv,
                                               const int it, T* __restrict__ cs) {
+  constexpr int R = RS25<T>;
   const int s = __builtin_amdgcn_readfirstlane(wv.x);
   const DShot& S = shots[s];
   const DModel& M = models[S.model];
@@ -2501,33 +2526,28 @@ __device__ __forceinline__ void el25_stress_tile(const DModel* __restrict__ mode
   const uint32_t p = (uint32_t)k * nx + ic;
   const T idx = T(1.0 / M.dx), idy = T(1.0 / M.dy), idz = T(1.0 / M.dz), dt = T(M.dt);
   const int lx = M.lx, ly = M.ly, lz = M.lz;
+  // a chunk lies inside a y slab or outside both
   const bool inx = PML && incol && in_slab(i, nx, lx), inz = PML && in_slab(k, nz, lz);
+  const bool iny = PML && in_slab(j0, ny, ly);
   const Prof<T> P(&M.prof[0][0]);
-  gcptr<T> iky = P[6 + PK], ay = P[6 + PA], by = P[6 + PB];
-  gcptr<T> ikyh = P[6 + PKH], ayh = P[6 + PAH], byh = P[6 + PBH];
+  const auto iky = kp<T>(M.prof[1][PK]), ay = kp<T>(M.prof[1][PA]), by = kp<T>(M.prof[1][PB]);
+  const auto ikyh = kp<T>(M.prof[1][PKH]), ayh = kp<T>(M.prof[1][PAH]), byh = kp<T>(M.prof[1][PBH]);
   const T bx_i = P[PB][ic], ax_i = P[PA][ic], ikx_i = P[PK][ic];
   const T bxh_i = P[PBH][ic], axh_i = P[PAH][ic], ikxh_i = P[PKH][ic];
-  const T bz_k = P[12 + PB][k], az_k = P[12 + PA][k], ikz_k = P[12 + PK][k];
-  const T bzh_k = P[12 + PBH][k], azh_k = P[12 + PAH][k], ikzh_k = P[12 + PKH][k];
+  const T bz_k = kp<T>(M.prof[2][PB])[k], az_k = kp<T>(M.prof[2][PA])[k], ikz_k = kp<T>(M.prof[2][PK])[k];
+  const T bzh_k = kp<T>(M.prof[2][PBH])[k], azh_k = kp<T>(M.prof[2][PAH])[k], ikzh_k = kp<T>(M.prof[2][PKH])[k];
   // loop ranges of the four legacy stress loops (seismicfdtd.f95:617, :677, :728, :771)
   const bool p1 = own && k >= 1 && i <= nx - 2, p2 = own && k >= 1 && i >= 1;
   const bool p3 = own && k <= nz - 2 && i >= 1, p4 = own && k <= nz - 2 && i <= nx - 2;
   // The 33 coefficients of the four loops at this column and plane do not
   // change along y: they are loaded once per work item into LDS, one slot per
-  // thread that only that thread reads back, and read where each loop uses
-  // them (volatile, so they are not held in registers for the whole walk);
-  // the registers go to a second set of row loads instead.  cs: the block's
-  // 33 * NT25 LDS slots.
+  // thread that only that thread reads back, and read once per row group where
+  // each loop uses them (volatile, so they are not held in registers for the
+  // whole walk).  cs: the block's 33 * NT25 LDS slots.
   {
     T* w = cs + threadIdx.x;
 #pragma unroll
-    for (int q = 0; q < 15; ++q) w[q * NT25] = p1 ? A32<const T>(M.coef[q])[p] : T(0);
-#pragma unroll
-    for (int q = 0; q < 6; ++q) {
-      w[(15 + q) * NT25] = p2 ? A32<const T>(M.coef[15 + q])[p] : T(0);
-      w[(21 + q) * NT25] = p3 ? A32<const T>(M.coef[21 + q])[p] : T(0);
-      w[(27 + q) * NT25] = p4 ? A32<const T>(M.coef[27 + q])[p] : T(0);
-    }
+    for (int q = 0; q < 33; ++q) w[q * NT25] = A32<const T>(M.coef[q])[p];
   }
   // coefficient q at C[q * NT25], read through an LDS pointer (ds_read)
   const __attribute__((address_space(3))) volatile T* C =
@@ -2542,182 +2562,213 @@ __device__ __forceinline__ void el25_stress_tile(const DModel* __restrict__ mode
   const A32<T> SXX = plane<T>(S.f[3], nxy, k), SYY = plane<T>(S.f[4], nxy, k);
   const A32<T> SZZ = plane<T>(S.f[5], nxy, k), SXY = plane<T>(S.f[6], nxy, k);
   const A32<T> SXZ = plane<T>(S.f[7], nxy, k), SYZ = plane<T>(S.f[8], nxy, k);
-  auto psi = mp<T>(S.psi);
-  const Slab3 L(nx, ny, nz, lx, ly, lz);
   const int xs = inx ? slab_pos(i, nx, lx) : 0, zs = inz ? slab_pos(k, nz, lz) : 0;
+  const PsiEl25<T> W(S.psi, Slab3(nx, ny, nz, lx, ly, lz), 0, nx, ny, lx, ly, k, zs);
 
-  // y window of the velocities: rows j-1 (m), j (c)
-  const uint32_t r0 = (uint32_t)j0 * nx + ic;
-  T vxm = 0, vym = 0, vzm = 0;
-  if (j0 >= 1) { vxm = VX[r0 - nx]; vym = VY[r0 - nx]; vzm = VZ[r0 - nx]; }
-  T vxc = VX[r0], vyc = VY[r0], vzc = VZ[r0];
-
-  // the loads of row j: velocities of row j+1 (n) and of planes k-1 (d) and
-  // k+1 (u), the row's stresses (rows past the last are clamped in bounds)
-  struct RowLd { T vxn, vyn, vzn, vxd, vyd, vzd, vxu, vyu, vzu, sxx, syy, szz, sxy, sxz, syz; };
-  auto load_row = [&](int j) {
-    RowLd R;
-    const uint32_t c = (uint32_t)(j < ny ? j : ny - 1) * nx + ic;
-    const uint32_t cn = j + 1 < ny ? c + nx : c;
-    R.vxn = VX[cn]; R.vyn = VY[cn]; R.vzn = VZ[cn];
-    R.vxd = VXD[c]; R.vyd = VYD[c]; R.vzd = VZD[c];
-    R.vxu = VXU[c]; R.vyu = VYU[c]; R.vzu = VZU[c];
-    R.sxx = SXX[c]; R.syy = SYY[c]; R.szz = SZZ[c];
-    R.sxy = SXY[c]; R.sxz = SXZ[c]; R.syz = SYZ[c];
-    return R;
-  };
-  auto row = [&](const int j, const RowLd& R) {
-    const uint32_t c = (uint32_t)j * nx + ic;
-    const T vxn = R.vxn, vyn = R.vyn, vzn = R.vzn;      // row j+1 (n)
-    const T vxd = R.vxd, vyd = R.vyd, vzd = R.vzd;      // plane k-1 (d)
-    const T vxu = R.vxu, vyu = R.vyu, vzu = R.vzu;      // plane k+1 (u)
-    const T sxx0 = R.sxx, syy0 = R.syy, szz0 = R.szz, sxy0 = R.sxy, sxz0 = R.sxz, syz0 = R.syz;
-    const T vxe = lane_next(vxc), vye = lane_next(vyc), vze = lane_next(vzc);  // i+1 (e)
-    const T vxw = lane_prev(vxc), vyw = lane_prev(vyc), vzw = lane_prev(vzc);  // i-1 (w)
-    const bool iny = PML && in_slab(j, ny, ly);
-    const long ox = L.bx + ((long)k * ny + j) * 2 * lx + xs;
-    const long oy = L.by + ((long)k * 2 * ly + (iny ? slab_pos(j, ny, ly) : 0)) * nx + ic;
-    const long oz = L.bz + ((long)zs * ny + j) * nx + ic;
+  // velocity rows jb-1 .. jb+R: [0], [1] carried from group to group
+  T vx[R + 2], vy[R + 2], vz[R + 2];
+  {
+    const uint32_t m = (uint32_t)max(j0 - 1, 0) * nx + ic, c = (uint32_t)j0 * nx + ic;
+    vx[0] = VX[m]; vy[0] = VY[m]; vz[0] = VZ[m];
+    vx[1] = VX[c]; vy[1] = VY[c]; vz[1] = VZ[c];
+  }
+#pragma unroll 1
+  for (int jb = j0; jb < j1; jb += R) {
+    T vxd[R], vyd[R], vzd[R], vxu[R], vyu[R], vzu[R];
+    T sxx[R], syy[R], szz[R], sxy[R], sxz[R], syz[R];
+    T mxx[R], myx[R], mzx[R], mxy[R], myy[R], mzy[R], mxz[R], myz[R], mzz[R];
+    uint32_t c[R];
+    // every load of the R rows before the first use (rows past the chunk
+    // reload its last row; velocities the row below it)
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const uint32_t n = (uint32_t)min(jb + q + 1, min(j1, ny - 1)) * nx + ic;
+      c[q] = (uint32_t)min(jb + q, j1 - 1) * nx + ic;
+      vx[q + 2] = VX[n]; vy[q + 2] = VY[n]; vz[q + 2] = VZ[n];
+      vxd[q] = VXD[c[q]]; vyd[q] = VYD[c[q]]; vzd[q] = VZD[c[q]];
+      vxu[q] = VXU[c[q]]; vyu[q] = VYU[c[q]]; vzu[q] = VZU[c[q]];
+      sxx[q] = SXX[c[q]]; syy[q] = SYY[c[q]]; szz[q] = SZZ[c[q]];
+      sxy[q] = SXY[c[q]]; sxz[q] = SXZ[c[q]]; syz[q] = SYZ[c[q]];
+    }
     // velocity-derivative memory variables (shared by all four loops: A1)
-    T mxx = 0, myx = 0, mzx = 0, mxy = 0, myy = 0, mzy = 0, mxz = 0, myz = 0, mzz = 0;
-    if (inx) { mxx = psi[ox]; myx = psi[ox + L.SX]; mzx = psi[ox + 2 * L.SX]; }
-    if (iny && incol) { mxy = psi[oy]; myy = psi[oy + L.SY]; mzy = psi[oy + 2 * L.SY]; }
-    if (inz && incol) { mxz = psi[oz]; myz = psi[oz + L.SZ]; mzz = psi[oz + 2 * L.SZ]; }
-
+    if (PML && iny) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const uint32_t o = (uint32_t)slab_pos(min(jb + q, j1 - 1), ny, ly) * nx + ic;
+        mxy[q] = W.y0[o]; myy[q] = W.y1[o]; mzy[q] = W.y2[o];
+      }
+    }
+    if (PML && inz) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) { mxz[q] = W.z0[c[q]]; myz[q] = W.z1[c[q]]; mzz[q] = W.z2[c[q]]; }
+    }
+    if (PML && inx) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const uint32_t o = (uint32_t)min(jb + q, j1 - 1) * 2 * lx + xs;
+        mxx[q] = W.x0[o]; myx[q] = W.x1[o]; mzx[q] = W.x2[o];
+      }
+    }
     // loop 1: sigma xx, yy, zz (seismicfdtd.f95:617-674)
-    if (p1 && j >= 1) {
-      T dvx_dx = (vxe - vxc) * idx, dvy_dx = (vye - vyc) * idx, dvz_dx = (vze - vzc) * idx;
-      T dvy_dy = (vyc - vym) * idy, dvx_dy = (vxc - vxm) * idy, dvz_dy = (vzc - vzm) * idy;
-      T dvz_dz = (vzc - vzd) * idz, dvx_dz = (vxc - vxd) * idz, dvy_dz = (vyc - vyd) * idz;
-      if (inx) {
-        mxx = bxh_i * mxx + axh_i * dvx_dx; myx = bxh_i * myx + axh_i * dvy_dx; mzx = bxh_i * mzx + axh_i * dvz_dx;
-        dvx_dx = dvx_dx * ikxh_i + mxx; dvy_dx = dvy_dx * ikxh_i + myx; dvz_dx = dvz_dx * ikxh_i + mzx;
-      }
-      if (iny) {
-        const T b = by[j], a = ay[j], ik = iky[j];
-        myy = b * myy + a * dvy_dy; mxy = b * mxy + a * dvx_dy; mzy = b * mzy + a * dvz_dy;
-        dvy_dy = dvy_dy * ik + myy; dvx_dy = dvx_dy * ik + mxy; dvz_dy = dvz_dy * ik + mzy;
-      }
-      if (inz) {
-        mzz = bz_k * mzz + az_k * dvz_dz; mxz = bz_k * mxz + az_k * dvx_dz; myz = bz_k * myz + az_k * dvy_dz;
-        dvz_dz = dvz_dz * ikz_k + mzz; dvx_dz = dvx_dz * ikz_k + mxz; dvy_dz = dvy_dz * ikz_k + myz;
-      }
+    {
       const T c0 = C[0], c1 = C[1 * NT25], c2 = C[2 * NT25], c3 = C[3 * NT25], c4 = C[4 * NT25];
       const T c5 = C[5 * NT25], c6 = C[6 * NT25], c7 = C[7 * NT25], c8 = C[8 * NT25], c9 = C[9 * NT25];
       const T c10 = C[10 * NT25], c11 = C[11 * NT25], c12 = C[12 * NT25], c13 = C[13 * NT25];
       const T c14 = C[14 * NT25];
-      SXX[c] = sxx0 + (c0 * dvx_dx + c1 * dvy_dy + c2 * dvz_dz + c3 * (dvy_dz + dvz_dy) +
-                       c4 * (dvx_dz + dvz_dx) + c5 * (dvx_dy + dvz_dy)) * dt;  // A3 (c16)
-      SYY[c] = syy0 + (c1 * dvx_dx + c6 * dvy_dy + c7 * dvz_dz + c8 * (dvy_dz + dvz_dy) +
-                       c9 * (dvx_dz + dvz_dx) + c10 * (dvy_dx + dvx_dy)) * dt;
-      SZZ[c] = szz0 + (c2 * dvx_dx + c7 * dvy_dy + c11 * dvz_dz + c12 * (dvy_dz + dvz_dy) +
-                       c13 * (dvx_dz + dvz_dx) + c14 * (dvy_dx + dvx_dy)) * dt;
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const int j = jb + q;
+        const T vxc = vx[q + 1], vyc = vy[q + 1], vzc = vz[q + 1];
+        const T vxe = dpp_next(vxc), vye = dpp_next(vyc), vze = dpp_next(vzc);  // i+1
+        if (p1 && j >= 1 && j < j1) {
+          T dvx_dx = (vxe - vxc) * idx, dvy_dx = (vye - vyc) * idx, dvz_dx = (vze - vzc) * idx;
+          T dvy_dy = (vyc - vy[q]) * idy, dvx_dy = (vxc - vx[q]) * idy, dvz_dy = (vzc - vz[q]) * idy;
+          T dvz_dz = (vzc - vzd[q]) * idz, dvx_dz = (vxc - vxd[q]) * idz, dvy_dz = (vyc - vyd[q]) * idz;
+          if (PML && inx) {
+            mxx[q] = bxh_i * mxx[q] + axh_i * dvx_dx; myx[q] = bxh_i * myx[q] + axh_i * dvy_dx; mzx[q] = bxh_i * mzx[q] + axh_i * dvz_dx;
+            dvx_dx = dvx_dx * ikxh_i + mxx[q]; dvy_dx = dvy_dx * ikxh_i + myx[q]; dvz_dx = dvz_dx * ikxh_i + mzx[q];
+          }
+          if (PML && iny) {
+            const T b = by[j], a = ay[j], ik = iky[j];
+            myy[q] = b * myy[q] + a * dvy_dy; mxy[q] = b * mxy[q] + a * dvx_dy; mzy[q] = b * mzy[q] + a * dvz_dy;
+            dvy_dy = dvy_dy * ik + myy[q]; dvx_dy = dvx_dy * ik + mxy[q]; dvz_dy = dvz_dy * ik + mzy[q];
+          }
+          if (PML && inz) {
+            mzz[q] = bz_k * mzz[q] + az_k * dvz_dz; mxz[q] = bz_k * mxz[q] + az_k * dvx_dz; myz[q] = bz_k * myz[q] + az_k * dvy_dz;
+            dvz_dz = dvz_dz * ikz_k + mzz[q]; dvx_dz = dvx_dz * ikz_k + mxz[q]; dvy_dz = dvy_dz * ikz_k + myz[q];
+          }
+          SXX[c[q]] = sxx[q] + (c0 * dvx_dx + c1 * dvy_dy + c2 * dvz_dz + c3 * (dvy_dz + dvz_dy) +
+                                c4 * (dvx_dz + dvz_dx) + c5 * (dvx_dy + dvz_dy)) * dt;  // A3 (c16)
+          SYY[c[q]] = syy[q] + (c1 * dvx_dx + c6 * dvy_dy + c7 * dvz_dz + c8 * (dvy_dz + dvz_dy) +
+                                c9 * (dvx_dz + dvz_dx) + c10 * (dvy_dx + dvx_dy)) * dt;
+          SZZ[c[q]] = szz[q] + (c2 * dvx_dx + c7 * dvy_dy + c11 * dvz_dz + c12 * (dvy_dz + dvz_dy) +
+                                c13 * (dvx_dz + dvz_dx) + c14 * (dvy_dx + dvx_dy)) * dt;
+        }
+      }
     }
     // loop 2: sigma xy (seismicfdtd.f95:677-725); dvz_dx and dvx_dz get no correction
-    if (p2 && j <= ny - 2) {
-      T dvx_dx = (vxc - vxw) * idx, dvy_dx = (vyc - vyw) * idx, dvz_dx = (vzc - vzw) * idx;
-      T dvy_dy = (vyn - vyc) * idy, dvx_dy = (vxn - vxc) * idy, dvz_dy = (vzn - vzc) * idy;
-      T dvz_dz = (vzc - vzd) * idz, dvx_dz = (vxc - vxd) * idz, dvy_dz = (vyc - vyd) * idz;
-      if (inx) {
-        mxx = bx_i * mxx + ax_i * dvx_dx; myx = bx_i * myx + ax_i * dvy_dx; mzx = bx_i * mzx + ax_i * dvz_dx;
-        dvx_dx = dvx_dx * ikx_i + mxx; dvy_dx = dvy_dx * ikx_i + myx;
+    {
+      const T c0 = C[15 * NT25], c1 = C[16 * NT25], c2 = C[17 * NT25], c3 = C[18 * NT25], c4 = C[19 * NT25], c5 = C[20 * NT25];
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const int j = jb + q;
+        const T vxc = vx[q + 1], vyc = vy[q + 1], vzc = vz[q + 1];
+        const T vxw = dpp_prev(vxc), vyw = dpp_prev(vyc), vzw = dpp_prev(vzc);  // i-1
+        if (p2 && j <= ny - 2 && j < j1) {
+          T dvx_dx = (vxc - vxw) * idx, dvy_dx = (vyc - vyw) * idx, dvz_dx = (vzc - vzw) * idx;
+          T dvy_dy = (vy[q + 2] - vyc) * idy, dvx_dy = (vx[q + 2] - vxc) * idy, dvz_dy = (vz[q + 2] - vzc) * idy;
+          T dvz_dz = (vzc - vzd[q]) * idz, dvx_dz = (vxc - vxd[q]) * idz, dvy_dz = (vyc - vyd[q]) * idz;
+          if (PML && inx) {
+            mxx[q] = bx_i * mxx[q] + ax_i * dvx_dx; myx[q] = bx_i * myx[q] + ax_i * dvy_dx; mzx[q] = bx_i * mzx[q] + ax_i * dvz_dx;
+            dvx_dx = dvx_dx * ikx_i + mxx[q]; dvy_dx = dvy_dx * ikx_i + myx[q];
+          }
+          if (PML && iny) {
+            const T b = byh[j], a = ayh[j], ik = ikyh[j];
+            myy[q] = b * myy[q] + a * dvy_dy; mxy[q] = b * mxy[q] + a * dvx_dy; mzy[q] = b * mzy[q] + a * dvz_dy;
+            dvy_dy = dvy_dy * ik + myy[q]; dvx_dy = dvx_dy * ik + mxy[q]; dvz_dy = dvz_dy * ik + mzy[q];
+          }
+          if (PML && inz) {
+            mzz[q] = bzh_k * mzz[q] + azh_k * dvz_dz; mxz[q] = bzh_k * mxz[q] + azh_k * dvx_dz; myz[q] = bzh_k * myz[q] + azh_k * dvy_dz;
+            dvz_dz = dvz_dz * ikzh_k + mzz[q]; dvy_dz = dvy_dz * ikzh_k + myz[q];
+          }
+          SXY[c[q]] = sxy[q] + (c0 * dvx_dx + c1 * dvy_dy + c2 * dvz_dz + c3 * (dvz_dy + dvy_dz) +
+                                c4 * (dvz_dx + dvx_dz) + c5 * (dvy_dx + dvx_dy)) * dt;
+        }
       }
-      if (iny) {
-        const T b = byh[j], a = ayh[j], ik = ikyh[j];
-        myy = b * myy + a * dvy_dy; mxy = b * mxy + a * dvx_dy; mzy = b * mzy + a * dvz_dy;
-        dvy_dy = dvy_dy * ik + myy; dvx_dy = dvx_dy * ik + mxy; dvz_dy = dvz_dy * ik + mzy;
-      }
-      if (inz) {
-        mzz = bzh_k * mzz + azh_k * dvz_dz; mxz = bzh_k * mxz + azh_k * dvx_dz; myz = bzh_k * myz + azh_k * dvy_dz;
-        dvz_dz = dvz_dz * ikzh_k + mzz; dvy_dz = dvy_dz * ikzh_k + myz;
-      }
-      const __attribute__((address_space(3))) volatile T* K = C + 15 * NT25;
-      SXY[c] = sxy0 + (K[0] * dvx_dx + K[NT25] * dvy_dy + K[2 * NT25] * dvz_dz + K[3 * NT25] * (dvz_dy + dvy_dz) +
-                       K[4 * NT25] * (dvz_dx + dvx_dz) + K[5 * NT25] * (dvy_dx + dvx_dy)) * dt;
     }
     // loop 3: sigma xz (seismicfdtd.f95:728-768)
-    if (p3 && j >= 1) {
-      T dvx_dx = (vxc - vxw) * idx, dvy_dx = (vyc - vyw) * idx, dvz_dx = (vzc - vzw) * idx;
-      T dvy_dy = (vyc - vym) * idy, dvz_dy = (vzc - vzm) * idy, dvx_dy = (vxc - vxm) * idy;
-      T dvz_dz = (vzu - vzc) * idz, dvx_dz = (vxu - vxc) * idz, dvy_dz = (vyu - vyc) * idz;
-      if (inx) {
-        mxx = bx_i * mxx + ax_i * dvx_dx; myx = bx_i * myx + ax_i * dvy_dx; mzx = bx_i * mzx + ax_i * dvz_dx;
-        dvx_dx = dvx_dx * ikx_i + mxx; dvy_dx = dvy_dx * ikx_i + myx; dvz_dx = dvz_dx * ikx_i + mzx;
+    {
+      const T c0 = C[21 * NT25], c1 = C[22 * NT25], c2 = C[23 * NT25], c3 = C[24 * NT25], c4 = C[25 * NT25], c5 = C[26 * NT25];
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const int j = jb + q;
+        const T vxc = vx[q + 1], vyc = vy[q + 1], vzc = vz[q + 1];
+        const T vxw = dpp_prev(vxc), vyw = dpp_prev(vyc), vzw = dpp_prev(vzc);
+        if (p3 && j >= 1 && j < j1) {
+          T dvx_dx = (vxc - vxw) * idx, dvy_dx = (vyc - vyw) * idx, dvz_dx = (vzc - vzw) * idx;
+          T dvy_dy = (vyc - vy[q]) * idy, dvz_dy = (vzc - vz[q]) * idy, dvx_dy = (vxc - vx[q]) * idy;
+          T dvz_dz = (vzu[q] - vzc) * idz, dvx_dz = (vxu[q] - vxc) * idz, dvy_dz = (vyu[q] - vyc) * idz;
+          if (PML && inx) {
+            mxx[q] = bx_i * mxx[q] + ax_i * dvx_dx; myx[q] = bx_i * myx[q] + ax_i * dvy_dx; mzx[q] = bx_i * mzx[q] + ax_i * dvz_dx;
+            dvx_dx = dvx_dx * ikx_i + mxx[q]; dvy_dx = dvy_dx * ikx_i + myx[q]; dvz_dx = dvz_dx * ikx_i + mzx[q];
+          }
+          if (PML && iny) {
+            const T b = by[j], a = ay[j], ik = iky[j];
+            myy[q] = b * myy[q] + a * dvy_dy; mxy[q] = b * mxy[q] + a * dvx_dy; mzy[q] = b * mzy[q] + a * dvz_dy;
+            dvy_dy = dvy_dy * ik + myy[q]; dvx_dy = dvx_dy * ik + mxy[q]; dvz_dy = dvz_dy * ik + mzy[q];
+          }
+          if (PML && inz) {
+            mzz[q] = bzh_k * mzz[q] + azh_k * dvz_dz; mxz[q] = bzh_k * mxz[q] + azh_k * dvx_dz; myz[q] = bzh_k * myz[q] + azh_k * dvy_dz;
+            dvz_dz = dvz_dz * ikzh_k + mzz[q]; dvx_dz = dvx_dz * ikzh_k + mxz[q]; dvy_dz = dvy_dz * ikzh_k + myz[q];
+          }
+          SXZ[c[q]] = sxz[q] + (c0 * dvx_dx + c1 * dvy_dy + c2 * dvz_dz + c3 * (dvx_dz + dvz_dx) +
+                                c4 * (dvx_dz + dvz_dx) + c5 * (dvx_dy + dvy_dx)) * dt;  // A3 (c45)
+        }
       }
-      if (iny) {
-        const T b = by[j], a = ay[j], ik = iky[j];
-        myy = b * myy + a * dvy_dy; mxy = b * mxy + a * dvx_dy; mzy = b * mzy + a * dvz_dy;
-        dvy_dy = dvy_dy * ik + myy; dvx_dy = dvx_dy * ik + mxy; dvz_dy = dvz_dy * ik + mzy;
-      }
-      if (inz) {
-        mzz = bzh_k * mzz + azh_k * dvz_dz; mxz = bzh_k * mxz + azh_k * dvx_dz; myz = bzh_k * myz + azh_k * dvy_dz;
-        dvz_dz = dvz_dz * ikzh_k + mzz; dvx_dz = dvx_dz * ikzh_k + mxz; dvy_dz = dvy_dz * ikzh_k + myz;
-      }
-      const __attribute__((address_space(3))) volatile T* K = C + 21 * NT25;
-      SXZ[c] = sxz0 + (K[0] * dvx_dx + K[NT25] * dvy_dy + K[2 * NT25] * dvz_dz + K[3 * NT25] * (dvx_dz + dvz_dx) +
-                       K[4 * NT25] * (dvx_dz + dvz_dx) + K[5 * NT25] * (dvx_dy + dvy_dx)) * dt;  // A3 (c45)
     }
     // loop 4: sigma yz (seismicfdtd.f95:771-813)
-    if (p4 && j <= ny - 2) {
-      T dvx_dx = (vxe - vxc) * idx, dvy_dx = (vye - vyc) * idx, dvz_dx = (vze - vzc) * idx;
-      T dvy_dy = (vyn - vyc) * idy, dvx_dy = (vxn - vxc) * idy, dvz_dy = (vzn - vzc) * idy;
-      T dvz_dz = (vzu - vzc) * idz, dvx_dz = (vxu - vxc) * idz, dvy_dz = (vyu - vyc) * idz;
-      if (inx) {
-        mxx = bxh_i * mxx + axh_i * dvx_dx; myx = bxh_i * myx + axh_i * dvy_dx; mzx = bxh_i * mzx + axh_i * dvz_dx;
-        dvx_dx = dvx_dx * ikxh_i + mxx; dvy_dx = dvy_dx * ikxh_i + myx; dvz_dx = dvz_dx * ikxh_i + mzx;
+    {
+      const T c0 = C[27 * NT25], c1 = C[28 * NT25], c2 = C[29 * NT25], c3 = C[30 * NT25], c4 = C[31 * NT25], c5 = C[32 * NT25];
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const int j = jb + q;
+        const T vxc = vx[q + 1], vyc = vy[q + 1], vzc = vz[q + 1];
+        const T vxe = dpp_next(vxc), vye = dpp_next(vyc), vze = dpp_next(vzc);
+        if (p4 && j <= ny - 2 && j < j1) {
+          T dvx_dx = (vxe - vxc) * idx, dvy_dx = (vye - vyc) * idx, dvz_dx = (vze - vzc) * idx;
+          T dvy_dy = (vy[q + 2] - vyc) * idy, dvx_dy = (vx[q + 2] - vxc) * idy, dvz_dy = (vz[q + 2] - vzc) * idy;
+          T dvz_dz = (vzu[q] - vzc) * idz, dvx_dz = (vxu[q] - vxc) * idz, dvy_dz = (vyu[q] - vyc) * idz;
+          if (PML && inx) {
+            mxx[q] = bxh_i * mxx[q] + axh_i * dvx_dx; myx[q] = bxh_i * myx[q] + axh_i * dvy_dx; mzx[q] = bxh_i * mzx[q] + axh_i * dvz_dx;
+            dvx_dx = dvx_dx * ikxh_i + mxx[q]; dvy_dx = dvy_dx * ikxh_i + myx[q]; dvz_dx = dvz_dx * ikxh_i + mzx[q];
+          }
+          if (PML && iny) {
+            const T b = byh[j], a = ayh[j], ik = ikyh[j];
+            myy[q] = b * myy[q] + a * dvy_dy; mxy[q] = b * mxy[q] + a * dvx_dy; mzy[q] = b * mzy[q] + a * dvz_dy;
+            dvy_dy = dvy_dy * ik + myy[q]; dvx_dy = dvx_dy * ik + mxy[q]; dvz_dy = dvz_dy * ik + mzy[q];
+          }
+          if (PML && inz) {
+            mzz[q] = bzh_k * mzz[q] + azh_k * dvz_dz; mxz[q] = bzh_k * mxz[q] + azh_k * dvx_dz; myz[q] = bzh_k * myz[q] + azh_k * dvy_dz;
+            dvz_dz = dvz_dz * ikzh_k + mzz[q]; dvx_dz = dvx_dz * ikzh_k + mxz[q]; dvy_dz = dvy_dz * ikzh_k + myz[q];
+          }
+          SYZ[c[q]] = syz[q] + (c0 * dvx_dx + c1 * dvy_dy + c2 * dvz_dz + c3 * (dvy_dz + dvz_dy) +
+                                c4 * (dvx_dz + dvz_dx) + c5 * (dvy_dx + dvx_dy)) * dt;
+        }
       }
-      if (iny) {
-        const T b = byh[j], a = ayh[j], ik = ikyh[j];
-        myy = b * myy + a * dvy_dy; mxy = b * mxy + a * dvx_dy; mzy = b * mzy + a * dvz_dy;
-        dvy_dy = dvy_dy * ik + myy; dvx_dy = dvx_dy * ik + mxy; dvz_dy = dvz_dy * ik + mzy;
-      }
-      if (inz) {
-        mzz = bzh_k * mzz + azh_k * dvz_dz; mxz = bzh_k * mxz + azh_k * dvx_dz; myz = bzh_k * myz + azh_k * dvy_dz;
-        dvz_dz = dvz_dz * ikzh_k + mzz; dvx_dz = dvx_dz * ikzh_k + mxz; dvy_dz = dvy_dz * ikzh_k + myz;
-      }
-      const __attribute__((address_space(3))) volatile T* K = C + 27 * NT25;
-      SYZ[c] = syz0 + (K[0] * dvx_dx + K[NT25] * dvy_dy + K[2 * NT25] * dvz_dz + K[3 * NT25] * (dvy_dz + dvz_dy) +
-                       K[4 * NT25] * (dvx_dz + dvz_dx) + K[5 * NT25] * (dvy_dx + dvx_dy)) * dt;
     }
     if (own) {
-      if (inx) { psi[ox] = mxx; psi[ox + L.SX] = myx; psi[ox + 2 * L.SX] = mzx; }
-      if (iny) { psi[oy] = mxy; psi[oy + L.SY] = myy; psi[oy + 2 * L.SY] = mzy; }
-      if (inz) { psi[oz] = mxz; psi[oz + L.SZ] = myz; psi[oz + 2 * L.SZ] = mzz; }
-      if (i == S.isrc && k == S.ksrc && j == S.jsrc) {  // stress-rate (moment-tensor) source
-        if (S.msrc[0]) SXX[c] = SXX[c] + cp<T>(S.msrc[0])[it];
-        if (S.msrc[1]) SYY[c] = SYY[c] + cp<T>(S.msrc[1])[it];
-        if (S.msrc[2]) SZZ[c] = SZZ[c] + cp<T>(S.msrc[2])[it];
-        if (S.msrc[3]) SXY[c] = SXY[c] + cp<T>(S.msrc[3])[it];
-        if (S.msrc[4]) SXZ[c] = SXZ[c] + cp<T>(S.msrc[4])[it];
-        if (S.msrc[5]) SYZ[c] = SYZ[c] + cp<T>(S.msrc[5])[it];
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const int j = jb + q;
+        if (j >= j1) break;
+        if (PML && inx) {
+          const uint32_t o = (uint32_t)j * 2 * lx + xs;
+          W.x0[o] = mxx[q]; W.x1[o] = myx[q]; W.x2[o] = mzx[q];
+        }
+        if (PML && iny) {
+          const uint32_t o = (uint32_t)slab_pos(j, ny, ly) * nx + ic;
+          W.y0[o] = mxy[q]; W.y1[o] = myy[q]; W.y2[o] = mzy[q];
+        }
+        if (PML && inz) { W.z0[c[q]] = mxz[q]; W.z1[c[q]] = myz[q]; W.z2[c[q]] = mzz[q]; }
+        if (i == S.isrc && k == S.ksrc && j == S.jsrc) {  // stress-rate (moment-tensor) source
+          if (S.msrc[0]) SXX[c[q]] = SXX[c[q]] + cp<T>(S.msrc[0])[it];
+          if (S.msrc[1]) SYY[c[q]] = SYY[c[q]] + cp<T>(S.msrc[1])[it];
+          if (S.msrc[2]) SZZ[c[q]] = SZZ[c[q]] + cp<T>(S.msrc[2])[it];
+          if (S.msrc[3]) SXY[c[q]] = SXY[c[q]] + cp<T>(S.msrc[3])[it];
+          if (S.msrc[4]) SXZ[c[q]] = SXZ[c[q]] + cp<T>(S.msrc[4])[it];
+          if (S.msrc[5]) SYZ[c[q]] = SYZ[c[q]] + cp<T>(S.msrc[5])[it];
+        }
       }
     }
-    vxm = vxc; vym = vyc; vzm = vzc;
-    vxc = vxn; vyc = vyn; vzc = vzn;
-  };
-  // two rows per iteration: the loads of row j+1 are in flight while row j
-  // computes, and those of row j+2 while row j+1 does
-  if constexpr (!PML || SDT_EL25_PF_PML) {
-    RowLd A = load_row(j0);
-    int j = j0;
-#pragma unroll 1
-    for (; j + 1 < j1; j += 2) {
-      const RowLd B = load_row(j + 1);
-      row(j, A);
-      A = load_row(j + 2);
-      row(j + 1, B);
-    }
-    if (j < j1) row(j, A);
-  } else {
-#pragma unroll 1
-    for (int j = j0; j < j1; ++j) row(j, load_row(j));
+    vx[0] = vx[R]; vy[0] = vy[R]; vz[0] = vz[R];
+    vx[1] = vx[R + 1]; vy[1] = vy[R + 1]; vz[1] = vz[R + 1];
   }
 }
 
 // A wavefront whose columns, plane and rows all lie outside the C-PML slabs
 // runs the body without memory variables.
 template <typename T>
-__global__ void __launch_bounds__(NT25, sizeof(T) == 4 ? SDT_EL25S_WAVES : 2)
+__global__ void __launch_bounds__(NT25, WS25<T>)
 k_el25_stress(const DModel* __restrict__ models, const DShot* __restrict__ shots,
           const int4* __restrict__ work, int n, const int* __restrict__ base, int rel) {
   const int q = item25(n);
@@ -2740,6 +2791,7 @@ k_el25_stress(const DModel* __restrict__ models, const DShot* __restrict__ shots
 template <typename T, bool PML>
 __device__ __forceinline__ void el25_vel_tile(const DModel* __restrict__ models,
                                               const DShot* __restrict__ shots, const int4 wv, const int* __restrict__ base, int rel) {
+  constexpr int R = RV25;
   const int s = __builtin_amdgcn_readfirstlane(wv.x);
   const DShot& S = shots[s];
   const DModel& M = models[S.model];
@@ -2757,18 +2809,18 @@ __device__ __forceinline__ void el25_vel_tile(const DModel* __restrict__ models,
   const T idx = T(1.0 / M.dx), idy = T(1.0 / M.dy), idz = T(1.0 / M.dz);
   const int lx = M.lx, ly = M.ly, lz = M.lz;
   const bool inx = PML && incol && in_slab(i, nx, lx), inz = PML && in_slab(k, nz, lz);
+  const bool iny = PML && in_slab(j0, ny, ly);
   const Prof<T> P(&M.prof[0][0]);
   const T bx_i = P[PB][ic], ax_i = P[PA][ic], ikx_i = P[PK][ic];
   const T bxh_i = P[PBH][ic], axh_i = P[PAH][ic], ikxh_i = P[PKH][ic];
-  const T bz_k = P[12 + PB][k], az_k = P[12 + PA][k], ikz_k = P[12 + PK][k];
-  const T bzh_k = P[12 + PBH][k], azh_k = P[12 + PAH][k], ikzh_k = P[12 + PKH][k];
-  gcptr<T> by = P[6 + PB], ay = P[6 + PA], iky = P[6 + PK];
-  gcptr<T> byh = P[6 + PBH], ayh = P[6 + PAH], ikyh = P[6 + PKH];
+  const T bz_k = kp<T>(M.prof[2][PB])[k], az_k = kp<T>(M.prof[2][PA])[k], ikz_k = kp<T>(M.prof[2][PK])[k];
+  const T bzh_k = kp<T>(M.prof[2][PBH])[k], azh_k = kp<T>(M.prof[2][PAH])[k], ikzh_k = kp<T>(M.prof[2][PKH])[k];
+  const auto iky = kp<T>(M.prof[1][PK]), ay = kp<T>(M.prof[1][PA]), by = kp<T>(M.prof[1][PB]);
+  const auto ikyh = kp<T>(M.prof[1][PKH]), ayh = kp<T>(M.prof[1][PAH]), byh = kp<T>(M.prof[1][PBH]);
   // loop ranges of the legacy velocity loops (seismicfdtd.f95:821, :848, :873)
   const bool ux = own && k >= 1 && i >= 1, uy = own && k >= 1 && i <= nx - 2;
   const bool uz = own && k <= nz - 2 && i <= nx - 2;
-  const T dtrx = ux ? A32<const T>(M.coef[33])[p] : T(0), dtry = uy ? A32<const T>(M.coef[34])[p] : T(0);
-  const T dtrz = uz ? A32<const T>(M.coef[35])[p] : T(0);
+  const T dtrx = A32<const T>(M.coef[33])[p], dtry = A32<const T>(M.coef[34])[p], dtrz = A32<const T>(M.coef[35])[p];
   const T omx = A32<const T>(M.coef[36])[p], omy = A32<const T>(M.coef[37])[p];
   const T omz = A32<const T>(M.coef[38])[p];
   const int kd = k >= 1 ? k - 1 : 0, ku = k <= nz - 2 ? k + 1 : nz - 1;
@@ -2778,103 +2830,107 @@ __device__ __forceinline__ void el25_vel_tile(const DModel* __restrict__ models,
   const A32<const T> SXZD = cplane<T>(S.f[7], nxy, kd), SYZD = cplane<T>(S.f[8], nxy, kd);
   const A32<const T> SZZU = cplane<T>(S.f[5], nxy, ku);
   const A32<T> VX = plane<T>(S.f[0], nxy, k), VY = plane<T>(S.f[1], nxy, k), VZ = plane<T>(S.f[2], nxy, k);
-  auto psi = mp<T>(S.psi);
-  const Slab3 L(nx, ny, nz, lx, ly, lz);
   const int xs = inx ? slab_pos(i, nx, lx) : 0, zs = inz ? slab_pos(k, nz, lz) : 0;
+  const PsiEl25<T> W(S.psi, Slab3(nx, ny, nz, lx, ly, lz), 3, nx, ny, lx, ly, k, zs);
   const bool kedge = (i == 0 || k == 0 || i == nx - 1 || k == nz - 1);
   const bool srccol = (i == S.isrc && k == S.ksrc);
+  bool bad = false;
 
-  // y window: sxy, syz of row j-1 and syy of row j
-  const uint32_t r0 = (uint32_t)j0 * nx + ic;
-  T sxym = 0, syzm = 0;
-  if (j0 >= 1) { sxym = SXY[r0 - nx]; syzm = SYZ[r0 - nx]; }
-  T syyc = SYY[r0];
-  // the loads of row j (rows past the last are clamped in bounds)
-  struct RowLd { T sxx, sxy, sxz, szz, syz, syyn, sxzd, syzd, szzu, vx, vy, vz; };
-  auto load_row = [&](int j) {
-    RowLd R;
-    const uint32_t c = (uint32_t)(j < ny ? j : ny - 1) * nx + ic;
-    const uint32_t cn = j + 1 < ny ? c + nx : c;
-    R.sxx = SXX[c]; R.sxy = SXY[c]; R.sxz = SXZ[c]; R.szz = SZZ[c]; R.syz = SYZ[c];
-    R.syyn = SYY[cn];
-    R.sxzd = SXZD[c]; R.syzd = SYZD[c]; R.szzu = SZZU[c];
-    R.vx = VX[c]; R.vy = VY[c]; R.vz = VZ[c];
-    return R;
-  };
-  auto row = [&](const int j, const RowLd& R) {
-    const uint32_t c = (uint32_t)j * nx + ic;
-    const T sxx = R.sxx, sxy = R.sxy, sxz = R.sxz, szz = R.szz, syz = R.syz;
-    const T syyn = R.syyn;
-    const T sxzd = R.sxzd, syzd = R.syzd, szzu = R.szzu;
-    const T sxxw = lane_prev(sxx), sxye = lane_next(sxy), sxze = lane_next(sxz);
-    T vxn = R.vx, vyn = R.vy, vzn = R.vz;
-    const bool iny = PML && in_slab(j, ny, ly);
-    const long ox = L.bx + ((long)k * ny + j) * 2 * lx + xs;
-    const long oy = L.by + ((long)k * 2 * ly + (iny ? slab_pos(j, ny, ly) : 0)) * nx + ic;
-    const long oz = L.bz + ((long)zs * ny + j) * nx + ic;
-    // vx, seismicfdtd.f95:821-846
-    if (ux && j >= 1) {
-      T a = (sxx - sxxw) * idx, b = (sxy - sxym) * idy, d = (sxz - sxzd) * idz;
-      if (inx) { T m = bx_i * psi[ox + 3 * L.SX] + ax_i * a; a = a * ikx_i + m; psi[ox + 3 * L.SX] = m; }
-      if (iny) { T m = by[j] * psi[oy + 4 * L.SY] + ay[j] * b; b = b * iky[j] + m; psi[oy + 4 * L.SY] = m; }
-      if (inz) { T m = bz_k * psi[oz + 4 * L.SZ] + az_k * d; d = d * ikz_k + m; psi[oz + 4 * L.SZ] = m; }
-      vxn = vxn * omx + (a + b + d) * dtrx;
-    }
-    // vy, seismicfdtd.f95:848-870
-    if (uy && j <= ny - 2) {
-      T a = (sxye - sxy) * idx, b = (syyn - syyc) * idy, d = (syz - syzd) * idz;
-      if (inx) { T m = bxh_i * psi[ox + 4 * L.SX] + axh_i * a; a = a * ikxh_i + m; psi[ox + 4 * L.SX] = m; }
-      if (iny) { T m = byh[j] * psi[oy + 3 * L.SY] + ayh[j] * b; b = b * ikyh[j] + m; psi[oy + 3 * L.SY] = m; }
-      if (inz) { T m = bz_k * psi[oz + 5 * L.SZ] + az_k * d; d = d * ikz_k + m; psi[oz + 5 * L.SZ] = m; }
-      vyn = vyn * omy + (a + b + d) * dtry;
-    }
-    // vz, seismicfdtd.f95:873-896
-    if (uz && j >= 1) {
-      T a = (sxze - sxz) * idx, b = (syz - syzm) * idy, d = (szzu - szz) * idz;
-      if (inx) { T m = bxh_i * psi[ox + 5 * L.SX] + axh_i * a; a = a * ikxh_i + m; psi[ox + 5 * L.SX] = m; }
-      if (iny) { T m = by[j] * psi[oy + 5 * L.SY] + ay[j] * b; b = b * iky[j] + m; psi[oy + 5 * L.SY] = m; }
-      if (inz) { T m = bzh_k * psi[oz + 3 * L.SZ] + azh_k * d; d = d * ikzh_k + m; psi[oz + 3 * L.SZ] = m; }
-      vzn = vzn * omz + (a + b + d) * dtrz;
-    }
-    // source, seismicfdtd.f95:898-900
-    if (srccol && j == S.jsrc) {
-      if (S.src[0]) vxn += cp<T>(S.src[0])[it];
-      if (S.src[1]) vyn += cp<T>(S.src[1])[it];
-      if (S.src[2]) vzn += cp<T>(S.src[2])[it];
-    }
-    // Dirichlet faces, seismicfdtd.f95:903-925
-    if (kedge || j == 0 || j == ny - 1) { vxn = 0; vyn = 0; vzn = 0; }
-    if (own) {
-      check_blowup((double)vxn * vxn + (double)vyn * vyn + (double)vzn * vzn, S.blowup, it);
-      VX[c] = vxn;
-      VY[c] = vyn;
-      VZ[c] = vzn;
-    }
-    sxym = sxy; syzm = syz; syyc = syyn;
-  };
-  // two rows per iteration, as in the stress pass (FP64: one row at a time,
-  // two would cost a wavefront per SIMD)
-  if constexpr (sizeof(T) == 4) {
-    RowLd A = load_row(j0);
-    int j = j0;
-#pragma unroll 1
-    for (; j + 1 < j1; j += 2) {
-      const RowLd B = load_row(j + 1);
-      row(j, A);
-      A = load_row(j + 2);
-      row(j + 1, B);
-    }
-    if (j < j1) row(j, A);
-  } else {
-#pragma unroll 1
-    for (int j = j0; j < j1; ++j) row(j, load_row(j));
+  // sxy, syz of rows jb-1 .. jb+R-1 and syy of rows jb .. jb+R: [0] carried
+  T sxy[R + 1], syz[R + 1], syy[R + 1];
+  {
+    const uint32_t m = (uint32_t)max(j0 - 1, 0) * nx + ic;
+    sxy[0] = SXY[m]; syz[0] = SYZ[m];
+    syy[0] = SYY[(uint32_t)j0 * nx + ic];
   }
+#pragma unroll 1
+  for (int jb = j0; jb < j1; jb += R) {
+    T sxx[R], sxz[R], szz[R], sxzd[R], syzd[R], szzu[R], vx[R], vy[R], vz[R];
+    T x0[R], x1[R], x2[R], y0[R], y1[R], y2[R], z0[R], z1[R], z2[R];
+    uint32_t c[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      c[q] = (uint32_t)min(jb + q, j1 - 1) * nx + ic;
+      sxx[q] = SXX[c[q]]; sxz[q] = SXZ[c[q]]; szz[q] = SZZ[c[q]];
+      sxy[q + 1] = SXY[c[q]]; syz[q + 1] = SYZ[c[q]];
+      syy[q + 1] = SYY[(uint32_t)min(jb + q + 1, min(j1, ny - 1)) * nx + ic];
+      sxzd[q] = SXZD[c[q]]; syzd[q] = SYZD[c[q]]; szzu[q] = SZZU[c[q]];
+      vx[q] = VX[c[q]]; vy[q] = VY[c[q]]; vz[q] = VZ[c[q]];
+    }
+    if (PML && iny) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const uint32_t o = (uint32_t)slab_pos(min(jb + q, j1 - 1), ny, ly) * nx + ic;
+        y0[q] = W.y0[o]; y1[q] = W.y1[o]; y2[q] = W.y2[o];
+      }
+    }
+    if (PML && inz) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) { z0[q] = W.z0[c[q]]; z1[q] = W.z1[c[q]]; z2[q] = W.z2[c[q]]; }
+    }
+    if (PML && inx) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const uint32_t o = (uint32_t)min(jb + q, j1 - 1) * 2 * lx + xs;
+        x0[q] = W.x0[o]; x1[q] = W.x1[o]; x2[q] = W.x2[o];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const int j = jb + q;
+      const T sxxw = dpp_prev(sxx[q]), sxye = dpp_next(sxy[q + 1]), sxze = dpp_next(sxz[q]);
+      if (j >= j1) break;
+      const uint32_t ox = (uint32_t)j * 2 * lx + xs;
+      const uint32_t oy = PML && iny ? (uint32_t)slab_pos(j, ny, ly) * nx + ic : 0;
+      T vxn = vx[q], vyn = vy[q], vzn = vz[q];
+      // vx, seismicfdtd.f95:821-846
+      if (ux && j >= 1) {
+        T a = (sxx[q] - sxxw) * idx, b = (sxy[q + 1] - sxy[q]) * idy, d = (sxz[q] - sxzd[q]) * idz;
+        if (PML && inx) { const T m = bx_i * x0[q] + ax_i * a; a = a * ikx_i + m; W.x0[ox] = m; }
+        if (PML && iny) { const T m = by[j] * y1[q] + ay[j] * b; b = b * iky[j] + m; W.y1[oy] = m; }
+        if (PML && inz) { const T m = bz_k * z1[q] + az_k * d; d = d * ikz_k + m; W.z1[c[q]] = m; }
+        vxn = vxn * omx + (a + b + d) * dtrx;
+      }
+      // vy, seismicfdtd.f95:848-870
+      if (uy && j <= ny - 2) {
+        T a = (sxye - sxy[q + 1]) * idx, b = (syy[q + 1] - syy[q]) * idy, d = (syz[q + 1] - syzd[q]) * idz;
+        if (PML && inx) { const T m = bxh_i * x1[q] + axh_i * a; a = a * ikxh_i + m; W.x1[ox] = m; }
+        if (PML && iny) { const T m = byh[j] * y0[q] + ayh[j] * b; b = b * ikyh[j] + m; W.y0[oy] = m; }
+        if (PML && inz) { const T m = bz_k * z2[q] + az_k * d; d = d * ikz_k + m; W.z2[c[q]] = m; }
+        vyn = vyn * omy + (a + b + d) * dtry;
+      }
+      // vz, seismicfdtd.f95:873-896
+      if (uz && j >= 1) {
+        T a = (sxze - sxz[q]) * idx, b = (syz[q + 1] - syz[q]) * idy, d = (szzu[q] - szz[q]) * idz;
+        if (PML && inx) { const T m = bxh_i * x2[q] + axh_i * a; a = a * ikxh_i + m; W.x2[ox] = m; }
+        if (PML && iny) { const T m = by[j] * y2[q] + ay[j] * b; b = b * iky[j] + m; W.y2[oy] = m; }
+        if (PML && inz) { const T m = bzh_k * z0[q] + azh_k * d; d = d * ikzh_k + m; W.z0[c[q]] = m; }
+        vzn = vzn * omz + (a + b + d) * dtrz;
+      }
+      // source, seismicfdtd.f95:898-900
+      if (srccol && j == S.jsrc) {
+        if (S.src[0]) vxn += cp<T>(S.src[0])[it];
+        if (S.src[1]) vyn += cp<T>(S.src[1])[it];
+        if (S.src[2]) vzn += cp<T>(S.src[2])[it];
+      }
+      // Dirichlet faces, seismicfdtd.f95:903-925
+      if (kedge || j == 0 || j == ny - 1) { vxn = 0; vyn = 0; vzn = 0; }
+      if (own) {
+        bad |= !((double)vxn * vxn + (double)vyn * vyn + (double)vzn * vzn <= 1.0e50);
+        VX[c[q]] = vxn;
+        VY[c[q]] = vyn;
+        VZ[c[q]] = vzn;
+      }
+    }
+    sxy[0] = sxy[R]; syz[0] = syz[R]; syy[0] = syy[R];
+  }
+  if (bad) atomicMin(S.blowup, it);
 }
 
 // A wavefront whose columns, plane and rows all lie outside the C-PML slabs
 // runs the body without memory variables.
 template <typename T>
-__global__ void __launch_bounds__(NT25, sizeof(T) == 4 ? SDT_EL25V_WAVES : 2)
+__global__ void __launch_bounds__(NT25, WV25<T>)
 k_el25_vel(const DModel* __restrict__ models, const DShot* __restrict__ shots,
           const int4* __restrict__ work, int n, const int* __restrict__ base, int rel) {
   const int q = item25(n);
@@ -4067,13 +4123,12 @@ std::vector<int> cuts25(const sdt_model& M, int rows) {
 // waiting for their loads, so tall chunks leave a small grid bound by the
 // latency of that walk with most of the device idle; short ones reload the
 // row above and below, and, in the elastic passes, the column's 39
-// coefficients, per chunk.  EM: 4 rows (measured per step in us, 8 / 4 / 2 rows:
-// 332x72x182 FP32 90 / 84 / 86, FP64 207 / 202 / 203, 133x57x79 FP64 35 / 31 /
-// 31; 544x96x416 FP32 439 / 428 / -).  Elastic (32 / 16 / 8 / 4 / 2 rows):
-// 832x96x432 FP32 1309 / 1281 / 1322 / 1474 / 1872, 332x72x182 FP32 170 / 191 /
-// 171 / 174 / 203, 182x69x107 FP64 145 / 146 / 125 / 126 / 135, 112x56x82 FP64
-// 137 / 127 / 82 / 62 / 70: 16 rows, 8 where that leaves fewer than 12000
-// wavefronts, 4 below 2500 and 2 below 2000.
+// coefficients, per chunk.  Measured per step (us):
+//   EM, 8 / 4 / 2 rows: 332x72x182 FP32 90 / 84 / 86, FP64 207 / 202 / 203,
+//   133x57x79 FP64 35 / 31 / 31, 544x96x416 FP32 439 / 428 / -;
+//   elastic FP32, 16 / 8 / 4 / 2 rows: 832x96x432 1161 / 1160 / - / -, 332x72x182
+//   160 / 148 / 135 / 136, 112x56x82 63 / 42 / 31 / 27; FP64: 832x96x432 2180 /
+//   2179 / - / -, 332x72x182 357 / 342 / 347 / 374, 171x57x95 70 / 70 / 68 / 68.
 int rows25(const Plan* p) {
   auto waves = [&](int rows) {
     long long n = 0;
@@ -4084,9 +4139,9 @@ int rows25(const Plan* p) {
     return n;
   };
   if (p->kind == SDT_EM25) return 4;
-  if (waves(16) >= 12000) return 16;
-  if (waves(8) >= 2500) return 8;
-  return waves(4) >= 2000 ? 4 : 2;
+  if (waves(16) >= 20000) return 16;
+  if (p->prec == SDT_FP64) return waves(8) >= 5000 ? 8 : 4;
+  return waves(4) >= 2500 ? 4 : 2;
 }
 
 // Work list of the 2.5-D kernels: one item (shot, x0, k, j0 | j1 << 16) per

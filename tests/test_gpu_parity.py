@@ -123,12 +123,15 @@ def test_3d_tiles_and_y_chunks(oracle_lib, kind):
 
 
 @pytest.mark.parametrize("ny,npml", [(4, 1), (7, 2), (9, 3), (13, 5), (20, 4), (21, 8)])
-def test_em25_row_groups(oracle_lib, ny, npml):
-    """The EM 2.5-D passes take the rows of a chunk in groups (4 in FP32, 2 in
-    FP64): chunks of 1 to 4 rows, slabs with a remainder, a last row that the
-    H pass leaves out; against the oracle with the bars of the other tests."""
-    p = tiny_problem("em25", seed=68 + ny, nx=70, ny=ny, nz=19, npml=npml, nt=25, nrec=9,
-                     src=(35, ny // 2, 9))
+@pytest.mark.parametrize("kind", ["em25", "elastic25"])
+def test_25d_row_groups(oracle_lib, kind, ny, npml):
+    """The 2.5-D passes take the rows of a chunk in groups (of 1, 2 or 4):
+    chunks of 1 to 4 rows, slabs with a remainder, a last row that the EM H
+    pass leaves out; against the oracle with the bars of the other tests."""
+    p = tiny_problem(kind, seed=68 + ny, nx=70, ny=ny, nz=19, npml=npml, nt=25, nrec=9,
+                     src=(35, ny // 2, 9), **({"gamma": 1e-3} if kind == "elastic25" else {}))
+    i, j, k = p.shots[0].src      # receivers the wave reaches within the run (FP32 range)
+    p.shots[0].rec = np.array([[i, j, k], [i + 2, j, k - 1], [i - 2, j - 1, k + 2]], dtype=np.int32)
     _compare(_sim(p, "fp64").run().check(), p, oracle_lib, FP64_TOL)
     sim = _sim(p, "fp32").run(graph_block=5).check()
     ref = oracle_lib.OracleRun(p).run()
