@@ -176,7 +176,10 @@ int sdt_plan_run(void* plan, int it0, int nsteps, int graph_block, void* stream)
  * columns (56 in the two-step ELASTIC2 kernel, 60 in the two-step EM2
  * one), walks `rows` rows (1..256).
  * Default: by the number of wavefronts the plan has (short tiles for small
- * plans, so that they fill the device).  Results do not depend on the shape.
+ * plans, so that they fill the device).  While the tiles, their order and the
+ * steps per launch are the defaults, sdt_plan_run and sdt_run_noalloc may also
+ * run a plan on square regions that take several steps per launch.  Results do
+ * not depend on the shape.
  * The adjoint's trail recomputation has a tile shape of its own.
  * Synchronises the device when the shape changes. */
 int sdt_plan_set_tiles(void* plan, int waves_per_block, int rows);

@@ -2949,6 +2949,435 @@ k_el25_vel(const DModel* __restrict__ models, const DShot* __restrict__ shots,
 }
 
 // ===========================================================================
+// ELASTIC2 and EM2, several time steps per launch on regions.
+//
+// A block of 1024 threads holds a region of RM x RM cells of one shot, one cell
+// per thread, with the state, the memory variables and the coefficients in
+// registers, and takes up to tm steps: rows are exchanged through LDS, columns
+// by DPP lane shifts (a wavefront is two rows of the region; what a shift
+// carries across their ends reaches only halo columns).  One elastic step makes
+// a cell depend on columns i-1 .. i+2 and rows k-2 .. k+1, one EM step on one
+// neighbour each way, so after tm steps the middle of the region is exact
+// (columns tm .. RM-2tm-1 and rows 2tm .. RM-tm-1; EM tm .. RM-tm-1 both ways):
+// the block owns that and the neighbouring blocks recompute the rest.  Every
+// expression is the one-step kernel's, in the same order: identical bits.  A
+// launch reads state buffer par and writes the other.
+// What bounds it: at most two blocks share a CU, so a SIMD has 4 or 8 wavefronts
+// whose instructions it issues one after the other (about 1.1 us per elastic
+// step and block), and each launch waits once for its loads (5 to 7 us).
+// Regions off the slabs and the outer rings run a body without memory
+// variables and edge predicates (EM FP32 1064x808 5.6 -> 5.1 us per step with it).
+// The budget of 8 wavefronts per SIMD (elastic FP64 4, at 110 registers) is what
+// lets two blocks share a CU: EM FP64 1064x808 8.3 -> 6.5 us per step.  Letting
+// the wavefronts whose rows no later step needs sit out measured 3 % slower.
+// ===========================================================================
+constexpr int RM = 32;       // region: RM x RM cells, one thread each
+constexpr int TM_MAX = 8;    // most steps per launch
+
+// The receivers of the block's owned cells (columns cx0.., rows cz0.. of the
+// region, own x own): per thread the first index entry on its cell (INT_MAX:
+// none) and the end of its row's entries.  Called by every thread.
+__device__ __forceinline__ void region_receivers(const DShot& S, int* slot, int x0, int z0, int nz, int cx0,
+                                                 int cz0, int own, bool mine, int& e0, int& e1, int& id0,
+                                                 bool& more) {
+  const int zr0 = z0 + cz0, zr1 = min(zr0 + own, nz);
+  e0 = INT_MAX;
+  e1 = id0 = 0;
+  more = false;
+  if (S.nrec <= 0 || S.rrow[zr1] <= S.rrow[zr0]) return;  // block-uniform
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  slot[threadIdx.x] = INT_MAX;
+  __syncthreads();
+  for (int h = 0; h < 2; ++h) {
+    const int row = z0 + 2 * w + h;
+    if (row < zr0 || row >= zr1) continue;
+    const int q0 = S.rrow[row], q1 = S.rrow[row + 1];
+    for (int e = q0 + lane; e < q1; e += 64) {
+      const int cx = S.rxid[2 * e] - x0;
+      if (cx >= cx0 && cx < cx0 + own) atomicMin(&slot[(2 * w + h) * RM + cx], e);
+    }
+  }
+  __syncthreads();
+  if (!mine) return;
+  e0 = slot[threadIdx.x];
+  if (e0 == INT_MAX) return;
+  const int i = x0 + (int)(threadIdx.x % RM);
+  e1 = S.rrow[z0 + (int)(threadIdx.x / RM) + 1];
+  id0 = S.rxid[2 * e0 + 1];
+  more = e0 + 1 < e1 && S.rxid[2 * e0 + 2] == i;
+}
+
+// This step's samples a, b of the receivers on column i's cell.
+template <typename T>
+__device__ __forceinline__ void region_sample(const DShot& S, int it, int i, int e0, int e1, int id0, bool more,
+                                              T a, T b) {
+  if (e0 == INT_MAX) return;
+  auto tr = mp<T>(S.trace) + (long)it * 2 * S.nrec;
+  tr[id0] = a;
+  tr[S.nrec + id0] = b;
+  if (!more) return;
+  for (int e = e0 + 1; e < e1 && S.rxid[2 * e] == i; ++e) {
+    const int id = S.rxid[2 * e + 1];
+    tr[id] = a;
+    tr[S.nrec + id] = b;
+  }
+}
+
+template <typename T>
+struct ElRegionLds {
+  T v[2][RM][RM], s[2][RM][RM];  // vx, vz; sxz, szz
+  T px[6][RM], pz[7][RM];        // C-PML profiles of the region's columns and rows
+  T src[5][TM_MAX];              // source increments of the steps: vx vz sxx szz sxz
+  int slot[RM * RM];
+};
+
+// PML false: no cell of the region lies in a C-PML slab or on the outer ring.
+template <typename T, bool SPLIT, bool PML>
+__device__ __forceinline__ void el2_region(const DModel& M, const DShot& S, const int x0, const int z0,
+                                           const int it0, const int nsteps, const int tm, const int par,
+                                           ElRegionLds<T>& L) {
+#pragma clang fp contract(off)
+  const int nx = M.nx, nz = M.nz;
+  const int tx = threadIdx.x & (RM - 1), ty = threadIdx.x / RM;
+  const int i = x0 + tx, r = z0 + ty, osz = RM - 3 * tm;
+  const bool in = !PML || (i >= 0 && i < nx && r >= 0 && r < nz);
+  const int ic = PML ? min(max(i, 0), nx - 1) : i, rc = PML ? min(max(r, 0), nz - 1) : r;
+  const bool own = in && tx >= tm && tx < tm + osz && ty >= 2 * tm && ty < 2 * tm + osz;
+  const uint32_t c = (uint32_t)rc * nx + ic;
+  T vx = A32<const T>(par ? S.g[0] : S.f[0])[c], vz = A32<const T>(par ? S.g[1] : S.f[1])[c];
+  T sxx = A32<const T>(par ? S.g[2] : S.f[2])[c], szz = A32<const T>(par ? S.g[3] : S.f[3])[c];
+  T sxz = A32<const T>(par ? S.g[4] : S.f[4])[c];
+  const A32<const T> pin(par ? S.psi2 : S.psi);
+  const bool mono = M.coef[2] != nullptr, atten = M.coef[10] != nullptr;
+  const T n11 = A32<const T>(M.coef[0])[c], n13 = A32<const T>(M.coef[1])[c], n33 = A32<const T>(M.coef[3])[c];
+  const T s55 = A32<const T>(M.coef[7])[c];
+  const T n15 = mono ? A32<const T>(M.coef[2])[c] : T(0), n35 = mono ? A32<const T>(M.coef[4])[c] : T(0);
+  const T s15 = mono ? A32<const T>(M.coef[5])[c] : T(0), s35 = mono ? A32<const T>(M.coef[6])[c] : T(0);
+  const T dtx = A32<const T>(M.coef[8])[c], dtz = A32<const T>(M.coef[9])[c];
+  const T omx = atten ? A32<const T>(M.coef[10])[c] : T(1), omz = atten ? A32<const T>(M.coef[11])[c] : T(1);
+  const int lx = M.lx, lz = M.lz;
+  const bool inx = PML && in && in_slab(i, nx, lx), inz = PML && in && in_slab(r, nz, lz);
+  const uint32_t SX = (uint32_t)nz * 2 * lx, SZ = (uint32_t)2 * lz * nx, ZB = (SPLIT ? 6 : 4) * SX;
+  const uint32_t ox = inx ? (uint32_t)r * 2 * lx + slab_pos(i, nx, lx) : 0;
+  const uint32_t oz = ZB + (inz ? (uint32_t)slab_pos(r, nz, lz) * nx + i : 0);
+  T m_vxx = 0, m_vzx = 0, m_sxx = 0, m_sxzx = 0, s_vxx = 0, s_vzx = 0;
+  T m_vzz = 0, m_vxz = 0, m_szz = 0, m_sxzz = 0, s_vzz = 0, s_vxz = 0;
+  if (inx) {
+    m_vxx = pin[ox]; m_vzx = pin[SX + ox]; m_sxx = pin[2 * SX + ox]; m_sxzx = pin[3 * SX + ox];
+    if (SPLIT) { s_vxx = pin[4 * SX + ox]; s_vzx = pin[5 * SX + ox]; }
+  }
+  if (inz) {
+    m_vzz = pin[oz]; m_vxz = pin[SZ + oz]; m_szz = pin[2 * SZ + oz]; m_sxzz = pin[3 * SZ + oz];
+    if (SPLIT) { s_vzz = pin[4 * SZ + oz]; s_vxz = pin[5 * SZ + oz]; }
+  }
+  if (PML) {
+    // (z entry 6: the legacy normal loop's decay of memory_dvx_dx, b_x_half by row)
+    if (threadIdx.x < 6 * RM) {
+      L.px[threadIdx.x / RM][tx] = cp<T>(M.prof[0][threadIdx.x / RM])[min(max(x0 + tx, 0), nx - 1)];
+    } else if (threadIdx.x >= 256 && threadIdx.x < 256 + 7 * RM) {
+      const int q = (threadIdx.x - 256) / RM, zr = min(max(z0 + tx, 0), nz - 1);
+      L.pz[q][tx] = q < 6 ? cp<T>(M.prof[2][q])[zr] : SPLIT ? T(0) : cp<T>(M.aux)[zr];
+    }
+  }
+  if (threadIdx.x >= 512 && threadIdx.x < 512 + 5 * TM_MAX) {  // (read after the first barrier)
+    const int q = (threadIdx.x - 512) / TM_MAX, t = (threadIdx.x - 512) % TM_MAX;
+    const void* a = q == 0 ? S.src[0] : q == 1 ? S.src[2] : S.msrc[q == 2 ? 0 : q == 3 ? 2 : 4];
+    L.src[q][t] = a && t < nsteps ? cp<T>(a)[it0 + t] : T(0);
+  }
+  const T idx = T(1.0 / M.dx), idz = T(1.0 / M.dz), dt = T(M.dt);
+  const bool issrc = in && i == S.isrc && r == S.ksrc;
+  const bool msrc = S.msrc[0] || S.msrc[2] || S.msrc[4];
+  int e0, e1, id0;
+  bool more;
+  region_receivers(S, L.slot, x0, z0, nz, tm, 2 * tm, osz, own, e0, e1, id0, more);
+  int bad = INT_MAX;
+  const int tu = ty > 0 ? ty - 1 : 0, td = ty < RM - 1 ? ty + 1 : RM - 1;
+  for (int t = 0; t < nsteps; ++t) {
+    // ---- stresses (seismicfdtd.f95:247-312) ----
+    L.v[0][ty][tx] = vx;
+    L.v[1][ty][tx] = vz;
+    __syncthreads();
+    {
+      const T vx_e = dpp_next(vx), vz_e = dpp_next(vz), vx_w = dpp_prev(vx), vz_w = dpp_prev(vz);
+      const T vx_m = L.v[0][tu][tx], vz_m = L.v[1][tu][tx], vx_n = L.v[0][td][tx], vz_n = L.v[1][td][tx];
+      if (!PML || (in && i <= nx - 2 && r >= 1)) {
+        T dvx_dx = (vx_e - vx) * idx;
+        T dvz_dz = (vz - vz_m) * idz;
+        T dvz_dx = (vz_e - vz) * idx;
+        T dvx_dz = (vx - vx_m) * idz;
+        if (inx) {
+          m_vxx = fma(SPLIT ? L.px[PBH][tx] : L.pz[6][ty], m_vxx, L.px[PAH][tx] * dvx_dx);  // :255
+          m_vzx = fma(L.px[PB][tx], m_vzx, L.px[PA][tx] * dvz_dx);
+          dvx_dx = fma(dvx_dx, L.px[PKH][tx], m_vxx);
+          dvz_dx = fma(dvz_dx, L.px[PK][tx], m_vzx);
+        }
+        if (inz) {
+          m_vzz = fma(L.pz[PB][ty], m_vzz, L.pz[PA][ty] * dvz_dz);
+          m_vxz = fma(L.pz[PBH][ty], m_vxz, L.pz[PAH][ty] * dvx_dz);
+          dvz_dz = fma(dvz_dz, L.pz[PK][ty], m_vzz);
+          dvx_dz = fma(dvx_dz, L.pz[PKH][ty], m_vxz);
+        }
+        const T sh = dvz_dx + dvx_dz;
+        sxx = fma(fma(n15, sh, fma(n13, dvz_dz, n11 * dvx_dx)), dt, sxx);
+        szz = fma(fma(n35, sh, fma(n33, dvz_dz, n13 * dvx_dx)), dt, szz);
+      }
+      if (!PML || (in && i >= 1 && r <= nz - 2)) {  // same psi arrays (A1) unless split
+        T& q_vxx = SPLIT ? s_vxx : m_vxx;
+        T& q_vzx = SPLIT ? s_vzx : m_vzx;
+        T& q_vzz = SPLIT ? s_vzz : m_vzz;
+        T& q_vxz = SPLIT ? s_vxz : m_vxz;
+        T dvx_dx = (vx - vx_w) * idx;
+        T dvz_dz = (vz_n - vz) * idz;
+        T dvz_dx = (vz - vz_w) * idx;
+        T dvx_dz = (vx_n - vx) * idz;
+        if (inx) {
+          q_vxx = fma(L.px[PBH][tx], q_vxx, L.px[PAH][tx] * dvx_dx);
+          q_vzx = fma(L.px[PB][tx], q_vzx, L.px[PA][tx] * dvz_dx);
+          dvx_dx = fma(dvx_dx, L.px[PKH][tx], q_vxx);
+          dvz_dx = fma(dvz_dx, L.px[PK][tx], q_vzx);
+        }
+        if (inz) {
+          q_vzz = fma(L.pz[PB][ty], q_vzz, L.pz[PA][ty] * dvz_dz);
+          q_vxz = fma(L.pz[PBH][ty], q_vxz, L.pz[PAH][ty] * dvx_dz);
+          dvz_dz = fma(dvz_dz, L.pz[PK][ty], q_vzz);
+          dvx_dz = fma(dvx_dz, L.pz[PKH][ty], q_vxz);
+        }
+        sxz = fma(fma(s55, dvz_dx + dvx_dz, fma(s35, dvz_dz, s15 * dvx_dx)), dt, sxz);
+      }
+      if (msrc && issrc) {
+        sxx += L.src[2][t];
+        szz += L.src[3][t];
+        sxz += L.src[4][t];
+      }
+    }
+    // ---- velocities (:317-375) ----
+    L.s[0][ty][tx] = sxz;
+    L.s[1][ty][tx] = szz;
+    __syncthreads();
+    {
+      const T sxx_w = dpp_prev(sxx), sxz_e = dpp_next(sxz);
+      const T sxz_u = L.s[0][tu][tx], szz_d = L.s[1][td][tx];
+      if (!PML || (in && i >= 1 && r >= 1)) {
+        T a = (sxx - sxx_w) * idx;
+        T b = (sxz - sxz_u) * idz;
+        if (inx) {
+          m_sxx = fma(L.px[PB][tx], m_sxx, L.px[PA][tx] * a);
+          a = fma(a, L.px[PK][tx], m_sxx);
+        }
+        if (inz) {
+          m_sxzz = fma(L.pz[PB][ty], m_sxzz, L.pz[PA][ty] * b);
+          b = fma(b, L.pz[PK][ty], m_sxzz);
+        }
+        vx = fma(vx, omx, (a + b) * dtx);
+      }
+      if (!PML || (in && i <= nx - 2 && r <= nz - 2)) {
+        T a = (sxz_e - sxz) * idx;
+        T b = (szz_d - szz) * idz;
+        if (inx) {
+          m_sxzx = fma(L.px[PBH][tx], m_sxzx, L.px[PAH][tx] * a);
+          a = fma(a, L.px[PKH][tx], m_sxzx);
+        }
+        if (inz) {
+          m_szz = fma(L.pz[PBH][ty], m_szz, L.pz[PAH][ty] * b);
+          b = fma(b, L.pz[PKH][ty], m_szz);
+        }
+        vz = fma(vz, omz, (a + b) * dtz);
+      }
+      if (issrc) {  // :359-361
+        vx += L.src[0][t];
+        vz += L.src[1][t];
+      }
+      if (PML && (i <= 0 || i >= nx - 1 || r <= 0 || r >= nz - 1)) { vx = 0; vz = 0; }  // :365-375
+      if (own) {
+        if (!((double)vx * vx + (double)vz * vz <= 1.0e50)) bad = min(bad, it0 + t);
+        region_sample<T>(S, it0 + t, i, e0, e1, id0, more, vx, vz);
+      }
+    }
+  }
+  if (own) {
+    A32<T>(par ? S.f[0] : S.g[0])[c] = vx;
+    A32<T>(par ? S.f[1] : S.g[1])[c] = vz;
+    A32<T>(par ? S.f[2] : S.g[2])[c] = sxx;
+    A32<T>(par ? S.f[3] : S.g[3])[c] = szz;
+    A32<T>(par ? S.f[4] : S.g[4])[c] = sxz;
+    const A32<T> pout(par ? S.psi : S.psi2);
+    if (inx) {
+      pout[ox] = m_vxx; pout[SX + ox] = m_vzx; pout[2 * SX + ox] = m_sxx; pout[3 * SX + ox] = m_sxzx;
+      if (SPLIT) { pout[4 * SX + ox] = s_vxx; pout[5 * SX + ox] = s_vzx; }
+    }
+    if (inz) {
+      pout[oz] = m_vzz; pout[SZ + oz] = m_vxz; pout[2 * SZ + oz] = m_szz; pout[3 * SZ + oz] = m_sxzz;
+      if (SPLIT) { pout[4 * SZ + oz] = s_vzz; pout[5 * SZ + oz] = s_vxz; }
+    }
+    if (bad != INT_MAX) atomicMin(S.blowup, bad);
+  }
+}
+
+// Whether no cell of the region at (x0, z0) lies in a slab or on the outer two
+// rows or columns (the rings of the EM fields' shorter extents included).
+__device__ __forceinline__ bool region_interior(const DModel& M, int x0, int z0) {
+  return x0 >= max(M.lx, 1) && x0 + RM <= M.nx - max(M.lx, 2) && z0 >= max(M.lz, 1) &&
+         z0 + RM <= M.nz - max(M.lz, 2);
+}
+
+template <typename T, bool SPLIT>
+__global__ void __launch_bounds__(RM* RM, sizeof(T) == 4 ? 8 : 4)
+k_el2_multi(const DModel* __restrict__ models, const DShot* __restrict__ shots, const int4* __restrict__ work,
+            int n, const int* __restrict__ base, int rel, int nsteps, int tm, int par) {
+  __shared__ ElRegionLds<T> L;
+  const int q = item25(n);
+  if (q < 0) return;
+  const int4 wv = work[q];
+  const DShot& S = shots[__builtin_amdgcn_readfirstlane(wv.x)];
+  const DModel& M = models[__builtin_amdgcn_readfirstlane(wv.w)];
+  const int it0 = __builtin_amdgcn_readfirstlane(*base + rel);
+  const int x0 = __builtin_amdgcn_readfirstlane(wv.y) - tm, z0 = __builtin_amdgcn_readfirstlane(wv.z) - 2 * tm;
+  if (region_interior(M, x0, z0))
+    el2_region<T, SPLIT, false>(M, S, x0, z0, it0, nsteps, tm, par, L);
+  else
+    el2_region<T, SPLIT, true>(M, S, x0, z0, it0, nsteps, tm, par, L);
+}
+
+template <typename T>
+struct EmRegionLds {
+  T ex[RM][RM], hy[RM][RM];
+  T px[6][RM], pz[6][RM];
+  T src[2][TM_MAX];  // source increments of the steps: Ex, Ez
+  int slot[RM * RM];
+};
+
+// psi slabs and stages of k_em2_step.
+template <typename T, bool PML>
+__device__ __forceinline__ void em2_region(const DModel& M, const DShot& S, const int x0, const int z0,
+                                           const int it0, const int nsteps, const int tm, const int par,
+                                           EmRegionLds<T>& L) {
+#pragma clang fp contract(off)
+  const int nx = M.nx, nz = M.nz;
+  const int tx = threadIdx.x & (RM - 1), ty = threadIdx.x / RM;
+  const int i = x0 + tx, r = z0 + ty, osz = RM - 2 * tm;
+  const bool in = !PML || (i >= 0 && i < nx && r >= 0 && r < nz);
+  const int ic = PML ? min(max(i, 0), nx - 1) : i, rc = PML ? min(max(r, 0), nz - 1) : r;
+  const bool own = in && tx >= tm && tx < tm + osz && ty >= tm && ty < tm + osz;
+  const uint32_t c = (uint32_t)rc * nx + ic;
+  T ex = A32<const T>(par ? S.g[0] : S.f[0])[c], ez = A32<const T>(par ? S.g[1] : S.f[1])[c];
+  T hy = A32<const T>(par ? S.g[2] : S.f[2])[c];
+  const A32<const T> pin(par ? S.psi2 : S.psi);
+  const T cax = A32<const T>(M.coef[0])[c], cbx = A32<const T>(M.coef[1])[c];
+  const T caz = A32<const T>(M.coef[2])[c], cbz = A32<const T>(M.coef[3])[c];
+  const int lx = M.lx, lz = M.lz;
+  const bool inx = PML && in && in_slab(i, nx, lx), inz = PML && in && in_slab(r, nz, lz);
+  const uint32_t SX = (uint32_t)nz * 2 * lx, SZ = (uint32_t)2 * lz * nx;
+  const uint32_t ox = inx ? (uint32_t)r * 2 * lx + slab_pos(i, nx, lx) : 0;
+  const uint32_t oz = 2 * SX + (inz ? (uint32_t)slab_pos(r, nz, lz) * nx + i : 0);
+  T m_ezx = 0, m_hyx = 0, m_exz = 0, m_hyz = 0;
+  if (inx) { m_ezx = pin[ox]; m_hyx = pin[SX + ox]; }
+  if (inz) { m_exz = pin[oz]; m_hyz = pin[SZ + oz]; }
+  if (PML) {
+    if (threadIdx.x < 6 * RM) {
+      L.px[threadIdx.x / RM][tx] = cp<T>(M.prof[0][threadIdx.x / RM])[min(max(x0 + tx, 0), nx - 1)];
+    } else if (threadIdx.x >= 256 && threadIdx.x < 256 + 6 * RM) {
+      L.pz[(threadIdx.x - 256) / RM][tx] = cp<T>(M.prof[2][(threadIdx.x - 256) / RM])[min(max(z0 + tx, 0), nz - 1)];
+    }
+  }
+  if (threadIdx.x >= 512 && threadIdx.x < 512 + 2 * TM_MAX) {  // (read after the first barrier)
+    const int q = (threadIdx.x - 512) / TM_MAX, t = (threadIdx.x - 512) % TM_MAX;
+    const void* a = q == 0 ? S.src[0] : S.src[2];
+    L.src[q][t] = a && t < nsteps ? cp<T>(a)[it0 + t] : T(0);
+  }
+  const T idx = T(1.0 / M.dx), idz = T(1.0 / M.dz), dbh = T(M.scal[0]);
+  const bool issrc = in && i == S.isrc && r == S.ksrc;
+  int e0, e1, id0;
+  bool more;
+  region_receivers(S, L.slot, x0, z0, nz, tm, tm, osz, own, e0, e1, id0, more);
+  int bad = INT_MAX;
+  const int tu = ty > 0 ? ty - 1 : 0, td = ty < RM - 1 ? ty + 1 : RM - 1;
+  for (int t = 0; t < nsteps; ++t) {
+    // ---- Hy (electromagfdtd.f95:249-266) ----
+    L.ex[ty][tx] = ex;
+    __syncthreads();
+    {
+      const T ez_e = dpp_next(ez), ex_n = L.ex[td][tx];
+      if (!PML || (in && i <= nx - 2 && r <= nz - 2)) {
+        T a = (ex_n - ex) * idz;
+        if (inz) {
+          m_exz = fma(L.pz[PB][ty], m_exz, L.pz[PA][ty] * a);
+          a = fma(a, L.pz[PK][ty], m_exz);
+        }
+        T b = (ez_e - ez) * idx;
+        if (inx) {
+          m_ezx = fma(L.px[PB][tx], m_ezx, L.px[PA][tx] * b);
+          b = fma(b, L.px[PK][tx], m_ezx);
+        }
+        // (the zeroing of the ring that ends the last step, :312-315)
+        const bool edge = PML && (i == 0 || i == nx - 2 || r == 0 || r == nz - 2);
+        hy = fma(dbh, b + a, edge ? T(0) : hy);
+      }
+    }
+    // ---- Ex, Ez (:273-295), source, Dirichlet ----
+    L.hy[ty][tx] = hy;
+    __syncthreads();
+    {
+      const T hy_w = dpp_prev(hy), hy_p = L.hy[tu][tx];
+      if (!PML || (in && i <= nx - 2 && r >= 1 && r <= nz - 2)) {
+        T d = (hy - hy_p) * idz;
+        if (inz) {
+          m_hyz = fma(L.pz[PBH][ty], m_hyz, L.pz[PAH][ty] * d);
+          d = fma(d, L.pz[PKH][ty], m_hyz);
+        }
+        ex = fma(cax, ex, cbx * d);
+      }
+      if (!PML || (in && i >= 1 && i <= nx - 2 && r <= nz - 2)) {
+        T d = (hy - hy_w) * idx;
+        if (inx) {
+          m_hyx = fma(L.px[PBH][tx], m_hyx, L.px[PAH][tx] * d);
+          d = fma(d, L.px[PKH][tx], m_hyx);
+        }
+        ez = fma(caz, ez, cbz * d);
+      }
+      if (issrc) {
+        ex += L.src[0][t];
+        ez += L.src[1][t];
+      }
+      if (PML) {  // :304-311, and the cells outside the fields' extents
+        if (i <= 0 || i >= nx - 2 || r <= 0 || r >= nz - 1) ex = 0;
+        if (i <= 0 || i >= nx - 1 || r <= 0 || r >= nz - 2) ez = 0;
+      }
+      if (own) {
+        if (!((double)ex * ex + (double)ez * ez <= 1.0e50)) bad = min(bad, it0 + t);
+        region_sample<T>(S, it0 + t, i, e0, e1, id0, more, ex, ez);
+      }
+    }
+  }
+  if (own) {
+    A32<T>(par ? S.f[0] : S.g[0])[c] = ex;
+    A32<T>(par ? S.f[1] : S.g[1])[c] = ez;
+    A32<T>(par ? S.f[2] : S.g[2])[c] = hy;
+    const A32<T> pout(par ? S.psi : S.psi2);
+    if (inx) { pout[ox] = m_ezx; pout[SX + ox] = m_hyx; }
+    if (inz) { pout[oz] = m_exz; pout[SZ + oz] = m_hyz; }
+    if (bad != INT_MAX) atomicMin(S.blowup, bad);
+  }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(RM* RM, 8)
+k_em2_multi(const DModel* __restrict__ models, const DShot* __restrict__ shots, const int4* __restrict__ work,
+            int n, const int* __restrict__ base, int rel, int nsteps, int tm, int par) {
+  __shared__ EmRegionLds<T> L;
+  const int q = item25(n);
+  if (q < 0) return;
+  const int4 wv = work[q];
+  const DShot& S = shots[__builtin_amdgcn_readfirstlane(wv.x)];
+  const DModel& M = models[__builtin_amdgcn_readfirstlane(wv.w)];
+  const int it0 = __builtin_amdgcn_readfirstlane(*base + rel);
+  const int x0 = __builtin_amdgcn_readfirstlane(wv.y) - tm, z0 = __builtin_amdgcn_readfirstlane(wv.z) - tm;
+  if (region_interior(M, x0, z0))
+    em2_region<T, false>(M, S, x0, z0, it0, nsteps, tm, par, L);
+  else
+    em2_region<T, true>(M, S, x0, z0, it0, nsteps, tm, par, L);
+}
+
+// ===========================================================================
 // EM2 adjoint: the transpose of one EM2 step (k_em2_step), for gradients
 // of a trace misfit with respect to the E-update coefficients (caEx cbEx
 // caEz cbEz, from permittivity and conductivity).  No counterpart in the
@@ -3756,7 +4185,13 @@ struct Plan {
   int el2x2_grid = 0, el2x2_grid_i = 0;
   int* dit0 = nullptr;         // first step of the current run of two-step launches
   int* drec = nullptr;         // receivers by row of every shot (DShot::rrow, rxid)
-  bool graph_two = false;      // the cached graph holds two-step launches
+  int graph_mode = 0;          // what the cached graph holds (run_mode)
+  // several steps per launch on regions (default_regions), while the launch
+  // shape is the one that the plan picked by its size (run_mode)
+  bool multi = false;
+  int def_spl = 0, def_wb = 0, def_eh = 0, def_order = 0;
+  int4* dwmulti = nullptr;     // work list: (shot, x0, z0, model) per region
+  int nmulti = 0, tm = 0;      // tm: most steps per launch, the width of the regions' halo
   bool b_holds = false;        // buffer B holds the current state too (ELASTIC2 / EM2)
   int* dflags = nullptr;  // per shot first unstable step (INT_MAX = none)
   int* dbase = nullptr;   // step index of rel = 0
@@ -3971,6 +4406,42 @@ long long waves2d(const Plan* p, int ew, int rows) {
   return n;
 }
 
+// Regions of a 2-D plan whose halo is tm steps wide.
+long long regions2d(const Plan* p, int tm) {
+  const int own = RM - (p->kind == SDT_EM2 ? 2 : 3) * tm;
+  long long n = 0;
+  for (const sdt_shot& S : p->hshots) {
+    const sdt_model& M = p->hmodels[S.model];
+    n += (long long)((M.nx + own - 1) / own) * ((M.nz + own - 1) / own);
+  }
+  return n;
+}
+
+// Whether a 2-D plan runs on regions (k_el2_multi, k_em2_multi) and the most
+// steps per launch there.  A region recomputes its halo (tm = 4 elastic: 40 % of
+// its cells are owned, tm = 5 EM: 47 %), which pays where the walking kernels
+// wait on launches and loads, not where they stream: measured (us per step,
+// walking kernels in the shape of default_shape, then regions) elastic FP64
+// 127x103 6.4 -> 2.3, 296^2 7.8 -> 3.5, 1064x808 27.3 -> 18.9, x 3 shots 57 -> 52,
+// x 4 shots 70 -> 70; elastic FP32 296^2 6.7 -> 2.8, 1064x808 17.9 -> 9.4, x 10
+// shots 85 -> 81, x 16 shots 119 -> 129; EM FP64 127x103 3.5 -> 1.5, 1064x808 11.9
+// -> 6.2, x 32 shots 207 -> 174; EM FP32 1064x808 7.6 -> 4.7, x 32 shots 120 ->
+// 117, 2088x808 x 32 shots 218 -> 227.
+// tm: a launch costs 5 to 7 us beside its steps, so the most steps for which the
+// regions still run all at once (one block of elastic FP64 per CU, else two):
+// 127x103 elastic FP64 5.1 / 2.8 / 2.3 with 2 / 4 / 7 steps, 296^2 5.2 / 3.4 / 5.8;
+// larger plans take the number whose owned share balances the launches.
+void default_regions(Plan* p, double bytes, bool big) {
+  const bool em = p->kind == SDT_EM2, f64 = p->prec == SDT_FP64;
+  p->tm = em ? 5 : f64 && regions2d(p, 4) > 2500 ? 3 : 4;
+  for (int t = TM_MAX; t >= (!em && f64 ? 2 : 3); --t)
+    if (regions2d(p, t) <= (!em && f64 ? 256 : 512)) {
+      p->tm = t;
+      break;
+    }
+  p->multi = em ? f64 || bytes < 900e6 : f64 ? !big : bytes < 400e6;
+}
+
 // Default launch shape of a 2-D plan: steps per launch, wavefronts per block,
 // rows per tile and tile order, from how many wavefronts the plan has and
 // whether its ping-pong fields fit the 256 MB last-level cache.  Fitted to the
@@ -4024,6 +4495,46 @@ void default_shape(Plan* p) {
       if (waves2d(p, ew, rows) >= (f64 ? 2000 : em ? 2800 : 4000)) p->el2_eh = rows;
     if (waves2d(p, ew, 16) >= (em ? 12000 : 8000)) p->el2_eh = 16;
   }
+  default_regions(p, cells * kind_fields(p->kind) * 2 * (f64 ? 8 : 4), big);
+  p->def_spl = p->spl;
+  p->def_wb = p->el2_wb;
+  p->def_eh = p->el2_eh;
+  p->def_order = p->el2_order;
+}
+
+// Work list of the region kernels: the regions of a model column by column,
+// so that the contiguous run an XCD takes (item25) is one part of the model.
+std::vector<int4> multi_work(const Plan* p) {
+  const int own = RM - (p->kind == SDT_EM2 ? 2 : 3) * p->tm;
+  std::vector<int4> w;
+  for (int s = 0; s < p->nshots; ++s) {
+    const int m = p->hshots[s].model;
+    const sdt_model& M = p->hmodels[m];
+    for (int x = 0; x < M.nx; x += own)
+      for (int z = 0; z < M.nz; z += own) w.push_back(make_int4(s, x, z, m));
+  }
+  return w;
+}
+
+// Steps of one run or graph block of n steps on regions: at most p->tm per
+// launch, in launches of nearly equal length, an even number of them if
+// `even` (a graph block must leave the state in the buffer it started from).
+// Returns the number of launches.
+template <typename T>
+int launch_multi(Plan* p, hipStream_t st, int n, bool even) {
+  int L = (n + p->tm - 1) / p->tm;
+  if (even) L += L & 1;
+  const dim3 g((p->nmulti + 7) / 8 * 8), b(RM * RM);
+  for (int l = 0; l < L; ++l) {
+    const int r = (int)((long long)n * l / L), k = (int)((long long)n * (l + 1) / L) - r;
+    if (p->kind == SDT_EM2)
+      hipLaunchKernelGGL(k_em2_multi<T>, g, b, 0, st, p->dmodels, p->dshots, p->dwmulti, p->nmulti, p->dbase, r, k, p->tm, l & 1);
+    else if (p->split)
+      hipLaunchKernelGGL((k_el2_multi<T, true>), g, b, 0, st, p->dmodels, p->dshots, p->dwmulti, p->nmulti, p->dbase, r, k, p->tm, l & 1);
+    else
+      hipLaunchKernelGGL((k_el2_multi<T, false>), g, b, 0, st, p->dmodels, p->dshots, p->dwmulti, p->nmulti, p->dbase, r, k, p->tm, l & 1);
+  }
+  return L;
 }
 
 // Row cuts of one model's tiles: rows of at most eh, and with zt < zb also
@@ -4381,6 +4892,27 @@ bool use_two(const Plan* p, int n, int graph_block) {
   return p->spl == 2 && n >= 2 && (graph_block <= 1 || n < graph_block || graph_block % 2 == 0);
 }
 
+// How a run of n steps goes: 0 one step per launch, 1 two, 2 several on regions
+// (only with the launch shape that the plan picked).
+int run_mode(const Plan* p, int n, int graph_block) {
+  if (p->multi && p->spl == p->def_spl && p->el2_wb == p->def_wb && p->el2_eh == p->def_eh &&
+      p->el2_order == p->def_order)
+    return 2;
+  return use_two(p, n, graph_block) ? 1 : 0;
+}
+
+// Enqueue n steps in mode `mode`; whether the state is then in buffer B, or -1
+// where the step index says so (mode 0).
+int launch_run(Plan* p, hipStream_t st, int n, int mode, bool even) {
+  if (mode == 2) return (p->prec == SDT_FP64 ? launch_multi<double>(p, st, n, even) : launch_multi<float>(p, st, n, even)) & 1;
+  if (mode == 1) {
+    launch_pairs(p, st, n);
+    return (n / 2 + (n & 1)) & 1;
+  }
+  launch_steps(p, st, n);
+  return -1;
+}
+
 int validate(int kind, bool split, int prec, const sdt_model* models, int nmodels,
              const sdt_shot* shots, int nshots, int nt) {
   const int kpsi = kind | (split ? SDT_SPLIT_CPML : 0);
@@ -4663,6 +5195,7 @@ struct Stage {
   std::vector<DShot> ds;
   std::vector<int4> work;       // one-step ELASTIC2 / EM2 list, or the 2.5-D list
   std::vector<int4> work2;      // two-step list (ELASTIC2, EM2)
+  std::vector<int4> workm;      // region list (ELASTIC2, EM2)
   std::vector<int> rows_cols;   // receivers by row (ELASTIC2, EM2)
   std::vector<long> rec_off;    // per shot offset into rows_cols, -1 = none
   long long rows_cols_size = 0; // known before the receivers are read
@@ -4737,7 +5270,10 @@ int stage_host(Plan* p, int kind, int prec, const sdt_model* models, int nmodels
     if (least_rows > p->el2_eh) {  // shorter lists for the fixed scratch
       p->el2_eh = least_rows;
       p->el2_wb = 4;
+      p->multi = false;
     }
+    if (p->multi) S.workm = multi_work(p);
+    p->nmulti = (int)S.workm.size();
     S.work = el2_work(p, p->el2_wb, p->el2_eh, p->el2_order);
     const int nblk = (int)S.work.size();
     p->el2_grid = std::max(8, std::min(nblk, SDT_EL2_GRID) / 8 * 8);
@@ -4842,7 +5378,7 @@ int scratch_ptr(unsigned char** out) {
 
 // Offsets of one call's arrays inside the scratch (256-byte aligned).
 struct ScratchLayout {
-  size_t models, shots, work, work2, rec, flags, ints, nel, npsi, total;
+  size_t models, shots, work, work2, workm, rec, flags, ints, nel, npsi, total;
 };
 ScratchLayout scratch_layout(const Plan* p, const Stage& S) {
   auto up = [](size_t v) { return (v + 255) & ~size_t(255); };
@@ -4852,6 +5388,7 @@ ScratchLayout scratch_layout(const Plan* p, const Stage& S) {
   L.shots = o;  o = up(o + sizeof(DShot) * p->nshots);
   L.work = o;   o = up(o + sizeof(int4) * S.work.size());
   L.work2 = o;  o = up(o + sizeof(int4) * S.work2.size());
+  L.workm = o;  o = up(o + sizeof(int4) * S.workm.size());
   L.rec = o;    o = up(o + sizeof(int) * (size_t)S.rows_cols_size);
   L.flags = o;  o = up(o + sizeof(int) * p->nshots);
   L.ints = o;   o = up(o + 2 * sizeof(int));
@@ -4923,6 +5460,12 @@ int sdt_plan_create(int kind, int prec, const sdt_model* models, int nmodels,
             hipSuccess)
       return bail(fail(SDT_EDEVICE, "hipMalloc/hipMemcpy failed (work list)"));
   }
+  if (!S.workm.empty()) {
+    if (hipMalloc(&p->dwmulti, sizeof(int4) * S.workm.size()) != hipSuccess ||
+        hipMemcpy(p->dwmulti, S.workm.data(), sizeof(int4) * S.workm.size(), hipMemcpyHostToDevice) !=
+            hipSuccess)
+      return bail(fail(SDT_EDEVICE, "hipMalloc/hipMemcpy failed (work list)"));
+  }
   hipLaunchKernelGGL(k_fill_int, dim3((nshots + 255) / 256), dim3(256), 0, nullptr, p->dflags,
                      nshots, INT_MAX);
   hipLaunchKernelGGL(k_set_int2, dim3(1), dim3(1), 0, nullptr, p->dbase, 0, p->dit0, 0);
@@ -4941,34 +5484,30 @@ int sdt_plan_run(void* plan, int it0, int nsteps, int graph_block, void* stream)
   hipStream_t st = static_cast<hipStream_t>(stream);
   p->last = st;
   if (nsteps == 0) return SDT_OK;
-  const bool two = use_two(p, nsteps, graph_block);
-  start_of_run(p, st, it0, two);
+  const int mode = run_mode(p, nsteps, graph_block);
+  start_of_run(p, st, it0, mode != 0);
   hipLaunchKernelGGL(k_set_int2, dim3(1), dim3(1), 0, st, p->dbase, it0, p->dit0, it0);
   int done = 0;
   if (graph_block > 1 && nsteps >= graph_block) {
-    if (p->graph_block != graph_block || !p->gexec || p->graph_two != two) {
+    if (p->graph_block != graph_block || !p->gexec || p->graph_mode != mode) {
       if (p->gexec) { (void)hipGraphExecDestroy(p->gexec); p->gexec = nullptr; }
       if (p->graph) { (void)hipGraphDestroy(p->graph); p->graph = nullptr; }
       HIP_TRY(hipStreamBeginCapture(p->cap, hipStreamCaptureModeThreadLocal));
-      if (two)
-        launch_pairs(p, p->cap, graph_block);
-      else
-        launch_steps(p, p->cap, graph_block);
+      launch_run(p, p->cap, graph_block, mode, true);
       hipLaunchKernelGGL(k_add_int, dim3(1), dim3(1), 0, p->cap, p->dbase, graph_block);
       HIP_TRY(hipStreamEndCapture(p->cap, &p->graph));
       HIP_TRY(hipGraphInstantiate(&p->gexec, p->graph, nullptr, nullptr, 0));
       p->graph_block = graph_block;
-      p->graph_two = two;
+      p->graph_mode = mode;
     }
     for (; done + graph_block <= nsteps; done += graph_block) HIP_TRY(hipGraphLaunch(p->gexec, st));
   }
+  int final_b = mode == 2 ? 0 : mode == 1 ? (nsteps / 2 + (nsteps & 1)) & 1 : -1;
   if (done < nsteps) {
-    if (two)
-      launch_pairs(p, st, nsteps - done);
-    else
-      launch_steps(p, st, nsteps - done);
+    const int b = launch_run(p, st, nsteps - done, mode, false);
+    if (mode == 2) final_b = b;
   }
-  end_of_run(p, st, it0 + nsteps, two ? ((nsteps / 2 + (nsteps & 1)) & 1) : -1);
+  end_of_run(p, st, it0 + nsteps, final_b);
   HIP_TRY(hipGetLastError());
   return SDT_OK;
 }
@@ -5097,6 +5636,7 @@ int sdt_run_noalloc(int kind, int prec, const sdt_model* models, int nmodels,
   p->dshots = reinterpret_cast<DShot*>(base + L.shots);
   p->dwork = reinterpret_cast<int4*>(base + L.work);
   p->dwork2 = S.work2.empty() ? nullptr : reinterpret_cast<int4*>(base + L.work2);
+  p->dwmulti = S.workm.empty() ? nullptr : reinterpret_cast<int4*>(base + L.workm);
   p->drec = S.rows_cols.empty() ? nullptr : reinterpret_cast<int*>(base + L.rec);
   p->dflags = reinterpret_cast<int*>(base + L.flags);
   p->dbase = reinterpret_cast<int*>(base + L.ints);
@@ -5113,6 +5653,9 @@ int sdt_run_noalloc(int kind, int prec, const sdt_model* models, int nmodels,
   if (p->dwork2)
     HIP_TRY(hipMemcpyAsync(p->dwork2, S.work2.data(), sizeof(int4) * S.work2.size(),
                            hipMemcpyHostToDevice, st));
+  if (p->dwmulti)
+    HIP_TRY(hipMemcpyAsync(p->dwmulti, S.workm.data(), sizeof(int4) * S.workm.size(),
+                           hipMemcpyHostToDevice, st));
   if (p->drec)
     HIP_TRY(hipMemcpyAsync(p->drec, S.rows_cols.data(), sizeof(int) * S.rows_cols.size(),
                            hipMemcpyHostToDevice, st));
@@ -5123,13 +5666,9 @@ int sdt_run_noalloc(int kind, int prec, const sdt_model* models, int nmodels,
   hipLaunchKernelGGL(k_fill_int, dim3((nshots + 255) / 256), dim3(256), 0, st, p->dflags, nshots, INT_MAX);
   hipLaunchKernelGGL(k_set_int2, dim3(1), dim3(1), 0, st, p->dbase, it0, p->dit0, it0);
   if (nsteps > 0) {
-    const bool two = use_two(p, nsteps, 0);
-    start_of_run(p, st, it0, two);
-    if (two)
-      launch_pairs(p, st, nsteps);
-    else
-      launch_steps(p, st, nsteps);
-    end_of_run(p, st, it0 + nsteps, two ? ((nsteps / 2 + (nsteps & 1)) & 1) : -1);
+    const int mode = run_mode(p, nsteps, 0);
+    start_of_run(p, st, it0, mode != 0);
+    end_of_run(p, st, it0 + nsteps, launch_run(p, st, nsteps, mode, false));
   }
   HIP_TRY(hipGetLastError());
   std::vector<int> f(nshots);
@@ -5489,6 +6028,7 @@ void sdt_plan_destroy(void* plan) {
   if (p->dshots) (void)hipFree(p->dshots);
   if (p->dwork) (void)hipFree(p->dwork);
   if (p->dwork2) (void)hipFree(p->dwork2);
+  if (p->dwmulti) (void)hipFree(p->dwmulti);
   if (p->dit0) (void)hipFree(p->dit0);
   if (p->drec) (void)hipFree(p->drec);
   if (p->dflags) (void)hipFree(p->dflags);
