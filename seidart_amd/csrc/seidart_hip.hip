@@ -180,6 +180,14 @@ __device__ __forceinline__ void check_blowup(double v2, int* flag, int it) {
   if (!(v2 <= 1.0e50)) atomicMin(flag, it);
 }
 
+// The work item of this block in a launch over n consecutive items, -1 for
+// none (the grid is n rounded up to a multiple of 8): each XCD (blockIdx % 8)
+// takes a contiguous run of them.
+__device__ __forceinline__ int item8(int n) {
+  const int run = (int)(gridDim.x >> 3), q = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
+  return q < n ? q : -1;
+}
+
 // slab offset helpers: position of column i inside the two x slabs
 __device__ __forceinline__ int slab_pos(int i, int n, int l) { return i < l ? i : i - n + 2 * l; }
 __device__ __forceinline__ bool in_slab(int i, int n, int l) { return i < l || i >= n - l; }
@@ -1194,16 +1202,6 @@ __device__ __forceinline__ void gadd(__attribute__((address_space(1))) double* g
 __device__ __forceinline__ void gadd(__attribute__((address_space(1))) float* g, double v) {
   gadd((float*)g, v);
 }
-// gradient products in FP32 (not FP64) before the FP32 staging add: a
-// measured option, off by default
-#ifndef SDT_ADJ_F32PROD
-#define SDT_ADJ_F32PROD 0
-#endif
-#if SDT_ADJ_F32PROD
-__device__ __forceinline__ void gadd(__attribute__((address_space(1))) float* g, float v) {
-  if (v != 0.0f) unsafeAtomicAdd((float*)g, v);
-}
-#endif
 template <typename T>
 struct GAcc;
 template <>
@@ -1539,414 +1537,345 @@ k_el2_adj_g(const DModel* __restrict__ models, const DShot* __restrict__ shots,
 
 // ---------------------------------------------------------------------------
 // Fused adjoint step: the same transpose as the three kernels above, in one
-// pass.  A wavefront owns AW columns (lanes 2..AW+1; two halo lanes on each
-// side) of eh rows of one shot and marches down them.  At march row r it
-// does V^T of row r, the stress gathers with S^T / N^T of row r-1 and the
-// velocity gather of row r-2, keeping the few rows each phase needs from
-// the previous ones in registers and taking x neighbours from the
-// neighbouring lanes.  The halo lanes and the two halo rows above and below
-// the tile are recomputed, so tiles are independent (lambda ping-pongs).
-// Only owned cells write lambda_t and add to the gradient.
+// launch.  A block holds 64 columns x AR rows of one shot, one cell per thread
+// and one row per wavefront, and owns all but a ring of them (AdjOwn): V^T of
+// every cell, then the stress gathers with S^T and N^T, then the velocity
+// gather.  x neighbours come from the neighbouring lanes, z neighbours through
+// LDS.  Blocks recompute the ring, so they are independent (lambda
+// ping-pongs); only owned cells write lambda_t and add to the gradient.  The
+// residual of the step is added to lambda_{t+1} as it is read.
+// All loads of a cell are issued before the first use, and no load follows a
+// store (loads and stores complete in order, so that a walk down the rows
+// waits for the gradient's atomics with every row).  Against wavefronts
+// walking tiles of 1 to 64 rows (us per step, elastic FP32 with six gradient
+// slots then EM FP64 with four): 120x90 14.7 -> 10.0 and 15.8 -> 5.1, 740x440
+// x 6 shots 73 -> 51 and 90 -> 53, 1064x552 x 16 shots 260 -> 209 and 322 -> 221;
+// elastic FP64 16.3 -> 10.5, 133 -> 107, 423 -> 422.  Bound at the largest: 0.53
+// GB of state (106 us at 5 TB/s, 186 without the gradient) and the atomics (22
+// us for six slots); at the smallest three dependent scalar loads, one round
+// of loads and two barriers.
 // ---------------------------------------------------------------------------
-#ifndef SDT_ADJ_WAVES_PER_SIMD
-#define SDT_ADJ_WAVES_PER_SIMD 3
-#endif
-#ifndef SDT_ADJ_AW
-#define SDT_ADJ_AW 60
-#endif
-constexpr int AW = SDT_ADJ_AW;   // owned columns per wavefront
-static_assert(AW >= 1 && AW <= 60, "adjoint wavefront: two halo lanes on each side");
-constexpr int AWB = 4;   // wavefronts per block, side by side in x
+// Rows of a block: 16 where two such blocks fit on a CU (elastic FP32, 64
+// registers), else 8, of which two to four fit.  Measured (us per step, blocks
+// of 8 / 12 / 16 rows): elastic FP32 120x90 8.4 / 9.6 / 9.9, 1064x552 x 16 shots 227
+// / 231 / 203 (legacy C-PML); FP64 740x440 x 6 shots 105 / 115 / 104, 120x90 10.0 /
+// 12.2 / 12.9; EM FP32 x 6 shots 29 / 31 / 29, FP64 54 / 53 / 59, 120x90 5.2 / 6.2 / 7.0.
+template <typename T, bool EM>
+constexpr int AR = !EM && sizeof(T) == 4 ? 16 : 8;
 
-// One march row of the fused adjoint, shared by the one-step kernel and by
-// both stages of the two-step kernel.  Inputs of march row r: lambda_{t+1}
-// of the velocities of row r, of the stresses of row q = r - 1, the memory
-// adjoints of row r (the stress-derivative memories the velocity update
-// uses) and of row q (the velocity-derivative memories, with the shear
-// loop's own four in the split variant).  Outputs: lambda_t of the
-// velocities of row r - 2, of the stresses of row q, and the memory adjoints
-// of rows r and q.
+// Owned cells of a block: columns x0 .. x0 + w - 1, rows 1 .. h of its 64 x AR.
+// The stress adjoints of a row and column need V^T one cell away, the
+// velocities those of their neighbours: a ring of one cell.  The legacy C-PML
+// passes the shear loop's memory adjoints on to the normal loop's, which
+// reaches one cell further to the west and to the south.
+template <int ROWS, bool LEGACY>
+struct AdjOwn {
+  static constexpr int x0 = LEGACY ? 2 : 1, w = 63 - x0, h = LEGACY ? ROWS - 3 : ROWS - 2;
+};
+template <typename T, bool SPLIT>
+using ElAdjOwn = AdjOwn<AR<T, false>, !SPLIT>;
 template <typename T>
-struct AdjRow {
-  T lvx = 0, lvz = 0, lsxx = 0, lszz = 0, lsxz = 0;
-  T x2 = 0, x3 = 0, z2 = 0, z3 = 0;                                  // row r
-  T x0 = 0, x1 = 0, z0 = 0, z1 = 0, sx0 = 0, sx1 = 0, sz0 = 0, sz1 = 0;  // row q
+using EmAdjOwn = AdjOwn<AR<T, true>, false>;
+
+// The residuals of step t of the receivers on this wavefront's row r of the
+// grid, summed per column: lane l's column is xl + l.  buf: 2 x 64 of the
+// wavefront's own.
+template <typename T>
+__device__ __forceinline__ void adj_residual(const DShot& S, const DAdj& A, int t, int r, int xl, int lane,
+                                             T* b0, T* b1, T& a0, T& a1) {
+  const int q0 = S.rrow[r], q1 = S.rrow[r + 1];
+  if (q1 <= q0) return;
+  const auto res = cp<T>(A.resid) + (long)t * 2 * S.nrec;
+  b0[lane] = 0;
+  b1[lane] = 0;
+  __builtin_amdgcn_wave_barrier();
+  for (int e = q0 + lane; e < q1; e += 64) {
+    const int l = S.rxid[2 * e] - xl, id = S.rxid[2 * e + 1];
+    if (l >= 0 && l < 64) {
+      atomicAdd(&b0[l], res[id]);
+      atomicAdd(&b1[l], res[S.nrec + id]);
+    }
+  }
+  __builtin_amdgcn_wave_barrier();
+  a0 += b0[lane];
+  a1 += b1[lane];
+}
+
+template <typename T>
+struct ElAdjLds {
+  static constexpr int R = AR<T, false>;
+  T u[4][R][64];   // u_t's vx, vz; u_{t+1}'s sxz, szz
+  T bd[2][R][64];  // V^T: adjoints of dsxz_dz (at vx), dszz_dz (at vz)
+  T ef[4][R][64];  // stress phase: adjoints of dvz_dz, dvx_dz (normal), dvz_dz, dvx_dz (shear)
 };
 
+// PML false: no cell of the block lies in a slab or outside the grid's inner cells.
 template <typename T, bool SPLIT, bool PML>
-struct AdjStage {
-  using GT = typename std::conditional<sizeof(T) == 4 && SDT_ADJ_F32PROD, float, double>::type;
-  using GP = typename std::remove_pointer<decltype(GAcc<T>::of(std::declval<const DAdj&>()))>::type;
-  const DShot& S;
-  const DAdj& A;
-  const int nx, nz, i, ic, lx, lz;
-  const bool incol, sl, inx;
-  const uint32_t n, SX, SZ, ZB, xs;
-  const A32<const T> u1, u0;
-  const A32<GP> G;
-  T ikx, ax, bx, ikxh, axh, bxh, idx, idz, dt;
-  gcptr<T> ikz, az, bz, ikzh, azh, bzh, brow;
-  const A32<const T> N11, N13, N15, N33, N35, S15, S35, S55, DTX, DTZ, OMX, OMZ;
-  const bool mono, atten;
-  // windows (rows relative to the march row r)
-  T A1 = 0, B1 = 0, C1 = 0, D1 = 0, D2 = 0;      // A, B, C, D of row r-1; D of r-2
-  T pvx1 = 0, pvz1 = 0, pvx2 = 0, pvz2 = 0;      // partial lambda_v of rows r-1, r-2
-  T vx_m = 0, vz_m = 0, vx_c = 0, vz_c = 0;      // u_t velocities of rows r-2, r-1
-  T sxz_p = 0, szz_c = 0;                        // u_{t+1} sxz of row r-1, szz of row r
-  T E1p = 0, E2p = 0, E3p = 0, E4p = 0, F1p = 0, F2p = 0, F3p = 0, F4p = 0;  // row r-2
-  T F2pp = 0, F4pp = 0;                                                      // row r-3
-  // per march row: rows, validity and memory offsets of rows r and q
-  int rs = 0, qs = 0;
-  bool vr = false, vq = false, inzr = false, inzq = false;
-  uint32_t cr = 0, cq = 0, cn = 0, oxr = 0, oxq = 0, ozr = 0, ozq = 0;
-
-  // u1 = the trail slot of u_{t+1}, u0 that of u_t; r0 = the first march row
-  __device__ __forceinline__ AdjStage(const DModel& M, const DShot& S_, const DAdj& A_, int xo, int lane,
-                                      const T* u1p, const T* u0p, int r0)
-      : S(S_), A(A_), nx(M.nx), nz(M.nz), i(xo - 2 + lane),
-        ic(i >= 0 && i < M.nx ? i : (i < 0 ? 0 : M.nx - 1)), lx(M.lx), lz(M.lz),
-        incol(i >= 0 && i < M.nx), sl(incol && lane >= 1 && lane <= 2 + AW),
-        inx(PML && incol && in_slab(i, M.nx, M.lx)), n((uint32_t)M.nx * M.nz),
-        SX((uint32_t)M.nz * 2 * M.lx), SZ((uint32_t)2 * M.lz * M.nx),
-        ZB(5 * n + (SPLIT ? 6 : 4) * SX), xs(5 * n + (inx ? slab_pos(i, M.nx, M.lx) : 0)),
-        u1(u1p), u0(u0p), G(GAcc<T>::of(A_)), N11(M.coef[0]), N13(M.coef[1]), N15(M.coef[2]),
-        N33(M.coef[3]), N35(M.coef[4]), S15(M.coef[5]), S35(M.coef[6]), S55(M.coef[7]),
-        DTX(M.coef[8]), DTZ(M.coef[9]), OMX(M.coef[10]), OMZ(M.coef[11]),
-        mono(M.coef[2] != nullptr), atten(M.coef[10] != nullptr) {
-    const Prof<T> P(&M.prof[0][0]);
+__device__ __forceinline__ void el2_adj_block(const DModel& M, const DShot& S, const DAdj& A, const int x0,
+                                              const int z0, const int t, const int t0, const int tb,
+                                              const unsigned gmask, ElAdjLds<T>& L) {
+  using Own = ElAdjOwn<T, SPLIT>;
+  constexpr int R = AR<T, false>;
+  const int nx = M.nx, nz = M.nz, lx = M.lx, lz = M.lz;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = x0 + lane, r = z0 + w;
+  const bool in = !PML || (i >= 0 && i < nx && r >= 0 && r < nz);
+  const int ic = PML ? min(max(i, 0), nx - 1) : i, rc = PML ? min(max(r, 0), nz - 1) : r;
+  const bool own = in && lane >= Own::x0 && lane < Own::x0 + Own::w && w >= 1 && w <= Own::h;
+  // 32-bit element offsets within one state / gradient array (checked at setup)
+  const uint32_t n = (uint32_t)nx * nz, c = (uint32_t)rc * nx + ic;
+  const A32<const T> Li(A.lam[(t + 1) & 1]);
+  const A32<T> Lo(A.lam[t & 1]);
+  const T* trail = static_cast<const T*>(A.trail[tb]);
+  const A32<const T> u1(trail + (long)(t + 1 - t0) * A.slot), u0(trail + (long)(t - t0) * A.slot);
+  T lvx = Li[c], lvz = Li[n + c];
+  T lsxx = Li[2 * n + c], lszz = Li[3 * n + c], lsxz = Li[4 * n + c];
+  const T sxx1 = u1[2 * n + c], szz1 = u1[3 * n + c], sxz1 = u1[4 * n + c];
+  const T vx = u0[c], vz = u0[n + c];
+  const bool mono = M.coef[2] != nullptr, atten = M.coef[10] != nullptr;
+  const T dtx = A32<const T>(M.coef[8])[c], dtz = A32<const T>(M.coef[9])[c];
+  const T omx = atten ? A32<const T>(M.coef[10])[c] : T(1), omz = atten ? A32<const T>(M.coef[11])[c] : T(1);
+  const T n11 = A32<const T>(M.coef[0])[c], n13 = A32<const T>(M.coef[1])[c], n33 = A32<const T>(M.coef[3])[c];
+  const T s55 = A32<const T>(M.coef[7])[c];
+  const T n15 = mono ? A32<const T>(M.coef[2])[c] : T(0), n35 = mono ? A32<const T>(M.coef[4])[c] : T(0);
+  const T s15 = mono ? A32<const T>(M.coef[5])[c] : T(0), s35 = mono ? A32<const T>(M.coef[6])[c] : T(0);
+  // memory variables: offsets, and profiles of the column and of the row
+  const bool inx = PML && in && in_slab(i, nx, lx), inz = PML && in && in_slab(r, nz, lz);
+  const uint32_t SX = (uint32_t)nz * 2 * lx, SZ = (uint32_t)2 * lz * nx;
+  const uint32_t ox = 5 * n + (inx ? (uint32_t)r * 2 * lx + slab_pos(i, nx, lx) : 0);
+  const uint32_t oz = 5 * n + (SPLIT ? 6 : 4) * SX + (inz ? (uint32_t)slab_pos(r, nz, lz) * nx + i : 0);
+  const Prof<T> P(&M.prof[0][0]);
+  T ikx = 0, ax = 0, bx = 0, ikxh = 0, axh = 0, bxh = 0, ikz = 0, az = 0, bz = 0, ikzh = 0, azh = 0, bzh = 0;
+  if (inx) {
     ikx = P[PK][ic]; ax = P[PA][ic]; bx = P[PB][ic];
     ikxh = P[PKH][ic]; axh = P[PAH][ic]; bxh = P[PBH][ic];
-    ikz = P[12 + PK]; az = P[12 + PA]; bz = P[12 + PB];
-    ikzh = P[12 + PKH]; azh = P[12 + PAH]; bzh = P[12 + PBH];
-    brow = cp<T>(M.aux);
-    idx = T(1.0 / M.dx); idz = T(1.0 / M.dz); dt = T(M.dt);
-    sxz_p = valid(r0 - 1) ? u1[4 * n + rowi(r0 - 1)] : T(0);
-    szz_c = valid(r0) ? u1[3 * n + rowi(r0)] : T(0);
   }
-  __device__ __forceinline__ uint32_t rowi(int r) const {
-    return (uint32_t)(r < 0 ? 0 : (r >= nz ? nz - 1 : r)) * nx + ic;
+  if (inz) {
+    ikz = P[12 + PK][rc]; az = P[12 + PA][rc]; bz = P[12 + PB][rc];
+    ikzh = P[12 + PKH][rc]; azh = P[12 + PAH][rc]; bzh = P[12 + PBH][rc];
   }
-  __device__ __forceinline__ bool valid(int r) const { return incol && r >= 0 && r < nz; }
-  __device__ __forceinline__ int clampr(int r) const { return r < 0 ? 0 : (r >= nz ? nz - 1 : r); }
+  const T idx = T(1.0 / M.dx), idz = T(1.0 / M.dz), dt = T(M.dt);
+  const A32<typename std::remove_pointer<decltype(GAcc<T>::of(A))>::type> G(GAcc<T>::of(A));
+  if (S.nrec > 0 && A.resid && r >= 0 && r < nz)
+    adj_residual<T>(S, A, t, r, x0, lane, L.ef[0][w], L.ef[1][w], lvx, lvz);
 
-  // rows, validity and memory offsets of march row r
-  __device__ __forceinline__ void prep(int r) {
-    const int q = r - 1;
-    cr = rowi(r); cq = rowi(q); cn = rowi(r + 1);
-    vr = valid(r); vq = valid(q);
-    rs = clampr(r); qs = clampr(q);
-    inzr = PML && incol && in_slab(rs, nz, lz);
-    inzq = PML && incol && in_slab(qs, nz, lz);
-    oxr = xs + (inx ? (uint32_t)rs * 2 * lx : 0);
-    oxq = xs + (inx ? (uint32_t)qs * 2 * lx : 0);
-    ozr = ZB + (inzr ? (uint32_t)slab_pos(rs, nz, lz) * nx + ic : 0);
-    ozq = ZB + (inzq ? (uint32_t)slab_pos(qs, nz, lz) * nx + ic : 0);
+  // ---- V^T: velocity updates, seismicfdtd.f95:317-375 ----
+  const bool edge = PML && (i <= 0 || i >= nx - 1 || r <= 0 || r >= nz - 1);
+  if (edge) lvx = lvz = 0;
+  if (own && i == S.isrc && r == S.ksrc && A.gsrc) {
+    A.gsrc[3 * (long)t + 0] = (double)lvx;
+    A.gsrc[3 * (long)t + 2] = (double)lvz;
   }
-
-  // the inputs of the prepared row from a lambda state (slab loads only
-  // where the cell has that memory: a zero-width slab has no storage)
-  __device__ __forceinline__ void load(const A32<const T>& L, AdjRow<T>& in) const {
-    in.lvx = L[cr]; in.lvz = L[n + cr];
-    in.lsxx = L[2 * n + cq]; in.lszz = L[3 * n + cq]; in.lsxz = L[4 * n + cq];
-    in.x2 = inx ? L[oxr + 2 * SX] : T(0); in.x3 = inx ? L[oxr + 3 * SX] : T(0);
-    in.z2 = inzr ? L[ozr + 2 * SZ] : T(0); in.z3 = inzr ? L[ozr + 3 * SZ] : T(0);
-    in.x0 = inx ? L[oxq] : T(0); in.x1 = inx ? L[oxq + SX] : T(0);
-    in.z0 = inzq ? L[ozq] : T(0); in.z1 = inzq ? L[ozq + SZ] : T(0);
-    if (SPLIT) {
-      in.sx0 = inx ? L[oxq + 4 * SX] : T(0);
-      in.sx1 = inx ? L[oxq + 5 * SX] : T(0);
-      in.sz0 = inzq ? L[ozq + 4 * SZ] : T(0);
-      in.sz1 = inzq ? L[ozq + 5 * SZ] : T(0);
+  const bool dox = !PML || (in && i >= 1 && r >= 1), doz = !PML || (in && i <= nx - 2 && r <= nz - 2);
+  T An = 0, Bn = 0, Cn = 0, Dn = 0, pvx = lvx, pvz = lvz;
+  if (dox) {
+    const T q = dtx * lvx;
+    An = q;
+    Bn = q;
+    pvx = omx * lvx;
+    if (inx) {
+      const T lr = Li[ox + 2 * SX] + q;
+      An = ikx * q + ax * lr;
+      if (own) Lo[ox + 2 * SX] = bx * lr;
     }
-  }
-
-  // One march row (prepared): V^T of row r, the stress gathers with S^T and
-  // N^T of row q (from march row qmin on), the velocity gather of row r-2.
-  // Gradient terms are added for the cells of rows [g0, g1) on the lanes
-  // where `own`; the source gradient of step tg likewise.
-  __device__ __forceinline__ void row(const int r, const AdjRow<T>& in, AdjRow<T>& o, const bool own,
-                                      const int g0, const int g1, const int qmin, const int tg,
-                                      const unsigned gmask) {
-    const int q = r - 1;
-    // ---- loads ----
-    const T dtx = DTX[cr], dtz = DTZ[cr];
-    const T omx = atten ? OMX[cr] : T(1), omz = atten ? OMZ[cr] : T(1);
-    const T sxx1 = u1[2 * n + cr], sxz1 = u1[4 * n + cr], szz1n = u1[3 * n + cn];
-    const T vx_n = vr ? u0[cr] : T(0), vz_n = vr ? u0[n + cr] : T(0);
-    const T n11 = N11[cq], n13 = N13[cq], n33 = N33[cq], s55 = S55[cq];
-    const T n15 = mono ? N15[cq] : T(0), n35 = mono ? N35[cq] : T(0);
-    const T s15 = mono ? S15[cq] : T(0), s35 = mono ? S35[cq] : T(0);
-    // psi of the velocity row r (stress-derivative memory) and of the stress
-    // row q (velocity-derivative memory)
-    const T Ux2 = inx ? u1[oxr + 2 * SX] : T(0), Ux3 = inx ? u1[oxr + 3 * SX] : T(0);
-    const T Uz2 = inzr ? u1[ozr + 2 * SZ] : T(0), Uz3 = inzr ? u1[ozr + 3 * SZ] : T(0);
-    const uint32_t xq2 = SPLIT ? 4 * SX : 0, zq2 = SPLIT ? 4 * SZ : 0;  // shear loop's arrays
-    const T Ox0 = inx ? u0[oxq] : T(0), Ox1 = inx ? u0[oxq + SX] : T(0);
-    const T Oz0 = inzq ? u0[ozq] : T(0), Oz1 = inzq ? u0[ozq + SZ] : T(0);
-    const T Qx0 = inx ? u1[oxq + xq2] : T(0), Qx1 = inx ? u1[oxq + xq2 + SX] : T(0);
-    const T Qz0 = inzq ? u1[ozq + zq2] : T(0), Qz1 = inzq ? u1[ozq + zq2 + SZ] : T(0);
-    const T browq = SPLIT ? bxh : brow[qs];
-    const T bzr = bz[rs], azr = az[rs], ikzr = ikz[rs], bzhr = bzh[rs], azhr = azh[rs], ikzhr = ikzh[rs];
-    const T bzq = bz[qs], azq = az[qs], ikzq = ikz[qs], bzhq = bzh[qs], azhq = azh[qs], ikzhq = ikzh[qs];
-    // neighbour values (wave-wide shuffles, outside any branch)
-    const T sxx1_w = lane_prev(sxx1), sxz1_e = lane_next(sxz1);
-    const T A1_e = lane_next(A1), C1_w = lane_prev(C1);
-    const T vx_cw = lane_prev(vx_c), vz_cw = lane_prev(vz_c);
-    const T vx_ce = lane_next(vx_c), vz_ce = lane_next(vz_c);
-    const T E1p_w = lane_prev(E1p), E3p_w = lane_prev(E3p);
-    const T F1p_e = lane_next(F1p), F3p_e = lane_next(F3p);
-
-    // ---- V^T of row r: velocity updates, seismicfdtd.f95:317-375 ----
-    const bool ownr = own && r >= g0 && r < g1;
-    const bool edge = (i == 0 || i == nx - 1 || r == 0 || r == nz - 1);
-    const T lvx = (vr && !edge) ? in.lvx : T(0), lvz = (vr && !edge) ? in.lvz : T(0);
-    T An = 0, Bn = 0, Cn = 0, Dn = 0, pvx = lvx, pvz = lvz;
-    if (ownr && i == S.isrc && r == S.ksrc && A.gsrc) {
-      A.gsrc[3 * (long)tg + 0] = (double)lvx;
-      A.gsrc[3 * (long)tg + 2] = (double)lvz;
+    if (inz) {
+      const T lr = Li[oz + 3 * SZ] + q;
+      Bn = ikz * q + az * lr;
+      if (own) Lo[oz + 3 * SZ] = bz * lr;
     }
-    o.x2 = in.x2; o.z3 = in.z3; o.x3 = in.x3; o.z2 = in.z2;
-    if (vr && i >= 1 && r >= 1) {
-      const T w = dtx * lvx;
-      An = w;
-      Bn = w;
-      T b1 = (sxx1 - sxx1_w) * idx, b2 = (sxz1 - sxz_p) * idz;
+  } else if (own) {
+    if (inx) Lo[ox + 2 * SX] = Li[ox + 2 * SX];
+    if (inz) Lo[oz + 3 * SZ] = Li[oz + 3 * SZ];
+  }
+  if (doz) {
+    const T q = dtz * lvz;
+    Cn = q;
+    Dn = q;
+    pvz = omz * lvz;
+    if (inx) {
+      const T lr = Li[ox + 3 * SX] + q;
+      Cn = ikxh * q + axh * lr;
+      if (own) Lo[ox + 3 * SX] = bxh * lr;
+    }
+    if (inz) {
+      const T lr = Li[oz + 2 * SZ] + q;
+      Dn = ikzh * q + azh * lr;
+      if (own) Lo[oz + 2 * SZ] = bzh * lr;
+    }
+  } else if (own) {
+    if (inx) Lo[ox + 3 * SX] = Li[ox + 3 * SX];
+    if (inz) Lo[oz + 2 * SZ] = Li[oz + 2 * SZ];
+  }
+  L.u[0][w][lane] = vx;
+  L.u[1][w][lane] = vz;
+  L.u[2][w][lane] = sxz1;
+  L.u[3][w][lane] = szz1;
+  L.bd[0][w][lane] = Bn;
+  L.bd[1][w][lane] = Dn;
+  __syncthreads();
+
+  // ---- stresses: gathers, then S^T and N^T, :247-312 ----
+  const int wu = w > 0 ? w - 1 : 0, wd = w < R - 1 ? w + 1 : R - 1;
+  const T A_e = dpp_next(An), C_w = dpp_prev(Cn);
+  const T vx_w = dpp_prev(vx), vz_w = dpp_prev(vz), vx_e = dpp_next(vx), vz_e = dpp_next(vz);
+  const T sxx_w = dpp_prev(sxx1), sxz_e = dpp_next(sxz1);
+  lsxx += idx * (An - A_e);
+  lszz += idz * (L.bd[1][wu][lane] - Dn);
+  lsxz += idz * (Bn - L.bd[0][wd][lane]) + idx * (C_w - Cn);
+  if (own) {
+    if (dox) {
+      T b1 = (sxx1 - sxx_w) * idx, b2 = (sxz1 - L.u[2][wu][lane]) * idz;
+      if (inx) b1 = ikx * b1 + u1[ox + 2 * SX];
+      if (inz) b2 = ikz * b2 + u1[oz + 3 * SZ];
+      if (gmask & (1u << 8)) gadd(&G[8 * n + c], (double)lvx * (double)(b1 + b2));
+      if (gmask & (1u << 10)) gadd(&G[10 * n + c], (double)lvx * (double)vx);
+    }
+    if (doz) {
+      T b1 = (sxz_e - sxz1) * idx, b2 = (L.u[3][wd][lane] - szz1) * idz;
+      if (inx) b1 = ikxh * b1 + u1[ox + 3 * SX];
+      if (inz) b2 = ikzh * b2 + u1[oz + 2 * SZ];
+      if (gmask & (1u << 9)) gadd(&G[9 * n + c], (double)lvz * (double)(b1 + b2));
+      if (gmask & (1u << 11)) gadd(&G[11 * n + c], (double)lvz * (double)vz);
+    }
+    Lo[2 * n + c] = lsxx;
+    Lo[3 * n + c] = lszz;
+    Lo[4 * n + c] = lsxz;
+  }
+  T E1 = 0, E2 = 0, E3 = 0, E4 = 0, F1 = 0, F2 = 0, F3 = 0, F4 = 0;
+  const bool dos = !PML || (in && r <= nz - 2 && i >= 1), don = !PML || (in && r >= 1 && i <= nx - 2);
+  // memory adjoints: the shear loop's own four if split, then the normal
+  // loop's; one set for both loops otherwise
+  const uint32_t xq = SPLIT ? 4 * SX : 0, zq = SPLIT ? 4 * SZ : 0;
+  T q1 = 0, q2 = 0, q3 = 0, q4 = 0;
+  if (inx) { q1 = Li[ox + xq]; q3 = Li[ox + xq + SX]; }
+  if (inz) { q2 = Li[oz + zq]; q4 = Li[oz + zq + SZ]; }
+  if (dos) {  // S^T
+    const T mu = dt * lsxz;
+    T g1 = (vx - vx_w) * idx, g2 = (L.u[1][wd][lane] - vz) * idz;
+    T g3 = (vz - vz_w) * idx, g4 = (L.u[0][wd][lane] - vx) * idz;
+    const T lg1 = s15 * mu, lg2 = s35 * mu, lg3 = s55 * mu;
+    F1 = lg1; F2 = lg2; F3 = lg3; F4 = lg3;
+    if (inx) {
+      T l = q1 + lg1;
+      F1 = ikxh * lg1 + axh * l;
+      q1 = bxh * l;
+      l = q3 + lg3;
+      F3 = ikx * lg3 + ax * l;
+      q3 = bx * l;
+    }
+    if (inz) {
+      T l = q2 + lg2;
+      F2 = ikz * lg2 + az * l;
+      q2 = bz * l;
+      l = q4 + lg3;
+      F4 = ikzh * lg3 + azh * l;
+      q4 = bzh * l;
+    }
+    if (own) {
       if (inx) {
-        const T lr = in.x2 + w;
-        An = ikx * w + ax * lr;
-        o.x2 = bx * lr;
-        b1 = ikx * b1 + Ux2;
+        g1 = ikxh * g1 + u1[ox + xq];
+        g3 = ikx * g3 + u1[ox + xq + SX];
       }
-      if (inzr) {
-        const T lr = in.z3 + w;
-        Bn = ikzr * w + azr * lr;
-        o.z3 = bzr * lr;
-        b2 = ikzr * b2 + Uz3;
+      if (inz) {
+        g2 = ikz * g2 + u1[oz + zq];
+        g4 = ikzh * g4 + u1[oz + zq + SZ];
       }
-      pvx = omx * lvx;
-      if (ownr) {
-        if (gmask & (1u << 8)) gadd(&G[8 * n + cr], (GT)lvx * (GT)(b1 + b2));
-        if (gmask & (1u << 10)) gadd(&G[10 * n + cr], (GT)lvx * (GT)vx_n);
-      }
-    }
-    if (vr && i <= nx - 2 && r <= nz - 2) {
-      const T w = dtz * lvz;
-      Cn = w;
-      Dn = w;
-      T b1 = (sxz1_e - sxz1) * idx, b2 = (szz1n - szz_c) * idz;
-      if (inx) {
-        const T lr = in.x3 + w;
-        Cn = ikxh * w + axh * lr;
-        o.x3 = bxh * lr;
-        b1 = ikxh * b1 + Ux3;
-      }
-      if (inzr) {
-        const T lr = in.z2 + w;
-        Dn = ikzhr * w + azhr * lr;
-        o.z2 = bzhr * lr;
-        b2 = ikzhr * b2 + Uz2;
-      }
-      pvz = omz * lvz;
-      if (ownr) {
-        if (gmask & (1u << 9)) gadd(&G[9 * n + cr], (GT)lvz * (GT)(b1 + b2));
-        if (gmask & (1u << 11)) gadd(&G[11 * n + cr], (GT)lvz * (GT)vz_n);
-      }
-    }
-
-    // ---- stresses of row q: gathers, then S^T and N^T, :247-312 ----
-    T Ee1 = 0, Ee2 = 0, Ee3 = 0, Ee4 = 0, Ff1 = 0, Ff2 = 0, Ff3 = 0, Ff4 = 0;
-    o.lsxx = 0; o.lszz = 0; o.lsxz = 0;
-    o.x0 = in.x0; o.x1 = in.x1; o.z0 = in.z0; o.z1 = in.z1;
-    o.sx0 = in.sx0; o.sx1 = in.sx1; o.sz0 = in.sz0; o.sz1 = in.sz1;
-    if (sl && vq && q >= qmin) {
-      const bool ownq = own && q >= g0 && q < g1;
-      const T lsxx = in.lsxx + idx * (A1 - A1_e);
-      const T lszz = in.lszz + idz * (D2 - D1);
-      const T lsxz = in.lsxz + idz * (B1 - Bn) + idx * (C1_w - C1);
-      o.lsxx = lsxx; o.lszz = lszz; o.lsxz = lsxz;
-      T lm1 = in.x0, lm3 = in.x1, lm2 = in.z0, lm4 = in.z1;     // normal loop's psi adjoints
-      T ls1 = in.sx0, ls3 = in.sx1, ls2 = in.sz0, ls4 = in.sz1;  // shear loop's (split)
-      T& k1 = SPLIT ? ls1 : lm1;
-      T& k2 = SPLIT ? ls2 : lm2;
-      T& k3 = SPLIT ? ls3 : lm3;
-      T& k4 = SPLIT ? ls4 : lm4;
-      if (q <= nz - 2 && i >= 1) {  // S^T
-        const T mu = dt * lsxz;
-        const T f1 = (vx_c - vx_cw) * idx, f2 = (vz_n - vz_c) * idz;
-        const T f3 = (vz_c - vz_cw) * idx, f4 = (vx_n - vx_c) * idz;
-        const T lg1 = s15 * mu, lg2 = s35 * mu, lg3 = s55 * mu;
-        T g1 = f1, g2 = f2, g3 = f3, g4 = f4;
-        Ff1 = lg1; Ff2 = lg2; Ff3 = lg3; Ff4 = lg3;
-        if (inx) {
-          g1 = ikxh * f1 + Qx0;
-          T l = k1 + lg1;
-          Ff1 = ikxh * lg1 + axh * l;
-          k1 = bxh * l;
-          g3 = ikx * f3 + Qx1;
-          l = k3 + lg3;
-          Ff3 = ikx * lg3 + ax * l;
-          k3 = bx * l;
-        }
-        if (inzq) {
-          g2 = ikzq * f2 + Qz0;
-          T l = k2 + lg2;
-          Ff2 = ikzq * lg2 + azq * l;
-          k2 = bzq * l;
-          g4 = ikzhq * f4 + Qz1;
-          l = k4 + lg3;
-          Ff4 = ikzhq * lg3 + azhq * l;
-          k4 = bzhq * l;
-        }
-        if (ownq) {
-          const GT m = (GT)mu;
-          if (gmask & (1u << 5)) gadd(&G[5 * n + cq], m * (GT)g1);
-          if (gmask & (1u << 6)) gadd(&G[6 * n + cq], m * (GT)g2);
-          if (gmask & (1u << 7)) gadd(&G[7 * n + cq], m * ((GT)g3 + (GT)g4));
-        }
-      }
-      if (q >= 1 && i <= nx - 2) {  // N^T
-        const T mux = dt * lsxx, muz = dt * lszz;
-        const T e1 = (vx_ce - vx_c) * idx, e2 = (vz_c - vz_m) * idz;
-        const T e3 = (vz_ce - vz_c) * idx, e4 = (vx_c - vx_m) * idz;
-        const T ld1 = n11 * mux + n13 * muz, ld2 = n13 * mux + n33 * muz, lsh = n15 * mux + n35 * muz;
-        T d1 = e1, d2 = e2, d3 = e3, d4 = e4;
-        Ee1 = ld1; Ee2 = ld2; Ee3 = lsh; Ee4 = lsh;
-        if (inx) {
-          d1 = ikxh * e1 + (browq * Ox0 + axh * e1);
-          T l = lm1 + ld1;
-          Ee1 = ikxh * ld1 + axh * l;
-          lm1 = browq * l;
-          d3 = ikx * e3 + (bx * Ox1 + ax * e3);
-          l = lm3 + lsh;
-          Ee3 = ikx * lsh + ax * l;
-          lm3 = bx * l;
-        }
-        if (inzq) {
-          d2 = ikzq * e2 + (bzq * Oz0 + azq * e2);
-          T l = lm2 + ld2;
-          Ee2 = ikzq * ld2 + azq * l;
-          lm2 = bzq * l;
-          d4 = ikzhq * e4 + (bzhq * Oz1 + azhq * e4);
-          l = lm4 + lsh;
-          Ee4 = ikzhq * lsh + azhq * l;
-          lm4 = bzhq * l;
-        }
-        if (ownq) {
-          const GT mx = (GT)mux, mz = (GT)muz, sh = (GT)d3 + (GT)d4;
-          if (gmask & (1u << 0)) gadd(&G[cq], mx * (GT)d1);
-          if (gmask & (1u << 1)) gadd(&G[n + cq], mx * (GT)d2 + mz * (GT)d1);
-          if (gmask & (1u << 2)) gadd(&G[2 * n + cq], mx * sh);
-          if (gmask & (1u << 3)) gadd(&G[3 * n + cq], mz * (GT)d2);
-          if (gmask & (1u << 4)) gadd(&G[4 * n + cq], mz * sh);
-        }
-      }
-      o.x0 = lm1; o.x1 = lm3; o.z0 = lm2; o.z1 = lm4;
-      o.sx0 = ls1; o.sx1 = ls3; o.sz0 = ls2; o.sz1 = ls4;
-    }
-
-    // ---- velocities of row r-2: gather of the stress-phase adjoints ----
-    o.lvx = pvx2 + idx * (E1p_w - E1p) + idz * (E4p - Ee4) + idx * (F1p - F1p_e) + idz * (F4pp - F4p);
-    o.lvz = pvz2 + idz * (E2p - Ee2) + idx * (E3p_w - E3p) + idz * (F2pp - F2p) + idx * (F3p - F3p_e);
-
-    // ---- shift the windows ----
-    F2pp = F2p; F4pp = F4p;
-    E1p = Ee1; E2p = Ee2; E3p = Ee3; E4p = Ee4;
-    F1p = Ff1; F2p = Ff2; F3p = Ff3; F4p = Ff4;
-    pvx2 = pvx1; pvz2 = pvz1; pvx1 = pvx; pvz1 = pvz;
-    A1 = An; B1 = Bn; C1 = Cn; D2 = D1; D1 = Dn;
-    vx_m = vx_c; vz_m = vz_c; vx_c = vx_n; vz_c = vz_n;
-    sxz_p = sxz1; szz_c = szz1n;
-  }
-
-  // Store the outputs of the prepared march row r into a lambda state for
-  // the cells of rows [g0, g1) on the lanes where `own`.
-  __device__ __forceinline__ void store(const A32<T>& L, const int r, const AdjRow<T>& o, const bool own,
-                                        const int g0, const int g1) const {
-    const int q = r - 1, pr = r - 2;
-    if (own && r >= g0 && r < g1) {
-      if (inx) { L[oxr + 2 * SX] = o.x2; L[oxr + 3 * SX] = o.x3; }
-      if (inzr) { L[ozr + 3 * SZ] = o.z3; L[ozr + 2 * SZ] = o.z2; }
-    }
-    if (own && q >= g0 && q < g1) {
-      L[2 * n + cq] = o.lsxx;
-      L[3 * n + cq] = o.lszz;
-      L[4 * n + cq] = o.lsxz;
-      if (inx) {
-        L[oxq] = o.x0;
-        L[oxq + SX] = o.x1;
-        if (SPLIT) {
-          L[oxq + 4 * SX] = o.sx0;
-          L[oxq + 5 * SX] = o.sx1;
-        }
-      }
-      if (inzq) {
-        L[ozq] = o.z0;
-        L[ozq + SZ] = o.z1;
-        if (SPLIT) {
-          L[ozq + 4 * SZ] = o.sz0;
-          L[ozq + 5 * SZ] = o.sz1;
-        }
-      }
-    }
-    if (own && pr >= g0 && pr < g1) {
-      const uint32_t cp_ = rowi(pr);
-      L[cp_] = o.lvx;
-      L[n + cp_] = o.lvz;
+      if (gmask & (1u << 5)) gadd(&G[5 * n + c], (double)mu * (double)g1);
+      if (gmask & (1u << 6)) gadd(&G[6 * n + c], (double)mu * (double)g2);
+      if (gmask & (1u << 7)) gadd(&G[7 * n + c], (double)mu * ((double)g3 + (double)g4));
     }
   }
-};
+  if (SPLIT) {
+    if (own && inx) { Lo[ox + xq] = q1; Lo[ox + xq + SX] = q3; }
+    if (own && inz) { Lo[oz + zq] = q2; Lo[oz + zq + SZ] = q4; }
+    if (inx) { q1 = Li[ox]; q3 = Li[ox + SX]; }
+    if (inz) { q2 = Li[oz]; q4 = Li[oz + SZ]; }
+  }
+  if (don) {  // N^T
+    const T mux = dt * lsxx, muz = dt * lszz;
+    const T ld1 = n11 * mux + n13 * muz, ld2 = n13 * mux + n33 * muz, lsh = n15 * mux + n35 * muz;
+    T d1 = (vx_e - vx) * idx, d2 = (vz - L.u[1][wu][lane]) * idz;
+    T d3 = (vz_e - vz) * idx, d4 = (vx - L.u[0][wu][lane]) * idz;
+    E1 = ld1; E2 = ld2; E3 = lsh; E4 = lsh;
+    // (the legacy normal loop's decay of memory_dvx_dx: b_x_half by row, :255)
+    T bxn = bxh;
+    if (inx) {
+      if (!SPLIT) bxn = cp<T>(M.aux)[rc];
+      T l = q1 + ld1;
+      E1 = ikxh * ld1 + axh * l;
+      q1 = bxn * l;
+      l = q3 + lsh;
+      E3 = ikx * lsh + ax * l;
+      q3 = bx * l;
+    }
+    if (inz) {
+      T l = q2 + ld2;
+      E2 = ikz * ld2 + az * l;
+      q2 = bz * l;
+      l = q4 + lsh;
+      E4 = ikzh * lsh + azh * l;
+      q4 = bzh * l;
+    }
+    if (own) {
+      if (inx) {
+        d1 = ikxh * d1 + (bxn * u0[ox] + axh * d1);
+        d3 = ikx * d3 + (bx * u0[ox + SX] + ax * d3);
+      }
+      if (inz) {
+        d2 = ikz * d2 + (bz * u0[oz] + az * d2);
+        d4 = ikzh * d4 + (bzh * u0[oz + SZ] + azh * d4);
+      }
+      const double mx = (double)mux, mz = (double)muz, sh = (double)d3 + (double)d4;
+      if (gmask & (1u << 0)) gadd(&G[c], mx * (double)d1);
+      if (gmask & (1u << 1)) gadd(&G[n + c], mx * (double)d2 + mz * (double)d1);
+      if (gmask & (1u << 2)) gadd(&G[2 * n + c], mx * sh);
+      if (gmask & (1u << 3)) gadd(&G[3 * n + c], mz * (double)d2);
+      if (gmask & (1u << 4)) gadd(&G[4 * n + c], mz * sh);
+    }
+  }
+  if (own && inx) { Lo[ox] = q1; Lo[ox + SX] = q3; }
+  if (own && inz) { Lo[oz] = q2; Lo[oz + SZ] = q4; }
+  L.ef[0][w][lane] = E2;
+  L.ef[1][w][lane] = E4;
+  L.ef[2][w][lane] = F2;
+  L.ef[3][w][lane] = F4;
+  __syncthreads();
 
-template <typename T, bool SPLIT, bool PML>
-__device__ __forceinline__ void el2_adj_tile(const DModel* __restrict__ models,
-                                             const DShot* __restrict__ shots,
-                                             const DAdj* __restrict__ adj, const int s, const int xo,
-                                             const int zo, const int eh, const int t, const int t0,
-                                             const unsigned gmask, const int lane, const int tb) {
-  const DShot& S = shots[s];
-  const DModel& M = models[S.model];
-  const DAdj& A = adj[s];
-  const int zend = min(zo + eh, M.nz);
-  const A32<const T> Lin(A.lam[(t + 1) & 1]);
-  const A32<T> Lout(A.lam[t & 1]);
-  const T* trail = static_cast<const T*>(A.trail[tb]);
-  AdjStage<T, SPLIT, PML> st(M, S, A, xo, lane, trail + (long)(t + 1 - t0) * A.slot,
-                             trail + (long)(t - t0) * A.slot, zo - 2);
-  const bool own = st.incol && lane >= 2 && lane < 2 + AW;
-  for (int r = zo - 2; r <= zend + 1; ++r) {
-    st.prep(r);
-    AdjRow<T> in, o;
-    st.load(Lin, in);
-    st.row(r, in, o, own, zo, zend, zo - 1, t, gmask);
-    st.store(Lout, r, o, own, zo, zend);
+  // ---- velocities: gather of the stress-phase adjoints ----
+  const T E1_w = dpp_prev(E1), E3_w = dpp_prev(E3), F1_e = dpp_next(F1), F3_e = dpp_next(F3);
+  if (own) {
+    Lo[c] = pvx + idx * (E1_w - E1) + idz * (E4 - L.ef[1][wd][lane]) + idx * (F1 - F1_e) +
+            idz * (L.ef[3][wu][lane] - F4);
+    Lo[n + c] = pvz + idz * (E2 - L.ef[0][wd][lane]) + idx * (E3_w - E3) + idz * (L.ef[2][wu][lane] - F2) +
+                idx * (F3 - F3_e);
   }
 }
 
+// Whether the block at (x0, z0) avoids every slab and the grid's outer cells:
+// it runs the body without memory variables and edge predicates.
+__device__ __forceinline__ bool adj_interior(const DModel& M, int x0, int z0, int rows) {
+  return x0 >= max(M.lx, 1) && x0 + 64 <= M.nx - max(M.lx, 2) && z0 >= max(M.lz, 1) &&
+         z0 + rows <= M.nz - max(M.lz, 2);
+}
+
 template <typename T, bool SPLIT>
-__global__ void __launch_bounds__(64 * AWB, sizeof(T) == 4 ? SDT_ADJ_WAVES_PER_SIMD : 2)
-k_el2_adj(const DModel* __restrict__ models, const DShot* __restrict__ shots,
-          const DAdj* __restrict__ adj, const int4* __restrict__ work, int nitems,
-          const int* __restrict__ tbase, int k, unsigned gmask, const int* __restrict__ tsel) {
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int t0 = __builtin_amdgcn_readfirstlane(*tbase);
-  const int tb = __builtin_amdgcn_readfirstlane(*tsel);
-  const int t = t0 + k;
-  for (int w = blockIdx.x; w < nitems; w += gridDim.x) {
-    const int4 wv = work[w];
-    const int s = __builtin_amdgcn_readfirstlane(wv.x);
-    const int xo = __builtin_amdgcn_readfirstlane(wv.y) + wave * AW;
-    const int zo = __builtin_amdgcn_readfirstlane(wv.z), eh = __builtin_amdgcn_readfirstlane(wv.w);
-    if (s < 0) continue;
-    const DModel& M = models[shots[s].model];
-    if (xo >= M.nx) continue;
-    // a wave whose columns and rows (halo included) avoid every C-PML slab
-    // runs the body without memory variables
-    const bool interior = xo - 2 >= M.lx && xo + 61 < M.nx - M.lx && zo - 3 >= M.lz &&
-                          zo + eh + 2 < M.nz - M.lz;
-    if (interior)
-      el2_adj_tile<T, SPLIT, false>(models, shots, adj, s, xo, zo, eh, t, t0, gmask, threadIdx.x & 63, tb);
-    else
-      el2_adj_tile<T, SPLIT, true>(models, shots, adj, s, xo, zo, eh, t, t0, gmask, threadIdx.x & 63, tb);
-  }
+__global__ void __launch_bounds__((64 * AR<T, false>), sizeof(T) == 4 ? 8 : 4)
+k_el2_adj(const DModel* __restrict__ models, const DShot* __restrict__ shots, const DAdj* __restrict__ adj,
+          const int4* __restrict__ work, int nitems, const int* __restrict__ tbase, int k, unsigned gmask,
+          const int* __restrict__ tsel) {
+  __shared__ ElAdjLds<T> L;
+  const int q = item8(nitems);
+  if (q < 0) return;
+  const int4 wv = work[q];
+  const int s = __builtin_amdgcn_readfirstlane(wv.x);
+  const int t0 = __builtin_amdgcn_readfirstlane(*tbase), tb = __builtin_amdgcn_readfirstlane(*tsel);
+  const DModel& M = models[__builtin_amdgcn_readfirstlane(wv.w)];
+  const int x0 = __builtin_amdgcn_readfirstlane(wv.y) - ElAdjOwn<T, SPLIT>::x0;
+  const int z0 = __builtin_amdgcn_readfirstlane(wv.z) - 1;
+  if (adj_interior(M, x0, z0, AR<T, false>))
+    el2_adj_block<T, SPLIT, false>(M, shots[s], adj[s], x0, z0, t0 + k, t0, tb, gmask, L);
+  else
+    el2_adj_block<T, SPLIT, true>(M, shots[s], adj[s], x0, z0, t0 + k, t0, tb, gmask, L);
 }
 
 // ===========================================================================
@@ -2446,14 +2375,6 @@ __host__ __device__ inline int ychunk_pack(int j0, int j1) {
 __host__ __device__ inline int ychunk_j0(int w) { return (int)((unsigned)w & 0xffffu); }
 __host__ __device__ inline int ychunk_j1(int w) { return (int)((unsigned)w >> 16); }
 
-// The work item of this block in a launch over n consecutive items, -1 for
-// none (the grid is n rounded up to a multiple of 8): each XCD (blockIdx % 8)
-// takes a contiguous run of them.
-__device__ __forceinline__ int item25(int n) {
-  const int run = (int)(gridDim.x >> 3), q = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
-  return q < n ? q : -1;
-}
-
 struct Slab3 {
   long SX, SY, SZ;       // elements per memory-variable array on each axis
   long bx, by, bz;       // base offsets of the x, y, z groups
@@ -2771,7 +2692,7 @@ template <typename T>
 __global__ void __launch_bounds__(NT25, WS25<T>)
 k_el25_stress(const DModel* __restrict__ models, const DShot* __restrict__ shots,
           const int4* __restrict__ work, int n, const int* __restrict__ base, int rel) {
-  const int q = item25(n);
+  const int q = item8(n);
   if (q < 0) return;
   const int4 wv = work[q];
   const int s = __builtin_amdgcn_readfirstlane(wv.x);
@@ -2933,7 +2854,7 @@ template <typename T>
 __global__ void __launch_bounds__(NT25, WV25<T>)
 k_el25_vel(const DModel* __restrict__ models, const DShot* __restrict__ shots,
           const int4* __restrict__ work, int n, const int* __restrict__ base, int rel) {
-  const int q = item25(n);
+  const int q = item8(n);
   if (q < 0) return;
   const int4 wv = work[q];
   const int s = __builtin_amdgcn_readfirstlane(wv.x);
@@ -3225,7 +3146,7 @@ __global__ void __launch_bounds__(RM* RM, sizeof(T) == 4 ? 8 : 4)
 k_el2_multi(const DModel* __restrict__ models, const DShot* __restrict__ shots, const int4* __restrict__ work,
             int n, const int* __restrict__ base, int rel, int nsteps, int tm, int par) {
   __shared__ ElRegionLds<T> L;
-  const int q = item25(n);
+  const int q = item8(n);
   if (q < 0) return;
   const int4 wv = work[q];
   const DShot& S = shots[__builtin_amdgcn_readfirstlane(wv.x)];
@@ -3364,7 +3285,7 @@ __global__ void __launch_bounds__(RM* RM, 8)
 k_em2_multi(const DModel* __restrict__ models, const DShot* __restrict__ shots, const int4* __restrict__ work,
             int n, const int* __restrict__ base, int rel, int nsteps, int tm, int par) {
   __shared__ EmRegionLds<T> L;
-  const int q = item25(n);
+  const int q = item8(n);
   if (q < 0) return;
   const int4 wv = work[q];
   const DShot& S = shots[__builtin_amdgcn_readfirstlane(wv.x)];
@@ -3542,201 +3463,167 @@ k_em2_adj_g(const DModel* __restrict__ models, const DShot* __restrict__ shots,
 }
 
 // ---------------------------------------------------------------------------
-// Fused EM2 adjoint step: the transpose of k_em2_adj_{e,h,g} in one pass,
-// the same arithmetic in the same order.  A wavefront owns AW columns
-// (lanes 2..AW+1; lane l holds column xo - 2 + l) of eh rows of one shot and
-// marches down them (eh rows: the plan picks the height that gives it
-// enough tiles): at march row q it does E^T of row q, H^T of row q-1
-// (which reads the E^T results of rows q-1 and q and of column i+1) and the
-// E gather of row q-1 (the H^T results of rows q-2 and q-1 and of column
-// i-1).  E^T at column i reads the new Hy of column i-1, so two halo lanes on
-// the left and one on the right give exact results on the owned lanes; the
-// halo row above the tile is recomputed, so tiles are independent (lambda
-// ping-pongs).  Only owned cells write lambda_t and add to the gradient.
+// Fused EM2 adjoint step: the transpose of k_em2_adj_{e,h,g} in one launch, on
+// blocks of 64 columns x AR rows like k_el2_adj: E^T of every cell, H^T (which
+// reads the E^T results of the cells to the east and south), the E gather
+// (the H^T results of the cells to the west and north).  Blocks own all but a
+// ring of one cell.
 // ---------------------------------------------------------------------------
+template <typename T>
+struct EmAdjLds {
+  static constexpr int R = AR<T, true>;
+  T wx[R][64], hy[R][64], la[R][64];  // E^T's adjoint of dHy_dz; u_{t+1}'s Hy; H^T's of dEx_dz
+  T rs[2][R][64];                     // adj_residual
+};
+
 template <typename T, bool PML>
-__device__ __forceinline__ void em2_adj_tile(const DModel* __restrict__ models,
-                                             const DShot* __restrict__ shots,
-                                             const DAdj* __restrict__ adj, const int s, const int xo,
-                                             const int zo, const int eh, const int t, const int t0,
-                                             const unsigned gmask, const int lane, const int tb) {
-  const DShot& S = shots[s];
-  const DModel& M = models[S.model];
-  const DAdj& A = adj[s];
-  const int nx = M.nx, nz = M.nz;
-  const int i = xo - 2 + lane;
-  const bool incol = (i >= 0 && i < nx);
-  const int ic = incol ? i : (i < 0 ? 0 : nx - 1);
-  const bool own = incol && lane >= 2 && lane < 2 + AW;
-  const int zend = min(zo + eh, nz);
+__device__ __forceinline__ void em2_adj_block(const DModel& M, const DShot& S, const DAdj& A, const int x0,
+                                              const int z0, const int t, const int t0, const int tb,
+                                              const unsigned gmask, EmAdjLds<T>& L) {
+  using Own = EmAdjOwn<T>;
+  constexpr int R = AR<T, true>;
+  const int nx = M.nx, nz = M.nz, lx = M.lx, lz = M.lz;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = x0 + lane, r = z0 + w;
+  const bool in = !PML || (i >= 0 && i < nx && r >= 0 && r < nz);
+  const int ic = PML ? min(max(i, 0), nx - 1) : i, rc = PML ? min(max(r, 0), nz - 1) : r;
+  const bool own = in && lane >= Own::x0 && lane < Own::x0 + Own::w && w >= 1 && w <= Own::h;
   // 32-bit element offsets within one state / gradient array (checked at setup)
-  const uint32_t n = (uint32_t)nx * nz;
-  const int lx = M.lx, lz = M.lz;
+  const uint32_t n = (uint32_t)nx * nz, c = (uint32_t)rc * nx + ic;
+  const A32<const T> Li(A.lam[(t + 1) & 1]);
+  const A32<T> Lo(A.lam[t & 1]);
+  const T* trail = static_cast<const T*>(A.trail[tb]);
+  const A32<const T> u1(trail + (long)(t + 1 - t0) * A.slot), u0(trail + (long)(t - t0) * A.slot);
+  T lex = Li[c], lez = Li[n + c], lh = Li[2 * n + c];
+  const T hy = u1[2 * n + c];
+  const T uex = u0[c], uez = u0[n + c];
+  const T cax = A32<const T>(M.coef[0])[c], cbx = A32<const T>(M.coef[1])[c];
+  const T caz = A32<const T>(M.coef[2])[c], cbz = A32<const T>(M.coef[3])[c];
+  const bool inx = PML && in && in_slab(i, nx, lx), inz = PML && in && in_slab(r, nz, lz);
   const uint32_t SX = (uint32_t)nz * 2 * lx, SZ = (uint32_t)2 * lz * nx;
-  const A32<const T> Lin(A.lam[(t + 1) & 1]);
-  const A32<T> Lout(A.lam[t & 1]);
-  const A32<const T> u1(static_cast<const T*>(A.trail[tb]) + (long)(t + 1 - t0) * A.slot);
-  const A32<const T> u0(static_cast<const T*>(A.trail[tb]) + (long)(t - t0) * A.slot);
-  const A32<typename std::remove_pointer<decltype(GAcc<T>::of(A))>::type> G(GAcc<T>::of(A));
+  const uint32_t ox = 3 * n + (inx ? (uint32_t)r * 2 * lx + slab_pos(i, nx, lx) : 0);
+  const uint32_t oz = 3 * n + 2 * SX + (inz ? (uint32_t)slab_pos(r, nz, lz) * nx + i : 0);
   const Prof<T> P(&M.prof[0][0]);
-  const bool inx = PML && incol && in_slab(i, nx, lx);
-  const uint32_t xs = inx ? slab_pos(i, nx, lx) : 0;
-  const T ikx = P[PK][ic], ax = P[PA][ic], bx = P[PB][ic];
-  const T ikxh = P[PKH][ic], axh = P[PAH][ic], bxh = P[PBH][ic];
-  const auto ikz = P[12 + PK], az = P[12 + PA], bz = P[12 + PB];
-  const auto ikzh = P[12 + PKH], azh = P[12 + PAH], bzh = P[12 + PBH];
-  const A32<const T> CAX(M.coef[0]), CBX(M.coef[1]), CAZ(M.coef[2]), CBZ(M.coef[3]);
+  T ikx = 0, ax = 0, bx = 0, ikxh = 0, axh = 0, bxh = 0, ikz = 0, az = 0, bz = 0, ikzh = 0, azh = 0, bzh = 0;
+  T lx0 = 0, lx1 = 0, lz0 = 0, lz1 = 0, ux1 = 0, uz1 = 0;
+  if (inx) {
+    ikx = P[PK][ic]; ax = P[PA][ic]; bx = P[PB][ic];
+    ikxh = P[PKH][ic]; axh = P[PAH][ic]; bxh = P[PBH][ic];
+    lx0 = Li[ox]; lx1 = Li[ox + SX]; ux1 = u1[ox + SX];
+  }
+  if (inz) {
+    ikz = P[12 + PK][rc]; az = P[12 + PA][rc]; bz = P[12 + PB][rc];
+    ikzh = P[12 + PKH][rc]; azh = P[12 + PAH][rc]; bzh = P[12 + PBH][rc];
+    lz0 = Li[oz]; lz1 = Li[oz + SZ]; uz1 = u1[oz + SZ];
+  }
   const T idx = T(1.0 / M.dx), idz = T(1.0 / M.dz), dbh = T(M.scal[0]);
-  auto row = [&](int r) { return (uint32_t)(r < 0 ? 0 : (r >= nz ? nz - 1 : r)) * nx + ic; };
-  auto clampr = [&](int r) { return r < 0 ? 0 : (r >= nz ? nz - 1 : r); };
+  const A32<typename std::remove_pointer<decltype(GAcc<T>::of(A))>::type> G(GAcc<T>::of(A));
+  if (S.nrec > 0 && A.resid && r >= 0 && r < nz)
+    adj_residual<T>(S, A, t, r, x0, lane, L.rs[0][w], L.rs[1][w], lex, lez);
 
-  // carried from the previous march row: E^T of row q-1 (adjoints of dHy_dz
-  // at the Ex node, of dHy_dx at the Ez node, and the partial lambda_E), the
-  // H^T result la of row q-2, and u_{t+1}'s Hy of row q-1
-  T wx_p = 0, wz_p = 0, ex_p = 0, ez_p = 0, la_pp = 0;
-  T hy1_p = (incol && zo - 2 >= 0) ? u1[2 * n + row(zo - 2)] : T(0);
-  for (int q = zo - 1; q <= zend; ++q) {
-    // ---- E^T of row q (k_em2_adj_e) ----
-    const bool vq = incol && q >= 0 && q < nz;
-    const int qs = clampr(q);
-    const uint32_t c = row(q);
-    const T hy1 = vq ? u1[2 * n + c] : T(0);
-    const T hy1_w = lane_prev(hy1);  // u_{t+1} Hy(i-1, q)
-    const bool ownq = own && q >= zo && q < zend;
-    T wx = 0, wz = 0, exq = 0, ezq = 0;
-    if (vq) {
-      const bool inz = PML && in_slab(qs, nz, lz);
-      const uint32_t ox = 3 * n + (inx ? (uint32_t)qs * 2 * lx + xs : 0);
-      const uint32_t oz = 3 * n + 2 * SX + (inz ? (uint32_t)slab_pos(qs, nz, lz) * nx + ic : 0);
-      // Dirichlet ring of Ex and Ez (and cells outside their Fortran extent)
-      const bool edx = (i == 0 || i >= nx - 2 || q == 0 || q == nz - 1);
-      const bool edz = (i == 0 || i == nx - 1 || q == 0 || q >= nz - 2);
-      const T lex = edx ? T(0) : Lin[c], lez = edz ? T(0) : Lin[n + c];
-      if (ownq && A.gsrc && i == S.isrc && q == S.ksrc) {
-        A.gsrc[3 * (long)t + 0] = (double)lex;
-        A.gsrc[3 * (long)t + 2] = (double)lez;
-      }
-      if (q >= 1 && q <= nz - 2 && i <= nx - 2) {  // Ex node, :273-283
-        const T ld = CBX[c] * lex;
-        const T d = (hy1 - hy1_p) * idz;
-        T D = d;
-        wx = ld;
-        if (inz) {
-          const T lr = Lin[oz + SZ] + ld;
-          wx = ikzh[qs] * ld + azh[qs] * lr;
-          if (ownq) Lout[oz + SZ] = bzh[qs] * lr;
-          D = ikzh[qs] * d + u1[oz + SZ];
-        }
-        if (ownq) {
-          if (gmask & 1u) gadd(&G[c], (double)lex * (double)u0[c]);
-          if (gmask & 2u) gadd(&G[n + c], (double)lex * (double)D);
-        }
-        exq = CAX[c] * lex;
-      } else {
-        if (ownq && inz) Lout[oz + SZ] = Lin[oz + SZ];
-        exq = lex;
-      }
-      if (q <= nz - 2 && i >= 1 && i <= nx - 2) {  // Ez node, :285-295
-        const T le = CBZ[c] * lez;
-        const T e = (hy1 - hy1_w) * idx;
-        T E = e;
-        wz = le;
-        if (inx) {
-          const T lr = Lin[ox + SX] + le;
-          wz = ikxh * le + axh * lr;
-          if (ownq) Lout[ox + SX] = bxh * lr;
-          E = ikxh * e + u1[ox + SX];
-        }
-        if (ownq) {
-          if (gmask & 4u) gadd(&G[2 * n + c], (double)lez * (double)u0[n + c]);
-          if (gmask & 8u) gadd(&G[3 * n + c], (double)lez * (double)E);
-        }
-        ezq = CAZ[c] * lez;
-      } else {
-        if (ownq && inx) Lout[ox + SX] = Lin[ox + SX];
-        ezq = lez;
-      }
+  // ---- E^T (k_em2_adj_e); the Dirichlet ring of Ex and Ez and the cells
+  // outside their extent pass nothing on ----
+  if (PML && (i <= 0 || i >= nx - 2 || r <= 0 || r >= nz - 1)) lex = 0;
+  if (PML && (i <= 0 || i >= nx - 1 || r <= 0 || r >= nz - 2)) lez = 0;
+  if (own && A.gsrc && i == S.isrc && r == S.ksrc) {
+    A.gsrc[3 * (long)t + 0] = (double)lex;
+    A.gsrc[3 * (long)t + 2] = (double)lez;
+  }
+  const bool dox = !PML || (in && r >= 1 && r <= nz - 2 && i <= nx - 2);            // Ex node, :273-283
+  const bool doz = !PML || (in && r <= nz - 2 && i >= 1 && i <= nx - 2);            // Ez node, :285-295
+  T wx = 0, wz = 0, exq = in ? lex : T(0), ezq = in ? lez : T(0);
+  if (dox) {
+    const T ld = cbx * lex;
+    wx = ld;
+    if (inz) {
+      const T lr = lz1 + ld;
+      wx = ikzh * ld + azh * lr;
+      lz1 = bzh * lr;
     }
-
-    // ---- H^T of row r = q-1 (k_em2_adj_h) ----
-    const int r = q - 1;
-    const T wz_e = lane_next(wz_p);  // E^T adjoint of dHy_dx at the Ez node (i+1, r)
-    T la = 0, lb = 0;
-    const bool vr = incol && r >= 0 && r < nz && q >= zo;
-    if (vr) {
-      const bool ownr = own && r >= zo && r < zend;
-      const uint32_t cr = row(r);
-      const bool inz = PML && in_slab(r, nz, lz);
-      const uint32_t ox = 3 * n + (inx ? (uint32_t)r * 2 * lx + xs : 0);
-      const uint32_t oz = 3 * n + 2 * SX + (inz ? (uint32_t)slab_pos(r, nz, lz) * nx + ic : 0);
-      // Hy' feeds the E updates through dHy_dz (Ex node c, c+nx) and dHy_dx (Ez node c, c+1)
-      const T lh = Lin[2 * n + cr] + idz * (wx_p - (r + 1 < nz ? wx : T(0))) +
-                   idx * (wz_p - (i + 1 < nx ? wz_e : T(0)));
-      if (i <= nx - 2 && r <= nz - 2) {  // Hy node, :249-266
-        const bool ring = (i == 0 || i == nx - 2 || r == 0 || r == nz - 2);
-        if (ownr) Lout[2 * n + cr] = ring ? T(0) : lh;
-        const T w = dbh * lh;
-        la = w;
-        lb = w;
-        if (inz) {
-          const T lr = Lin[oz] + w;
-          la = ikz[r] * w + az[r] * lr;
-          if (ownr) Lout[oz] = bz[r] * lr;
-        }
-        if (inx) {
-          const T lr = Lin[ox] + w;
-          lb = ikx * w + ax * lr;
-          if (ownr) Lout[ox] = bx * lr;
-        }
-      } else if (ownr) {
-        Lout[2 * n + cr] = lh;
-        if (inz) Lout[oz] = Lin[oz];
-        if (inx) Lout[ox] = Lin[ox];
-      }
+    exq = cax * lex;
+  }
+  if (doz) {
+    const T le = cbz * lez;
+    wz = le;
+    if (inx) {
+      const T lr = lx1 + le;
+      wz = ikxh * le + axh * lr;
+      lx1 = bxh * lr;
     }
+    ezq = caz * lez;
+  }
+  L.wx[w][lane] = wx;
+  L.hy[w][lane] = hy;
+  __syncthreads();
 
-    // ---- E gather of row r (k_em2_adj_g) ----
-    const T lb_w = lane_prev(lb);  // H^T adjoint of dEz_dx at the Hy node (i-1, r)
-    if (own && r >= zo && r < zend) {
-      const uint32_t cr = row(r);
-      Lout[cr] = ex_p + idz * ((r >= 1 ? la_pp : T(0)) - la);
-      Lout[n + cr] = ez_p + idx * ((i >= 1 ? lb_w : T(0)) - lb);
+  // ---- H^T (k_em2_adj_h): Hy' feeds the E updates through dHy_dz (Ex nodes
+  // of this row and the next) and dHy_dx (Ez nodes of this column and the next) ----
+  const int wu = w > 0 ? w - 1 : 0, wd = w < R - 1 ? w + 1 : R - 1;
+  const T wz_e = dpp_next(wz), hy_w = dpp_prev(hy);
+  lh += idz * (wx - L.wx[wd][lane]) + idx * (wz - wz_e);
+  T la = 0, lb = 0, out = lh;
+  if (!PML || (in && i <= nx - 2 && r <= nz - 2)) {  // Hy node, :249-266
+    if (PML && (i == 0 || i == nx - 2 || r == 0 || r == nz - 2)) out = 0;
+    const T q = dbh * lh;
+    la = q;
+    lb = q;
+    if (inz) {
+      const T lr = lz0 + q;
+      la = ikz * q + az * lr;
+      lz0 = bz * lr;
     }
+    if (inx) {
+      const T lr = lx0 + q;
+      lb = ikx * q + ax * lr;
+      lx0 = bx * lr;
+    }
+  }
+  if (own) {
+    if (dox) {
+      T D = (hy - L.hy[wu][lane]) * idz;
+      if (inz) D = ikzh * D + uz1;
+      if (gmask & 1u) gadd(&G[c], (double)lex * (double)uex);
+      if (gmask & 2u) gadd(&G[n + c], (double)lex * (double)D);
+    }
+    if (doz) {
+      T E = (hy - hy_w) * idx;
+      if (inx) E = ikxh * E + ux1;
+      if (gmask & 4u) gadd(&G[2 * n + c], (double)lez * (double)uez);
+      if (gmask & 8u) gadd(&G[3 * n + c], (double)lez * (double)E);
+    }
+    Lo[2 * n + c] = out;
+    if (inx) { Lo[ox] = lx0; Lo[ox + SX] = lx1; }
+    if (inz) { Lo[oz] = lz0; Lo[oz + SZ] = lz1; }
+  }
+  L.la[w][lane] = la;
+  __syncthreads();
 
-    // ---- shift the windows ----
-    wx_p = wx; wz_p = wz; ex_p = exq; ez_p = ezq;
-    la_pp = la;
-    hy1_p = hy1;
+  // ---- E gather (k_em2_adj_g) ----
+  const T lb_w = dpp_prev(lb);
+  if (own) {
+    Lo[c] = exq + idz * (L.la[wu][lane] - la);
+    Lo[n + c] = ezq + idx * (lb_w - lb);
   }
 }
 
 template <typename T>
-__global__ void __launch_bounds__(64 * AWB)
-k_em2_adj(const DModel* __restrict__ models, const DShot* __restrict__ shots,
-          const DAdj* __restrict__ adj, const int4* __restrict__ work, int nitems,
-          const int* __restrict__ tbase, int k, unsigned gmask, const int* __restrict__ tsel) {
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int t0 = __builtin_amdgcn_readfirstlane(*tbase);
-  const int tb = __builtin_amdgcn_readfirstlane(*tsel);
-  const int t = t0 + k;
-  for (int w = blockIdx.x; w < nitems; w += gridDim.x) {
-    const int4 wv = work[w];
-    const int s = __builtin_amdgcn_readfirstlane(wv.x);
-    const int xo = __builtin_amdgcn_readfirstlane(wv.y) + wave * AW;
-    const int zo = __builtin_amdgcn_readfirstlane(wv.z);
-    const int eh = __builtin_amdgcn_readfirstlane(wv.w);  // tile height
-    if (s < 0) continue;
-    const DModel& M = models[shots[s].model];
-    if (xo >= M.nx) continue;
-    // a wave whose columns and rows (halo included) avoid every C-PML slab
-    // runs the body without memory variables
-    const bool interior = xo - 2 >= M.lx && xo + 61 < M.nx - M.lx && zo - 1 >= M.lz &&
-                          zo + eh < M.nz - M.lz;
-    if (interior)
-      em2_adj_tile<T, false>(models, shots, adj, s, xo, zo, eh, t, t0, gmask, threadIdx.x & 63, tb);
-    else
-      em2_adj_tile<T, true>(models, shots, adj, s, xo, zo, eh, t, t0, gmask, threadIdx.x & 63, tb);
-  }
+__global__ void __launch_bounds__((64 * AR<T, true>), sizeof(T) == 4 ? 8 : 6)
+k_em2_adj(const DModel* __restrict__ models, const DShot* __restrict__ shots, const DAdj* __restrict__ adj,
+          const int4* __restrict__ work, int nitems, const int* __restrict__ tbase, int k, unsigned gmask,
+          const int* __restrict__ tsel) {
+  __shared__ EmAdjLds<T> L;
+  const int q = item8(nitems);
+  if (q < 0) return;
+  const int4 wv = work[q];
+  const int s = __builtin_amdgcn_readfirstlane(wv.x);
+  const int t0 = __builtin_amdgcn_readfirstlane(*tbase), tb = __builtin_amdgcn_readfirstlane(*tsel);
+  const DModel& M = models[__builtin_amdgcn_readfirstlane(wv.w)];
+  const int x0 = __builtin_amdgcn_readfirstlane(wv.y) - EmAdjOwn<T>::x0;
+  const int z0 = __builtin_amdgcn_readfirstlane(wv.z) - 1;
+  if (adj_interior(M, x0, z0, AR<T, true>))
+    em2_adj_block<T, false>(M, shots[s], adj[s], x0, z0, t0 + k, t0, tb, gmask, L);
+  else
+    em2_adj_block<T, true>(M, shots[s], adj[s], x0, z0, t0 + k, t0, tb, gmask, L);
 }
 
 // ===========================================================================
@@ -4047,7 +3934,7 @@ template <typename T>
 __global__ void __launch_bounds__(64)
 k_em25_h(const DModel* __restrict__ models, const DShot* __restrict__ shots,
          const int4* __restrict__ work, int n) {
-  const int q = item25(n);
+  const int q = item8(n);
   if (q < 0) return;
   const int4 wv = work[q];
   const int s = __builtin_amdgcn_readfirstlane(wv.x);
@@ -4063,7 +3950,7 @@ template <typename T>
 __global__ void __launch_bounds__(64)
 k_em25_e(const DModel* __restrict__ models, const DShot* __restrict__ shots,
          const int4* __restrict__ work, int n, const int* __restrict__ base, int rel) {
-  const int q = item25(n);
+  const int q = item8(n);
   if (q < 0) return;
   const int4 wv = work[q];
   const int s = __builtin_amdgcn_readfirstlane(wv.x);
@@ -5043,15 +4930,15 @@ void launch_adjoint_steps(Plan* p, hipStream_t st, int khi, int klo) {
   const dim3 grd((p->maxnx + TX - 1) / TX, (p->maxnz + TZ - 1) / TZ, p->nshots);
   const int* tb = p->dtbase;
   for (int k = khi - 1; k >= klo; --k) {
-    if (p->maxrec > 0)
-      hipLaunchKernelGGL(k_el2_adj_inject<T>, dim3((p->maxrec + 63) / 64, p->nshots), dim3(64), 0,
-                         st, p->dmodels, p->dshots, p->dadj, p->nshots, tb, k);
     if (!(p->adj_flags & SDT_ADJ_REFERENCE)) {
-      hipLaunchKernelGGL((k_el2_adj<T, SPLIT>), dim3(p->nadjwork), dim3(64 * AWB), 0, st,
+      hipLaunchKernelGGL((k_el2_adj<T, SPLIT>), dim3((p->nadjwork + 7) / 8 * 8), dim3(64 * AR<T, false>), 0, st,
                          p->dmodels, p->dshots, p->dadj, p->dadjwork, p->nadjwork, tb, k, p->gmask,
                          p->dtsel_adj);
       continue;
     }
+    if (p->maxrec > 0)
+      hipLaunchKernelGGL(k_el2_adj_inject<T>, dim3((p->maxrec + 63) / 64, p->nshots), dim3(64), 0,
+                         st, p->dmodels, p->dshots, p->dadj, p->nshots, tb, k);
     hipLaunchKernelGGL((k_el2_adj_v<T, SPLIT>), grd, blk, 0, st, p->dmodels, p->dshots, p->dadj,
                        p->nshots, tb, k, p->dtsel_adj);
     hipLaunchKernelGGL((k_el2_adj_s<T, SPLIT>), grd, blk, 0, st, p->dmodels, p->dshots, p->dadj,
@@ -5085,14 +4972,14 @@ void launch_adjoint_em2(Plan* p, hipStream_t st, int khi, int klo) {
   const dim3 grd((p->maxnx + TX - 1) / TX, (p->maxnz + TZ - 1) / TZ, p->nshots);
   const int* tb = p->dtbase;
   for (int k = khi - 1; k >= klo; --k) {
-    if (p->maxrec > 0)
-      hipLaunchKernelGGL(k_el2_adj_inject<T>, dim3((p->maxrec + 63) / 64, p->nshots), dim3(64), 0,
-                         st, p->dmodels, p->dshots, p->dadj, p->nshots, tb, k);
     if (!(p->adj_flags & SDT_ADJ_REFERENCE)) {
-      hipLaunchKernelGGL(k_em2_adj<T>, dim3(p->nadjwork), dim3(64 * AWB), 0, st, p->dmodels,
+      hipLaunchKernelGGL(k_em2_adj<T>, dim3((p->nadjwork + 7) / 8 * 8), dim3(64 * AR<T, true>), 0, st, p->dmodels,
                          p->dshots, p->dadj, p->dadjwork, p->nadjwork, tb, k, p->gmask, p->dtsel_adj);
       continue;
     }
+    if (p->maxrec > 0)
+      hipLaunchKernelGGL(k_el2_adj_inject<T>, dim3((p->maxrec + 63) / 64, p->nshots), dim3(64), 0,
+                         st, p->dmodels, p->dshots, p->dadj, p->nshots, tb, k);
     hipLaunchKernelGGL(k_em2_adj_e<T>, grd, blk, 0, st, p->dmodels, p->dshots, p->dadj, p->nshots,
                        tb, k, p->dtsel_adj, p->gmask);
     hipLaunchKernelGGL(k_em2_adj_h<T>, grd, blk, 0, st, p->dmodels, p->dshots, p->dadj, p->nshots,
@@ -5909,54 +5796,23 @@ int sdt_adjoint_setup(void* plan, const sdt_adj_shot* adj, int nshots, unsigned 
     p->tr_grid = std::max(8, std::min(p->ntrwork, SDT_EL2_GRID) / 8 * 8);
   }
   if (!p->dadjwork) {
-    // (shot, x0, z0, rows) items of AWB * AW columns x rows; the items of one
-    // tile over all shots of its model share blockIdx % 8 (one XCD's L2).
-    // Rows per tile: a tile is a serial walk, so a small plan needs short
-    // ones to fill the device, a large one tall ones (the elastic walk reads
-    // five halo rows per tile).  Elastic: the rows whose walk, times the rounds
-    // the device needs for all blocks at three (FP64 two) blocks per CU, is
-    // shortest.  EM: the tallest that give 1300 blocks.  Measured for one
-    // backward pass of 128 steps (ms; 1 / 2 / 4 / 8 / 16 / 32 / 64 rows): elastic
-    // FP32 160x130 2.6 / 3.0 / 4.3 / 5.1 / 7.7 / 13.3 / 23.1, FP64 740x440 x 2
-    // shots 15.8 / 12.3 / 10.7 / 9.8 / 12.1 / 18.0 / 29.7, x 6 shots 43.1 / 32.4 /
-    // 28.4 / 25.4 / 24.8 / 30.1 / 36.8; EM FP64 1064x808 x 2 shots 12.8 / 11.7 /
-    // 11.9 / 14.1 / 18.2 / 27.5 / 45.8.
-    const int bw = AW * AWB;
-    auto blocks = [&](int rows) {
-      long long n = 0;
-      for (const sdt_shot& S : p->hshots) {
-        const sdt_model& M = p->hmodels[S.model];
-        n += (long long)((M.nx + bw - 1) / bw) * ((M.nz + rows - 1) / rows);
-      }
-      return n;
-    };
-    int eh = 1;
-    if (p->kind == SDT_EM2) {
-      for (int rows : {2, 4, 8, 16, 32})
-        if (blocks(rows) >= 1300) eh = rows;
-    } else {
-      const double room = 256.0 * (p->prec == SDT_FP32 ? 3 : 2);
-      double best = 1e300;
-      for (int rows : {1, 2, 4, 8, 16, 24, 32, 64}) {
-        const double cost = std::max(1.0, blocks(rows) / room) * (rows + 5);
-        if (cost < best) { best = cost; eh = rows; }
-      }
-    }
+    // (shot, x0, z0, model) blocks of the fused adjoint kernel, shot by shot:
+    // an XCD (item8) then works on one shot's states at a time, about 20 arrays
+    // whose pages its translation caches hold.  Measured for 16 shots of 1064x552
+    // elastic FP32 (us per step, blocks of 12 rows): 238, with the blocks of one
+    // tile over all shots next to each other 283 (fewer coefficients and gradient
+    // cells to fetch, but every array of 16 shots in use at once), shots in turn
+    // dealt to all XCDs 245.
+    const bool f32 = p->prec == SDT_FP32, em = p->kind == SDT_EM2;
+    const int bw = em || p->split ? ElAdjOwn<float, true>::w : ElAdjOwn<float, false>::w;
+    const int bh = em ? (f32 ? EmAdjOwn<float>::h : EmAdjOwn<double>::h)
+                 : p->split ? (f32 ? ElAdjOwn<float, true>::h : ElAdjOwn<double, true>::h)
+                            : (f32 ? ElAdjOwn<float, false>::h : ElAdjOwn<double, false>::h);
     std::vector<int4> work;
-    for (int m = 0; m < p->nmodels; ++m) {
-      const sdt_model& M = p->hmodels[m];
-      const int tx = (M.nx + bw - 1) / bw, tz = (M.nz + eh - 1) / eh, ntile = tx * tz;
-      std::vector<int> ms;
-      for (int s = 0; s < p->nshots; ++s)
-        if (p->hshots[s].model == m) ms.push_back(s);
-      if (ms.empty()) continue;
-      for (int tg = 0; tg < (ntile + 7) / 8; ++tg)
-        for (int s : ms)
-          for (int tt = 0; tt < 8; ++tt) {
-            const int t = tg * 8 + tt;
-            work.push_back(t < ntile ? make_int4(s, (t % tx) * bw, (t / tx) * eh, eh)
-                                     : make_int4(-1, 0, 0, 0));
-          }
+    for (int s = 0; s < p->nshots; ++s) {
+      const int m = p->hshots[s].model;
+      for (int z = 0; z < p->hmodels[m].nz; z += bh)
+        for (int x = 0; x < p->hmodels[m].nx; x += bw) work.push_back(make_int4(s, x, z, m));
     }
     HIP_TRY(hipMalloc(&p->dadjwork, sizeof(int4) * work.size()));
     HIP_TRY(hipMemcpy(p->dadjwork, work.data(), sizeof(int4) * work.size(), hipMemcpyHostToDevice));

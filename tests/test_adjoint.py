@@ -604,3 +604,35 @@ def test_adjoint_tile_heights_match_reference_kernels(kind, nx, nz, nshots):
         assert rel_l2(g0[q], g1[q]) < 1e-12, (q, rel_l2(g0[q], g1[q]))
     for a, b in zip(l0, l1):
         assert rel_l2(a, b) < 1e-12
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("fp32", 3e-5)])  # 10 steps of ~50 roundings
+@pytest.mark.parametrize("kind,split", [("elastic2", False), ("elastic2", True), ("em2", False)])
+@pytest.mark.parametrize("nx,nz,npml,nshots", [(12, 9, 2, 1), (63, 15, 4, 2), (124, 27, 1, 1), (187, 70, 8, 3)])
+def test_adjoint_blocks_match_reference_kernels(kind, split, precision, tol, nx, nz, npml, nshots):
+    """The fused adjoint (blocks of 64 columns by 8 or 16 rows) against the
+    unfused kernels at grids of one block, of whole blocks and with
+    remainders; receivers on the rings, the source cell and twice on one
+    cell, more of them on one row than a wavefront has lanes."""
+    p = tiny_problem(kind, seed=96, nx=nx, nz=nz, npml=npml, nt=10, nshots=nshots, nrec=5,
+                     src=(nx // 2, 0, nz // 2), gamma=1e-3 if kind == "elastic2" else 0.0)
+    p.cpml_split = split
+    row = [(i, nz // 3) for i in range(nx)]
+    for sh in p.shots:
+        i, _, k = sh.src
+        pts = [(0, 0), (nx - 1, nz - 1), (nx - 2, 1), (i, k), (i, k), (i, k), (1, nz - 2)] + row[::-1]
+        sh.rec = np.array([[x, 0, z] for x, z in pts], dtype=np.int32)
+    out = []
+    for ref in (False, True):
+        eng = _engine(p, precision, every=4, reference=ref)
+        g = torch.Generator().manual_seed(13)
+        for s in range(eng.nshots):
+            eng.init[s].copy_(torch.randn(eng.init[s].numel(), generator=g, dtype=torch.float64))
+        tr = eng.forward()
+        grad, gsrc = eng.backward([torch.randn(t.shape, generator=g, dtype=torch.float64) for t in tr])
+        out.append([x.cpu().numpy().copy() for x in [*grad[0], *gsrc]] +
+                   [eng.adjoint_state(s).cpu().double().numpy() for s in range(nshots)])
+        eng.close()
+    for q, (a, b) in enumerate(zip(*out)):
+        assert rel_l2(a, b) < tol, (q, rel_l2(a, b))
