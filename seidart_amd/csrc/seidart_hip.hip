@@ -285,20 +285,16 @@ __device__ __forceinline__ T dpp_prev(T v) {
   }
 }
 
-template <typename T, bool TRAIL, bool SPLIT, bool PML, bool R1>
+template <typename T, bool SPLIT, bool PML, bool R1>
 __device__ __forceinline__ void el2_tile(const DModel* __restrict__ models,
                                          const DShot* __restrict__ shots, const int4 wi, const int it,
-                                         const int lane, const DAdj* __restrict__ adj, const int slot,
-                                         const int tb, const int eh, const int par);
+                                         const int lane, const int eh, const int par);
 
 // Work: a block of WB wavefronts takes one item (shot, xo, zo): wave w owns
 // columns xo + w*EW .. +EW-1 of rows zo .. zo+eh-1, so the block's row
 // accesses are WB*EW contiguous cells of each array.  The grid is
 // persistent: block b takes items b, b + gridDim.x, ...; gridDim.x is a
 // multiple of 8, so item w always runs on XCD w % 8.
-// TRAIL: read the state of step it from trail slot rel (the run starts at
-// slot 0) and write the new state into the next slot (forward recomputation
-// for the adjoint).
 // SPLIT: the split C-PML variant (see SDT_SPLIT_CPML).
 // R1: tiles of one row (eh == 1), whose three row steps take their loads
 // all at once (a latency-bound shape: register budget of one wavefront per
@@ -307,12 +303,11 @@ __device__ __forceinline__ void el2_tile(const DModel* __restrict__ models,
 // field_b/psi_b) and written to the other; with prun (the first step of a
 // run of two-step launches, k_el2_step2) it is read from buffer
 // ((it - *prun) / 2) & 1 instead, the buffer those launches leave it in.
-template <typename T, bool TRAIL, bool SPLIT, int WB, bool R1 = false>
+template <typename T, bool SPLIT, int WB, bool R1 = false>
 __global__ void __launch_bounds__(64 * WB, R1 ? 1 : (sizeof(T) == 4 ? SDT_EL2_WAVES_PER_SIMD : 3))
 k_el2_step(const DModel* __restrict__ models, const DShot* __restrict__ shots,
            const int4* __restrict__ work, int nitems, const int* __restrict__ base, int rel,
-           const DAdj* __restrict__ adj, const int* __restrict__ tsel, int eh,
-           const int* __restrict__ prun) {
+           int eh, const int* __restrict__ prun) {
   // wave-uniform values kept in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int it = __builtin_amdgcn_readfirstlane(*base + rel);
@@ -330,19 +325,17 @@ k_el2_step(const DModel* __restrict__ models, const DShot* __restrict__ shots,
     // runs the body without memory variables
     const bool interior = wi.y - 1 >= M.lx && wi.y + 62 < M.nx - M.lx && wi.z - 2 >= M.lz &&
                           wi.z + eh + 1 < M.nz - M.lz;
-    const int tb = TRAIL ? __builtin_amdgcn_readfirstlane(*tsel) : 0;
     if (interior)
-      el2_tile<T, TRAIL, SPLIT, false, R1>(models, shots, wi, it, threadIdx.x & 63, adj, rel, tb, eh, par);
+      el2_tile<T, SPLIT, false, R1>(models, shots, wi, it, threadIdx.x & 63, eh, par);
     else
-      el2_tile<T, TRAIL, SPLIT, true, R1>(models, shots, wi, it, threadIdx.x & 63, adj, rel, tb, eh, par);
+      el2_tile<T, SPLIT, true, R1>(models, shots, wi, it, threadIdx.x & 63, eh, par);
   }
 }
 
-template <typename T, bool TRAIL, bool SPLIT, bool PML, bool R1>
+template <typename T, bool SPLIT, bool PML, bool R1>
 __device__ __forceinline__ void el2_tile(const DModel* __restrict__ models,
                                          const DShot* __restrict__ shots, const int4 wi, const int it,
-                                         const int lane, const DAdj* __restrict__ adj, const int slot,
-                                         const int tb, const int eh, const int par) {
+                                         const int lane, const int eh, const int par) {
   // Every fused multiply-add is written out; nothing else is contracted, so
   // the interior and C-PML bodies (and every tile shape) round identically.
 #pragma clang fp contract(off)
@@ -355,27 +348,20 @@ __device__ __forceinline__ void el2_tile(const DModel* __restrict__ models,
   const int ic = incol ? i : (i < 0 ? 0 : nx - 1);  // clamped column: every load stays in bounds
   const bool own = incol && lane >= 1 && lane <= EW;
   const int zend = min(zo + eh, nz);
-  const bool has_rec = !TRAIL && S.nrec > 0 && S.rrow[zend] > S.rrow[zo];  // receivers on own rows
+  const bool has_rec = S.nrec > 0 && S.rrow[zend] > S.rrow[zo];  // receivers on own rows
   const long nn = (long)nx * nz;
-  const T* tin = nullptr;
-  T* tout = nullptr;
-  if (TRAIL) {
-    const DAdj& A = adj[wi.x];
-    tin = static_cast<const T*>(A.trail[tb]) + (long)slot * A.slot;
-    tout = static_cast<T*>(A.trail[tb]) + (long)(slot + 1) * A.slot;
-  }
-  const A32<const T> vxi(TRAIL ? tin : (par ? S.g[0] : S.f[0]));
-  const A32<const T> vzi(TRAIL ? tin + nn : (par ? S.g[1] : S.f[1]));
-  const A32<const T> sxxi(TRAIL ? tin + 2 * nn : (par ? S.g[2] : S.f[2]));
-  const A32<const T> szzi(TRAIL ? tin + 3 * nn : (par ? S.g[3] : S.f[3]));
-  const A32<const T> sxzi(TRAIL ? tin + 4 * nn : (par ? S.g[4] : S.f[4]));
-  const A32<T> vxo(TRAIL ? tout : (par ? S.f[0] : S.g[0]));
-  const A32<T> vzo(TRAIL ? tout + nn : (par ? S.f[1] : S.g[1]));
-  const A32<T> sxxo(TRAIL ? tout + 2 * nn : (par ? S.f[2] : S.g[2]));
-  const A32<T> szzo(TRAIL ? tout + 3 * nn : (par ? S.f[3] : S.g[3]));
-  const A32<T> sxzo(TRAIL ? tout + 4 * nn : (par ? S.f[4] : S.g[4]));
-  const A32<const T> pin(TRAIL ? tin + 5 * nn : (par ? S.psi2 : S.psi));
-  const A32<T> pout(TRAIL ? tout + 5 * nn : (par ? S.psi : S.psi2));
+  const A32<const T> vxi(par ? S.g[0] : S.f[0]);
+  const A32<const T> vzi(par ? S.g[1] : S.f[1]);
+  const A32<const T> sxxi(par ? S.g[2] : S.f[2]);
+  const A32<const T> szzi(par ? S.g[3] : S.f[3]);
+  const A32<const T> sxzi(par ? S.g[4] : S.f[4]);
+  const A32<T> vxo(par ? S.f[0] : S.g[0]);
+  const A32<T> vzo(par ? S.f[1] : S.g[1]);
+  const A32<T> sxxo(par ? S.f[2] : S.g[2]);
+  const A32<T> szzo(par ? S.f[3] : S.g[3]);
+  const A32<T> sxzo(par ? S.f[4] : S.g[4]);
+  const A32<const T> pin(par ? S.psi2 : S.psi);
+  const A32<T> pout(par ? S.psi : S.psi2);
   const T idx = T(1.0 / M.dx), idz = T(1.0 / M.dz), dt = T(M.dt);
   const int lx = M.lx, lz = M.lz;
   const uint32_t SX = (uint32_t)nz * 2 * lx, SZ = (uint32_t)2 * lz * nx;
@@ -1893,11 +1879,10 @@ k_el2_adj(const DModel* __restrict__ models, const DShot* __restrict__ shots, co
 // boundary Hy as 0, and by k_em2_edges at the end of a run.
 // Every fused multiply-add is written out (contraction off).
 // ===========================================================================
-template <typename T, bool TRAIL, bool PML>
+template <typename T, bool PML>
 __device__ __forceinline__ void em2_tile(const DModel* __restrict__ models,
                                          const DShot* __restrict__ shots, const int4 wi, const int it,
-                                         const int lane, const DAdj* __restrict__ adj, const int slot,
-                                         const int tb, const int eh, const int par) {
+                                         const int lane, const int eh, const int par) {
 #pragma clang fp contract(off)
   const DShot& S = shots[wi.x];
   const DModel& M = models[S.model];
@@ -1908,23 +1893,16 @@ __device__ __forceinline__ void em2_tile(const DModel* __restrict__ models,
   const int ic = incol ? i : (i < 0 ? 0 : nx - 1);  // clamped column: every load stays in bounds
   const bool own = incol && lane >= 1 && lane <= EW;
   const int zend = min(zo + eh, nz);
-  const bool has_rec = !TRAIL && S.nrec > 0 && S.rrow[zend] > S.rrow[zo];  // receivers on own rows
+  const bool has_rec = S.nrec > 0 && S.rrow[zend] > S.rrow[zo];  // receivers on own rows
   const long nn = (long)nx * nz;
-  const T* tin = nullptr;
-  T* tout = nullptr;
-  if (TRAIL) {
-    const DAdj& A = adj[wi.x];
-    tin = static_cast<const T*>(A.trail[tb]) + (long)slot * A.slot;
-    tout = static_cast<T*>(A.trail[tb]) + (long)(slot + 1) * A.slot;
-  }
-  const A32<const T> exi(TRAIL ? tin : (par ? S.g[0] : S.f[0]));
-  const A32<const T> ezi(TRAIL ? tin + nn : (par ? S.g[1] : S.f[1]));
-  const A32<const T> hyi(TRAIL ? tin + 2 * nn : (par ? S.g[2] : S.f[2]));
-  const A32<T> exo(TRAIL ? tout : (par ? S.f[0] : S.g[0]));
-  const A32<T> ezo(TRAIL ? tout + nn : (par ? S.f[1] : S.g[1]));
-  const A32<T> hyo(TRAIL ? tout + 2 * nn : (par ? S.f[2] : S.g[2]));
-  const A32<const T> pin(TRAIL ? tin + 3 * nn : (par ? S.psi2 : S.psi));
-  const A32<T> pout(TRAIL ? tout + 3 * nn : (par ? S.psi : S.psi2));
+  const A32<const T> exi(par ? S.g[0] : S.f[0]);
+  const A32<const T> ezi(par ? S.g[1] : S.f[1]);
+  const A32<const T> hyi(par ? S.g[2] : S.f[2]);
+  const A32<T> exo(par ? S.f[0] : S.g[0]);
+  const A32<T> ezo(par ? S.f[1] : S.g[1]);
+  const A32<T> hyo(par ? S.f[2] : S.g[2]);
+  const A32<const T> pin(par ? S.psi2 : S.psi);
+  const A32<T> pout(par ? S.psi : S.psi2);
   const T idx = T(1.0 / M.dx), idz = T(1.0 / M.dz), dbh = T(M.scal[0]);
   const int lx = M.lx, lz = M.lz;
   const uint32_t SX = (uint32_t)nz * 2 * lx, SZ = (uint32_t)2 * lz * nx;
@@ -2026,12 +2004,11 @@ __device__ __forceinline__ void em2_tile(const DModel* __restrict__ models,
 
 // Same work list and launch shape as k_el2_step, and the same buffer
 // choice (prun: the single step that ends a run of two-step launches).
-template <typename T, bool TRAIL, int WB>
+template <typename T, int WB>
 __global__ void __launch_bounds__(64 * WB)
 k_em2_step(const DModel* __restrict__ models, const DShot* __restrict__ shots,
            const int4* __restrict__ work, int nitems, const int* __restrict__ base, int rel,
-           const DAdj* __restrict__ adj, const int* __restrict__ tsel, int eh,
-           const int* __restrict__ prun) {
+           int eh, const int* __restrict__ prun) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int it = __builtin_amdgcn_readfirstlane(*base + rel);
   const int par = prun ? __builtin_amdgcn_readfirstlane(((it - *prun) >> 1) & 1) : (it & 1);
@@ -2046,11 +2023,10 @@ k_em2_step(const DModel* __restrict__ models, const DShot* __restrict__ shots,
     // columns (halo included) and rows zo-1 .. zo+eh-1 clear of every slab
     const bool interior = wi.y - 1 >= M.lx && wi.y + 62 < M.nx - M.lx && wi.z - 1 >= M.lz &&
                           wi.z + eh <= M.nz - M.lz;
-    const int tb = TRAIL ? __builtin_amdgcn_readfirstlane(*tsel) : 0;
     if (interior)
-      em2_tile<T, TRAIL, false>(models, shots, wi, it, threadIdx.x & 63, adj, rel, tb, eh, par);
+      em2_tile<T, false>(models, shots, wi, it, threadIdx.x & 63, eh, par);
     else
-      em2_tile<T, TRAIL, true>(models, shots, wi, it, threadIdx.x & 63, adj, rel, tb, eh, par);
+      em2_tile<T, true>(models, shots, wi, it, threadIdx.x & 63, eh, par);
   }
 }
 
@@ -2944,19 +2920,33 @@ __device__ __forceinline__ void region_sample(const DShot& S, int it, int i, int
   }
 }
 
-template <typename T>
+template <typename T, bool SPLIT>
 struct ElRegionLds {
   T v[2][RM][RM], s[2][RM][RM];  // vx, vz; sxz, szz
   T px[6][RM], pz[7][RM];        // C-PML profiles of the region's columns and rows
   T src[5][TM_MAX];              // source increments of the steps: vx vz sxx szz sxz
+  // split C-PML, FP32: the shear loop's memory variables of each cell, used by
+  // its own thread only (in registers two blocks would not fit on a CU; FP64,
+  // whose single block has registers to spare, 709 -> 657 us per 300 steps of
+  // a 139x113 plan without them here)
+  static constexpr bool SH = SPLIT && sizeof(T) == 4;
+  T sh[SH ? 4 : 1][SH ? RM : 1][SH ? RM : 1];
   int slot[RM * RM];
 };
 
 // PML false: no cell of the region lies in a C-PML slab or on the outer ring.
-template <typename T, bool SPLIT, bool PML>
+// TRAIL: the state is read from trail buffer ts.tb's slot ts.slot, every step's
+// new one written to the next; no samples, no blow-up check (the forward has
+// done both).
+struct TrailSlot {
+  const DAdj* adj;
+  int tb, slot;
+};
+
+template <typename T, bool SPLIT, bool PML, bool TRAIL>
 __device__ __forceinline__ void el2_region(const DModel& M, const DShot& S, const int x0, const int z0,
                                            const int it0, const int nsteps, const int tm, const int par,
-                                           ElRegionLds<T>& L) {
+                                           const TrailSlot ts, ElRegionLds<T, SPLIT>& L) {
 #pragma clang fp contract(off)
   const int nx = M.nx, nz = M.nz;
   const int tx = threadIdx.x & (RM - 1), ty = threadIdx.x / RM;
@@ -2965,10 +2955,14 @@ __device__ __forceinline__ void el2_region(const DModel& M, const DShot& S, cons
   const int ic = PML ? min(max(i, 0), nx - 1) : i, rc = PML ? min(max(r, 0), nz - 1) : r;
   const bool own = in && tx >= tm && tx < tm + osz && ty >= 2 * tm && ty < 2 * tm + osz;
   const uint32_t c = (uint32_t)rc * nx + ic;
-  T vx = A32<const T>(par ? S.g[0] : S.f[0])[c], vz = A32<const T>(par ? S.g[1] : S.f[1])[c];
-  T sxx = A32<const T>(par ? S.g[2] : S.f[2])[c], szz = A32<const T>(par ? S.g[3] : S.f[3])[c];
-  T sxz = A32<const T>(par ? S.g[4] : S.f[4])[c];
-  const A32<const T> pin(par ? S.psi2 : S.psi);
+  const long n = (long)nx * nz;
+  T* const trail = TRAIL ? static_cast<T*>(ts.adj->trail[ts.tb]) + ts.slot * ts.adj->slot : nullptr;
+  T vx = A32<const T>(TRAIL ? trail : par ? S.g[0] : S.f[0])[c];
+  T vz = A32<const T>(TRAIL ? trail + n : par ? S.g[1] : S.f[1])[c];
+  T sxx = A32<const T>(TRAIL ? trail + 2 * n : par ? S.g[2] : S.f[2])[c];
+  T szz = A32<const T>(TRAIL ? trail + 3 * n : par ? S.g[3] : S.f[3])[c];
+  T sxz = A32<const T>(TRAIL ? trail + 4 * n : par ? S.g[4] : S.f[4])[c];
+  const A32<const T> pin(TRAIL ? trail + 5 * n : par ? S.psi2 : S.psi);
   const bool mono = M.coef[2] != nullptr, atten = M.coef[10] != nullptr;
   const T n11 = A32<const T>(M.coef[0])[c], n13 = A32<const T>(M.coef[1])[c], n33 = A32<const T>(M.coef[3])[c];
   const T s55 = A32<const T>(M.coef[7])[c];
@@ -2980,16 +2974,22 @@ __device__ __forceinline__ void el2_region(const DModel& M, const DShot& S, cons
   const bool inx = PML && in && in_slab(i, nx, lx), inz = PML && in && in_slab(r, nz, lz);
   const uint32_t SX = (uint32_t)nz * 2 * lx, SZ = (uint32_t)2 * lz * nx, ZB = (SPLIT ? 6 : 4) * SX;
   const uint32_t ox = inx ? (uint32_t)r * 2 * lx + slab_pos(i, nx, lx) : 0;
-  const uint32_t oz = ZB + (inz ? (uint32_t)slab_pos(r, nz, lz) * nx + i : 0);
-  T m_vxx = 0, m_vzx = 0, m_sxx = 0, m_sxzx = 0, s_vxx = 0, s_vzx = 0;
-  T m_vzz = 0, m_vxz = 0, m_szz = 0, m_sxzz = 0, s_vzz = 0, s_vxz = 0;
+  const uint32_t oz = inz ? (uint32_t)slab_pos(r, nz, lz) * nx + i : 0;
+  T m_vxx = 0, m_vzx = 0, m_sxx = 0, m_sxzx = 0, m_vzz = 0, m_vxz = 0, m_szz = 0, m_sxzz = 0;
+  constexpr bool SH = ElRegionLds<T, SPLIT>::SH;
+  T sh[4] = {0, 0, 0, 0};
+  T& s_vxx = SH ? L.sh[0][ty][tx] : sh[0];
+  T& s_vzx = SH ? L.sh[SH ? 1 : 0][ty][tx] : sh[1];
+  T& s_vzz = SH ? L.sh[SH ? 2 : 0][ty][tx] : sh[2];
+  T& s_vxz = SH ? L.sh[SH ? 3 : 0][ty][tx] : sh[3];
   if (inx) {
     m_vxx = pin[ox]; m_vzx = pin[SX + ox]; m_sxx = pin[2 * SX + ox]; m_sxzx = pin[3 * SX + ox];
     if (SPLIT) { s_vxx = pin[4 * SX + ox]; s_vzx = pin[5 * SX + ox]; }
   }
   if (inz) {
-    m_vzz = pin[oz]; m_vxz = pin[SZ + oz]; m_szz = pin[2 * SZ + oz]; m_sxzz = pin[3 * SZ + oz];
-    if (SPLIT) { s_vzz = pin[4 * SZ + oz]; s_vxz = pin[5 * SZ + oz]; }
+    const uint32_t q = ZB + oz;
+    m_vzz = pin[q]; m_vxz = pin[SZ + q]; m_szz = pin[2 * SZ + q]; m_sxzz = pin[3 * SZ + q];
+    if (SPLIT) { s_vzz = pin[4 * SZ + q]; s_vxz = pin[5 * SZ + q]; }
   }
   if (PML) {
     // (z entry 6: the legacy normal loop's decay of memory_dvx_dx, b_x_half by row)
@@ -3010,8 +3010,28 @@ __device__ __forceinline__ void el2_region(const DModel& M, const DShot& S, cons
   const bool msrc = S.msrc[0] || S.msrc[2] || S.msrc[4];
   int e0, e1, id0;
   bool more;
-  region_receivers(S, L.slot, x0, z0, nz, tm, 2 * tm, osz, own, e0, e1, id0, more);
+  if (!TRAIL) region_receivers(S, L.slot, x0, z0, nz, tm, 2 * tm, osz, own, e0, e1, id0, more);
   int bad = INT_MAX;
+  auto store = [&](void* o0, void* o1, void* o2, void* o3, void* o4, void* o5) {
+    A32<T>{o0}[c] = vx;
+    A32<T>{o1}[c] = vz;
+    A32<T>{o2}[c] = sxx;
+    A32<T>{o3}[c] = szz;
+    A32<T>{o4}[c] = sxz;
+    // (array q by its scalar base: one offset register for all)
+    T* const px = static_cast<T*>(o5);
+    T* const pz = px + ZB;
+    if (inx) {
+      A32<T>{px}[ox] = m_vxx; A32<T>{px + SX}[ox] = m_vzx; A32<T>{px + 2 * SX}[ox] = m_sxx;
+      A32<T>{px + 3 * SX}[ox] = m_sxzx;
+      if (SPLIT) { A32<T>{px + 4 * SX}[ox] = s_vxx; A32<T>{px + 5 * SX}[ox] = s_vzx; }
+    }
+    if (inz) {
+      A32<T>{pz}[oz] = m_vzz; A32<T>{pz + SZ}[oz] = m_vxz; A32<T>{pz + 2 * SZ}[oz] = m_szz;
+      A32<T>{pz + 3 * SZ}[oz] = m_sxzz;
+      if (SPLIT) { A32<T>{pz + 4 * SZ}[oz] = s_vzz; A32<T>{pz + 5 * SZ}[oz] = s_vxz; }
+    }
+  };
   const int tu = ty > 0 ? ty - 1 : 0, td = ty < RM - 1 ? ty + 1 : RM - 1;
   for (int t = 0; t < nsteps; ++t) {
     // ---- stresses (seismicfdtd.f95:247-312) ----
@@ -3109,27 +3129,20 @@ __device__ __forceinline__ void el2_region(const DModel& M, const DShot& S, cons
         vz += L.src[1][t];
       }
       if (PML && (i <= 0 || i >= nx - 1 || r <= 0 || r >= nz - 1)) { vx = 0; vz = 0; }  // :365-375
-      if (own) {
+      if (TRAIL && own) {
+        T* const o = trail + (t + 1) * ts.adj->slot;
+        store(o, o + n, o + 2 * n, o + 3 * n, o + 4 * n, o + 5 * n);
+      } else if (own) {
         if (!((double)vx * vx + (double)vz * vz <= 1.0e50)) bad = min(bad, it0 + t);
         region_sample<T>(S, it0 + t, i, e0, e1, id0, more, vx, vz);
       }
     }
   }
-  if (own) {
-    A32<T>(par ? S.f[0] : S.g[0])[c] = vx;
-    A32<T>(par ? S.f[1] : S.g[1])[c] = vz;
-    A32<T>(par ? S.f[2] : S.g[2])[c] = sxx;
-    A32<T>(par ? S.f[3] : S.g[3])[c] = szz;
-    A32<T>(par ? S.f[4] : S.g[4])[c] = sxz;
-    const A32<T> pout(par ? S.psi : S.psi2);
-    if (inx) {
-      pout[ox] = m_vxx; pout[SX + ox] = m_vzx; pout[2 * SX + ox] = m_sxx; pout[3 * SX + ox] = m_sxzx;
-      if (SPLIT) { pout[4 * SX + ox] = s_vxx; pout[5 * SX + ox] = s_vzx; }
-    }
-    if (inz) {
-      pout[oz] = m_vzz; pout[SZ + oz] = m_vxz; pout[2 * SZ + oz] = m_szz; pout[3 * SZ + oz] = m_sxzz;
-      if (SPLIT) { pout[4 * SZ + oz] = s_vzz; pout[5 * SZ + oz] = s_vxz; }
-    }
+  if (!TRAIL && own) {
+    if (par)
+      store(S.f[0], S.f[1], S.f[2], S.f[3], S.f[4], S.psi);
+    else
+      store(S.g[0], S.g[1], S.g[2], S.g[3], S.g[4], S.psi2);
     if (bad != INT_MAX) atomicMin(S.blowup, bad);
   }
 }
@@ -3141,22 +3154,25 @@ __device__ __forceinline__ bool region_interior(const DModel& M, int x0, int z0)
          z0 + RM <= M.nz - max(M.lz, 2);
 }
 
-template <typename T, bool SPLIT>
+template <typename T, bool SPLIT, bool TRAIL>
 __global__ void __launch_bounds__(RM* RM, sizeof(T) == 4 ? 8 : 4)
 k_el2_multi(const DModel* __restrict__ models, const DShot* __restrict__ shots, const int4* __restrict__ work,
-            int n, const int* __restrict__ base, int rel, int nsteps, int tm, int par) {
-  __shared__ ElRegionLds<T> L;
+            int n, const int* __restrict__ base, int rel, int nsteps, int tm, int par,
+            const DAdj* __restrict__ adj, const int* __restrict__ tsel) {
+  __shared__ ElRegionLds<T, SPLIT> L;
   const int q = item8(n);
   if (q < 0) return;
   const int4 wv = work[q];
-  const DShot& S = shots[__builtin_amdgcn_readfirstlane(wv.x)];
+  const int s = __builtin_amdgcn_readfirstlane(wv.x);
+  const DShot& S = shots[s];
   const DModel& M = models[__builtin_amdgcn_readfirstlane(wv.w)];
   const int it0 = __builtin_amdgcn_readfirstlane(*base + rel);
   const int x0 = __builtin_amdgcn_readfirstlane(wv.y) - tm, z0 = __builtin_amdgcn_readfirstlane(wv.z) - 2 * tm;
+  const TrailSlot ts{TRAIL ? adj + s : nullptr, TRAIL ? __builtin_amdgcn_readfirstlane(*tsel) : 0, rel};
   if (region_interior(M, x0, z0))
-    el2_region<T, SPLIT, false>(M, S, x0, z0, it0, nsteps, tm, par, L);
+    el2_region<T, SPLIT, false, TRAIL>(M, S, x0, z0, it0, nsteps, tm, par, ts, L);
   else
-    el2_region<T, SPLIT, true>(M, S, x0, z0, it0, nsteps, tm, par, L);
+    el2_region<T, SPLIT, true, TRAIL>(M, S, x0, z0, it0, nsteps, tm, par, ts, L);
 }
 
 template <typename T>
@@ -3168,10 +3184,10 @@ struct EmRegionLds {
 };
 
 // psi slabs and stages of k_em2_step.
-template <typename T, bool PML>
+template <typename T, bool PML, bool TRAIL>
 __device__ __forceinline__ void em2_region(const DModel& M, const DShot& S, const int x0, const int z0,
                                            const int it0, const int nsteps, const int tm, const int par,
-                                           EmRegionLds<T>& L) {
+                                           const TrailSlot ts, EmRegionLds<T>& L) {
 #pragma clang fp contract(off)
   const int nx = M.nx, nz = M.nz;
   const int tx = threadIdx.x & (RM - 1), ty = threadIdx.x / RM;
@@ -3180,9 +3196,12 @@ __device__ __forceinline__ void em2_region(const DModel& M, const DShot& S, cons
   const int ic = PML ? min(max(i, 0), nx - 1) : i, rc = PML ? min(max(r, 0), nz - 1) : r;
   const bool own = in && tx >= tm && tx < tm + osz && ty >= tm && ty < tm + osz;
   const uint32_t c = (uint32_t)rc * nx + ic;
-  T ex = A32<const T>(par ? S.g[0] : S.f[0])[c], ez = A32<const T>(par ? S.g[1] : S.f[1])[c];
-  T hy = A32<const T>(par ? S.g[2] : S.f[2])[c];
-  const A32<const T> pin(par ? S.psi2 : S.psi);
+  const long n = (long)nx * nz;
+  T* const trail = TRAIL ? static_cast<T*>(ts.adj->trail[ts.tb]) + ts.slot * ts.adj->slot : nullptr;
+  T ex = A32<const T>(TRAIL ? trail : par ? S.g[0] : S.f[0])[c];
+  T ez = A32<const T>(TRAIL ? trail + n : par ? S.g[1] : S.f[1])[c];
+  T hy = A32<const T>(TRAIL ? trail + 2 * n : par ? S.g[2] : S.f[2])[c];
+  const A32<const T> pin(TRAIL ? trail + 3 * n : par ? S.psi2 : S.psi);
   const T cax = A32<const T>(M.coef[0])[c], cbx = A32<const T>(M.coef[1])[c];
   const T caz = A32<const T>(M.coef[2])[c], cbz = A32<const T>(M.coef[3])[c];
   const int lx = M.lx, lz = M.lz;
@@ -3209,8 +3228,16 @@ __device__ __forceinline__ void em2_region(const DModel& M, const DShot& S, cons
   const bool issrc = in && i == S.isrc && r == S.ksrc;
   int e0, e1, id0;
   bool more;
-  region_receivers(S, L.slot, x0, z0, nz, tm, tm, osz, own, e0, e1, id0, more);
+  if (!TRAIL) region_receivers(S, L.slot, x0, z0, nz, tm, tm, osz, own, e0, e1, id0, more);
   int bad = INT_MAX;
+  auto store = [&](void* o0, void* o1, void* o2, void* o3) {
+    A32<T>{o0}[c] = ex;
+    A32<T>{o1}[c] = ez;
+    A32<T>{o2}[c] = hy;
+    const A32<T> pout(o3);
+    if (inx) { pout[ox] = m_ezx; pout[SX + ox] = m_hyx; }
+    if (inz) { pout[oz] = m_exz; pout[SZ + oz] = m_hyz; }
+  };
   const int tu = ty > 0 ? ty - 1 : 0, td = ty < RM - 1 ? ty + 1 : RM - 1;
   for (int t = 0; t < nsteps; ++t) {
     // ---- Hy (electromagfdtd.f95:249-266) ----
@@ -3263,39 +3290,43 @@ __device__ __forceinline__ void em2_region(const DModel& M, const DShot& S, cons
         if (i <= 0 || i >= nx - 2 || r <= 0 || r >= nz - 1) ex = 0;
         if (i <= 0 || i >= nx - 1 || r <= 0 || r >= nz - 2) ez = 0;
       }
-      if (own) {
+      if (TRAIL && own) {
+        T* const o = trail + (t + 1) * ts.adj->slot;
+        store(o, o + n, o + 2 * n, o + 3 * n);
+      } else if (own) {
         if (!((double)ex * ex + (double)ez * ez <= 1.0e50)) bad = min(bad, it0 + t);
         region_sample<T>(S, it0 + t, i, e0, e1, id0, more, ex, ez);
       }
     }
   }
-  if (own) {
-    A32<T>(par ? S.f[0] : S.g[0])[c] = ex;
-    A32<T>(par ? S.f[1] : S.g[1])[c] = ez;
-    A32<T>(par ? S.f[2] : S.g[2])[c] = hy;
-    const A32<T> pout(par ? S.psi : S.psi2);
-    if (inx) { pout[ox] = m_ezx; pout[SX + ox] = m_hyx; }
-    if (inz) { pout[oz] = m_exz; pout[SZ + oz] = m_hyz; }
+  if (!TRAIL && own) {
+    if (par)
+      store(S.f[0], S.f[1], S.f[2], S.psi);
+    else
+      store(S.g[0], S.g[1], S.g[2], S.psi2);
     if (bad != INT_MAX) atomicMin(S.blowup, bad);
   }
 }
 
-template <typename T>
+template <typename T, bool TRAIL>
 __global__ void __launch_bounds__(RM* RM, 8)
 k_em2_multi(const DModel* __restrict__ models, const DShot* __restrict__ shots, const int4* __restrict__ work,
-            int n, const int* __restrict__ base, int rel, int nsteps, int tm, int par) {
+            int n, const int* __restrict__ base, int rel, int nsteps, int tm, int par,
+            const DAdj* __restrict__ adj, const int* __restrict__ tsel) {
   __shared__ EmRegionLds<T> L;
   const int q = item8(n);
   if (q < 0) return;
   const int4 wv = work[q];
-  const DShot& S = shots[__builtin_amdgcn_readfirstlane(wv.x)];
+  const int s = __builtin_amdgcn_readfirstlane(wv.x);
+  const DShot& S = shots[s];
   const DModel& M = models[__builtin_amdgcn_readfirstlane(wv.w)];
   const int it0 = __builtin_amdgcn_readfirstlane(*base + rel);
   const int x0 = __builtin_amdgcn_readfirstlane(wv.y) - tm, z0 = __builtin_amdgcn_readfirstlane(wv.z) - tm;
+  const TrailSlot ts{TRAIL ? adj + s : nullptr, TRAIL ? __builtin_amdgcn_readfirstlane(*tsel) : 0, rel};
   if (region_interior(M, x0, z0))
-    em2_region<T, false>(M, S, x0, z0, it0, nsteps, tm, par, L);
+    em2_region<T, false, TRAIL>(M, S, x0, z0, it0, nsteps, tm, par, ts, L);
   else
-    em2_region<T, true>(M, S, x0, z0, it0, nsteps, tm, par, L);
+    em2_region<T, true, TRAIL>(M, S, x0, z0, it0, nsteps, tm, par, ts, L);
 }
 
 // ===========================================================================
@@ -4092,8 +4123,8 @@ struct Plan {
   DAdj* dadj = nullptr;          // adjoint descriptors (sdt_adjoint_setup)
   std::vector<DAdj> hadj;
   int4* dadjwork = nullptr;      // work list of the fused adjoint kernel
-  int4* dtrwork = nullptr;       // work list of the trail recomputation, with its own tile shape
-  int ntrwork = 0, tr_grid = 0, tr_wb = 4, tr_eh = 4;
+  int4* dtrwork = nullptr;       // work list of the trail recomputation (regions)
+  int ntrwork = 0, tr_tm = 0;    // its length and its steps per launch
   int* dtbase = nullptr;         // first step of the trail (adjoint kernels)
   int* dtsel_trail = nullptr;    // trail buffer the recomputation writes
   int* dtsel_adj = nullptr;      // trail buffer the adjoint reads
@@ -4154,42 +4185,40 @@ long long psi_elems(int kind, long long nx, long long ny, long long nz, long lon
 }
 
 // One launch of the single-pass ELASTIC2 step with the plan's tile shape.
-template <typename T, bool TRAIL, bool SPLIT>
-void launch_el2(Plan* p, hipStream_t st, int rel, const int* tsel, const int* prun = nullptr) {
-  const DAdj* adj = TRAIL ? p->dadj : nullptr;
-  const dim3 g(TRAIL ? p->tr_grid : p->el2_grid);
-  const int4* w = TRAIL ? p->dtrwork : p->dwork;
-  const int n = TRAIL ? p->ntrwork : p->nwork, wb = TRAIL ? p->tr_wb : p->el2_wb;
-  const int eh = TRAIL ? p->tr_eh : p->el2_eh;
-  if (!TRAIL && eh == 1) {  // tiles of one row: all loads at once
+template <typename T, bool SPLIT>
+void launch_el2(Plan* p, hipStream_t st, int rel, const int* prun = nullptr) {
+  const dim3 g(p->el2_grid);
+  const int4* w = p->dwork;
+  const int n = p->nwork, wb = p->el2_wb, eh = p->el2_eh;
+  if (eh == 1) {  // tiles of one row: all loads at once
     switch (wb) {
       case 1:
-        hipLaunchKernelGGL((k_el2_step<T, false, SPLIT, 1, true>), g, dim3(64), 0, st, p->dmodels,
-                           p->dshots, w, n, p->dbase, rel, adj, tsel, 1, prun);
+        hipLaunchKernelGGL((k_el2_step<T, SPLIT, 1, true>), g, dim3(64), 0, st, p->dmodels,
+                           p->dshots, w, n, p->dbase, rel, 1, prun);
         break;
       case 2:
-        hipLaunchKernelGGL((k_el2_step<T, false, SPLIT, 2, true>), g, dim3(128), 0, st, p->dmodels,
-                           p->dshots, w, n, p->dbase, rel, adj, tsel, 1, prun);
+        hipLaunchKernelGGL((k_el2_step<T, SPLIT, 2, true>), g, dim3(128), 0, st, p->dmodels,
+                           p->dshots, w, n, p->dbase, rel, 1, prun);
         break;
       default:
-        hipLaunchKernelGGL((k_el2_step<T, false, SPLIT, 4, true>), g, dim3(256), 0, st, p->dmodels,
-                           p->dshots, w, n, p->dbase, rel, adj, tsel, 1, prun);
+        hipLaunchKernelGGL((k_el2_step<T, SPLIT, 4, true>), g, dim3(256), 0, st, p->dmodels,
+                           p->dshots, w, n, p->dbase, rel, 1, prun);
         break;
     }
     return;
   }
   switch (wb) {
     case 1:
-      hipLaunchKernelGGL((k_el2_step<T, TRAIL, SPLIT, 1>), g, dim3(64), 0, st, p->dmodels,
-                         p->dshots, w, n, p->dbase, rel, adj, tsel, eh, prun);
+      hipLaunchKernelGGL((k_el2_step<T, SPLIT, 1>), g, dim3(64), 0, st, p->dmodels,
+                         p->dshots, w, n, p->dbase, rel, eh, prun);
       break;
     case 2:
-      hipLaunchKernelGGL((k_el2_step<T, TRAIL, SPLIT, 2>), g, dim3(128), 0, st, p->dmodels,
-                         p->dshots, w, n, p->dbase, rel, adj, tsel, eh, prun);
+      hipLaunchKernelGGL((k_el2_step<T, SPLIT, 2>), g, dim3(128), 0, st, p->dmodels,
+                         p->dshots, w, n, p->dbase, rel, eh, prun);
       break;
     default:
-      hipLaunchKernelGGL((k_el2_step<T, TRAIL, SPLIT, 4>), g, dim3(256), 0, st, p->dmodels,
-                         p->dshots, w, n, p->dbase, rel, adj, tsel, eh, prun);
+      hipLaunchKernelGGL((k_el2_step<T, SPLIT, 4>), g, dim3(256), 0, st, p->dmodels,
+                         p->dshots, w, n, p->dbase, rel, eh, prun);
       break;
   }
 }
@@ -4222,25 +4251,23 @@ void launch_el2x2(Plan* p, hipStream_t st, int rel) {
                                      p->el2x2_grid);
 }
 
-template <typename T, bool TRAIL>
-void launch_em2(Plan* p, hipStream_t st, int rel, const int* tsel, const int* prun = nullptr) {
-  const DAdj* adj = TRAIL ? p->dadj : nullptr;
-  const dim3 g(TRAIL ? p->tr_grid : p->el2_grid);
-  const int4* w = TRAIL ? p->dtrwork : p->dwork;
-  const int n = TRAIL ? p->ntrwork : p->nwork, wb = TRAIL ? p->tr_wb : p->el2_wb;
-  const int eh = TRAIL ? p->tr_eh : p->el2_eh;
+template <typename T>
+void launch_em2(Plan* p, hipStream_t st, int rel, const int* prun = nullptr) {
+  const dim3 g(p->el2_grid);
+  const int4* w = p->dwork;
+  const int n = p->nwork, wb = p->el2_wb, eh = p->el2_eh;
   switch (wb) {
     case 1:
-      hipLaunchKernelGGL((k_em2_step<T, TRAIL, 1>), g, dim3(64), 0, st, p->dmodels, p->dshots,
-                         w, n, p->dbase, rel, adj, tsel, eh, prun);
+      hipLaunchKernelGGL((k_em2_step<T, 1>), g, dim3(64), 0, st, p->dmodels, p->dshots,
+                         w, n, p->dbase, rel, eh, prun);
       break;
     case 2:
-      hipLaunchKernelGGL((k_em2_step<T, TRAIL, 2>), g, dim3(128), 0, st, p->dmodels, p->dshots,
-                         w, n, p->dbase, rel, adj, tsel, eh, prun);
+      hipLaunchKernelGGL((k_em2_step<T, 2>), g, dim3(128), 0, st, p->dmodels, p->dshots,
+                         w, n, p->dbase, rel, eh, prun);
       break;
     default:
-      hipLaunchKernelGGL((k_em2_step<T, TRAIL, 4>), g, dim3(256), 0, st, p->dmodels, p->dshots,
-                         w, n, p->dbase, rel, adj, tsel, eh, prun);
+      hipLaunchKernelGGL((k_em2_step<T, 4>), g, dim3(256), 0, st, p->dmodels, p->dshots,
+                         w, n, p->dbase, rel, eh, prun);
       break;
   }
 }
@@ -4309,16 +4336,16 @@ long long regions2d(const Plan* p, int tm) {
 // its cells are owned, tm = 5 EM: 47 %), which pays where the walking kernels
 // wait on launches and loads, not where they stream: measured (us per step,
 // walking kernels in the shape of default_shape, then regions) elastic FP64
-// 127x103 6.4 -> 2.3, 296^2 7.8 -> 3.5, 1064x808 27.3 -> 18.9, x 3 shots 57 -> 52,
-// x 4 shots 70 -> 70; elastic FP32 296^2 6.7 -> 2.8, 1064x808 17.9 -> 9.4, x 10
-// shots 85 -> 81, x 16 shots 119 -> 129; EM FP64 127x103 3.5 -> 1.5, 1064x808 11.9
-// -> 6.2, x 32 shots 207 -> 174; EM FP32 1064x808 7.6 -> 4.7, x 32 shots 120 ->
-// 117, 2088x808 x 32 shots 218 -> 227.
+// 127x103 6.4 -> 2.3, 296^2 7.8 -> 3.4, 1064x808 27 -> 19, x 4 shots 71 -> 67, x 6
+// shots (413 MB of fields) 92 -> 100; elastic FP32 296^2 6.7 -> 2.8, 1064x808 17.9
+// -> 9.4, x 16 shots 125 -> 120, x 24 shots 177 -> 173, x 32 shots (1.1 GB) 229 ->
+// 229; EM FP64 127x103 3.5 -> 1.5, 1064x808 11.9 -> 6.1, x 32 shots 207 -> 174; EM
+// FP32 1064x808 7.6 -> 4.7, x 32 shots 123 -> 109, 2088x1540 x 32 shots 397 -> 376.
 // tm: a launch costs 5 to 7 us beside its steps, so the most steps for which the
 // regions still run all at once (one block of elastic FP64 per CU, else two):
 // 127x103 elastic FP64 5.1 / 2.8 / 2.3 with 2 / 4 / 7 steps, 296^2 5.2 / 3.4 / 5.8;
 // larger plans take the number whose owned share balances the launches.
-void default_regions(Plan* p, double bytes, bool big) {
+void default_regions(Plan* p, double bytes) {
   const bool em = p->kind == SDT_EM2, f64 = p->prec == SDT_FP64;
   p->tm = em ? 5 : f64 && regions2d(p, 4) > 2500 ? 3 : 4;
   for (int t = TM_MAX; t >= (!em && f64 ? 2 : 3); --t)
@@ -4326,7 +4353,7 @@ void default_regions(Plan* p, double bytes, bool big) {
       p->tm = t;
       break;
     }
-  p->multi = em ? f64 || bytes < 900e6 : f64 ? !big : bytes < 400e6;
+  p->multi = em || bytes < (f64 ? 350e6 : 900e6);
 }
 
 // Default launch shape of a 2-D plan: steps per launch, wavefronts per block,
@@ -4382,23 +4409,26 @@ void default_shape(Plan* p) {
       if (waves2d(p, ew, rows) >= (f64 ? 2000 : em ? 2800 : 4000)) p->el2_eh = rows;
     if (waves2d(p, ew, 16) >= (em ? 12000 : 8000)) p->el2_eh = 16;
   }
-  default_regions(p, cells * kind_fields(p->kind) * 2 * (f64 ? 8 : 4), big);
+  default_regions(p, cells * kind_fields(p->kind) * 2 * (f64 ? 8 : 4));
   p->def_spl = p->spl;
   p->def_wb = p->el2_wb;
   p->def_eh = p->el2_eh;
   p->def_order = p->el2_order;
 }
 
-// Work list of the region kernels: the regions of a model column by column,
-// so that the contiguous run an XCD takes (item25) is one part of the model.
-std::vector<int4> multi_work(const Plan* p) {
-  const int own = RM - (p->kind == SDT_EM2 ? 2 : 3) * p->tm;
+// Work list of the region kernels: the regions of a model row by row, so that
+// the run an XCD takes (item8) is one part of the model and neighbours in x,
+// which write parts of the same cache lines, run together (column by column:
+// EM FP32 32 shots of 1064x808 118 us per step against 107, elastic FP32 16 of
+// 1064x552 84 against 77, their recomputation 142 against 114).
+std::vector<int4> multi_work(const Plan* p, int tm) {
+  const int own = RM - (p->kind == SDT_EM2 ? 2 : 3) * tm;
   std::vector<int4> w;
   for (int s = 0; s < p->nshots; ++s) {
     const int m = p->hshots[s].model;
     const sdt_model& M = p->hmodels[m];
-    for (int x = 0; x < M.nx; x += own)
-      for (int z = 0; z < M.nz; z += own) w.push_back(make_int4(s, x, z, m));
+    for (int z = 0; z < M.nz; z += own)
+      for (int x = 0; x < M.nx; x += own) w.push_back(make_int4(s, x, z, m));
   }
   return w;
 }
@@ -4407,19 +4437,24 @@ std::vector<int4> multi_work(const Plan* p) {
 // launch, in launches of nearly equal length, an even number of them if
 // `even` (a graph block must leave the state in the buffer it started from).
 // Returns the number of launches.
-template <typename T>
+template <typename T, bool TRAIL = false>
 int launch_multi(Plan* p, hipStream_t st, int n, bool even) {
-  int L = (n + p->tm - 1) / p->tm;
+  const int tm = TRAIL ? p->tr_tm : p->tm, nw = TRAIL ? p->ntrwork : p->nmulti;
+  const int4* w = TRAIL ? p->dtrwork : p->dwmulti;
+  int L = (n + tm - 1) / tm;
   if (even) L += L & 1;
-  const dim3 g((p->nmulti + 7) / 8 * 8), b(RM * RM);
+  const dim3 g((nw + 7) / 8 * 8), b(RM * RM);
   for (int l = 0; l < L; ++l) {
     const int r = (int)((long long)n * l / L), k = (int)((long long)n * (l + 1) / L) - r;
     if (p->kind == SDT_EM2)
-      hipLaunchKernelGGL(k_em2_multi<T>, g, b, 0, st, p->dmodels, p->dshots, p->dwmulti, p->nmulti, p->dbase, r, k, p->tm, l & 1);
+      hipLaunchKernelGGL((k_em2_multi<T, TRAIL>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k, tm,
+                         l & 1, p->dadj, p->dtsel_trail);
     else if (p->split)
-      hipLaunchKernelGGL((k_el2_multi<T, true>), g, b, 0, st, p->dmodels, p->dshots, p->dwmulti, p->nmulti, p->dbase, r, k, p->tm, l & 1);
+      hipLaunchKernelGGL((k_el2_multi<T, true, TRAIL>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k,
+                         tm, l & 1, p->dadj, p->dtsel_trail);
     else
-      hipLaunchKernelGGL((k_el2_multi<T, false>), g, b, 0, st, p->dmodels, p->dshots, p->dwmulti, p->nmulti, p->dbase, r, k, p->tm, l & 1);
+      hipLaunchKernelGGL((k_el2_multi<T, false, TRAIL>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k,
+                         tm, l & 1, p->dadj, p->dtsel_trail);
   }
   return L;
 }
@@ -4690,14 +4725,14 @@ void launch_one(Plan* p, hipStream_t st, int rel, int which) {
   switch (p->kind * 2 + which) {
     case SDT_ELASTIC2 * 2:
       if (p->split)
-        launch_el2<T, false, true>(p, st, rel, nullptr);
+        launch_el2<T, true>(p, st, rel);
       else
-        launch_el2<T, false, false>(p, st, rel, nullptr);
+        launch_el2<T, false>(p, st, rel);
       break;
     case SDT_ELASTIC2 * 2 + 1:
       break;  // the fused step kernel does both phases
     case SDT_EM2 * 2:
-      launch_em2<T, false>(p, st, rel, nullptr);
+      launch_em2<T>(p, st, rel);
       break;
     case SDT_EM2 * 2 + 1:
       break;  // the fused step kernel does both phases
@@ -4756,11 +4791,11 @@ void launch_two(Plan* p, hipStream_t st, int r, bool single) {
     return;
   }
   if (em)
-    launch_em2<T, false>(p, st, r, nullptr, p->dit0);
+    launch_em2<T>(p, st, r, p->dit0);
   else if (p->split)
-    launch_el2<T, false, true>(p, st, r, nullptr, p->dit0);
+    launch_el2<T, true>(p, st, r, p->dit0);
   else
-    launch_el2<T, false, false>(p, st, r, nullptr, p->dit0);
+    launch_el2<T, false>(p, st, r, p->dit0);
 }
 
 void launch_pairs(Plan* p, hipStream_t st, int n) {
@@ -4912,16 +4947,6 @@ long long state_elems(int kind, long long nx, long long ny, long long nz, long l
   return np < 0 ? -1 : kind_fields(kind & ~SDT_SPLIT_CPML) * nx * ny * nz + np;
 }
 
-template <typename T>
-void launch_trail_steps(Plan* p, hipStream_t st, int it0, int nsteps) {
-  for (int r = 0; r < nsteps; ++r) {
-    if (p->split)
-      launch_el2<T, true, true>(p, st, r, p->dtsel_trail);
-    else
-      launch_el2<T, true, false>(p, st, r, p->dtsel_trail);
-  }
-}
-
 // Adjoint steps t = tbase + k for k = khi-1 down to klo (tbase = the trail's
 // first step, held on the device so a captured segment replays anywhere).
 template <typename T, bool SPLIT>
@@ -4947,23 +4972,11 @@ void launch_adjoint_steps(Plan* p, hipStream_t st, int khi, int klo) {
   }
 }
 
-template <typename T>
-void launch_trail_em2(Plan* p, hipStream_t st, int nsteps) {
-  for (int r = 0; r < nsteps; ++r) launch_em2<T, true>(p, st, r, p->dtsel_trail);
-}
-
 void launch_trail(Plan* p, hipStream_t st, int nsteps) {
-  if (p->kind == SDT_EM2) {
-    if (p->prec == SDT_FP64)
-      launch_trail_em2<double>(p, st, nsteps);
-    else
-      launch_trail_em2<float>(p, st, nsteps);
-    return;
-  }
   if (p->prec == SDT_FP64)
-    launch_trail_steps<double>(p, st, 0, nsteps);
+    launch_multi<double, true>(p, st, nsteps, false);
   else
-    launch_trail_steps<float>(p, st, 0, nsteps);
+    launch_multi<float, true>(p, st, nsteps, false);
 }
 
 template <typename T>
@@ -5159,7 +5172,7 @@ int stage_host(Plan* p, int kind, int prec, const sdt_model* models, int nmodels
       p->el2_wb = 4;
       p->multi = false;
     }
-    if (p->multi) S.workm = multi_work(p);
+    if (p->multi) S.workm = multi_work(p, p->tm);
     p->nmulti = (int)S.workm.size();
     S.work = el2_work(p, p->el2_wb, p->el2_eh, p->el2_order);
     const int nblk = (int)S.work.size();
@@ -5775,16 +5788,18 @@ int sdt_adjoint_setup(void* plan, const sdt_adj_shot* adj, int nshots, unsigned 
   if (!p->dtsel_trail) HIP_TRY(hipMalloc(&p->dtsel_trail, sizeof(int)));
   if (!p->dtsel_adj) HIP_TRY(hipMalloc(&p->dtsel_adj, sizeof(int)));
   if (!p->dtrwork) {
-    // The recomputation has a tile shape of its own (it steps one at a time,
-    // beside the adjoint kernel): 4 rows, 2 where the plan then has fewer than
-    // 4000 wavefronts, tiles dealt to the XCDs in turn.  Measured for one
-    // backward pass (ms, tiles of 1 / 2 / 4 / 8 / 32 rows): 16 shots of
-    // 1064x552 FP32 86.5 / 73.9 / 70.1 / 71.2 / 75.0 (73.6 with 4 rows in column
-    // strips), 6 shots of 740x440 FP64 32.7 / 30.0 / 28.9 / 29.0 / 32.2 with two
-    // wavefronts per block (30.1 with four).
-    p->tr_wb = p->prec == SDT_FP64 ? 2 : 4;
-    p->tr_eh = waves2d(p, EW, 4) >= 4000 ? 4 : 2;
-    const std::vector<int4> work = el2_work(p, p->tr_wb, p->tr_eh, 0);
+    // The recomputation runs on regions at every size, at the plan's steps per
+    // launch where they all run at once, else at 3 (EM: 4).  It writes every
+    // step's state, so that at the largest plans the writes bound it (elastic
+    // FP32 16 shots of 1064x552: 188 MB, 40 us at 5 TB/s) and a wider ring costs
+    // more than fewer reads give.  Measured (us per step, one launch of tiled
+    // wavefronts per step, then regions of 2 / 3 / 4 / 5 steps): elastic FP32
+    // 120x90 9.8, 3.9 / 3.2 / 2.8 / 2.6, 740x440 x 6 shots 41, 25 / 27 / 28 / 34,
+    // 1064x552 x 16 shots 160, 140 / 121 / 138 / 164; FP64 64, 53 / 52 / 49 / 61 and 255,
+    // 245 / 211 / 233 / 266; EM FP64 1064x808 x 2 shots 30, 22 / 21 / 20 / 22.
+    const bool em = p->kind == SDT_EM2;
+    p->tr_tm = p->tm > (em ? 5 : 4) ? p->tm : em ? 4 : 3;
+    const std::vector<int4> work = multi_work(p, p->tr_tm);
     int4* dw = nullptr;
     HIP_TRY(hipMalloc(&dw, sizeof(int4) * work.size()));
     if (hipMemcpy(dw, work.data(), sizeof(int4) * work.size(), hipMemcpyHostToDevice) != hipSuccess) {
@@ -5793,7 +5808,6 @@ int sdt_adjoint_setup(void* plan, const sdt_adj_shot* adj, int nshots, unsigned 
     }
     p->dtrwork = dw;
     p->ntrwork = (int)work.size();
-    p->tr_grid = std::max(8, std::min(p->ntrwork, SDT_EL2_GRID) / 8 * 8);
   }
   if (!p->dadjwork) {
     // (shot, x0, z0, model) blocks of the fused adjoint kernel, shot by shot:

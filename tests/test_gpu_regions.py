@@ -104,3 +104,37 @@ def test_regions_report_the_same_unstable_step(kind):
         with pytest.raises(UnstableError):
             s.check()
     assert a.unstable == b.unstable and a.unstable[0] >= 0
+
+
+@pytest.mark.parametrize("kind,split", [("elastic2", False), ("elastic2", True), ("em2", False)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("nx,nz,npml,nshots", [(16, 16, 3, 1), (57, 90, 6, 3), (400, 270, 9, 2)])
+def test_region_recomputation_equals_one_step_kernel(kind, split, precision, nx, nz, npml, nshots):
+    """Every state of a trail (segments of one, of several launches and with a
+    remainder) against the one-step kernel stepping the same shots."""
+    import ctypes as C
+
+    from seidart_amd import _hip
+    from seidart_amd.adjoint import AdjointEngine
+    p = _ring(tiny_problem(kind, seed=450 + nx, nx=nx, nz=nz, npml=npml, nt=40, nshots=nshots,
+                           gamma=1e-3 if kind == "elastic2" else 0.0))
+    p.cpml_split = split
+    e = AdjointEngine(p, precision=precision, every=23)
+    a = _walk(p, precision)
+    st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for it0, n, buf in ((0, 1, 0), (1, 23, 1), (24, 16, 0)):
+        for s, (_, _, b) in enumerate(a.shots):
+            e.trail[s][buf][0].copy_(b["state"])
+        _hip.check(_hip.lib().sdt_plan_run_trail(e.sim._plan, it0, n, buf, st))
+        for k in range(1, n + 1):
+            a.run(1)
+            for s, (_, _, b) in enumerate(a.shots):
+                got = e.trail[s][buf][k]
+                if kind == "em2":  # Hy's ring, zeroed at the end of a run and read as zero
+                    got = got.clone()
+                    hy = got[2 * p.cells:3 * p.cells].view(nz, nx)
+                    hy[0, : nx - 1] = hy[nz - 2, : nx - 1] = 0
+                    hy[: nz - 1, 0] = hy[: nz - 1, nx - 2] = 0
+                assert torch.equal(b["state"], got), (it0, k, s)
+    a.close()
+    e.close()
