@@ -2859,7 +2859,8 @@ k_el25_vel(const DModel* __restrict__ models, const DShot* __restrict__ shots,
 // the block owns that and the neighbouring blocks recompute the rest.  Every
 // expression is the one-step kernel's, in the same order: identical bits.  A
 // launch reads state buffer par and writes the other.
-// What bounds it: at most two blocks share a CU, so a SIMD has 4 or 8 wavefronts
+// What bounds it: at most two blocks (four of the EM blocks of two rows per
+// thread) share a CU, so a SIMD has 4 or 8 wavefronts
 // whose instructions it issues one after the other (about 1.1 us per elastic
 // step and block), and each launch waits once for its loads (5 to 7 us).
 // Regions off the slabs and the outer rings run a body without memory
@@ -2871,49 +2872,53 @@ k_el25_vel(const DModel* __restrict__ models, const DShot* __restrict__ shots,
 constexpr int RM = 32;       // region: RM x RM cells, one thread each
 constexpr int TM_MAX = 8;    // most steps per launch
 
-// The receivers of the block's owned cells (columns cx0.., rows cz0.. of the
-// region, own x own): per thread the first index entry on its cell (INT_MAX:
-// none) and the end of its row's entries.  Called by every thread.
+// The receivers of a thread's K cells (rows z0 + K * (threadIdx.x / RM) + k of
+// the region at x0, z0): per cell the first index entry on it (INT_MAX: none),
+// that receiver, and whether more follow.  The block owns own x own cells from
+// column cx0, row cz0 on; mine: the thread's cell is one of them.  Called by
+// every thread; slot: one entry per cell.
+struct RegionRec {
+  int e0, id0;
+  bool more;
+};
+template <int K>
 __device__ __forceinline__ void region_receivers(const DShot& S, int* slot, int x0, int z0, int nz, int cx0,
-                                                 int cz0, int own, bool mine, int& e0, int& e1, int& id0,
-                                                 bool& more) {
+                                                 int cz0, int own, const bool (&mine)[K], RegionRec (&rec)[K]) {
   const int zr0 = z0 + cz0, zr1 = min(zr0 + own, nz);
-  e0 = INT_MAX;
-  e1 = id0 = 0;
-  more = false;
+  for (int k = 0; k < K; ++k) rec[k] = {INT_MAX, 0, false};
   if (S.nrec <= 0 || S.rrow[zr1] <= S.rrow[zr0]) return;  // block-uniform
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  slot[threadIdx.x] = INT_MAX;
+  const int tx = threadIdx.x % RM, ty = K * (int)(threadIdx.x / RM);
+  for (int k = 0; k < K; ++k) slot[(ty + k) * RM + tx] = INT_MAX;
   __syncthreads();
-  for (int h = 0; h < 2; ++h) {
-    const int row = z0 + 2 * w + h;
+  for (int h = 0; h < 2 * K; ++h) {  // a wavefront's own rows
+    const int row = z0 + 2 * K * w + h;
     if (row < zr0 || row >= zr1) continue;
     const int q0 = S.rrow[row], q1 = S.rrow[row + 1];
     for (int e = q0 + lane; e < q1; e += 64) {
       const int cx = S.rxid[2 * e] - x0;
-      if (cx >= cx0 && cx < cx0 + own) atomicMin(&slot[(2 * w + h) * RM + cx], e);
+      if (cx >= cx0 && cx < cx0 + own) atomicMin(&slot[(2 * K * w + h) * RM + cx], e);
     }
   }
   __syncthreads();
-  if (!mine) return;
-  e0 = slot[threadIdx.x];
-  if (e0 == INT_MAX) return;
-  const int i = x0 + (int)(threadIdx.x % RM);
-  e1 = S.rrow[z0 + (int)(threadIdx.x / RM) + 1];
-  id0 = S.rxid[2 * e0 + 1];
-  more = e0 + 1 < e1 && S.rxid[2 * e0 + 2] == i;
+  for (int k = 0; k < K; ++k) {
+    const int e0 = slot[(ty + k) * RM + tx];
+    if (!mine[k] || e0 == INT_MAX) continue;
+    rec[k] = {e0, S.rxid[2 * e0 + 1], e0 + 1 < S.rrow[z0 + ty + k + 1] && S.rxid[2 * e0 + 2] == x0 + tx};
+  }
 }
 
-// This step's samples a, b of the receivers on column i's cell.
+// This step's samples a, b of the receivers on a cell of column i, row r.
 template <typename T>
-__device__ __forceinline__ void region_sample(const DShot& S, int it, int i, int e0, int e1, int id0, bool more,
-                                              T a, T b) {
-  if (e0 == INT_MAX) return;
+__device__ __forceinline__ void region_sample(const DShot& S, int it, int i, int r, const RegionRec& rec, T a,
+                                              T b) {
+  if (rec.e0 == INT_MAX) return;
   auto tr = mp<T>(S.trace) + (long)it * 2 * S.nrec;
-  tr[id0] = a;
-  tr[S.nrec + id0] = b;
-  if (!more) return;
-  for (int e = e0 + 1; e < e1 && S.rxid[2 * e] == i; ++e) {
+  tr[rec.id0] = a;
+  tr[S.nrec + rec.id0] = b;
+  if (!rec.more) return;
+  const int e1 = S.rrow[r + 1];
+  for (int e = rec.e0 + 1; e < e1 && S.rxid[2 * e] == i; ++e) {
     const int id = S.rxid[2 * e + 1];
     tr[id] = a;
     tr[S.nrec + id] = b;
@@ -3008,9 +3013,8 @@ __device__ __forceinline__ void el2_region(const DModel& M, const DShot& S, cons
   const T idx = T(1.0 / M.dx), idz = T(1.0 / M.dz), dt = T(M.dt);
   const bool issrc = in && i == S.isrc && r == S.ksrc;
   const bool msrc = S.msrc[0] || S.msrc[2] || S.msrc[4];
-  int e0, e1, id0;
-  bool more;
-  if (!TRAIL) region_receivers(S, L.slot, x0, z0, nz, tm, 2 * tm, osz, own, e0, e1, id0, more);
+  RegionRec rec[1];
+  if (!TRAIL) region_receivers<1>(S, L.slot, x0, z0, nz, tm, 2 * tm, osz, {own}, rec);
   int bad = INT_MAX;
   auto store = [&](void* o0, void* o1, void* o2, void* o3, void* o4, void* o5) {
     A32<T>{o0}[c] = vx;
@@ -3134,7 +3138,7 @@ __device__ __forceinline__ void el2_region(const DModel& M, const DShot& S, cons
         store(o, o + n, o + 2 * n, o + 3 * n, o + 4 * n, o + 5 * n);
       } else if (own) {
         if (!((double)vx * vx + (double)vz * vz <= 1.0e50)) bad = min(bad, it0 + t);
-        region_sample<T>(S, it0 + t, i, e0, e1, id0, more, vx, vz);
+        region_sample<T>(S, it0 + t, i, r, rec[0], vx, vz);
       }
     }
   }
@@ -3175,145 +3179,174 @@ k_el2_multi(const DModel* __restrict__ models, const DShot* __restrict__ shots, 
     el2_region<T, SPLIT, true, TRAIL>(M, S, x0, z0, it0, nsteps, tm, par, ts, L);
 }
 
-template <typename T>
+// EK: rows per thread.  With two, the z neighbour of one of them is in the
+// thread's own registers and four FP32 regions share a CU (59 registers), so
+// that the loads of one run beside the steps of the others; a plan whose
+// regions all run at once wants the wavefronts of one row per thread, and two
+// FP64 rows take 84 registers.  Measured (us per step, EK 1 then 2): FP32 32
+// shots of 1064x808 107 -> 87, 8 of 740x540 13.6 -> 11.4, 32 of 2088x1540 374 ->
+// 313, 3 of 340x240 2.8 -> 3.0, 130x110 1.5 -> 2.0; FP64 1064x808 6.1 -> 6.5, 32 shots
+// 156 -> 164; the recomputation, which its stores bound, 52 -> 52.
+template <typename T, int EK>
 struct EmRegionLds {
-  T ex[RM][RM], hy[RM][RM];
+  T ex[RM / EK][RM], hy[RM / EK][RM];  // the threads' first rows' Ex, last rows' Hy
   T px[6][RM], pz[6][RM];
   T src[2][TM_MAX];  // source increments of the steps: Ex, Ez
   int slot[RM * RM];
 };
 
 // psi slabs and stages of k_em2_step.
-template <typename T, bool PML, bool TRAIL>
+template <typename T, bool PML, bool TRAIL, int EK>
 __device__ __forceinline__ void em2_region(const DModel& M, const DShot& S, const int x0, const int z0,
                                            const int it0, const int nsteps, const int tm, const int par,
-                                           const TrailSlot ts, EmRegionLds<T>& L) {
+                                           const TrailSlot ts, EmRegionLds<T, EK>& L) {
 #pragma clang fp contract(off)
-  const int nx = M.nx, nz = M.nz;
-  const int tx = threadIdx.x & (RM - 1), ty = threadIdx.x / RM;
-  const int i = x0 + tx, r = z0 + ty, osz = RM - 2 * tm;
-  const bool in = !PML || (i >= 0 && i < nx && r >= 0 && r < nz);
-  const int ic = PML ? min(max(i, 0), nx - 1) : i, rc = PML ? min(max(r, 0), nz - 1) : r;
-  const bool own = in && tx >= tm && tx < tm + osz && ty >= tm && ty < tm + osz;
-  const uint32_t c = (uint32_t)rc * nx + ic;
+  const int nx = M.nx, nz = M.nz, lx = M.lx, lz = M.lz;
+  const int tx = threadIdx.x & (RM - 1), tq = threadIdx.x / RM;
+  const int i = x0 + tx, osz = RM - 2 * tm;
+  const uint32_t SX = (uint32_t)nz * 2 * lx, SZ = (uint32_t)2 * lz * nx;
   const long n = (long)nx * nz;
   T* const trail = TRAIL ? static_cast<T*>(ts.adj->trail[ts.tb]) + ts.slot * ts.adj->slot : nullptr;
-  T ex = A32<const T>(TRAIL ? trail : par ? S.g[0] : S.f[0])[c];
-  T ez = A32<const T>(TRAIL ? trail + n : par ? S.g[1] : S.f[1])[c];
-  T hy = A32<const T>(TRAIL ? trail + 2 * n : par ? S.g[2] : S.f[2])[c];
+  const A32<const T> exi(TRAIL ? trail : par ? S.g[0] : S.f[0]);
+  const A32<const T> ezi(TRAIL ? trail + n : par ? S.g[1] : S.f[1]);
+  const A32<const T> hyi(TRAIL ? trail + 2 * n : par ? S.g[2] : S.f[2]);
   const A32<const T> pin(TRAIL ? trail + 3 * n : par ? S.psi2 : S.psi);
-  const T cax = A32<const T>(M.coef[0])[c], cbx = A32<const T>(M.coef[1])[c];
-  const T caz = A32<const T>(M.coef[2])[c], cbz = A32<const T>(M.coef[3])[c];
-  const int lx = M.lx, lz = M.lz;
-  const bool inx = PML && in && in_slab(i, nx, lx), inz = PML && in && in_slab(r, nz, lz);
-  const uint32_t SX = (uint32_t)nz * 2 * lx, SZ = (uint32_t)2 * lz * nx;
-  const uint32_t ox = inx ? (uint32_t)r * 2 * lx + slab_pos(i, nx, lx) : 0;
-  const uint32_t oz = 2 * SX + (inz ? (uint32_t)slab_pos(r, nz, lz) * nx + i : 0);
-  T m_ezx = 0, m_hyx = 0, m_exz = 0, m_hyz = 0;
-  if (inx) { m_ezx = pin[ox]; m_hyx = pin[SX + ox]; }
-  if (inz) { m_exz = pin[oz]; m_hyz = pin[SZ + oz]; }
+  const A32<const T> CAX(M.coef[0]), CBX(M.coef[1]), CAZ(M.coef[2]), CBZ(M.coef[3]);
+  bool in[EK], own[EK], inx[EK], inz[EK], issrc[EK];
+  uint32_t c[EK], ox[EK], oz[EK];
+  T ex[EK], ez[EK], hy[EK], cax[EK], cbx[EK], caz[EK], cbz[EK];
+  T m_ezx[EK], m_hyx[EK], m_exz[EK], m_hyz[EK];
+#pragma unroll
+  for (int k = 0; k < EK; ++k) {
+    const int ty = EK * tq + k, r = z0 + ty;
+    in[k] = !PML || (i >= 0 && i < nx && r >= 0 && r < nz);
+    const int ic = PML ? min(max(i, 0), nx - 1) : i, rc = PML ? min(max(r, 0), nz - 1) : r;
+    own[k] = in[k] && tx >= tm && tx < tm + osz && ty >= tm && ty < tm + osz;
+    issrc[k] = in[k] && i == S.isrc && r == S.ksrc;
+    c[k] = (uint32_t)rc * nx + ic;
+    ex[k] = exi[c[k]];
+    ez[k] = ezi[c[k]];
+    hy[k] = hyi[c[k]];
+    cax[k] = CAX[c[k]];
+    cbx[k] = CBX[c[k]];
+    caz[k] = CAZ[c[k]];
+    cbz[k] = CBZ[c[k]];
+    inx[k] = PML && in[k] && in_slab(i, nx, lx);
+    inz[k] = PML && in[k] && in_slab(r, nz, lz);
+    ox[k] = inx[k] ? (uint32_t)r * 2 * lx + slab_pos(i, nx, lx) : 0;
+    oz[k] = 2 * SX + (inz[k] ? (uint32_t)slab_pos(r, nz, lz) * nx + i : 0);
+    m_ezx[k] = inx[k] ? pin[ox[k]] : T(0);
+    m_hyx[k] = inx[k] ? pin[SX + ox[k]] : T(0);
+    m_exz[k] = inz[k] ? pin[oz[k]] : T(0);
+    m_hyz[k] = inz[k] ? pin[SZ + oz[k]] : T(0);
+  }
   if (PML) {
     if (threadIdx.x < 6 * RM) {
-      L.px[threadIdx.x / RM][tx] = cp<T>(M.prof[0][threadIdx.x / RM])[min(max(x0 + tx, 0), nx - 1)];
+      L.px[tq][tx] = cp<T>(M.prof[0][tq])[min(max(x0 + tx, 0), nx - 1)];
     } else if (threadIdx.x >= 256 && threadIdx.x < 256 + 6 * RM) {
-      L.pz[(threadIdx.x - 256) / RM][tx] = cp<T>(M.prof[2][(threadIdx.x - 256) / RM])[min(max(z0 + tx, 0), nz - 1)];
+      L.pz[tq - 8][tx] = cp<T>(M.prof[2][tq - 8])[min(max(z0 + tx, 0), nz - 1)];
     }
   }
-  if (threadIdx.x >= 512 && threadIdx.x < 512 + 2 * TM_MAX) {  // (read after the first barrier)
-    const int q = (threadIdx.x - 512) / TM_MAX, t = (threadIdx.x - 512) % TM_MAX;
+  if (threadIdx.x >= 480 && threadIdx.x < 480 + 2 * TM_MAX) {  // (read after the first barrier)
+    const int q = (threadIdx.x - 480) / TM_MAX, t = (threadIdx.x - 480) % TM_MAX;
     const void* a = q == 0 ? S.src[0] : S.src[2];
     L.src[q][t] = a && t < nsteps ? cp<T>(a)[it0 + t] : T(0);
   }
   const T idx = T(1.0 / M.dx), idz = T(1.0 / M.dz), dbh = T(M.scal[0]);
-  const bool issrc = in && i == S.isrc && r == S.ksrc;
-  int e0, e1, id0;
-  bool more;
-  if (!TRAIL) region_receivers(S, L.slot, x0, z0, nz, tm, tm, osz, own, e0, e1, id0, more);
+  RegionRec rec[EK];
+  if (!TRAIL) region_receivers<EK>(S, L.slot, x0, z0, nz, tm, tm, osz, own, rec);
   int bad = INT_MAX;
-  auto store = [&](void* o0, void* o1, void* o2, void* o3) {
-    A32<T>{o0}[c] = ex;
-    A32<T>{o1}[c] = ez;
-    A32<T>{o2}[c] = hy;
+  auto store = [&](int k, void* o0, void* o1, void* o2, void* o3) {
+    A32<T>{o0}[c[k]] = ex[k];
+    A32<T>{o1}[c[k]] = ez[k];
+    A32<T>{o2}[c[k]] = hy[k];
     const A32<T> pout(o3);
-    if (inx) { pout[ox] = m_ezx; pout[SX + ox] = m_hyx; }
-    if (inz) { pout[oz] = m_exz; pout[SZ + oz] = m_hyz; }
+    if (inx[k]) { pout[ox[k]] = m_ezx[k]; pout[SX + ox[k]] = m_hyx[k]; }
+    if (inz[k]) { pout[oz[k]] = m_exz[k]; pout[SZ + oz[k]] = m_hyz[k]; }
   };
-  const int tu = ty > 0 ? ty - 1 : 0, td = ty < RM - 1 ? ty + 1 : RM - 1;
+  const int tu = tq > 0 ? tq - 1 : 0, td = tq < RM / EK - 1 ? tq + 1 : RM / EK - 1;
   for (int t = 0; t < nsteps; ++t) {
     // ---- Hy (electromagfdtd.f95:249-266) ----
-    L.ex[ty][tx] = ex;
+    L.ex[tq][tx] = ex[0];
     __syncthreads();
-    {
-      const T ez_e = dpp_next(ez), ex_n = L.ex[td][tx];
-      if (!PML || (in && i <= nx - 2 && r <= nz - 2)) {
-        T a = (ex_n - ex) * idz;
-        if (inz) {
-          m_exz = fma(L.pz[PB][ty], m_exz, L.pz[PA][ty] * a);
-          a = fma(a, L.pz[PK][ty], m_exz);
+#pragma unroll
+    for (int k = 0; k < EK; ++k) {
+      const int ty = EK * tq + k, r = z0 + ty;
+      const T ez_e = dpp_next(ez[k]), ex_n = k + 1 < EK ? ex[(k + 1) % EK] : L.ex[td][tx];
+      if (!PML || (in[k] && i <= nx - 2 && r <= nz - 2)) {
+        T a = (ex_n - ex[k]) * idz;
+        if (inz[k]) {
+          m_exz[k] = fma(L.pz[PB][ty], m_exz[k], L.pz[PA][ty] * a);
+          a = fma(a, L.pz[PK][ty], m_exz[k]);
         }
-        T b = (ez_e - ez) * idx;
-        if (inx) {
-          m_ezx = fma(L.px[PB][tx], m_ezx, L.px[PA][tx] * b);
-          b = fma(b, L.px[PK][tx], m_ezx);
+        T b = (ez_e - ez[k]) * idx;
+        if (inx[k]) {
+          m_ezx[k] = fma(L.px[PB][tx], m_ezx[k], L.px[PA][tx] * b);
+          b = fma(b, L.px[PK][tx], m_ezx[k]);
         }
         // (the zeroing of the ring that ends the last step, :312-315)
         const bool edge = PML && (i == 0 || i == nx - 2 || r == 0 || r == nz - 2);
-        hy = fma(dbh, b + a, edge ? T(0) : hy);
+        hy[k] = fma(dbh, b + a, edge ? T(0) : hy[k]);
       }
     }
     // ---- Ex, Ez (:273-295), source, Dirichlet ----
-    L.hy[ty][tx] = hy;
+    L.hy[tq][tx] = hy[EK - 1];
     __syncthreads();
-    {
-      const T hy_w = dpp_prev(hy), hy_p = L.hy[tu][tx];
-      if (!PML || (in && i <= nx - 2 && r >= 1 && r <= nz - 2)) {
-        T d = (hy - hy_p) * idz;
-        if (inz) {
-          m_hyz = fma(L.pz[PBH][ty], m_hyz, L.pz[PAH][ty] * d);
-          d = fma(d, L.pz[PKH][ty], m_hyz);
+#pragma unroll
+    for (int k = 0; k < EK; ++k) {
+      const int ty = EK * tq + k, r = z0 + ty;
+      const T hy_w = dpp_prev(hy[k]), hy_p = k > 0 ? hy[(k + EK - 1) % EK] : L.hy[tu][tx];
+      if (!PML || (in[k] && i <= nx - 2 && r >= 1 && r <= nz - 2)) {
+        T d = (hy[k] - hy_p) * idz;
+        if (inz[k]) {
+          m_hyz[k] = fma(L.pz[PBH][ty], m_hyz[k], L.pz[PAH][ty] * d);
+          d = fma(d, L.pz[PKH][ty], m_hyz[k]);
         }
-        ex = fma(cax, ex, cbx * d);
+        ex[k] = fma(cax[k], ex[k], cbx[k] * d);
       }
-      if (!PML || (in && i >= 1 && i <= nx - 2 && r <= nz - 2)) {
-        T d = (hy - hy_w) * idx;
-        if (inx) {
-          m_hyx = fma(L.px[PBH][tx], m_hyx, L.px[PAH][tx] * d);
-          d = fma(d, L.px[PKH][tx], m_hyx);
+      if (!PML || (in[k] && i >= 1 && i <= nx - 2 && r <= nz - 2)) {
+        T d = (hy[k] - hy_w) * idx;
+        if (inx[k]) {
+          m_hyx[k] = fma(L.px[PBH][tx], m_hyx[k], L.px[PAH][tx] * d);
+          d = fma(d, L.px[PKH][tx], m_hyx[k]);
         }
-        ez = fma(caz, ez, cbz * d);
+        ez[k] = fma(caz[k], ez[k], cbz[k] * d);
       }
-      if (issrc) {
-        ex += L.src[0][t];
-        ez += L.src[1][t];
+      if (issrc[k]) {
+        ex[k] += L.src[0][t];
+        ez[k] += L.src[1][t];
       }
       if (PML) {  // :304-311, and the cells outside the fields' extents
-        if (i <= 0 || i >= nx - 2 || r <= 0 || r >= nz - 1) ex = 0;
-        if (i <= 0 || i >= nx - 1 || r <= 0 || r >= nz - 2) ez = 0;
+        if (i <= 0 || i >= nx - 2 || r <= 0 || r >= nz - 1) ex[k] = 0;
+        if (i <= 0 || i >= nx - 1 || r <= 0 || r >= nz - 2) ez[k] = 0;
       }
-      if (TRAIL && own) {
+      if (TRAIL && own[k]) {
         T* const o = trail + (t + 1) * ts.adj->slot;
-        store(o, o + n, o + 2 * n, o + 3 * n);
-      } else if (own) {
-        if (!((double)ex * ex + (double)ez * ez <= 1.0e50)) bad = min(bad, it0 + t);
-        region_sample<T>(S, it0 + t, i, e0, e1, id0, more, ex, ez);
+        store(k, o, o + n, o + 2 * n, o + 3 * n);
+      } else if (own[k]) {
+        if (!((double)ex[k] * ex[k] + (double)ez[k] * ez[k] <= 1.0e50)) bad = min(bad, it0 + t);
+        region_sample<T>(S, it0 + t, i, r, rec[k], ex[k], ez[k]);
       }
     }
   }
-  if (!TRAIL && own) {
-    if (par)
-      store(S.f[0], S.f[1], S.f[2], S.psi);
-    else
-      store(S.g[0], S.g[1], S.g[2], S.psi2);
-    if (bad != INT_MAX) atomicMin(S.blowup, bad);
-  }
+  if (TRAIL) return;
+#pragma unroll
+  for (int k = 0; k < EK; ++k)
+    if (own[k]) {
+      if (par)
+        store(k, S.f[0], S.f[1], S.f[2], S.psi);
+      else
+        store(k, S.g[0], S.g[1], S.g[2], S.psi2);
+    }
+  if (bad != INT_MAX) atomicMin(S.blowup, bad);
 }
 
-template <typename T, bool TRAIL>
-__global__ void __launch_bounds__(RM* RM, 8)
+template <typename T, bool TRAIL, int EK>
+__global__ void __launch_bounds__(RM* RM / EK, 8)
 k_em2_multi(const DModel* __restrict__ models, const DShot* __restrict__ shots, const int4* __restrict__ work,
             int n, const int* __restrict__ base, int rel, int nsteps, int tm, int par,
             const DAdj* __restrict__ adj, const int* __restrict__ tsel) {
-  __shared__ EmRegionLds<T> L;
+  __shared__ EmRegionLds<T, EK> L;
   const int q = item8(n);
   if (q < 0) return;
   const int4 wv = work[q];
@@ -3324,9 +3357,9 @@ k_em2_multi(const DModel* __restrict__ models, const DShot* __restrict__ shots, 
   const int x0 = __builtin_amdgcn_readfirstlane(wv.y) - tm, z0 = __builtin_amdgcn_readfirstlane(wv.z) - tm;
   const TrailSlot ts{TRAIL ? adj + s : nullptr, TRAIL ? __builtin_amdgcn_readfirstlane(*tsel) : 0, rel};
   if (region_interior(M, x0, z0))
-    em2_region<T, false, TRAIL>(M, S, x0, z0, it0, nsteps, tm, par, ts, L);
+    em2_region<T, false, TRAIL, EK>(M, S, x0, z0, it0, nsteps, tm, par, ts, L);
   else
-    em2_region<T, true, TRAIL>(M, S, x0, z0, it0, nsteps, tm, par, ts, L);
+    em2_region<T, true, TRAIL, EK>(M, S, x0, z0, it0, nsteps, tm, par, ts, L);
 }
 
 // ===========================================================================
@@ -4340,7 +4373,7 @@ long long regions2d(const Plan* p, int tm) {
 // shots (413 MB of fields) 92 -> 100; elastic FP32 296^2 6.7 -> 2.8, 1064x808 17.9
 // -> 9.4, x 16 shots 125 -> 120, x 24 shots 177 -> 173, x 32 shots (1.1 GB) 229 ->
 // 229; EM FP64 127x103 3.5 -> 1.5, 1064x808 11.9 -> 6.1, x 32 shots 207 -> 174; EM
-// FP32 1064x808 7.6 -> 4.7, x 32 shots 123 -> 109, 2088x1540 x 32 shots 397 -> 376.
+// FP32 1064x808 7.6 -> 4.4, x 32 shots 123 -> 87, 2088x1540 x 32 shots 397 -> 313.
 // tm: a launch costs 5 to 7 us beside its steps, so the most steps for which the
 // regions still run all at once (one block of elastic FP64 per CU, else two):
 // 127x103 elastic FP64 5.1 / 2.8 / 2.3 with 2 / 4 / 7 steps, 296^2 5.2 / 3.4 / 5.8;
@@ -4446,8 +4479,11 @@ int launch_multi(Plan* p, hipStream_t st, int n, bool even) {
   const dim3 g((nw + 7) / 8 * 8), b(RM * RM);
   for (int l = 0; l < L; ++l) {
     const int r = (int)((long long)n * l / L), k = (int)((long long)n * (l + 1) / L) - r;
-    if (p->kind == SDT_EM2)
-      hipLaunchKernelGGL((k_em2_multi<T, TRAIL>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k, tm,
+    if (p->kind == SDT_EM2 && !TRAIL && sizeof(T) == 4 && nw > 512)  // (see EmRegionLds)
+      hipLaunchKernelGGL((k_em2_multi<float, false, 2>), g, dim3(RM * RM / 2), 0, st, p->dmodels, p->dshots, w, nw,
+                         p->dbase, r, k, tm, l & 1, p->dadj, p->dtsel_trail);
+    else if (p->kind == SDT_EM2)
+      hipLaunchKernelGGL((k_em2_multi<T, TRAIL, 1>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k, tm,
                          l & 1, p->dadj, p->dtsel_trail);
     else if (p->split)
       hipLaunchKernelGGL((k_el2_multi<T, true, TRAIL>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k,

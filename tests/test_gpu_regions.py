@@ -138,3 +138,18 @@ def test_region_recomputation_equals_one_step_kernel(kind, split, precision, nx,
                 assert torch.equal(b["state"], got), (it0, k, s)
     a.close()
     e.close()
+
+
+@pytest.mark.parametrize("nx,nz,npml,nshots", [(400, 270, 9, 3), (803, 611, 13, 1), (660, 23, 6, 18)])
+def test_em_regions_of_two_rows_per_thread(nx, nz, npml, nshots):
+    """FP32 EM plans of more than 512 regions (two rows per thread, remainders
+    of odd heights) against the one-step kernel."""
+    from seidart_amd.solver import Simulation
+    p = _ring(tiny_problem("em2", seed=460 + nx, nx=nx, nz=nz, npml=npml, nt=48, nshots=nshots))
+    a, b = _walk(p, "fp32"), Simulation(p, precision="fp32")
+    for n, gb in ((1, 0), (7, 0), (22, 11), (18, 5)):
+        a.run(n)
+        b.run(n, graph_block=gb)
+        _same(a, b)
+    a.close()
+    b.close()
