@@ -487,19 +487,23 @@ def main(argv=None):
     gpu_ms = ev0.elapsed_time(ev1)
     sim.check()
     value = cells_per_step * K / wall / 1e9
-    # per-kernel durations (HIP events around each launch, same stream)
-    k_ms = sim.profile(PROFILE_STEPS)
+    # The shape the plan started with runs the region kernel, several steps per
+    # launch: its time per step is the timed run's.  Other shapes: per-kernel
+    # durations (HIP events around each launch, same stream).
+    regions = (sim_spl, *sim_tiles, sim_order) == sim._own_shape
+    k_ms = (gpu_ms / K, 0.0, 0.0) if regions else sim.profile(PROFILE_STEPS)
     sim.check()
-    # one launch of the step kernel advances `spl` steps (two by default: the
-    # state of the first stays in registers), so its algorithmic bytes are
-    # spl times those of one step
-    spl = sim.steps_per_launch
+    # one launch of the step kernel advances `spl` steps (two: the state of the
+    # first stays in registers), so its algorithmic bytes are spl times those of
+    # one step (regions: both per step)
+    spl = 1 if regions else sim.steps_per_launch
     dom_bytes = spl * algorithmic_bytes(problems, shots, 4)
     achieved = dom_bytes / (k_ms[0] * 1e-3) / 1e9
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": measured_traffic(dom_bytes),
-                "kernel": "k_el2_step2<float>" if spl == 2 else "k_el2_step<float>",
+                "kernel": "k_el2_multi<float>, per step" if regions else
+                          "k_el2_step2<float>" if spl == 2 else "k_el2_step<float>",
                 "kernel_ms": round(k_ms[0], 4), "steps_per_launch": spl,
                 "alg_bytes_per_launch": int(dom_bytes),
                 "alg_bytes_per_cell_update": round(dom_bytes / spl / cells_per_step, 2),

@@ -2852,10 +2852,14 @@ k_el25_vel(const DModel* __restrict__ models, const DShot* __restrict__ shots,
 // per thread, with the state, the memory variables and the coefficients in
 // registers, and takes up to tm steps: rows are exchanged through LDS, columns
 // by DPP lane shifts (a wavefront is two rows of the region; what a shift
-// carries across their ends reaches only halo columns).  One elastic step makes
-// a cell depend on columns i-1 .. i+2 and rows k-2 .. k+1, one EM step on one
-// neighbour each way, so after tm steps the middle of the region is exact
-// (columns tm .. RM-2tm-1 and rows 2tm .. RM-tm-1; EM tm .. RM-tm-1 both ways):
+// carries across their ends reaches only halo columns).  One step makes a cell
+// depend on one neighbour each way; with the legacy C-PML, whose shear loop uses
+// the memory the normal loop has just updated, an elastic cell also on column
+// i+2 and row k-2.  So after tm steps the middle of the region is exact (columns
+// and rows tm .. RM-tm-1; legacy elastic columns tm .. RM-2tm-1, rows 2tm ..
+// RM-tm-1; the split C-PML with its own ring instead of that one, us per step:
+// FP32 48 shots of 39 M cells 350 -> 248, 16 of 1064x552 77 -> 61, FP64 296^2 3.4 ->
+// 2.9, 4 of 1064x808 67 -> 50):
 // the block owns that and the neighbouring blocks recompute the rest.  Every
 // expression is the one-step kernel's, in the same order: identical bits.  A
 // launch reads state buffer par and writes the other.
@@ -2871,6 +2875,11 @@ k_el25_vel(const DModel* __restrict__ models, const DShot* __restrict__ shots,
 // ===========================================================================
 constexpr int RM = 32;       // region: RM x RM cells, one thread each
 constexpr int TM_MAX = 8;    // most steps per launch
+
+// Elastic regions of tm steps: rows above the owned cells (tm columns to their
+// left), owned cells a side.
+__host__ __device__ constexpr int el_top(bool split, int tm) { return split ? tm : 2 * tm; }
+__host__ __device__ constexpr int el_own(bool split, int tm) { return RM - (split ? 2 : 3) * tm; }
 
 // The receivers of a thread's K cells (rows z0 + K * (threadIdx.x / RM) + k of
 // the region at x0, z0): per cell the first index entry on it (INT_MAX: none),
@@ -2955,10 +2964,10 @@ __device__ __forceinline__ void el2_region(const DModel& M, const DShot& S, cons
 #pragma clang fp contract(off)
   const int nx = M.nx, nz = M.nz;
   const int tx = threadIdx.x & (RM - 1), ty = threadIdx.x / RM;
-  const int i = x0 + tx, r = z0 + ty, osz = RM - 3 * tm;
+  const int i = x0 + tx, r = z0 + ty, osz = el_own(SPLIT, tm), zt = el_top(SPLIT, tm);
   const bool in = !PML || (i >= 0 && i < nx && r >= 0 && r < nz);
   const int ic = PML ? min(max(i, 0), nx - 1) : i, rc = PML ? min(max(r, 0), nz - 1) : r;
-  const bool own = in && tx >= tm && tx < tm + osz && ty >= 2 * tm && ty < 2 * tm + osz;
+  const bool own = in && tx >= tm && tx < tm + osz && ty >= zt && ty < zt + osz;
   const uint32_t c = (uint32_t)rc * nx + ic;
   const long n = (long)nx * nz;
   T* const trail = TRAIL ? static_cast<T*>(ts.adj->trail[ts.tb]) + ts.slot * ts.adj->slot : nullptr;
@@ -3014,7 +3023,7 @@ __device__ __forceinline__ void el2_region(const DModel& M, const DShot& S, cons
   const bool issrc = in && i == S.isrc && r == S.ksrc;
   const bool msrc = S.msrc[0] || S.msrc[2] || S.msrc[4];
   RegionRec rec[1];
-  if (!TRAIL) region_receivers<1>(S, L.slot, x0, z0, nz, tm, 2 * tm, osz, {own}, rec);
+  if (!TRAIL) region_receivers<1>(S, L.slot, x0, z0, nz, tm, zt, osz, {own}, rec);
   int bad = INT_MAX;
   auto store = [&](void* o0, void* o1, void* o2, void* o3, void* o4, void* o5) {
     A32<T>{o0}[c] = vx;
@@ -3171,7 +3180,7 @@ k_el2_multi(const DModel* __restrict__ models, const DShot* __restrict__ shots, 
   const DShot& S = shots[s];
   const DModel& M = models[__builtin_amdgcn_readfirstlane(wv.w)];
   const int it0 = __builtin_amdgcn_readfirstlane(*base + rel);
-  const int x0 = __builtin_amdgcn_readfirstlane(wv.y) - tm, z0 = __builtin_amdgcn_readfirstlane(wv.z) - 2 * tm;
+  const int x0 = __builtin_amdgcn_readfirstlane(wv.y) - tm, z0 = __builtin_amdgcn_readfirstlane(wv.z) - el_top(SPLIT, tm);
   const TrailSlot ts{TRAIL ? adj + s : nullptr, TRAIL ? __builtin_amdgcn_readfirstlane(*tsel) : 0, rel};
   if (region_interior(M, x0, z0))
     el2_region<T, SPLIT, false, TRAIL>(M, S, x0, z0, it0, nsteps, tm, par, ts, L);
@@ -4354,8 +4363,9 @@ long long waves2d(const Plan* p, int ew, int rows) {
 }
 
 // Regions of a 2-D plan whose halo is tm steps wide.
+int region_own(const Plan* p, int tm) { return el_own(p->kind == SDT_EM2 || p->split, tm); }
 long long regions2d(const Plan* p, int tm) {
-  const int own = RM - (p->kind == SDT_EM2 ? 2 : 3) * tm;
+  const int own = region_own(p, tm);
   long long n = 0;
   for (const sdt_shot& S : p->hshots) {
     const sdt_model& M = p->hmodels[S.model];
@@ -4365,10 +4375,11 @@ long long regions2d(const Plan* p, int tm) {
 }
 
 // Whether a 2-D plan runs on regions (k_el2_multi, k_em2_multi) and the most
-// steps per launch there.  A region recomputes its halo (tm = 4 elastic: 40 % of
-// its cells are owned, tm = 5 EM: 47 %), which pays where the walking kernels
-// wait on launches and loads, not where they stream: measured (us per step,
-// walking kernels in the shape of default_shape, then regions) elastic FP64
+// steps per launch there.  A region recomputes its halo (tm = 4 legacy elastic:
+// 40 % of its cells are owned, tm = 5 else: 47 %).  Measured (us per step, walking
+// kernels in the shape of default_shape, then regions): split elastic FP32 39 M
+// cells of 48 shots 312 -> 248, 32 shots of 1064x808 234 -> 159, FP64 12 shots 163 ->
+// 144, 8 of 2088x808 216 -> 185, 296^2 7.7 -> 2.9.  Legacy elastic FP64
 // 127x103 6.4 -> 2.3, 296^2 7.8 -> 3.4, 1064x808 27 -> 19, x 4 shots 71 -> 67, x 6
 // shots (413 MB of fields) 92 -> 100; elastic FP32 296^2 6.7 -> 2.8, 1064x808 17.9
 // -> 9.4, x 16 shots 125 -> 120, x 24 shots 177 -> 173, x 32 shots (1.1 GB) 229 ->
@@ -4380,13 +4391,13 @@ long long regions2d(const Plan* p, int tm) {
 // larger plans take the number whose owned share balances the launches.
 void default_regions(Plan* p, double bytes) {
   const bool em = p->kind == SDT_EM2, f64 = p->prec == SDT_FP64;
-  p->tm = em ? 5 : f64 && regions2d(p, 4) > 2500 ? 3 : 4;
+  p->tm = em || p->split ? 5 : f64 && regions2d(p, 4) > 2500 ? 3 : 4;
   for (int t = TM_MAX; t >= (!em && f64 ? 2 : 3); --t)
     if (regions2d(p, t) <= (!em && f64 ? 256 : 512)) {
       p->tm = t;
       break;
     }
-  p->multi = em || bytes < (f64 ? 350e6 : 900e6);
+  p->multi = em || p->split || bytes < (f64 ? 350e6 : 900e6);
 }
 
 // Default launch shape of a 2-D plan: steps per launch, wavefronts per block,
@@ -4455,7 +4466,7 @@ void default_shape(Plan* p) {
 // EM FP32 32 shots of 1064x808 118 us per step against 107, elastic FP32 16 of
 // 1064x552 84 against 77, their recomputation 142 against 114).
 std::vector<int4> multi_work(const Plan* p, int tm) {
-  const int own = RM - (p->kind == SDT_EM2 ? 2 : 3) * tm;
+  const int own = region_own(p, tm);
   std::vector<int4> w;
   for (int s = 0; s < p->nshots; ++s) {
     const int m = p->hshots[s].model;
@@ -5825,7 +5836,7 @@ int sdt_adjoint_setup(void* plan, const sdt_adj_shot* adj, int nshots, unsigned 
   if (!p->dtsel_adj) HIP_TRY(hipMalloc(&p->dtsel_adj, sizeof(int)));
   if (!p->dtrwork) {
     // The recomputation runs on regions at every size, at the plan's steps per
-    // launch where they all run at once, else at 3 (EM: 4).  It writes every
+    // launch where they all run at once, else at 4 (legacy C-PML: 3).  It writes every
     // step's state, so that at the largest plans the writes bound it (elastic
     // FP32 16 shots of 1064x552: 188 MB, 40 us at 5 TB/s) and a wider ring costs
     // more than fewer reads give.  Measured (us per step, one launch of tiled
@@ -5833,8 +5844,8 @@ int sdt_adjoint_setup(void* plan, const sdt_adj_shot* adj, int nshots, unsigned 
     // 120x90 9.8, 3.9 / 3.2 / 2.8 / 2.6, 740x440 x 6 shots 41, 25 / 27 / 28 / 34,
     // 1064x552 x 16 shots 160, 140 / 121 / 138 / 164; FP64 64, 53 / 52 / 49 / 61 and 255,
     // 245 / 211 / 233 / 266; EM FP64 1064x808 x 2 shots 30, 22 / 21 / 20 / 22.
-    const bool em = p->kind == SDT_EM2;
-    p->tr_tm = p->tm > (em ? 5 : 4) ? p->tm : em ? 4 : 3;
+    const bool wide = p->kind == SDT_ELASTIC2 && !p->split;
+    p->tr_tm = p->tm > (wide ? 4 : 5) ? p->tm : wide ? 3 : 4;
     const std::vector<int4> work = multi_work(p, p->tr_tm);
     int4* dw = nullptr;
     HIP_TRY(hipMalloc(&dw, sizeof(int4) * work.size()));
