@@ -2855,11 +2855,11 @@ k_el25_vel(const DModel* __restrict__ models, const DShot* __restrict__ shots,
 // carries across their ends reaches only halo columns).  One step makes a cell
 // depend on one neighbour each way; with the legacy C-PML, whose shear loop uses
 // the memory the normal loop has just updated, an elastic cell also on column
-// i+2 and row k-2.  So after tm steps the middle of the region is exact (columns
-// and rows tm .. RM-tm-1; legacy elastic columns tm .. RM-2tm-1, rows 2tm ..
-// RM-tm-1; the split C-PML with its own ring instead of that one, us per step:
-// FP32 48 shots of 39 M cells 350 -> 248, 16 of 1064x552 77 -> 61, FP64 296^2 3.4 ->
-// 2.9, 4 of 1064x808 67 -> 50):
+// i+2 (in an x slab) and row k-2 (in a z slab).  So after tm steps the middle of
+// the region is exact (columns and rows tm .. RM-tm-1; where a legacy region
+// touches an x slab columns tm .. RM-2tm-1, a z slab rows 2tm .. RM-tm-1; with
+// that wider ring everywhere, us per step: FP32 48 shots of 39 M cells 350, now
+// 248, 16 of 1064x552 77, 61, FP64 9 uneven shots 26, 21, 4 of 1064x808 67, 50):
 // the block owns that and the neighbouring blocks recompute the rest.  Every
 // expression is the one-step kernel's, in the same order: identical bits.  A
 // launch reads state buffer par and writes the other.
@@ -2876,14 +2876,18 @@ k_el25_vel(const DModel* __restrict__ models, const DShot* __restrict__ shots,
 constexpr int RM = 32;       // region: RM x RM cells, one thread each
 constexpr int TM_MAX = 8;    // most steps per launch
 
-// Elastic regions of tm steps: rows above the owned cells (tm columns to their
-// left), owned cells a side.
-__host__ __device__ constexpr int el_top(bool split, int tm) { return split ? tm : 2 * tm; }
-__host__ __device__ constexpr int el_own(bool split, int tm) { return RM - (split ? 2 : 3) * tm; }
+// Regions of tm steps, along one axis: rows above the owned cells (tm columns to
+// their left), owned cells.  one: a step reaches one cell each way; otherwise
+// the legacy elastic C-PML, on the axis whose slab the region touches.
+__host__ __device__ constexpr int region_top(bool one, int tm) { return one ? tm : 2 * tm; }
+__host__ __device__ constexpr int region_own(bool one, int tm) { return RM - (one ? 2 : 3) * tm; }
+// Flags of a legacy elastic work item beside its model: the region keeps off
+// the x slabs, off the z slabs.
+constexpr int REGION_X1 = 1 << 30, REGION_Z1 = 1 << 29;
 
 // The receivers of a thread's K cells (rows z0 + K * (threadIdx.x / RM) + k of
 // the region at x0, z0): per cell the first index entry on it (INT_MAX: none),
-// that receiver, and whether more follow.  The block owns own x own cells from
+// that receiver, and whether more follow.  The block owns ownx x ownz cells from
 // column cx0, row cz0 on; mine: the thread's cell is one of them.  Called by
 // every thread; slot: one entry per cell.
 struct RegionRec {
@@ -2892,8 +2896,9 @@ struct RegionRec {
 };
 template <int K>
 __device__ __forceinline__ void region_receivers(const DShot& S, int* slot, int x0, int z0, int nz, int cx0,
-                                                 int cz0, int own, const bool (&mine)[K], RegionRec (&rec)[K]) {
-  const int zr0 = z0 + cz0, zr1 = min(zr0 + own, nz);
+                                                 int cz0, int ownx, int ownz, const bool (&mine)[K],
+                                                 RegionRec (&rec)[K]) {
+  const int zr0 = z0 + cz0, zr1 = min(zr0 + ownz, nz);
   for (int k = 0; k < K; ++k) rec[k] = {INT_MAX, 0, false};
   if (S.nrec <= 0 || S.rrow[zr1] <= S.rrow[zr0]) return;  // block-uniform
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -2906,7 +2911,7 @@ __device__ __forceinline__ void region_receivers(const DShot& S, int* slot, int 
     const int q0 = S.rrow[row], q1 = S.rrow[row + 1];
     for (int e = q0 + lane; e < q1; e += 64) {
       const int cx = S.rxid[2 * e] - x0;
-      if (cx >= cx0 && cx < cx0 + own) atomicMin(&slot[(2 * K * w + h) * RM + cx], e);
+      if (cx >= cx0 && cx < cx0 + ownx) atomicMin(&slot[(2 * K * w + h) * RM + cx], e);
     }
   }
   __syncthreads();
@@ -2959,15 +2964,16 @@ struct TrailSlot {
 
 template <typename T, bool SPLIT, bool PML, bool TRAIL>
 __device__ __forceinline__ void el2_region(const DModel& M, const DShot& S, const int x0, const int z0,
-                                           const int it0, const int nsteps, const int tm, const int par,
+                                           const bool x1, const bool z1, const int it0, const int nsteps, const int tm, const int par,
                                            const TrailSlot ts, ElRegionLds<T, SPLIT>& L) {
 #pragma clang fp contract(off)
   const int nx = M.nx, nz = M.nz;
   const int tx = threadIdx.x & (RM - 1), ty = threadIdx.x / RM;
-  const int i = x0 + tx, r = z0 + ty, osz = el_own(SPLIT, tm), zt = el_top(SPLIT, tm);
+  const int i = x0 + tx, r = z0 + ty;
+  const int osx = region_own(x1, tm), osz = region_own(z1, tm), zt = region_top(z1, tm);
   const bool in = !PML || (i >= 0 && i < nx && r >= 0 && r < nz);
   const int ic = PML ? min(max(i, 0), nx - 1) : i, rc = PML ? min(max(r, 0), nz - 1) : r;
-  const bool own = in && tx >= tm && tx < tm + osz && ty >= zt && ty < zt + osz;
+  const bool own = in && tx >= tm && tx < tm + osx && ty >= zt && ty < zt + osz;
   const uint32_t c = (uint32_t)rc * nx + ic;
   const long n = (long)nx * nz;
   T* const trail = TRAIL ? static_cast<T*>(ts.adj->trail[ts.tb]) + ts.slot * ts.adj->slot : nullptr;
@@ -3023,7 +3029,7 @@ __device__ __forceinline__ void el2_region(const DModel& M, const DShot& S, cons
   const bool issrc = in && i == S.isrc && r == S.ksrc;
   const bool msrc = S.msrc[0] || S.msrc[2] || S.msrc[4];
   RegionRec rec[1];
-  if (!TRAIL) region_receivers<1>(S, L.slot, x0, z0, nz, tm, zt, osz, {own}, rec);
+  if (!TRAIL) region_receivers<1>(S, L.slot, x0, z0, nz, tm, zt, osx, osz, {own}, rec);
   int bad = INT_MAX;
   auto store = [&](void* o0, void* o1, void* o2, void* o3, void* o4, void* o5) {
     A32<T>{o0}[c] = vx;
@@ -3178,14 +3184,17 @@ k_el2_multi(const DModel* __restrict__ models, const DShot* __restrict__ shots, 
   const int4 wv = work[q];
   const int s = __builtin_amdgcn_readfirstlane(wv.x);
   const DShot& S = shots[s];
-  const DModel& M = models[__builtin_amdgcn_readfirstlane(wv.w)];
+  const int mf = __builtin_amdgcn_readfirstlane(wv.w);
+  const bool x1 = SPLIT || (mf & REGION_X1), z1 = SPLIT || (mf & REGION_Z1);
+  const DModel& M = models[mf & (REGION_Z1 - 1)];
   const int it0 = __builtin_amdgcn_readfirstlane(*base + rel);
-  const int x0 = __builtin_amdgcn_readfirstlane(wv.y) - tm, z0 = __builtin_amdgcn_readfirstlane(wv.z) - el_top(SPLIT, tm);
+  const int x0 = __builtin_amdgcn_readfirstlane(wv.y) - tm;
+  const int z0 = __builtin_amdgcn_readfirstlane(wv.z) - region_top(z1, tm);
   const TrailSlot ts{TRAIL ? adj + s : nullptr, TRAIL ? __builtin_amdgcn_readfirstlane(*tsel) : 0, rel};
   if (region_interior(M, x0, z0))
-    el2_region<T, SPLIT, false, TRAIL>(M, S, x0, z0, it0, nsteps, tm, par, ts, L);
+    el2_region<T, SPLIT, false, TRAIL>(M, S, x0, z0, x1, z1, it0, nsteps, tm, par, ts, L);
   else
-    el2_region<T, SPLIT, true, TRAIL>(M, S, x0, z0, it0, nsteps, tm, par, ts, L);
+    el2_region<T, SPLIT, true, TRAIL>(M, S, x0, z0, x1, z1, it0, nsteps, tm, par, ts, L);
 }
 
 // EK: rows per thread.  With two, the z neighbour of one of them is in the
@@ -3263,7 +3272,7 @@ __device__ __forceinline__ void em2_region(const DModel& M, const DShot& S, cons
   }
   const T idx = T(1.0 / M.dx), idz = T(1.0 / M.dz), dbh = T(M.scal[0]);
   RegionRec rec[EK];
-  if (!TRAIL) region_receivers<EK>(S, L.slot, x0, z0, nz, tm, tm, osz, own, rec);
+  if (!TRAIL) region_receivers<EK>(S, L.slot, x0, z0, nz, tm, tm, osz, osz, own, rec);
   int bad = INT_MAX;
   auto store = [&](int k, void* o0, void* o1, void* o2, void* o3) {
     A32<T>{o0}[c[k]] = ex[k];
@@ -4363,41 +4372,60 @@ long long waves2d(const Plan* p, int ew, int rows) {
 }
 
 // Regions of a 2-D plan whose halo is tm steps wide.
-int region_own(const Plan* p, int tm) { return el_own(p->kind == SDT_EM2 || p->split, tm); }
-long long regions2d(const Plan* p, int tm) {
-  const int own = region_own(p, tm);
-  long long n = 0;
-  for (const sdt_shot& S : p->hshots) {
-    const sdt_model& M = p->hmodels[S.model];
-    n += (long long)((M.nx + own - 1) / own) * ((M.nz + own - 1) / own);
+// Where the regions of one axis of n cells with slabs of l start owning cells,
+// and whether a step reaches one cell each way in them (region_own).
+std::vector<std::pair<int, bool>> region_cuts(const Plan* p, int n, int l, int tm) {
+  const bool legacy = p->kind == SDT_ELASTIC2 && !p->split;
+  std::vector<std::pair<int, bool>> c;
+  for (int o = 0; o < n; o += region_own(c.back().second, tm)) {
+    const int a = o - region_top(true, tm);  // (first cell of the region)
+    c.push_back({o, !legacy || (a >= l && a + RM <= n - l)});
   }
+  return c;
+}
+long long regions2d(const Plan* p, int tm) {
+  std::vector<long long> per(p->nmodels);
+  for (int m = 0; m < p->nmodels; ++m) {
+    const sdt_model& M = p->hmodels[m];
+    per[m] = (long long)(region_cuts(p, M.nx, M.lx, tm).size() * region_cuts(p, M.nz, M.lz, tm).size());
+  }
+  long long n = 0;
+  for (const sdt_shot& S : p->hshots) n += per[S.model];
   return n;
 }
 
-// Whether a 2-D plan runs on regions (k_el2_multi, k_em2_multi) and the most
-// steps per launch there.  A region recomputes its halo (tm = 4 legacy elastic:
-// 40 % of its cells are owned, tm = 5 else: 47 %).  Measured (us per step, walking
-// kernels in the shape of default_shape, then regions): split elastic FP32 39 M
-// cells of 48 shots 312 -> 248, 32 shots of 1064x808 234 -> 159, FP64 12 shots 163 ->
-// 144, 8 of 2088x808 216 -> 185, 296^2 7.7 -> 2.9.  Legacy elastic FP64
-// 127x103 6.4 -> 2.3, 296^2 7.8 -> 3.4, 1064x808 27 -> 19, x 4 shots 71 -> 67, x 6
-// shots (413 MB of fields) 92 -> 100; elastic FP32 296^2 6.7 -> 2.8, 1064x808 17.9
-// -> 9.4, x 16 shots 125 -> 120, x 24 shots 177 -> 173, x 32 shots (1.1 GB) 229 ->
-// 229; EM FP64 127x103 3.5 -> 1.5, 1064x808 11.9 -> 6.1, x 32 shots 207 -> 174; EM
-// FP32 1064x808 7.6 -> 4.4, x 32 shots 123 -> 87, 2088x1540 x 32 shots 397 -> 313.
-// tm: a launch costs 5 to 7 us beside its steps, so the most steps for which the
-// regions still run all at once (one block of elastic FP64 per CU, else two):
-// 127x103 elastic FP64 5.1 / 2.8 / 2.3 with 2 / 4 / 7 steps, 296^2 5.2 / 3.4 / 5.8;
-// larger plans take the number whose owned share balances the launches.
-void default_regions(Plan* p, double bytes) {
-  const bool em = p->kind == SDT_EM2, f64 = p->prec == SDT_FP64;
-  p->tm = em || p->split ? 5 : f64 && regions2d(p, 4) > 2500 ? 3 : 4;
-  for (int t = TM_MAX; t >= (!em && f64 ? 2 : 3); --t)
-    if (regions2d(p, t) <= (!em && f64 ? 256 : 512)) {
+// The most steps per launch of a 2-D plan on regions (k_el2_multi, k_em2_multi),
+// its default at every size.  A region recomputes its halo: with five steps per
+// launch 47 % of its cells are owned.  Measured (us per step, walking kernels in
+// the shape of default_shape, then regions): elastic FP64 127x103 6.3 -> 2.4, 296^2
+// 8.3 -> 3.0, 12 shots of 1064x808 158 -> 150, 8 of 2088x808 208 -> 196; FP32 1064x808
+// 18.7 -> 7.0, x 32 shots 227 -> 160, 48 shots of 39 M cells 312 -> 248; EM FP64
+// 127x103 3.5 -> 1.5, 1064x808 11.9 -> 6.1, x 32 shots 207 -> 156; EM FP32 1064x808 7.6
+// -> 4.4, x 32 shots 123 -> 87.
+// Where the regions run all at once (one block of elastic FP64 per CU, else two),
+// the most steps: a launch costs 5 to 7 us beside its steps (127x103 elastic FP64
+// 5.1 / 2.8 / 2.3 us per step with 2 / 4 / 7).  Larger plans: a launch's time is its
+// regions', whatever their steps, so the steps with the fewest regions times
+// launches in a block of 50 steps (an even number of launches): FP32 32 shots of
+// 1064x808 3 / 4 / 5 steps 211 / 188 / 159 (18 / 14 / 10 launches).
+void default_regions(Plan* p) {
+  auto cost = [&](int t) {
+    const int n = (50 + t - 1) / t;
+    return regions2d(p, t) * (n + (n & 1));
+  };
+  const int room = p->kind == SDT_ELASTIC2 && p->prec == SDT_FP64 ? 256 : 512;
+  p->tm = 5;
+  long long best = cost(5);
+  for (int t = 3; t <= TM_MAX; ++t) {
+    const long long c = cost(t);
+    if (c < best) { best = c; p->tm = t; }
+  }
+  for (int t = TM_MAX; t >= 3; --t)
+    if (regions2d(p, t) <= room) {
       p->tm = t;
       break;
     }
-  p->multi = em || p->split || bytes < (f64 ? 350e6 : 900e6);
+  p->multi = true;
 }
 
 // Default launch shape of a 2-D plan: steps per launch, wavefronts per block,
@@ -4453,7 +4481,7 @@ void default_shape(Plan* p) {
       if (waves2d(p, ew, rows) >= (f64 ? 2000 : em ? 2800 : 4000)) p->el2_eh = rows;
     if (waves2d(p, ew, 16) >= (em ? 12000 : 8000)) p->el2_eh = 16;
   }
-  default_regions(p, cells * kind_fields(p->kind) * 2 * (f64 ? 8 : 4));
+  default_regions(p);
   p->def_spl = p->spl;
   p->def_wb = p->el2_wb;
   p->def_eh = p->el2_eh;
@@ -4466,13 +4494,17 @@ void default_shape(Plan* p) {
 // EM FP32 32 shots of 1064x808 118 us per step against 107, elastic FP32 16 of
 // 1064x552 84 against 77, their recomputation 142 against 114).
 std::vector<int4> multi_work(const Plan* p, int tm) {
-  const int own = region_own(p, tm);
+  const bool legacy = p->kind == SDT_ELASTIC2 && !p->split;
   std::vector<int4> w;
+  w.reserve(regions2d(p, tm));
   for (int s = 0; s < p->nshots; ++s) {
     const int m = p->hshots[s].model;
     const sdt_model& M = p->hmodels[m];
-    for (int z = 0; z < M.nz; z += own)
-      for (int x = 0; x < M.nx; x += own) w.push_back(make_int4(s, x, z, m));
+    const auto xs = region_cuts(p, M.nx, M.lx, tm), zs = region_cuts(p, M.nz, M.lz, tm);
+    for (const auto& z : zs)
+      for (const auto& x : xs)
+        w.push_back(make_int4(s, x.first, z.first,
+                              m | (legacy && x.second ? REGION_X1 : 0) | (legacy && z.second ? REGION_Z1 : 0)));
   }
   return w;
 }
@@ -5836,7 +5868,7 @@ int sdt_adjoint_setup(void* plan, const sdt_adj_shot* adj, int nshots, unsigned 
   if (!p->dtsel_adj) HIP_TRY(hipMalloc(&p->dtsel_adj, sizeof(int)));
   if (!p->dtrwork) {
     // The recomputation runs on regions at every size, at the plan's steps per
-    // launch where they all run at once, else at 4 (legacy C-PML: 3).  It writes every
+    // launch where those are six or more, else at 4.  It writes every
     // step's state, so that at the largest plans the writes bound it (elastic
     // FP32 16 shots of 1064x552: 188 MB, 40 us at 5 TB/s) and a wider ring costs
     // more than fewer reads give.  Measured (us per step, one launch of tiled
@@ -5844,8 +5876,7 @@ int sdt_adjoint_setup(void* plan, const sdt_adj_shot* adj, int nshots, unsigned 
     // 120x90 9.8, 3.9 / 3.2 / 2.8 / 2.6, 740x440 x 6 shots 41, 25 / 27 / 28 / 34,
     // 1064x552 x 16 shots 160, 140 / 121 / 138 / 164; FP64 64, 53 / 52 / 49 / 61 and 255,
     // 245 / 211 / 233 / 266; EM FP64 1064x808 x 2 shots 30, 22 / 21 / 20 / 22.
-    const bool wide = p->kind == SDT_ELASTIC2 && !p->split;
-    p->tr_tm = p->tm > (wide ? 4 : 5) ? p->tm : wide ? 3 : 4;
+    p->tr_tm = p->tm > 5 ? p->tm : 4;
     const std::vector<int4> work = multi_work(p, p->tr_tm);
     int4* dw = nullptr;
     HIP_TRY(hipMalloc(&dw, sizeof(int4) * work.size()));
