@@ -219,7 +219,9 @@ class Simulation:
         events; return mean ms per launch of (first field kernel, second
         field kernel, receiver gather).  With two steps per launch
         (``steps_per_launch``) the first is the two-step kernel, per launch,
-        and the gather is 0 (the kernel writes the receiver samples)."""
+        and the gather is 0 (the kernel writes the receiver samples).  These
+        are the kernels of the launch shape also where ``run`` takes regions
+        (several steps per launch, the default of the 2-D kinds)."""
         if stream is None:
             stream = torch.cuda.current_stream(self.device)
         out = (C.c_double * 3)()
@@ -232,7 +234,8 @@ class Simulation:
     def steps_per_launch(self) -> int:
         """Time steps one launch of the ELASTIC2 / EM2 step kernel advances
         (2 by default, 1 for small ELASTIC2 plans; ``autotune`` times both);
-        results do not depend on it."""
+        while the whole launch shape is the plan's own, ``run`` takes regions,
+        up to 8 steps per launch.  Results do not depend on it."""
         v = C.c_int()
         _hip.check(_hip.lib().sdt_plan_get_steps_per_launch(self._plan, C.byref(v)))
         return v.value
