@@ -4958,10 +4958,13 @@ int validate(int kind, bool split, int prec, const sdt_model* models, int nmodel
       if ((long long)M.nx * M.nz * es >= (1LL << 32) || np * es >= (1LL << 32))
         return fail(SDT_EINVAL, tag + "grid too large (every array must stay under 4 GiB)");
     }
-    if (kind == SDT_ELASTIC25) {
-      // the kernels address one z plane of a field with 32-bit byte offsets
+    if (d3) {
+      // the kernels address one z plane of a field or memory variable, and a
+      // coefficient array, with 32-bit byte offsets (slabs that cover an odd
+      // axis hold one cell more than it), and pack a y chunk in 16-bit halves
       const long long es = prec == SDT_FP64 ? 8 : 4;
-      if ((long long)M.nx * M.ny * es >= (1LL << 32) || (long long)M.nx * M.nz * es >= (1LL << 32))
+      const long long wide = std::max(M.nx, 2 * M.lx), tall = std::max(M.ny, 2 * M.ly);
+      if (std::max(wide * M.ny, M.nx * tall) * es >= (1LL << 32) || (long long)M.nx * M.nz * es >= (1LL << 32))
         return fail(SDT_EINVAL, tag + "grid too large (an x-y plane must stay under 4 GiB)");
       if (M.ny > 65535) return fail(SDT_EINVAL, tag + "ny above 65535");
     }

@@ -154,6 +154,36 @@ def test_plan_create_rejects_bad_input(mutate, msg):
     assert not plan.value
 
 
+@pytest.mark.parametrize("kind,ncoef", [(_hip.SDT_ELASTIC25, 39), (_hip.SDT_EM25, 6)])
+@pytest.mark.parametrize("prec,dims,slabs,msg", [
+    (_hip.SDT_FP32, (3, 65536, 3), (0, 0, 0), "ny above 65535"),
+    (_hip.SDT_FP64, (40000, 15000, 3), (0, 0, 0), "grid too large"),          # x-y plane
+    (_hip.SDT_FP64, (600000, 3, 900), (0, 0, 0), "grid too large"),           # coefficients
+    (_hip.SDT_FP64, (32767, 16384, 3), (16384, 0, 0), "grid too large"),      # x slabs of nx + 1 cells
+    (_hip.SDT_FP64, (16384, 32767, 3), (0, 16384, 0), "grid too large"),      # y slabs of ny + 1 rows
+])
+def test_plan_create_rejects_25d_planes_beyond_the_offsets(kind, ncoef, prec, dims, slabs, msg):
+    """What the 2.5-D kernels cannot address (32-bit byte offsets in a plane,
+    y chunks in 16-bit halves) is refused, for both kinds."""
+    M, S = _model(), _shot()
+    M.nx, M.ny, M.nz = dims
+    M.lx, M.ly, M.lz = slabs
+    S.isrc, S.jsrc, S.ksrc = 1, 1, 1
+    for q in range(ncoef):
+        M.coef[q] = 0x1000
+    for q in range(6):
+        M.prof[1][q] = 0x1000
+    for f in range(9):
+        S.field[f] = 0x1000
+    models = (_hip.SdtModel * 1)(M)
+    shots = (_hip.SdtShot * 1)(S)
+    plan = C.c_void_p()
+    rc = _hip.lib().sdt_plan_create(kind, prec, models, 1, shots, 1, 10, C.byref(plan))
+    assert rc == _hip.SDT_EINVAL
+    assert msg in _hip.lib().sdt_last_error().decode()
+    assert not plan.value
+
+
 def test_plan_run_rejects_null_plan():
     rc = _hip.lib().sdt_plan_run(None, 0, 1, 0, None)
     assert rc == _hip.SDT_EINVAL
