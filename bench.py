@@ -490,7 +490,7 @@ def main(argv=None):
     # The shape the plan started with runs the region kernel, several steps per
     # launch: its time per step is the timed run's.  Other shapes: per-kernel
     # durations (HIP events around each launch, same stream).
-    regions = (sim_spl, *sim_tiles, sim_order) == sim._own_shape
+    regions = sim.regions
     k_ms = (gpu_ms / K, 0.0, 0.0) if regions else sim.profile(PROFILE_STEPS)
     sim.check()
     # one launch of the step kernel advances `spl` steps (two: the state of the

@@ -176,11 +176,10 @@ int sdt_plan_run(void* plan, int it0, int nsteps, int graph_block, void* stream)
  * columns (56 in the two-step ELASTIC2 kernel, 60 in the two-step EM2
  * one), walks `rows` rows (1..256).
  * Default: by the number of wavefronts the plan has (short tiles for small
- * plans, so that they fill the device).  While the tiles, their order and the
- * steps per launch are the defaults, sdt_plan_run and sdt_run_noalloc may also
- * run a plan on square regions that take several steps per launch.  Results do
- * not depend on the shape.
- * The adjoint's trail recomputation has a tile shape of its own.
+ * plans, so that they fill the device).  A call of this function, of
+ * sdt_plan_set_tile_order or of sdt_plan_set_steps_per_launch takes a plan off
+ * regions (sdt_plan_set_regions), whatever the values.  Results do not depend
+ * on the shape.  The adjoint's trail recomputation does not use it.
  * Synchronises the device when the shape changes. */
 int sdt_plan_set_tiles(void* plan, int waves_per_block, int rows);
 int sdt_plan_get_tiles(void* plan, int* waves_per_block, int* rows);
@@ -205,12 +204,23 @@ int sdt_plan_get_tile_order(void* plan, int* order);
  * crosses HBM once per two steps; 1 is the one-step kernel.  Results are
  * identical bit for bit.  A run of an odd number of steps ends with one
  * single step; with hipGraph blocks, two-step launches need an even
- * graph_block (odd blocks fall back to one step per launch).  The adjoint's
- * trail recomputation always steps one at a time.  In two-step mode
+ * graph_block (odd blocks fall back to one step per launch).  In two-step mode
  * sdt_plan_profile's out_ms[0] is the mean per two-step launch and
  * out_ms[2] is 0 (the kernel writes the receiver samples itself). */
 int sdt_plan_set_steps_per_launch(void* plan, int steps);
 int sdt_plan_get_steps_per_launch(void* plan, int* steps);
+
+/* ELASTIC2 / EM2 regions (no counterpart in the reference): blocks of 32 x 32
+ * cells that take several steps per launch and recompute their halo, the
+ * default.  on = 1 takes a plan back to them after a launch shape was set, 0
+ * runs the step kernels in the plan's launch shape.  sdt_plan_get_regions:
+ * whether the plan runs on regions, the most steps one launch takes and the
+ * number of regions (both optional).  Results do not depend on it.
+ * sdt_plan_get_run_mode: how sdt_plan_run with these arguments advances the
+ * plan: 0 one step per launch, 1 two, 2 several on regions (2.5-D: 0). */
+int sdt_plan_set_regions(void* plan, int on);
+int sdt_plan_get_regions(void* plan, int* on, int* most_steps, int* count);
+int sdt_plan_get_run_mode(void* plan, int nsteps, int graph_block, int* mode);
 
 /* Synchronise the plan's last stream and report instability: *first_step
  * gets the first step at which any shot's field exceeded 1e25 in magnitude

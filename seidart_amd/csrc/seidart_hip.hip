@@ -4155,10 +4155,9 @@ struct Plan {
   int* dit0 = nullptr;         // first step of the current run of two-step launches
   int* drec = nullptr;         // receivers by row of every shot (DShot::rrow, rxid)
   int graph_mode = 0;          // what the cached graph holds (run_mode)
-  // several steps per launch on regions (default_regions), while the launch
-  // shape is the one that the plan picked by its size (run_mode)
-  bool multi = false;
-  int def_spl = 0, def_wb = 0, def_eh = 0, def_order = 0;
+  // several steps per launch on regions (default_regions, run_mode): whether the
+  // plan has their list, and whether it may take them (no launch shape asked for)
+  bool multi = false, regions = true;
   int4* dwmulti = nullptr;     // work list: (shot, x0, z0, model) per region
   int nmulti = 0, tm = 0;      // tm: most steps per launch, the width of the regions' halo
   bool b_holds = false;        // buffer B holds the current state too (ELASTIC2 / EM2)
@@ -4482,10 +4481,6 @@ void default_shape(Plan* p) {
     if (waves2d(p, ew, 16) >= (em ? 12000 : 8000)) p->el2_eh = 16;
   }
   default_regions(p);
-  p->def_spl = p->spl;
-  p->def_wb = p->el2_wb;
-  p->def_eh = p->el2_eh;
-  p->def_order = p->el2_order;
 }
 
 // Work list of the region kernels: the regions of a model row by row, so that
@@ -4894,11 +4889,9 @@ bool use_two(const Plan* p, int n, int graph_block) {
 }
 
 // How a run of n steps goes: 0 one step per launch, 1 two, 2 several on regions
-// (only with the launch shape that the plan picked).
+// (unless a launch shape was asked for).
 int run_mode(const Plan* p, int n, int graph_block) {
-  if (p->multi && p->spl == p->def_spl && p->el2_wb == p->def_wb && p->el2_eh == p->def_eh &&
-      p->el2_order == p->def_order)
-    return 2;
+  if (p->multi && p->regions) return 2;
   return use_two(p, n, graph_block) ? 1 : 0;
 }
 
@@ -5724,8 +5717,12 @@ int sdt_plan_set_tiles(void* plan, int waves_per_block, int rows) {
   if (waves_per_block != 1 && waves_per_block != 2 && waves_per_block != 4)
     return fail(SDT_EINVAL, "waves_per_block must be 1, 2 or 4");
   if (rows < 1 || rows > 256) return fail(SDT_EINVAL, "rows must be in [1, 256]");
-  if (waves_per_block == p->el2_wb && rows == p->el2_eh) return SDT_OK;
-  return retile(p, waves_per_block, rows, p->el2_order);
+  if (waves_per_block != p->el2_wb || rows != p->el2_eh) {
+    const int rc = retile(p, waves_per_block, rows, p->el2_order);
+    if (rc) return rc;
+  }
+  p->regions = false;
+  return SDT_OK;
 }
 
 int sdt_plan_set_tile_order(void* plan, int order) {
@@ -5733,8 +5730,12 @@ int sdt_plan_set_tile_order(void* plan, int order) {
   if (!p) return fail(SDT_EINVAL, "plan is null");
   if (!pingpong(p->kind)) return fail(SDT_EINVAL, "tile orders apply to ELASTIC2 and EM2 plans");
   if (order != 0 && order != 1) return fail(SDT_EINVAL, "tile order must be 0 or 1");
-  if (order == p->el2_order) return SDT_OK;
-  return retile(p, p->el2_wb, p->el2_eh, order);
+  if (order != p->el2_order) {
+    const int rc = retile(p, p->el2_wb, p->el2_eh, order);
+    if (rc) return rc;
+  }
+  p->regions = false;
+  return SDT_OK;
 }
 
 int sdt_plan_get_tile_order(void* plan, int* order) {
@@ -5751,6 +5752,33 @@ int sdt_plan_set_steps_per_launch(void* plan, int steps) {
   if (steps == 2 && p->kind != SDT_ELASTIC2 && p->kind != SDT_EM2)
     return fail(SDT_EINVAL, "two steps per launch apply to ELASTIC2 and EM2 plans");
   p->spl = steps;
+  p->regions = false;
+  return SDT_OK;
+}
+
+int sdt_plan_set_regions(void* plan, int on) {
+  Plan* p = static_cast<Plan*>(plan);
+  if (!p) return fail(SDT_EINVAL, "plan is null");
+  if (!pingpong(p->kind)) return fail(SDT_EINVAL, "regions apply to ELASTIC2 and EM2 plans");
+  if (on != 0 && on != 1) return fail(SDT_EINVAL, "on must be 0 or 1");
+  p->regions = on == 1;
+  return SDT_OK;
+}
+
+int sdt_plan_get_regions(void* plan, int* on, int* most_steps, int* count) {
+  Plan* p = static_cast<Plan*>(plan);
+  if (!p || !on) return fail(SDT_EINVAL, "null argument");
+  *on = p->multi && p->regions;
+  if (most_steps) *most_steps = p->tm;
+  if (count) *count = p->nmulti;
+  return SDT_OK;
+}
+
+int sdt_plan_get_run_mode(void* plan, int nsteps, int graph_block, int* mode) {
+  Plan* p = static_cast<Plan*>(plan);
+  if (!p || !mode) return fail(SDT_EINVAL, "null argument");
+  if (nsteps < 1) return fail(SDT_EINVAL, "nsteps must be positive");
+  *mode = run_mode(p, nsteps, graph_block);
   return SDT_OK;
 }
 

@@ -233,9 +233,9 @@ class Simulation:
     @property
     def steps_per_launch(self) -> int:
         """Time steps one launch of the ELASTIC2 / EM2 step kernel advances
-        (2 by default, 1 for small ELASTIC2 plans; ``autotune`` times both);
-        while the whole launch shape is the plan's own, ``run`` takes regions,
-        up to 8 steps per launch.  Results do not depend on it."""
+        (2 by default, 1 for small ELASTIC2 plans; ``autotune`` times both)
+        where the plan does not run on ``regions``.  Setting it, the tiles or
+        their order leaves the regions.  Results do not depend on it."""
         v = C.c_int()
         _hip.check(_hip.lib().sdt_plan_get_steps_per_launch(self._plan, C.byref(v)))
         return v.value
@@ -243,6 +243,30 @@ class Simulation:
     @steps_per_launch.setter
     def steps_per_launch(self, steps: int):
         _hip.check(_hip.lib().sdt_plan_set_steps_per_launch(self._plan, int(steps)))
+
+    @property
+    def regions(self) -> bool:
+        """Whether ``run`` takes regions, up to 8 steps per launch (the default
+        of ELASTIC2 and EM2 until a launch shape is set)."""
+        return self.region_info()[0]
+
+    @regions.setter
+    def regions(self, on: bool):
+        _hip.check(_hip.lib().sdt_plan_set_regions(self._plan, int(bool(on))))
+
+    def region_info(self):
+        """(whether the plan runs on regions, most steps per launch on them,
+        their number)."""
+        v = [C.c_int() for _ in range(3)]
+        _hip.check(_hip.lib().sdt_plan_get_regions(self._plan, *(C.byref(x) for x in v)))
+        return bool(v[0].value), v[1].value, v[2].value
+
+    def run_mode(self, nsteps: int, graph_block: int = 0) -> int:
+        """How ``run(nsteps, graph_block)`` advances the plan: 0 one step per
+        launch, 1 two, 2 several on regions."""
+        v = C.c_int()
+        _hip.check(_hip.lib().sdt_plan_get_run_mode(self._plan, int(nsteps), int(graph_block), C.byref(v)))
+        return v.value
 
     # ------------------------------------------------------------------
     TILE_CANDIDATES = tuple((wb, rows) for wb in (4, 2, 1) for rows in (1, 2, 4, 8, 16, 32, 64))
@@ -275,11 +299,14 @@ class Simulation:
 
     def use(self, key):
         """Apply an ``autotune`` key (steps per launch, waves per block,
-        rows, tile order)."""
+        rows, tile order); the key of the shape that the plan started with
+        stands for regions."""
         spl, wb, rows, order = key
         self.steps_per_launch = spl
         self.tile_order = order
-        return self.set_tiles(wb, rows)
+        self.set_tiles(wb, rows)
+        self.regions = tuple(key) == self._own_shape
+        return self
 
     def autotune(self, steps: int = 8, candidates=None):
         """Pick the tile shape of the single-pass step kernel (ELASTIC2, EM2),

@@ -1,0 +1,77 @@
+"""Which kernels a run takes (sdt_plan_get_run_mode: 0 one step per launch, 1
+two, 2 regions), and that each of them is the one that a caller asked for."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import tiny_problem
+
+pytestmark = pytest.mark.gpu
+
+
+def _problem(kind, seed, nt, **kw):
+    p = tiny_problem(kind, seed=seed, nt=nt, nrec=9, **kw)
+    for sh in p.shots:  # the corners and the source cell too
+        i, _, k = sh.src
+        sh.rec = np.concatenate([sh.rec, np.array([[0, 0, 0], [p.nx - 1, 0, p.nz - 1], [i, 0, k]], dtype=np.int32)])
+    return p
+
+
+def _same(a, b):
+    torch.cuda.synchronize()
+    for (_, _, x), (_, _, y) in zip(a.shots, b.shots):
+        assert torch.equal(x["state"], y["state"])
+        assert torch.equal(x["trace"], y["trace"])
+
+
+@pytest.mark.parametrize("kind", ["elastic2", "em2"])
+def test_a_launch_shape_that_is_set_runs(kind):
+    """Also one that the plan had already: every setter leaves the regions."""
+    from seidart_amd.solver import Simulation
+    s = Simulation(_problem(kind, 500, 60, nx=70, nz=50, npml=5), precision="fp32")
+    own = (s.steps_per_launch, *s.tiles(), s.tile_order)
+    assert s.regions and s.run_mode(60) == 2 and s.run_mode(60, 20) == 2
+    for set_own in (lambda: setattr(s, "steps_per_launch", own[0]), lambda: s.set_tiles(*own[1:3]),
+                    lambda: setattr(s, "tile_order", own[3])):
+        set_own()
+        assert not s.regions and s.run_mode(60) == own[0] - 1
+        s.use(own)
+        assert s.regions and s.run_mode(60) == 2
+    s.steps_per_launch = 1
+    assert s.run_mode(60) == 0
+    s.steps_per_launch = 2
+    assert (s.run_mode(60), s.run_mode(60, 20), s.run_mode(60, 15), s.run_mode(1)) == (1, 1, 0, 0)
+    s.regions = True
+    assert s.run_mode(60) == 2
+    s.regions = False
+    assert s.run_mode(60) == 1
+    s.close()
+
+
+@pytest.mark.parametrize("kind", ["elastic2", "em2"])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("tiles", [None, (1, 2), (4, 8)])
+def test_two_step_kernel_over_segments(kind, precision, tiles):
+    """The two-step kernel over odd segments, odd and even graph blocks, from
+    odd steps and after switches, against the one-step kernel."""
+    from seidart_amd.solver import Simulation
+    p = _problem(kind, 510, 64, nx=150, nz=75, npml=6, nshots=2)
+    a, b = Simulation(p, precision=precision), Simulation(p, precision=precision)
+    a.use((1, 4, 32, 0))
+    b.steps_per_launch = 2
+    if tiles:
+        b.set_tiles(*tiles)
+    for n, gb, mode in ((1, 0, 0), (3, 0, 1), (6, 4, 1), (5, 5, 0), (9, 2, 1), (2, 2, 1), (11, 11, 0), (8, 8, 1)):
+        assert b.run_mode(n, gb) == mode and a.run_mode(n, gb) == 0
+        a.run(n)
+        b.run(n, graph_block=gb)
+        _same(a, b)
+    b.regions = True   # regions and back
+    a.run(7)
+    b.run(7)
+    b.regions = False
+    a.run(12)
+    b.run(12, graph_block=4)
+    _same(a, b)
+    a.close()
+    b.close()
