@@ -4504,16 +4504,21 @@ std::vector<int4> multi_work(const Plan* p, int tm) {
   return w;
 }
 
-// Steps of one run or graph block of n steps on regions: at most p->tm per
-// launch, in launches of nearly equal length, an even number of them if
-// `even` (a graph block must leave the state in the buffer it started from).
-// Returns the number of launches.
+// Launches of one run or graph block of n steps on regions: at most tm steps
+// each, an even number of them if `even` (a graph block must leave the state in
+// the buffer it started from).
+int region_launches(int n, int tm, bool even) {
+  const int L = (n + tm - 1) / tm;
+  return even ? L + (L & 1) : L;
+}
+
+// Steps of one run or graph block on regions, in launches of nearly equal
+// length.  Returns the number of launches.
 template <typename T, bool TRAIL = false>
 int launch_multi(Plan* p, hipStream_t st, int n, bool even) {
   const int tm = TRAIL ? p->tr_tm : p->tm, nw = TRAIL ? p->ntrwork : p->nmulti;
   const int4* w = TRAIL ? p->dtrwork : p->dwmulti;
-  int L = (n + tm - 1) / tm;
-  if (even) L += L & 1;
+  const int L = region_launches(n, tm, even);
   const dim3 g((nw + 7) / 8 * 8), b(RM * RM);
   for (int l = 0; l < L; ++l) {
     const int r = (int)((long long)n * l / L), k = (int)((long long)n * (l + 1) / L) - r;
@@ -4888,10 +4893,39 @@ bool use_two(const Plan* p, int n, int graph_block) {
   return p->spl == 2 && n >= 2 && (graph_block <= 1 || n < graph_block || graph_block % 2 == 0);
 }
 
+// Whether runs of n steps are faster on regions than with the walking kernels.
+// A region loads its whole halo however few steps it takes, and an odd number
+// of launches ends in buffer B, from where the state is copied back (a run of
+// one step on the walkers: every second time).  Small plans wait for launches
+// most of the time and gain from two steps on (us per step, walkers then
+// regions: elastic FP64 127x103 runs of 1 / 2 / 3 steps 10.6 / 8.1 / 8.4, 13.2 / 7.1 /
+// 5.2; 1064x808 49 / 42 / 36, 62 / 34 / 25; EM FP32 21 / 15.4 / 10.4, 29 / 15.3 /
+// 10.7; graph blocks of 2 / 3 / 4 steps 10.8 / 14.6 / 9.3, 16.2 / 11.4 / 9.0).  Plans
+// of many regions (6 and 36 shots of 1064x808) compare what both ways cost in
+// units of one pair of steps on the walkers, fitted to runs and blocks of 1 to 20
+// steps: a launch of k steps on regions a + b k, the copy c, a single step s.  36
+// elastic FP64 shots: runs of 1 / 2 / 4 / 5 / 6 / 8 / 12 steps 1212 / 809 / 538 / 726 / 628 /
+// 537 / 538, on regions 2140 / 1151 / 661 / 564 / 644 / 526 / 571.
+bool regions_pay(const Plan* p, int n, int graph_block) {
+  const bool blocks = graph_block > 1 && n >= graph_block;
+  const int k = blocks ? graph_block : n;
+  if (p->nmulti <= 4096) return k >= (blocks ? 3 : 2);
+  // a up to 32768 regions, a beyond, b, c, s: elastic FP64, FP32, EM FP64, FP32
+  static const double cost[4][5] = {{1.15, 1.32, 0.155, 0.50, 0.85}, {0.90, 1.22, 0.09, 0.65, 0.85},
+                                    {1.28, 1.46, 0.065, 0.67, 0.96}, {1.20, 1.38, 0.11, 0.85, 0.89}};
+  const double* t = cost[(p->kind == SDT_EM2 ? 2 : 0) + (p->prec == SDT_FP32 ? 1 : 0)];
+  const double a = t[p->nmulti > 32768], b = t[2], c = blocks ? 0 : t[3], s = t[4];
+  const int L = region_launches(k, p->tm, blocks);
+  const bool two = use_two(p, n, graph_block);
+  const int W = two ? k / 2 + (k & 1) : k;
+  const double walk = two ? k / 2 + (k & 1) * s + (W & 1) * c : k * s + (W & 1) * c / 2;
+  return L * a + k * b + (L & 1) * c < walk;
+}
+
 // How a run of n steps goes: 0 one step per launch, 1 two, 2 several on regions
 // (unless a launch shape was asked for).
 int run_mode(const Plan* p, int n, int graph_block) {
-  if (p->multi && p->regions) return 2;
+  if (p->multi && p->regions && regions_pay(p, n, graph_block)) return 2;
   return use_two(p, n, graph_block) ? 1 : 0;
 }
 

@@ -75,3 +75,46 @@ def test_two_step_kernel_over_segments(kind, precision, tiles):
     _same(a, b)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("kind", ["elastic2", "em2"])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_short_runs_take_the_walking_kernels(kind, precision):
+    """A run or graph block of too few steps for a region's halo goes to the
+    walkers (one step: every plan), longer ones to regions, with the same bits
+    whatever the sequence."""
+    from seidart_amd.solver import Simulation
+    p = _problem(kind, 520, 46, nx=90, nz=60, npml=6)
+    a, b = Simulation(p, precision=precision), Simulation(p, precision=precision)
+    a.use((1, 4, 32, 0))
+    assert [b.run_mode(n) for n in (1, 2, 3, 50)] == [0, 2, 2, 2]
+    assert b.run_mode(10, 2) != 2 and b.run_mode(12, 3) == b.run_mode(50, 50) == 2
+    for n, gb in ((1, 0), (1, 0), (2, 0), (1, 0), (4, 2), (5, 0), (1, 0), (1, 1), (9, 3), (1, 0), (6, 2), (13, 13), (1, 0)):
+        a.run(n)
+        b.run(n, graph_block=gb)
+        _same(a, b)
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("kind", ["elastic2", "em2"])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_short_runs_of_many_regions(kind, precision):
+    """More than 4096 regions: pairs of steps on the two-step kernel, the plan
+    path and the allocation-free one."""
+    from seidart_amd.solver import Simulation
+    p = _problem(kind, 530, 30, nx=400, nz=300, npml=6, nshots=34)
+    p.cpml_split = kind == "elastic2"
+    a, b, c = (Simulation(p, precision=precision) for _ in range(3))
+    assert b.region_info()[2] > 4096
+    a.use((1, 4, 32, 0))
+    assert [b.run_mode(n) for n in (1, 2, 5, 50)] == [0, 1, 2, 2]
+    assert b.run_mode(4, 4) == 1 and b.run_mode(50, 10) == 2
+    for n, gb in ((2, 0), (1, 0), (2, 0), (4, 4), (5, 0), (2, 0), (1, 0), (8, 2), (5, 0)):
+        a.run(n)
+        b.run(n, graph_block=gb)
+        c.run_noalloc(n)
+        _same(a, b)
+        _same(a, c)
+    for s in (a, b, c):
+        s.close()
