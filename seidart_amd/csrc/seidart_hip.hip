@@ -1123,29 +1123,37 @@ k_el2_step2(const DModel* __restrict__ models, const DShot* __restrict__ shots,
 // so the caller always finds the state in field[] / psi (A); B keeps an
 // identical copy, which the next (odd) step reads.  With to_b the copy runs
 // the other way (a run of two-step launches that ends in A before an odd
-// step).
+// step).  blockIdx.z: the field, or psi after the last.  Every short run with an
+// odd number of launches waits for it: 16 bytes per lane where the two arrays
+// are aligned alike (us, element by element with a division per element, then
+// so: 36 shots of 1064x808 elastic FP32 475, 259, FP64 541, 496, where it reaches
+// 5 TB/s; 32 shots EM FP32 257, 139; 6 shots 33, 19).
 template <typename T>
-__global__ void k_copy_back(const DShot* __restrict__ shots, int nfield, const long* __restrict__ nel,
-                            const long* __restrict__ npsi, int to_b) {
-  const int s = blockIdx.y;
+__global__ void __launch_bounds__(256)
+k_copy_back(const DShot* __restrict__ shots, int nfield, const long* __restrict__ nel,
+            const long* __restrict__ npsi, int to_b) {
+  using V = __attribute__((ext_vector_type(4))) uint32_t;
+  constexpr int E = 16 / sizeof(T);
+  const int s = blockIdx.y, f = blockIdx.z;
   const DShot& S = shots[s];
-  const long n = nel[s], np = npsi[s];
-  const long tot = nfield * n + np;
-  for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < tot; q += (long)gridDim.x * blockDim.x) {
-    if (q < nfield * n) {
-      const int f = (int)(q / n);
-      const long e = q - (long)f * n;
-      if (to_b)
-        mp<T>(S.g[f])[e] = cp<T>(S.f[f])[e];
-      else
-        mp<T>(S.f[f])[e] = cp<T>(S.g[f])[e];
-    } else {
-      const long e = q - nfield * n;
-      if (to_b)
-        mp<T>(S.psi2)[e] = cp<T>(S.psi)[e];
-      else
-        mp<T>(S.psi)[e] = cp<T>(S.psi2)[e];
-    }
+  const long n = f < nfield ? nel[s] : npsi[s];
+  void* const a = f < nfield ? S.f[f] : S.psi;
+  void* const b = f < nfield ? S.g[f] : S.psi2;
+  void* const src = to_b ? a : b;
+  void* const dst = to_b ? b : a;
+  // elements before the first 16-byte boundary, then whole vectors
+  long head = n, nv = 0;
+  if ((((uintptr_t)src ^ (uintptr_t)dst) & 15) == 0) {
+    head = min(n, (long)((16 - ((uintptr_t)src & 15)) & 15) / (long)sizeof(T));
+    nv = (n - head) / E;
+  }
+  const long t0 = (long)blockIdx.x * blockDim.x + threadIdx.x, step = (long)gridDim.x * blockDim.x;
+  const auto sv = (gcptr<V>)((const T*)src + head);
+  const auto dv = (gptr<V>)((T*)dst + head);
+  for (long q = t0; q < nv; q += step) dv[q] = sv[q];
+  for (long q = t0; q < n - nv * E; q += step) {
+    const long e = q < head ? q : q + nv * E;
+    mp<T>(dst)[e] = cp<T>(src)[e];
   }
 }
 
@@ -4194,6 +4202,7 @@ struct Plan {
   unsigned gmask = 0xfffu;       // gradient slots to accumulate
   int adj_flags = 0;
   int maxnx = 0, maxnz = 0;
+  long long maxel = 0;           // elements of the largest field or psi
 };
 
 int kind_fields(int kind) {
@@ -4820,8 +4829,11 @@ void launch_one(Plan* p, hipStream_t st, int rel, int which) {
 
 template <typename T>
 void launch_copy_back(Plan* p, hipStream_t st, int to_b = 0) {
-  hipLaunchKernelGGL(k_copy_back<T>, dim3(1024, p->nshots), dim3(256), 0, st, p->dshots,
-                     kind_fields(p->kind), p->dnel, p->dnpsi, to_b);
+  // four vectors per thread of the largest array
+  const int nf = kind_fields(p->kind);
+  const int blocks = (int)std::min<long long>(512, p->maxel * (long long)sizeof(T) / (16 * 256 * 4) + 1);
+  hipLaunchKernelGGL(k_copy_back<T>, dim3(blocks, p->nshots, nf + 1), dim3(256), 0, st, p->dshots, nf, p->dnel,
+                     p->dnpsi, to_b);
 }
 
 template <typename T>
@@ -4904,15 +4916,15 @@ bool use_two(const Plan* p, int n, int graph_block) {
 // of many regions (6 and 36 shots of 1064x808) compare what both ways cost in
 // units of one pair of steps on the walkers, fitted to runs and blocks of 1 to 20
 // steps: a launch of k steps on regions a + b k, the copy c, a single step s.  36
-// elastic FP64 shots: runs of 1 / 2 / 4 / 5 / 6 / 8 / 12 steps 1212 / 809 / 538 / 726 / 628 /
-// 537 / 538, on regions 2140 / 1151 / 661 / 564 / 644 / 526 / 571.
+// elastic FP64 shots: runs of 1 / 2 / 4 / 5 / 6 / 8 / 12 steps 1190 / 786 / 538 / 717 / 620 /
+// 537 / 538, on regions 2095 / 1130 / 650 / 555 / 644 / 526 / 567.
 bool regions_pay(const Plan* p, int n, int graph_block) {
   const bool blocks = graph_block > 1 && n >= graph_block;
   const int k = blocks ? graph_block : n;
   if (p->nmulti <= 4096) return k >= (blocks ? 3 : 2);
   // a up to 32768 regions, a beyond, b, c, s: elastic FP64, FP32, EM FP64, FP32
-  static const double cost[4][5] = {{1.15, 1.32, 0.155, 0.50, 0.85}, {0.90, 1.22, 0.09, 0.65, 0.85},
-                                    {1.28, 1.46, 0.065, 0.67, 0.96}, {1.20, 1.38, 0.11, 0.85, 0.89}};
+  static const double cost[4][5] = {{1.15, 1.32, 0.155, 0.42, 0.85}, {0.90, 1.22, 0.09, 0.38, 0.83},
+                                    {1.28, 1.46, 0.065, 0.55, 0.96}, {1.20, 1.38, 0.11, 0.48, 0.89}};
   const double* t = cost[(p->kind == SDT_EM2 ? 2 : 0) + (p->prec == SDT_FP32 ? 1 : 0)];
   const double a = t[p->nmulti > 32768], b = t[2], c = blocks ? 0 : t[3], s = t[4];
   const int L = region_launches(k, p->tm, blocks);
@@ -5299,6 +5311,7 @@ int stage_host(Plan* p, int kind, int prec, const sdt_model* models, int nmodels
     S.nel[s] = (long)M.nx * M.ny * M.nz;
     S.npsi[s] = (long)psi_elems(kind | (split ? SDT_SPLIT_CPML : 0), M.nx, M.ny, M.nz, M.lx,
                                 kind_3d(kind) ? M.ly : 0, M.lz);
+    p->maxel = std::max<long long>(p->maxel, std::max(S.nel[s], S.npsi[s]));
   }
   return SDT_OK;
 }
