@@ -4436,9 +4436,11 @@ void default_regions(Plan* p) {
   p->multi = true;
 }
 
-// Default launch shape of a 2-D plan: steps per launch, wavefronts per block,
-// rows per tile and tile order, from how many wavefronts the plan has and
-// whether its ping-pong fields fit the 256 MB last-level cache.  Fitted to the
+// Default launch shape of a 2-D plan's walking kernels, which take the runs that
+// are too short for regions (regions_pay) and those of a plan taken off them:
+// steps per launch, wavefronts per block, rows per tile and tile order, from how
+// many wavefronts the plan has and whether its ping-pong fields fit the 256 MB
+// last-level cache.  Fitted to the
 // times of every shape on 30 plans (6 k to 27 M cells per step, 1 to 36 shots)
 // per kind and precision: within 2 to 4 % of the fastest shape in the mean.
 // Against tiles of 32 .. 2 rows for 1024 blocks of four wavefronts, one step
@@ -4452,7 +4454,10 @@ void default_regions(Plan* p) {
 //    the one-step kernel's one-row tiles win (296^2 FP64 9.0 against 12.4).
 //  - Rows: the tallest of 8, 4, 2 (EM also 1) that still give 2000 (FP64) or
 //    4000 (elastic FP32; EM 2800) wavefronts; 16 and 32 only with many of them
-//    (1064x808 x 6 shots EM FP64 46.6 with 8, 51.4 with 16).
+//    (1064x808 x 6 shots EM FP64 46.6 with 8, 51.4 with 16).  EM plans of up to
+//    4096 regions, whose walking runs are of one step or blocks of two, halve 8
+//    rows (FP64 also 4): the one-step kernel's walk is the longer one (5 shots of
+//    670x330 FP64 24.3 us with 8 rows, 18.3 with 4; of 438x624 FP32 20.0, 18.1).
 //  - Column strips per XCD (order 1) while the fields fit the cache, tiles
 //    dealt in turn beyond (1064x808 x 12 shots elastic FP64 157 against 178).
 //  - Wide blocks waste wavefronts at the edge of a narrow grid and take its
@@ -4490,6 +4495,7 @@ void default_shape(Plan* p) {
     if (waves2d(p, ew, 16) >= (em ? 12000 : 8000)) p->el2_eh = 16;
   }
   default_regions(p);
+  if (em && p->el2_eh <= 8 && p->el2_eh >= (f64 ? 4 : 8) && regions2d(p, p->tm) <= 4096) p->el2_eh /= 2;
 }
 
 // Work list of the region kernels: the regions of a model row by row, so that
@@ -4916,8 +4922,9 @@ bool use_two(const Plan* p, int n, int graph_block) {
 // of many regions (6 and 36 shots of 1064x808) compare what both ways cost in
 // units of one pair of steps on the walkers, fitted to runs and blocks of 1 to 20
 // steps: a launch of k steps on regions a + b k, the copy c, a single step s.  36
-// elastic FP64 shots: runs of 1 / 2 / 4 / 5 / 6 / 8 / 12 steps 1190 / 786 / 538 / 717 / 620 /
-// 537 / 538, on regions 2095 / 1130 / 650 / 555 / 644 / 526 / 567.
+// elastic FP64 shots: runs of 1 / 2 / 4 / 5 / 6 / 8 / 12 steps 1212 / 809 / 538 / 726 / 628 /
+// 537 / 538, on regions 2140 / 1151 / 661 / 564 / 644 / 526 / 571 (with copies of 541 us,
+// now 496).
 bool regions_pay(const Plan* p, int n, int graph_block) {
   const bool blocks = graph_block > 1 && n >= graph_block;
   const int k = blocks ? graph_block : n;
