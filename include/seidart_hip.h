@@ -254,7 +254,9 @@ long long sdt_noalloc_scratch_bytes(void);
  * it0+nsteps-1 like sdt_plan_run (no graph), bracketing every kernel with
  * HIP events on `stream`, and return the mean duration in ms of
  * out_ms[0] the first field update (stress / H), out_ms[1] the second
- * (velocity / E) and out_ms[2] the receiver gather. */
+ * (velocity / E) and out_ms[2] the receiver gather.  On regions out_ms[0] is
+ * the mean per launch of as few launches as sdt_plan_get_regions' most steps
+ * allow, and the others are 0. */
 int sdt_plan_profile(void* plan, int it0, int nsteps, void* stream, double* out_ms);
 
 /* Measurement hook (no counterpart in the reference): enqueue on `stream` a

@@ -4527,28 +4527,34 @@ int region_launches(int n, int tm, bool even) {
   return even ? L + (L & 1) : L;
 }
 
+// One launch of k steps from step base + r on regions, reading state buffer par.
+template <typename T, bool TRAIL = false>
+void launch_region(Plan* p, hipStream_t st, int r, int k, int par) {
+  const int tm = TRAIL ? p->tr_tm : p->tm, nw = TRAIL ? p->ntrwork : p->nmulti;
+  const int4* w = TRAIL ? p->dtrwork : p->dwmulti;
+  const dim3 g((nw + 7) / 8 * 8), b(RM * RM);
+  if (p->kind == SDT_EM2 && !TRAIL && sizeof(T) == 4 && nw > 512)  // (see EmRegionLds)
+    hipLaunchKernelGGL((k_em2_multi<float, false, 2>), g, dim3(RM * RM / 2), 0, st, p->dmodels, p->dshots, w, nw,
+                       p->dbase, r, k, tm, par, p->dadj, p->dtsel_trail);
+  else if (p->kind == SDT_EM2)
+    hipLaunchKernelGGL((k_em2_multi<T, TRAIL, 1>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k, tm,
+                       par, p->dadj, p->dtsel_trail);
+  else if (p->split)
+    hipLaunchKernelGGL((k_el2_multi<T, true, TRAIL>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k,
+                       tm, par, p->dadj, p->dtsel_trail);
+  else
+    hipLaunchKernelGGL((k_el2_multi<T, false, TRAIL>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k,
+                       tm, par, p->dadj, p->dtsel_trail);
+}
+
 // Steps of one run or graph block on regions, in launches of nearly equal
 // length.  Returns the number of launches.
 template <typename T, bool TRAIL = false>
 int launch_multi(Plan* p, hipStream_t st, int n, bool even) {
-  const int tm = TRAIL ? p->tr_tm : p->tm, nw = TRAIL ? p->ntrwork : p->nmulti;
-  const int4* w = TRAIL ? p->dtrwork : p->dwmulti;
-  const int L = region_launches(n, tm, even);
-  const dim3 g((nw + 7) / 8 * 8), b(RM * RM);
+  const int L = region_launches(n, TRAIL ? p->tr_tm : p->tm, even);
   for (int l = 0; l < L; ++l) {
-    const int r = (int)((long long)n * l / L), k = (int)((long long)n * (l + 1) / L) - r;
-    if (p->kind == SDT_EM2 && !TRAIL && sizeof(T) == 4 && nw > 512)  // (see EmRegionLds)
-      hipLaunchKernelGGL((k_em2_multi<float, false, 2>), g, dim3(RM * RM / 2), 0, st, p->dmodels, p->dshots, w, nw,
-                         p->dbase, r, k, tm, l & 1, p->dadj, p->dtsel_trail);
-    else if (p->kind == SDT_EM2)
-      hipLaunchKernelGGL((k_em2_multi<T, TRAIL, 1>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k, tm,
-                         l & 1, p->dadj, p->dtsel_trail);
-    else if (p->split)
-      hipLaunchKernelGGL((k_el2_multi<T, true, TRAIL>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k,
-                         tm, l & 1, p->dadj, p->dtsel_trail);
-    else
-      hipLaunchKernelGGL((k_el2_multi<T, false, TRAIL>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k,
-                         tm, l & 1, p->dadj, p->dtsel_trail);
+    const int r = (int)((long long)n * l / L);
+    launch_region<T, TRAIL>(p, st, r, (int)((long long)n * (l + 1) / L) - r, l & 1);
   }
   return L;
 }
@@ -5551,21 +5557,25 @@ int sdt_plan_profile(void* plan, int it0, int nsteps, void* stream, double* out_
   hipEvent_t ev[4];
   for (int q = 0; q < 4; ++q) HIP_TRY(hipEventCreate(&ev[q]));
   double acc[3] = {0, 0, 0};
-  const bool two = use_two(p, nsteps, 0);
-  start_of_run(p, st, it0, two);
+  const int mode = run_mode(p, nsteps, 0);
+  start_of_run(p, st, it0, mode != 0);
   hipLaunchKernelGGL(k_set_int2, dim3(1), dim3(1), 0, st, p->dbase, it0, p->dit0, it0);
   int rc = SDT_OK;
-  if (two) {
-    // two-step launches: slot 0 is the mean per launch (two steps); the
-    // single step that ends an odd run is not timed
-    int npair = 0;
-    for (int s = 0; s < nsteps && rc == SDT_OK; s += 2) {
-      const bool single = s + 1 == nsteps;
+  if (mode != 0) {
+    // several steps per launch: slot 0 is the mean per launch; the single
+    // step that ends an odd run of pairs is not timed
+    const int L = mode == 2 ? region_launches(nsteps, p->tm, false) : nsteps / 2 + (nsteps & 1);
+    int timed = 0;
+    for (int l = 0; l < L && rc == SDT_OK; ++l) {
+      const bool single = mode == 1 && 2 * l + 1 == nsteps;
+      const int r = (int)((long long)nsteps * l / L), k = (int)((long long)nsteps * (l + 1) / L) - r;
       if (hipEventRecord(ev[0], st) != hipSuccess) { rc = fail(SDT_EDEVICE, "hipEventRecord"); break; }
-      if (p->prec == SDT_FP64)
-        launch_two<double>(p, st, s, single);
+      if (mode == 2)
+        p->prec == SDT_FP64 ? launch_region<double>(p, st, r, k, l & 1) : launch_region<float>(p, st, r, k, l & 1);
+      else if (p->prec == SDT_FP64)
+        launch_two<double>(p, st, 2 * l, single);
       else
-        launch_two<float>(p, st, s, single);
+        launch_two<float>(p, st, 2 * l, single);
       if (hipEventRecord(ev[1], st) != hipSuccess || hipEventSynchronize(ev[1]) != hipSuccess) {
         rc = fail(SDT_EDEVICE, "event sync failed");
         break;
@@ -5574,12 +5584,12 @@ int sdt_plan_profile(void* plan, int it0, int nsteps, void* stream, double* out_
       float ms = 0.f;
       if (hipEventElapsedTime(&ms, ev[0], ev[1]) != hipSuccess) { rc = fail(SDT_EDEVICE, "elapsed"); break; }
       acc[0] += ms;
-      ++npair;
+      ++timed;
     }
-    if (rc == SDT_OK) end_of_run(p, st, it0 + nsteps, (nsteps / 2 + (nsteps & 1)) & 1);
+    if (rc == SDT_OK) end_of_run(p, st, it0 + nsteps, L & 1);
     for (int q = 0; q < 4; ++q) (void)hipEventDestroy(ev[q]);
     if (rc) return rc;
-    out_ms[0] = npair ? acc[0] / npair : 0.0;
+    out_ms[0] = timed ? acc[0] / timed : 0.0;
     out_ms[1] = 0.0;
     out_ms[2] = 0.0;
     HIP_TRY(hipGetLastError());

@@ -217,11 +217,11 @@ class Simulation:
     def profile(self, nsteps: int, stream=None):
         """Run the next ``nsteps`` steps with every kernel bracketed by HIP
         events; return mean ms per launch of (first field kernel, second
-        field kernel, receiver gather).  With two steps per launch
-        (``steps_per_launch``) the first is the two-step kernel, per launch,
-        and the gather is 0 (the kernel writes the receiver samples).  These
-        are the kernels of the launch shape also where ``run`` takes regions
-        (several steps per launch, the default of the 2-D kinds)."""
+        field kernel, receiver gather).  With several steps per launch (two,
+        ``steps_per_launch``, or on ``regions``: the ``run_mode`` of
+        ``nsteps``) the first is the kernel per launch, on regions of the
+        fewest launches that ``region_info`` allows, and the gather is 0 (the
+        kernel writes the receiver samples)."""
         if stream is None:
             stream = torch.cuda.current_stream(self.device)
         out = (C.c_double * 3)()

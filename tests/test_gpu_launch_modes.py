@@ -150,3 +150,30 @@ def test_copies_between_the_state_buffers(kind, precision, nx, nz, offset):
         assert offset == 0 or float(st[:offset].min()) == 7.0
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("kind", ["elastic2", "em2"])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_profile_times_the_kernels_that_run_takes(kind, precision):
+    """In each mode: the state that a run of as many steps leaves, and the time
+    of the kernel per launch in the first slot."""
+    from seidart_amd.solver import Simulation
+    p = _problem(kind, 560, 120, nx=300, nz=260, npml=6, nshots=2)
+    a, b = Simulation(p, precision=precision), Simulation(p, precision=precision)
+    a.use((1, 4, 32, 0))
+    most = b.region_info()[1]
+    for setup, n in ((None, 3 * most), (None, 2 * most - 1), (2, 6), (2, 7), (1, 5), (None, 1)):
+        if setup:
+            b.steps_per_launch = setup
+        else:
+            b.regions = True
+        mode = b.run_mode(n)
+        assert mode == (0 if n == 1 else 2 if setup is None else setup - 1)
+        a.run(n)
+        ms = b.profile(n)
+        _same(a, b)
+        assert ms[0] > 0 and ms[1] >= 0 and ms[2] >= 0
+        if mode:
+            assert ms[1] == ms[2] == 0
+    a.close()
+    b.close()
