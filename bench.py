@@ -255,9 +255,10 @@ def config_lines(survey_steps: int = 200, ref_steps: int = 0, only=None):
     steps, gpr 4000, aniso25 3000) in FP32 and FP64, after the hipGraph of
     their block is captured; the two measured lines that are not reference
     configurations (gpr25, gpr_survey) run `survey_steps` steps.  Each line
-    gives Gcell-updates/s, the algorithmic bytes per cell-update, the
-    fraction of the HBM peak and the FP32 trace error against the FP64 run
-    over the same steps.  For profiling runs, `ref_steps` > 0 shortens the
+    gives Gcell-updates/s, the algorithmic bytes per cell-update (what one
+    step per launch must move), their rate, that over the HBM peak (no
+    fraction of it where launches take several steps) and the FP32 trace
+    error against the FP64 run over the same steps.  For profiling runs, `ref_steps` > 0 shortens the
     reference configurations to that many steps and `only` (names) keeps
     only those lines."""
     import torch
@@ -296,7 +297,7 @@ def config_lines(survey_steps: int = 200, ref_steps: int = 0, only=None):
             gcs = cells * K / el / 1e9
             bpc = alg_bytes_per_step([p], size) / cells
             rec[prec] = {"Gcell_updates_s": round(gcs, 3), "alg_B_per_cell_update": round(bpc, 2),
-                         "alg_GBs": round(gcs * bpc, 1), "frac_hbm": round(gcs * bpc / HBM_PEAK_GBS, 4)}
+                         "alg_GBs": round(gcs * bpc, 1), "alg_over_hbm_peak": round(gcs * bpc / HBM_PEAK_GBS, 4)}
         t32, t64 = traces["fp32"], traces["fp64"]
         rec["fp32_trace_rel_l2_vs_fp64"] = float(f"{np.linalg.norm(t32 - t64) / np.linalg.norm(t64):.3e}")
         if p.kind == "elastic25" and K > 1000:
@@ -312,16 +313,17 @@ def config_lines(survey_steps: int = 200, ref_steps: int = 0, only=None):
     return out
 
 
-def measured_traffic(alg_bytes: int):
-    """HBM bytes per launch of the headline kernel measured by rocprofv3 byte
-    counters (profiles/el2_step_batched_layered_fp32_hbm_bytes.md, scaled by
-    the copy calibration there), if that profile was taken on this workload
-    (same algorithmic bytes per launch); else None."""
-    path = os.path.join(ROOT, "profiles", "el2_step_batched_layered_fp32_hbm_bytes.md")
+def measured_traffic(regions: bool, alg_bytes: int):
+    """HBM bytes per launch of the headline kernel (a two-step launch pair, or
+    a launch of several steps on regions) measured by rocprofv3 byte counters
+    and scaled by the copy calibration there, if that profile was taken on
+    this workload (same algorithmic bytes per step); else None."""
+    name = "el2_regions" if regions else "el2_step"
+    path = os.path.join(ROOT, "profiles", name + "_batched_layered_fp32_hbm_bytes.md")
     try:
         kv = dict(line.split(":", 1) for line in open(path) if line.count(":") == 1
-                  and line.split(":")[0] in ("traffic_bytes_per_launch", "alg_bytes_per_launch"))
-        if int(kv["alg_bytes_per_launch"]) == int(alg_bytes):
+                  and line.split(":")[0] in ("traffic_bytes_per_launch", "alg_bytes_per_step"))
+        if int(kv["alg_bytes_per_step"]) == int(alg_bytes):
             return int(kv["traffic_bytes_per_launch"])
     except (OSError, KeyError, ValueError):
         pass
@@ -466,12 +468,15 @@ def main(argv=None):
 
     sim = Simulation(problems, precision="fp32")
     fixed = tuple(int(v) for v in a.tiles.split("x")) if a.tiles else None
+    own_shape = (sim.steps_per_launch, *sim.tiles(), sim.tile_order)  # (stands for regions)
     if fixed:
         sim.set_tiles(*fixed)
         tune = {(sim.steps_per_launch, *fixed, sim.tile_order): float("nan")}
     else:
         tune = sim.autotune(steps=10)   # tile shape of the step kernel (setup, untimed)
     sim_spl, sim_tiles, sim_order = sim.steps_per_launch, sim.tiles(), sim.tile_order
+    # most steps per launch of the timed run on regions, 0 off them
+    on_regions = sim.region_info()[1] if sim.run_mode(K, gb) == 2 else 0
     captured = sim.capture_graph(gb) if gb else False
     sim.run(W, graph_block=gb if W >= gb else 0)
     torch.cuda.synchronize()
@@ -487,29 +492,34 @@ def main(argv=None):
     gpu_ms = ev0.elapsed_time(ev1)
     sim.check()
     value = cells_per_step * K / wall / 1e9
-    # The shape the plan started with runs the region kernel, several steps per
-    # launch: its time per step is the timed run's.  Other shapes: per-kernel
-    # durations (HIP events around each launch, same stream).
-    regions = sim.regions
-    k_ms = (gpu_ms / K, 0.0, 0.0) if regions else sim.profile(PROFILE_STEPS)
+    # per-kernel durations (HIP events around each launch, same stream)
+    regions = sim.run_mode(PROFILE_STEPS) == 2
+    k_ms = sim.profile(PROFILE_STEPS)
     sim.check()
-    # one launch of the step kernel advances `spl` steps (two: the state of the
-    # first stays in registers), so its algorithmic bytes are spl times those of
-    # one step (regions: both per step)
-    spl = 1 if regions else sim.steps_per_launch
-    dom_bytes = spl * algorithmic_bytes(problems, shots, 4)
-    achieved = dom_bytes / (k_ms[0] * 1e-3) / 1e9
-    roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
+    # A launch moves the state in and out and the coefficients in once, however
+    # many steps it takes: that is what it must move.  The rate of the bytes
+    # that one step per launch would move is given beside it; with several
+    # steps per launch it is no share of the HBM peak.
+    spl = sim.steps_per_launch
+    if regions:
+        spl = PROFILE_STEPS / -(-PROFILE_STEPS // sim.region_info()[1])
+    alg = algorithmic_bytes(problems, shots, 4)
+    achieved = alg / (k_ms[0] * 1e-3) / 1e9
+    roofline = {"bound": "latency and issue of a region's steps" if regions else
+                         "hbm and issue" if spl == 2 else "hbm",
+                "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                "traffic": measured_traffic(dom_bytes),
-                "kernel": "k_el2_multi<float>, per step" if regions else
+                "traffic": measured_traffic(regions, alg) if spl > 1 else None,
+                "kernel": "k_el2_multi<float>" if regions else
                           "k_el2_step2<float>" if spl == 2 else "k_el2_step<float>",
-                "kernel_ms": round(k_ms[0], 4), "steps_per_launch": spl,
-                "alg_bytes_per_launch": int(dom_bytes),
-                "alg_bytes_per_cell_update": round(dom_bytes / spl / cells_per_step, 2),
+                "kernel_ms": round(k_ms[0], 4), "steps_per_launch": round(spl, 2),
+                "alg_bytes_per_launch": int(alg),
+                "alg_bytes_per_cell_update": round(alg / cells_per_step, 2),
+                "alg_step_rate_GBs": round(achieved * spl, 1),
                 "gather_ms": round(k_ms[2], 4)}
     if roofline["traffic"]:
         # measured bytes per launch over the launch time, against a plain copy
+        # (the profile's launches: two steps, or five on regions)
         cgbs = copy_rate()
         tgbs = roofline["traffic"] / (k_ms[0] * 1e-3) / 1e9
         roofline.update({"traffic_GBs": round(tgbs, 1), "copy_GBs": round(cgbs, 1),
@@ -641,10 +651,12 @@ def main(argv=None):
                                 if gb else ", direct launches"),
                    "cells_per_step": cells_per_step, "shots": sum(shots),
                    "graph_block": gb if captured else 0,
-                   "tiles": {"chosen": {"steps_per_launch": sim_spl, "waves": sim_tiles[0],
-                                        "rows": sim_tiles[1], "order": sim_order},
+                   "tiles": {"chosen": {"regions": on_regions} if on_regions else
+                             {"steps_per_launch": sim_spl, "waves": sim_tiles[0],
+                              "rows": sim_tiles[1], "order": sim_order},
                              "ms_per_step": {} if fixed else
-                             {f"{n}-step {w}x{r} order {o}": round(v, 4)
+                             {"regions" if (n, w, r, o) == own_shape else
+                              f"{n}-step {w}x{r} order {o}": round(v, 4)
                               for (n, w, r, o), v in tune.items()}}},
         "gpu_ms_events": round(gpu_ms, 3),
         "roofline": roofline,
