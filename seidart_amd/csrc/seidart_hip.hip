@@ -1571,6 +1571,13 @@ using ElAdjOwn = AdjOwn<AR<T, false>, !SPLIT>;
 template <typename T>
 using EmAdjOwn = AdjOwn<AR<T, true>, false>;
 
+// Orders a wavefront's LDS accesses before and after it, lanes among each other
+// (the hardware takes them in order; this keeps the compiler to it).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // The residuals of step t of the receivers on this wavefront's row r of the
 // grid, summed per column: lane l's column is xl + l.  buf: 2 x 64 of the
 // wavefront's own.
@@ -1582,7 +1589,7 @@ __device__ __forceinline__ void adj_residual(const DShot& S, const DAdj& A, int 
   const auto res = cp<T>(A.resid) + (long)t * 2 * S.nrec;
   b0[lane] = 0;
   b1[lane] = 0;
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_fence();
   for (int e = q0 + lane; e < q1; e += 64) {
     const int l = S.rxid[2 * e] - xl, id = S.rxid[2 * e + 1];
     if (l >= 0 && l < 64) {
@@ -1590,7 +1597,7 @@ __device__ __forceinline__ void adj_residual(const DShot& S, const DAdj& A, int 
       atomicAdd(&b1[l], res[S.nrec + id]);
     }
   }
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_fence();
   a0 += b0[lane];
   a1 += b1[lane];
 }
