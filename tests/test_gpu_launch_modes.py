@@ -177,3 +177,23 @@ def test_profile_times_the_kernels_that_run_takes(kind, precision):
             assert ms[1] == ms[2] == 0
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("nx,nz,nshots", [(660, 23, 20), (23, 650, 20), (47, 31, 140)])
+def test_em_regions_of_two_rows_on_thin_grids(nx, nz, nshots):
+    """FP32 EM plans of more than 512 regions (two rows per thread) whose
+    regions overhang a thin grid on both sides, its height odd, against the
+    one-step kernel."""
+    from seidart_amd.solver import Simulation
+    p = _problem("em2", 570 + nx, 40, nx=nx, nz=nz, npml=6, nshots=nshots)
+    a, b = Simulation(p, precision="fp32"), Simulation(p, precision="fp32")
+    on, most, count = b.region_info()
+    assert on and count > 512 and 3 <= most <= 8
+    a.use((1, 4, 32, 0))
+    for n, gb in ((7, 0), (22, 11), (11, 5)):
+        assert b.run_mode(n, gb) == 2
+        a.run(n)
+        b.run(n, graph_block=gb)
+        _same(a, b)
+    a.close()
+    b.close()
