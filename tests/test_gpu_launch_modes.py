@@ -179,7 +179,7 @@ def test_profile_times_the_kernels_that_run_takes(kind, precision):
     b.close()
 
 
-@pytest.mark.parametrize("nx,nz,nshots", [(660, 23, 20), (23, 650, 20), (47, 31, 140)])
+@pytest.mark.parametrize("nx,nz,nshots", [(660, 23, 20), (23, 691, 20), (47, 31, 140)])
 def test_em_regions_of_two_rows_on_thin_grids(nx, nz, nshots):
     """FP32 EM plans of more than 512 regions (two rows per thread) whose
     regions overhang a thin grid on both sides, its height odd, against the
