@@ -284,7 +284,8 @@ def config_lines(survey_steps: int = 200, ref_steps: int = 0, only=None):
         for prec, size in (("fp32", 4), ("fp64", 8)):
             sim = Simulation(p, precision=prec)
             if p.kind in ("elastic2", "em2"):
-                rec.setdefault("tiles", {})[prec] = list(min((r := sim.autotune(steps=10)), key=r.get))
+                best = list(min((r := sim.autotune(steps=10)), key=r.get))
+                rec.setdefault("tiles", {})[prec] = "regions" if sim.regions else best
             sim.capture_graph(50)
             torch.cuda.synchronize()
             t0 = time.perf_counter()

@@ -132,7 +132,8 @@ typedef struct sdt_model {
  *      moment-tensor series of sourcefunction.py:296-372; the reference's
  *      solver that consumes them is not in its sources, so this injection
  *      is this library's definition.  2-D kinds use xx, zz and xz.
- * rec: nrec triples (i, j, k), 0-based padded; trace: nt * ncomp * nrec,
+ * rec: nrec triples (i, j, k), 0-based padded, read when the plan is created
+ *      (do not change them while it lives); trace: nt * ncomp * nrec,
  *      trace[it][c][r] = component c at receiver r after step it, with
  *      ncomp = 2 (ELASTIC2: vx vz, EM2: Ex Ez) or 3 (vx vy vz / Ex Ey Ez).
  */
@@ -244,7 +245,8 @@ int sdt_plan_check(void* plan, int* first_step, int* per_shot);
  * GPU (other threads, other streams) race.  Kernels run on `stream`; the
  * call synchronises it before returning, and reports instability like
  * sdt_plan_check (first_step, per_shot optional).  No hipGraph is used;
- * two steps per launch as in sdt_plan_create's default. */
+ * steps per launch as in sdt_plan_create's default (taller tiles and no regions
+ * where the lists would not fit the array). */
 int sdt_run_noalloc(int kind, int precision, const sdt_model* models, int nmodels,
                     const sdt_shot* shots, int nshots, int nt, int it0, int nsteps, void* stream,
                     int* first_step, int* per_shot);

@@ -16,14 +16,17 @@
 //                 interior carries no C-PML state at all.
 //   traces        [it][comp][rec] per shot
 //
-// Execution: every time step is one field-update launch (2-D elastic, a
-// single pass) or two (stress then velocity, or H then E) over one
-// (shot, tile) work list covering every shot of every model, plus one
-// receiver-gather launch.  Work items are ordered so that all shots of one
-// tile land on the same XCD (blocks are dealt to the 8 XCDs round-robin),
-// so a model's coefficient tile is read from HBM once and served from that
-// XCD's L2 to the other shots.  The adjoint kernels (2-D elastic and EM)
-// sit after the forward kernels of their scheme.
+// Execution: the 2-D kinds take several time steps per launch on regions
+// (k_el2_multi, k_em2_multi), or one or two with the walking kernels (short
+// runs, and launch shapes that a caller sets), and write their receiver
+// samples themselves.  A 2.5-D step is two launches (stress then velocity, or
+// H then E) and a receiver gather.  Every launch goes over one work list that
+// covers the shots of every model.  The walking kernels' items are ordered so
+// that all shots of one tile land on the same XCD (blocks are dealt to the 8
+// XCDs round-robin), which serves the model's coefficients from its L2; the
+// other lists give each XCD a contiguous run of neighbouring items.  The
+// adjoint kernels (2-D elastic and EM) sit after the forward kernels of their
+// scheme.
 
 #include <hip/hip_runtime.h>
 
@@ -1538,9 +1541,11 @@ k_el2_adj_g(const DModel* __restrict__ models, const DShot* __restrict__ shots,
 // LDS.  Blocks recompute the ring, so they are independent (lambda
 // ping-pongs); only owned cells write lambda_t and add to the gradient.  The
 // residual of the step is added to lambda_{t+1} as it is read.
-// All loads of a cell are issued before the first use, and no load follows a
-// store (loads and stores complete in order, so that a walk down the rows
-// waits for the gradient's atomics with every row).  Against wavefronts
+// The interior body (and the whole EM kernel) issues all loads of a cell before
+// the first use, and no load follows a store (loads and stores complete in
+// order, so that a walk down the rows waits for the gradient's atomics with
+// every row).  The elastic slab body still loads memory variables and their
+// adjoints between its phases, after stores.  Against wavefronts
 // walking tiles of 1 to 64 rows (us per step, elastic FP32 with six gradient
 // slots then EM FP64 with four): 120x90 14.7 -> 10.0 and 15.8 -> 5.1, 740x440
 // x 6 shots 73 -> 51 and 90 -> 53, 1064x552 x 16 shots 260 -> 209 and 322 -> 221;
@@ -4360,9 +4365,6 @@ void launch_em2x2(Plan* p, hipStream_t st, int rel) {
   }
 }
 
-// Work list of the ELASTIC2 step kernel for the plan's tile shape: one item
-// (shot, x0, z0) per block of el2_wb adjacent x tiles; the items of one
-// block-tile over all shots of its model share blockIdx % 8 (one XCD's L2).
 // Whether every wavefront of the two-step kernel's block at (x0, z0) takes
 // the interior body (the test of k_el2_step2 for each of its wavefronts).
 bool el2x2_interior(const sdt_model& M, int x0, int z0, int wb, int eh) {
@@ -4386,7 +4388,6 @@ long long waves2d(const Plan* p, int ew, int rows) {
   return n;
 }
 
-// Regions of a 2-D plan whose halo is tm steps wide.
 // Where the regions of one axis of n cells with slabs of l start owning cells,
 // and whether a step reaches one cell each way in them (region_own).
 std::vector<std::pair<int, bool>> region_cuts(const Plan* p, int n, int l, int tm) {
@@ -4398,6 +4399,7 @@ std::vector<std::pair<int, bool>> region_cuts(const Plan* p, int n, int l, int t
   }
   return c;
 }
+// Regions of a 2-D plan whose halo is tm steps wide.
 long long regions2d(const Plan* p, int tm) {
   std::vector<long long> per(p->nmodels);
   for (int m = 0; m < p->nmodels; ++m) {
@@ -4410,7 +4412,7 @@ long long regions2d(const Plan* p, int tm) {
 }
 
 // The most steps per launch of a 2-D plan on regions (k_el2_multi, k_em2_multi),
-// its default at every size.  A region recomputes its halo: with five steps per
+// its default at every size (short runs aside: regions_pay).  A region recomputes its halo: with five steps per
 // launch 47 % of its cells are owned.  Measured (us per step, walking kernels in
 // the shape of default_shape, then regions): elastic FP64 127x103 6.3 -> 2.4, 296^2
 // 8.3 -> 3.0, 12 shots of 1064x808 158 -> 150, 8 of 2088x808 208 -> 196; FP32 1064x808
@@ -4419,10 +4421,13 @@ long long regions2d(const Plan* p, int tm) {
 // -> 4.4, x 32 shots 123 -> 87.
 // Where the regions run all at once (one block of elastic FP64 per CU, else two),
 // the most steps: a launch costs 5 to 7 us beside its steps (127x103 elastic FP64
-// 5.1 / 2.8 / 2.3 us per step with 2 / 4 / 7).  Larger plans: a launch's time is its
-// regions', whatever their steps, so the steps with the fewest regions times
-// launches in a block of 50 steps (an even number of launches): FP32 32 shots of
-// 1064x808 3 / 4 / 5 steps 211 / 188 / 159 (18 / 14 / 10 launches).
+// 5.1 / 2.8 / 2.3 us per step with 2 / 4 / 7).  Larger plans: the steps with the
+// fewest regions times launches in a block of 50 steps (an even number of
+// launches): FP32 32 shots of 1064x808 3 / 4 / 5 steps 211 / 188 / 159 (18 / 14 / 10
+// launches).  That leaves out what the steps of a region cost beside its loads,
+// a tenth of them per step in FP32 and a seventh in elastic FP64 (regions_pay);
+// 9 uneven elastic FP64 shots take 21.1 us per step with 4 steps, 22.7 with the 5
+// that this picks.
 void default_regions(Plan* p) {
   auto cost = [&](int t) {
     const int n = (50 + t - 1) / t;
@@ -4727,10 +4732,10 @@ double shot_bytes(const Plan* p, int s) {
 // 409; 6 shots of 232x96x182 FP32 508 -> 476; 24 shots of 152x62x112 FP64 1156 ->
 // 1064 (groups of 150 MB: 1257; a launch over four of them leaves the device
 // half empty at its end).  100 and 200 MB for blocks of planes: 378 and 357 on
-// the first grid, 600 and 613 on the third.  The elastic passes gain nothing
-// (832x96x432 FP32 1281 whole, 1398 .. 1750 in blocks of 40 .. 140 planes):
-// resident in the cache they run at 41 instead of 35 Gcell-updates/s, less than
-// the launches' tails cost.
+// the first grid, 600 and 613 on the third.  The elastic passes are not run so:
+// before their row groups they lost by it (832x96x432 FP32 1281 whole, 1398 ..
+// 1750 in blocks of 40 .. 140 planes); as they are (1160 whole) it has not been
+// measured.
 constexpr int STEPS25 = 16;
 constexpr double PLANES25_BYTES = 160e6, SHOTS25_BYTES = 200e6;
 
@@ -5167,9 +5172,6 @@ void drop_adjoint_graphs(Plan* p) {
   p->seg_graphs.clear();
 }
 
-// Replay (capturing on first use) the segment graph (kind, key) on st.
-// (Re)build the work list of the two-step ELASTIC2 kernel for the plan's
-// tile shape.
 // Work list of the two-step kernels for the plan's tile shape.  ELASTIC2:
 // interior blocks first (their count in *ni), then the others; EM2: one list.
 std::vector<int4> build_work2(const Plan* p, int* ni) {
@@ -5191,6 +5193,7 @@ void set_work2_grids(Plan* p, int nw, int ni) {
   p->el2x2_grid = std::max(8, std::min(p->nwork2 - ni, SDT_EL2_GRID) / 8 * 8);
 }
 
+// Rebuild that list for the plan's tile shape.
 int upload_work2(Plan* p) {
   int ni = 0;
   const std::vector<int4> work = build_work2(p, &ni);
@@ -5206,6 +5209,7 @@ int upload_work2(Plan* p) {
   return SDT_OK;
 }
 
+// Replay (capturing on first use) the segment graph (kind, key) on st.
 template <typename F>
 int replay_segment(Plan* p, int kind, long long key, hipStream_t st, F&& enqueue) {
   for (auto& x : p->seg_graphs)
