@@ -4539,24 +4539,38 @@ int region_launches(int n, int tm, bool even) {
   return even ? L + (L & 1) : L;
 }
 
-// One launch of k steps from step base + r on regions, reading state buffer par.
+// Items per launch of the kernels that take one item per block: a launch holds
+// fewer than 2^32 threads, which 4.2 M blocks of 1024 reach (2 G cells per step
+// on regions), so longer lists go in several launches.  At this length (0.13 G
+// cells, 3 ms per elastic launch of five steps) a further launch costs nothing
+// against the work.
+constexpr int LAUNCH_ITEMS = 1 << 18;
+template <typename F>
+void in_slices(int n, F&& launch) {
+  for (int o = 0; o < n; o += LAUNCH_ITEMS) launch(o, std::min(LAUNCH_ITEMS, n - o));
+}
+
+// k steps from step base + r on regions, reading state buffer par.
 template <typename T, bool TRAIL = false>
 void launch_region(Plan* p, hipStream_t st, int r, int k, int par) {
-  const int tm = TRAIL ? p->tr_tm : p->tm, nw = TRAIL ? p->ntrwork : p->nmulti;
-  const int4* w = TRAIL ? p->dtrwork : p->dwmulti;
-  const dim3 g((nw + 7) / 8 * 8), b(RM * RM);
-  if (p->kind == SDT_EM2 && !TRAIL && sizeof(T) == 4 && nw > 512)  // (see EmRegionLds)
-    hipLaunchKernelGGL((k_em2_multi<float, false, 2>), g, dim3(RM * RM / 2), 0, st, p->dmodels, p->dshots, w, nw,
-                       p->dbase, r, k, tm, par, p->dadj, p->dtsel_trail);
-  else if (p->kind == SDT_EM2)
-    hipLaunchKernelGGL((k_em2_multi<T, TRAIL, 1>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k, tm,
-                       par, p->dadj, p->dtsel_trail);
-  else if (p->split)
-    hipLaunchKernelGGL((k_el2_multi<T, true, TRAIL>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k,
-                       tm, par, p->dadj, p->dtsel_trail);
-  else
-    hipLaunchKernelGGL((k_el2_multi<T, false, TRAIL>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k,
-                       tm, par, p->dadj, p->dtsel_trail);
+  const int tm = TRAIL ? p->tr_tm : p->tm, items = TRAIL ? p->ntrwork : p->nmulti;
+  const dim3 b(RM * RM);
+  in_slices(items, [&](int o, int nw) {
+    const int4* w = (TRAIL ? p->dtrwork : p->dwmulti) + o;
+    const dim3 g((nw + 7) / 8 * 8);
+    if (p->kind == SDT_EM2 && !TRAIL && sizeof(T) == 4 && items > 512)  // (see EmRegionLds)
+      hipLaunchKernelGGL((k_em2_multi<float, false, 2>), g, dim3(RM * RM / 2), 0, st, p->dmodels, p->dshots, w, nw,
+                         p->dbase, r, k, tm, par, p->dadj, p->dtsel_trail);
+    else if (p->kind == SDT_EM2)
+      hipLaunchKernelGGL((k_em2_multi<T, TRAIL, 1>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k, tm,
+                         par, p->dadj, p->dtsel_trail);
+    else if (p->split)
+      hipLaunchKernelGGL((k_el2_multi<T, true, TRAIL>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k,
+                         tm, par, p->dadj, p->dtsel_trail);
+    else
+      hipLaunchKernelGGL((k_el2_multi<T, false, TRAIL>), g, b, 0, st, p->dmodels, p->dshots, w, nw, p->dbase, r, k,
+                         tm, par, p->dadj, p->dtsel_trail);
+  });
 }
 
 // Steps of one run or graph block on regions, in launches of nearly equal
@@ -5102,9 +5116,10 @@ void launch_adjoint_steps(Plan* p, hipStream_t st, int khi, int klo) {
   const int* tb = p->dtbase;
   for (int k = khi - 1; k >= klo; --k) {
     if (!(p->adj_flags & SDT_ADJ_REFERENCE)) {
-      hipLaunchKernelGGL((k_el2_adj<T, SPLIT>), dim3((p->nadjwork + 7) / 8 * 8), dim3(64 * AR<T, false>), 0, st,
-                         p->dmodels, p->dshots, p->dadj, p->dadjwork, p->nadjwork, tb, k, p->gmask,
-                         p->dtsel_adj);
+      in_slices(p->nadjwork, [&](int o, int n) {
+        hipLaunchKernelGGL((k_el2_adj<T, SPLIT>), dim3((n + 7) / 8 * 8), dim3(64 * AR<T, false>), 0, st, p->dmodels,
+                           p->dshots, p->dadj, p->dadjwork + o, n, tb, k, p->gmask, p->dtsel_adj);
+      });
       continue;
     }
     if (p->maxrec > 0)
@@ -5132,8 +5147,10 @@ void launch_adjoint_em2(Plan* p, hipStream_t st, int khi, int klo) {
   const int* tb = p->dtbase;
   for (int k = khi - 1; k >= klo; --k) {
     if (!(p->adj_flags & SDT_ADJ_REFERENCE)) {
-      hipLaunchKernelGGL(k_em2_adj<T>, dim3((p->nadjwork + 7) / 8 * 8), dim3(64 * AR<T, true>), 0, st, p->dmodels,
-                         p->dshots, p->dadj, p->dadjwork, p->nadjwork, tb, k, p->gmask, p->dtsel_adj);
+      in_slices(p->nadjwork, [&](int o, int n) {
+        hipLaunchKernelGGL(k_em2_adj<T>, dim3((n + 7) / 8 * 8), dim3(64 * AR<T, true>), 0, st, p->dmodels, p->dshots,
+                           p->dadj, p->dadjwork + o, n, tb, k, p->gmask, p->dtsel_adj);
+      });
       continue;
     }
     if (p->maxrec > 0)

@@ -197,3 +197,52 @@ def test_em_regions_of_two_rows_on_thin_grids(nx, nz, nshots):
         _same(a, b)
     a.close()
     b.close()
+
+
+def _copies(kind, seed, nt, n):
+    """n equal shots on one model: more items than one launch takes (262,144)."""
+    p = _problem(kind, seed, nt, nx=600, nz=500, npml=6)
+    return p, p.with_shots(list(p.shots) * n)
+
+
+@pytest.mark.parametrize("kind", ["elastic2", "em2"])
+def test_regions_in_several_launches(kind):
+    """A list of more regions than one launch takes: every shot equals the
+    shot alone, bit for bit."""
+    from seidart_amd.solver import Simulation
+    one, many = _copies(kind, 580, 12, 510)
+    a, b = Simulation(one, precision="fp32"), Simulation(many, precision="fp32")
+    assert b.region_info()[2] > 1 << 18 and b.run_mode(12, 10) == 2
+    a.run()
+    b.run(graph_block=10).check()
+    torch.cuda.synchronize()
+    ref = a.shots[0][2]
+    assert float(ref["trace"].abs().max()) > 0
+    for _, _, x in b.shots:
+        assert torch.equal(x["state"], ref["state"]) and torch.equal(x["trace"], ref["trace"])
+    a.close()
+    b.close()
+
+
+def test_recomputation_and_adjoint_in_several_launches():
+    """The same of the trail recomputation and the adjoint: lambda_0 of every
+    shot equals that of the shot alone, and the gradient is their sum."""
+    from seidart_amd.adjoint import AdjointEngine
+    one, many = _copies("em2", 590, 10, 520)
+    lam, grad = [], []
+    for p in (one, many):
+        e = AdjointEngine(p, precision="fp32", every=5)
+        tr = e.forward()
+        g, _ = e.backward([t + 1.0 for t in tr])
+        grad.append(g[0].cpu())
+        lam.append([e.adjoint_state(s) for s in range(len(p.shots))])
+        keep = lam[0][0].clone()
+        if p is many:
+            for s, x in enumerate(lam[1]):
+                assert torch.equal(x, ref), s
+        ref = keep
+        e.close()
+    assert float(ref.abs().max()) > 0
+    n, scale = len(many.shots), grad[0].abs().amax(dim=(1, 2), keepdim=True)
+    # FP32 atomics: n values of one size per step and cell, 10 steps, in any order
+    assert float(((grad[1] - n * grad[0]).abs() / (n * scale)).max()) < 10 * n * 2.0 ** -24
