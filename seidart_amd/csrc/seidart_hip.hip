@@ -5264,11 +5264,18 @@ struct Stage {
   std::vector<long> nel, npsi;
 };
 
+// bytes of the fixed scratch of sdt_run_noalloc
+#ifndef SDT_NOALLOC_SCRATCH_BYTES
+#define SDT_NOALLOC_SCRATCH_BYTES (8u << 20)
+#endif
+
 // Host half of plan creation: validate the inputs and fill the plan's
 // settings and everything of `S` except the receivers-by-row index.  Reads
-// no device memory.
+// no device memory.  once: for one run of that many steps in the fixed scratch
+// (0: any runs); least_rows > 0: with shorter lists, without regions and with
+// tiles or chunks of at least that many rows.
 int stage_host(Plan* p, int kind, int prec, const sdt_model* models, int nmodels,
-               const sdt_shot* shots, int nshots, int nt, Stage& S, int least_rows = 0) {
+               const sdt_shot* shots, int nshots, int nt, Stage& S, int once = 0, int least_rows = 0) {
   const bool split = (kind & SDT_SPLIT_CPML) != 0;
   kind &= ~SDT_SPLIT_CPML;
   if (split && kind != SDT_ELASTIC2) return fail(SDT_EINVAL, "SDT_SPLIT_CPML applies to ELASTIC2 only");
@@ -5329,13 +5336,15 @@ int stage_host(Plan* p, int kind, int prec, const sdt_model* models, int nmodels
   }
   if (pingpong(kind)) {
     default_shape(p);
-    if (least_rows > p->el2_eh) {  // shorter lists for the fixed scratch
+    if (least_rows > 0) p->multi = false;
+    if (least_rows > p->el2_eh) {
       p->el2_eh = least_rows;
       p->el2_wb = 4;
-      p->multi = false;
     }
+    p->nmulti = (int)regions2d(p, p->tm);
+    if (once > 0 && (run_mode(p, once, 0) != 2 || sizeof(int4) * p->nmulti > SDT_NOALLOC_SCRATCH_BYTES))
+      p->multi = false;
     if (p->multi) S.workm = multi_work(p, p->tm);
-    p->nmulti = (int)S.workm.size();
     S.work = el2_work(p, p->el2_wb, p->el2_eh, p->el2_order);
     const int nblk = (int)S.work.size();
     p->el2_grid = std::max(8, std::min(nblk, SDT_EL2_GRID) / 8 * 8);
@@ -5414,9 +5423,6 @@ void stage_bind(const Plan* p, Stage& S) {
 // itself to the device: it uses the address hipGetSymbolAddress returns for
 // the current device (scratch_ptr).
 // ---------------------------------------------------------------------------
-#ifndef SDT_NOALLOC_SCRATCH_BYTES
-#define SDT_NOALLOC_SCRATCH_BYTES (8u << 20)
-#endif
 __device__ __align__(256) unsigned char scratch[SDT_NOALLOC_SCRATCH_BYTES];
 
 constexpr int kMaxDevices = 64;
@@ -5678,14 +5684,15 @@ int sdt_run_noalloc(int kind, int prec, const sdt_model* models, int nmodels,
   Plan P;
   Plan* p = &P;
   Stage S;
-  int rc = stage_host(p, kind, prec, models, nmodels, shots, nshots, nt, S);
+  int rc = stage_host(p, kind, prec, models, nmodels, shots, nshots, nt, S, nsteps);
   if (rc) return rc;
   ScratchLayout L = scratch_layout(p, S);
-  // work lists too long for the scratch: taller tiles, as far as that helps
-  for (int rows = 4; L.total > (size_t)SDT_NOALLOC_SCRATCH_BYTES && rows <= 65536; rows *= 2) {
+  // work lists too long for the scratch: no regions, then taller tiles, as far as
+  // that helps
+  for (int rows = kind_3d(p->kind) ? 8 : 1; L.total > (size_t)SDT_NOALLOC_SCRATCH_BYTES && rows <= 65536; rows *= 2) {
     P = Plan();
     S = Stage();
-    rc = stage_host(p, kind, prec, models, nmodels, shots, nshots, nt, S, rows);
+    rc = stage_host(p, kind, prec, models, nmodels, shots, nshots, nt, S, nsteps, rows);
     if (rc) return rc;
     L = scratch_layout(p, S);
   }
