@@ -4542,7 +4542,7 @@ int region_launches(int n, int tm, bool even) {
 // Items per launch of the kernels that take one item per block: a launch holds
 // fewer than 2^32 threads, which 4.2 M blocks of 1024 reach (2 G cells per step
 // on regions), so longer lists go in several launches.  At this length (0.13 G
-// cells, 3 ms per elastic launch of five steps) a further launch costs nothing
+// cells, 4 ms per elastic FP32 launch of five steps) a further launch costs nothing
 // against the work.
 constexpr int LAUNCH_ITEMS = 1 << 18;
 template <typename F>
