@@ -2337,7 +2337,7 @@ __global__ void k_em2_edges(const DModel* __restrict__ models, const DShot* __re
 // edges, and a wavefront clear of every slab runs a body without memory
 // variables.  z neighbours are plain loads of the adjacent planes.
 // What bounds it: on large grids the bytes (the second pass re-reads what the
-// first wrote; 832x96x432 FP32 moves 5.0 GB per step at 4.3 TB/s, a copy
+// first wrote; 832x96x432 FP32 moves 5.8 GB per step at 5.2 TB/s, a copy
 // reaches 4.9 .. 5.3), on small ones the latency of a row's loads.  So the loads
 // of a row group, C-PML memory included, are all issued before the first use,
 // and the stress pass reads the 33 y-invariant coefficients of its column from
